@@ -7,6 +7,7 @@ overlap) into one library next to this file.  Called by
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -40,8 +41,7 @@ DEVICE = [
 def build(verbose=True):
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
-    objs = []
-    for src in SOURCES:
+    def compile_one(src):
         path = os.path.join(CSRC, src)
         obj = os.path.join(objdir, src.replace("/", "_") + ".o")
         if src.endswith(".hip"):
@@ -51,7 +51,11 @@ def build(verbose=True):
         if verbose:
             print("[build]", " ".join(cmd), flush=True)
         subprocess.run(cmd, check=True, stderr=subprocess.PIPE if not verbose else None)
-        objs.append(obj)
+        return obj
+
+    # the unrolled Coulomb kernels alone take over a minute: compile the sources side by side
+    with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1)) as pool:
+        objs = list(pool.map(compile_one, SOURCES))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fopenmp", "-o", tmp] + objs
     if verbose:

@@ -24,369 +24,553 @@ namespace sxc {
 
 namespace {
 
-// packed index of (t, u, v), s = t + u + v: all s' < s first, then t descending, u descending
-__device__ inline int hidx(int t, int u, int v) {
-  const int s = t + u + v;
-  const int q = s - t;
-  return s * (s + 1) * (s + 2) / 6 + q * (q + 1) / 2 + (q - u);
+// Packed Hermite indices of order <= kJMaxL (all orders below s = t + u + v first, then t descending,
+// u descending) as tables: (t, u, v) of index i, and the recursion of
+// i >= 1 in its first non-zero direction dir: R_i = x_dir R_m1 + mul R_m2 (m2 = m1 where mul = 0).
+// Read with constant indices in unrolled loops only, so that the arrays they index stay in registers.
+struct HermiteTable {
+  int t[kJMaxH], u[kJMaxH], v[kJMaxH], dir[kJMaxH], m1[kJMaxH], m2[kJMaxH], mul[kJMaxH];
+};
+constexpr int hidx_c(int t, int u, int v) {
+  return (t + u + v) * (t + u + v + 1) * (t + u + v + 2) / 6 + (u + v) * (u + v + 1) / 2 + v;
 }
-__device__ inline int hcount(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
+constexpr int hcount_c(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
+constexpr HermiteTable make_hermite_table() {
+  HermiteTable h{};
+  int i = 0;
+  for (int s = 0; s <= kJMaxL; ++s)
+    for (int t = s; t >= 0; --t)
+      for (int u = s - t; u >= 0; --u, ++i) {
+        const int v = s - t - u;
+        h.t[i] = t;
+        h.u[i] = u;
+        h.v[i] = v;
+        const int d = t > 0 ? 0 : u > 0 ? 1 : 2, e = d == 0 ? t : d == 1 ? u : v;
+        h.dir[i] = d;
+        h.mul[i] = e > 1 ? e - 1 : 0;
+        h.m1[i] = i == 0 ? 0 : hidx_c(t - (d == 0), u - (d == 1), v - (d == 2));
+        h.m2[i] = e > 1 ? hidx_c(t - 2 * (d == 0), u - 2 * (d == 1), v - 2 * (d == 2)) : h.m1[i];
+      }
+  return h;
+}
+__device__ constexpr HermiteTable kHerm = make_hermite_table();
 
-// Boys function F_0..F_m (m <= kJMaxL): series with downward recursion below T = 35,
-// asymptotic form with upward recursion above.
-__device__ void boys(int m, double T, double* F) {
-  const double e = exp(-T);
-  if (T < 35.0) {
-    double term = 1.0 / (2 * m + 1), sum = term;
-    for (int k = 1; k < 200; ++k) {
-      term *= 2.0 * T / (2 * m + 2 * k + 1);
-      sum += term;
-      if (term < 1e-17 * sum) break;
+// Boys functions F_0..F_M at T.  Below kBoysEnd: F_M by its Taylor expansion about the nearest node
+// of a table (dF_m/dT = -F_(m+1); |T - T_i| <= 0.05, nine terms: truncation below 1e-17 F_M) and
+// downward recursion, with e^-T from the same node.  Above: F_0 = sqrt(pi / T) / 2 (its
+// complement is below 1e-16 there) and upward recursion.
+template <int M>
+__device__ __forceinline__ void boys_table(double T, const double* __restrict__ tab, double (&F)[M + 1]) {
+  if (T < kBoysEnd) {
+    const int i = (int)(T * kBoysPerUnit + 0.5);
+    const double d = i * (1.0 / kBoysPerUnit) - T;
+    const gmem<const double>* row = to_global(tab) + i * kBoysCols;
+    double f = row[1 + M + 8], e = 1.0;
+#pragma unroll
+    for (int k = 8; k >= 1; --k) {
+      f = row[M + k] + f * (d * (1.0 / k));
+      e = 1.0 + e * (d * (1.0 / k));
     }
-    F[m] = e * sum;
-    for (int j = m; j > 0; --j) F[j - 1] = (2.0 * T * F[j] + e) / (2 * j - 1);
+    e *= row[0];
+    F[M] = f;
+#pragma unroll
+    for (int j = M; j > 0; --j) F[j - 1] = (2.0 * T * F[j] + e) * (1.0 / (2 * j - 1));
   } else {
-    F[0] = 0.5 * sqrt(M_PI / T);
-    for (int j = 0; j < m; ++j) F[j + 1] = ((2 * j + 1) * F[j] - e) / (2.0 * T);
+    const double r = rsqrt(T), o2t = 0.5 * r * r;
+    const double e = T < 100.0 ? exp(-T) : 0.0;  // beyond: below 1e-26 of every F_m kept
+    F[0] = 0.88622692545275801365 * r;           // sqrt(pi) / 2
+#pragma unroll
+    for (int j = 0; j < M; ++j) F[j + 1] = ((2 * j + 1) * F[j] - e) * o2t;
   }
 }
 
-// R^(0)_tuv(a, X, Y, Z) for t + u + v <= L, packed (hidx); buf: 2 hcount(kJMaxL) doubles.
-__device__ void hermite_R(int L, double a, double X, double Y, double Z, double* R, double* buf) {
-  double F[kJMaxL + 1];
-  boys(L, a * (X * X + Y * Y + Z * Z), F);
-  double* cur = buf;
-  double* nxt = buf + hcount(kJMaxL);
-  double pw = 1.0;
-  for (int n = 0; n < L; ++n) pw *= -2.0 * a;
-  // nxt holds level n + 1, cur is built for level n (entries with s <= L - n)
-  for (int n = L; n >= 0; --n) {
-    cur[0] = pw * F[n];
-    const int top = L - n;
-    for (int s = 1; s <= top; ++s)
-      for (int t = s; t >= 0; --t)
-        for (int u = s - t; u >= 0; --u) {
-          const int v = s - t - u;
-          double val;
-          if (t > 0) {
-            val = X * nxt[hidx(t - 1, u, v)];
-            if (t > 1) val += (t - 1) * nxt[hidx(t - 2, u, v)];
-          } else if (u > 0) {
-            val = Y * nxt[hidx(t, u - 1, v)];
-            if (u > 1) val += (u - 1) * nxt[hidx(t, u - 2, v)];
-          } else {
-            val = Z * nxt[hidx(t, u, v - 1)];
-            if (v > 1) val += (v - 1) * nxt[hidx(t, u, v - 2)];
-          }
-          cur[hidx(t, u, v)] = val;
-        }
-    double* tmp = cur;
-    cur = nxt;
-    nxt = tmp;
-    if (n > 0) pw /= -2.0 * a;
+// One level n of the Hermite Coulomb recursion, in place: entries of order <= M - n from those of
+// level n + 1 (descending, so an entry's sources of lower order are still of that level).
+template <int M, int N>
+__device__ __forceinline__ void r_level(const double (&x)[3], const double (&F)[M + 1], double (&R)[hcount_c(M)]) {
+#pragma unroll
+  for (int i = hcount_c(M - N) - 1; i >= 1; --i) {
+    double val = x[kHerm.dir[i]] * R[kHerm.m1[i]];
+    if (kHerm.mul[i] > 0) val += (double)kHerm.mul[i] * R[kHerm.m2[i]];
+    R[i] = val;
   }
-  const int cnt = hcount(L);
-  for (int i = 0; i < cnt; ++i) R[i] = nxt[i];
+  R[0] = F[N];
+  if constexpr (N > 0) r_level<M, N - 1>(x, F, R);
 }
 
-// Hermite expansion E[i][j][t] (i <= la, j <= lb, t <= i + j) of one direction,
-// stored at E[(i * (lb + 1) + j) * (la + lb + 1) + t].
-__device__ void hermite_E(int la, int lb, double p, double XPA, double XPB, double* E) {
-  const int nt = la + lb + 1;
+// scale R_tuv(alpha, x) for t + u + v <= M, packed, in registers.
+template <int M>
+__device__ __forceinline__ void r_tensor(double alpha, double scale, const double (&x)[3],
+                                         const double* __restrict__ tab, double (&R)[hcount_c(M)]) {
+  double F[M + 1];
+  boys_table<M>(alpha * (x[0] * x[0] + x[1] * x[1] + x[2] * x[2]), tab, F);
+  double pw = scale;
+#pragma unroll
+  for (int n = 0; n <= M; ++n) {
+    F[n] *= pw;
+    pw *= -2.0 * alpha;
+  }
+  r_level<M, M>(x, F, R);
+}
+
+// Hermite expansion E[i][j][t] (i <= LA, j <= LB, t <= i + j) of one direction.
+template <int LA, int LB>
+__device__ __forceinline__ void hermite_E(double p, double XPA, double XPB,
+                                          double (&E)[LA + 1][LB + 1][LA + LB + 1]) {
   const double o2p = 0.5 / p;
-  for (int k = 0; k < (la + 1) * (lb + 1) * nt; ++k) E[k] = 0.0;
-  auto at = [&](int i, int j, int t) -> double& { return E[(i * (lb + 1) + j) * nt + t]; };
-  at(0, 0, 0) = 1.0;
-  for (int i = 0; i <= la; ++i)
-    for (int j = 0; j <= lb; ++j) {
-      if (i == 0 && j == 0) continue;
-      for (int t = 0; t <= i + j; ++t) {
-        double v;
-        if (i > 0) {
-          v = XPA * at(i - 1, j, t);
-          if (t > 0) v += o2p * at(i - 1, j, t - 1);
-          if (t + 1 <= i - 1 + j) v += (t + 1) * at(i - 1, j, t + 1);
-        } else {
-          v = XPB * at(i, j - 1, t);
-          if (t > 0) v += o2p * at(i, j - 1, t - 1);
-          if (t + 1 <= i + j - 1) v += (t + 1) * at(i, j - 1, t + 1);
+#pragma unroll
+  for (int i = 0; i <= LA; ++i)
+#pragma unroll
+    for (int j = 0; j <= LB; ++j)
+#pragma unroll
+      for (int t = 0; t <= LA + LB; ++t) {
+        double v = 0.0;
+        if (i + j == 0) {
+          v = t == 0 ? 1.0 : 0.0;
+        } else if (t <= i + j) {
+          const double* old = i > 0 ? E[i > 0 ? i - 1 : 0][j] : E[i][j > 0 ? j - 1 : 0];
+          v = (i > 0 ? XPA : XPB) * old[t];
+          if (t > 0) v += o2p * old[t - 1];
+          if (t + 1 <= i + j - 1) v += (t + 1) * old[t + 1];
         }
-        at(i, j, t) = v;
+        E[i][j][t] = v;
       }
-    }
 }
 
-// Cartesian exponents of component c of a shell of angular momentum l (a = l..0, b = l-a..0)
-__device__ inline void cart_of(int l, int c, int& ax, int& ay, int& az) {
-  int k = 0;
-  for (int a = l; a >= 0; --a)
-    for (int b = l - a; b >= 0; --b, ++k)
-      if (k == c) {
-        ax = a;
-        ay = b;
-        az = l - a - b;
-        return;
+// Cartesian exponents of every component up to the auxiliary shells, as tables for unrolled loops.
+struct CartTable {
+  int x[kJMaxLAux + 1][kJMaxNcartAux], y[kJMaxLAux + 1][kJMaxNcartAux], z[kJMaxLAux + 1][kJMaxNcartAux];
+};
+constexpr CartTable make_cart_table() {
+  CartTable c{};
+  for (int l = 0; l <= kJMaxLAux; ++l) {
+    int k = 0;
+    for (int a = l; a >= 0; --a)
+      for (int b = l - a; b >= 0; --b, ++k) {
+        c.x[l][k] = a;
+        c.y[l][k] = b;
+        c.z[l][k] = l - a - b;
       }
-  ax = ay = az = 0;
+  }
+  return c;
 }
+__device__ constexpr CartTable kCart = make_cart_table();
 
-// Hermite expansion of x^n exp(-a x^2) about its own centre, n <= l: Ea[n * (l + 1) + tau].
-__device__ void aux_E(int l, double a, double* Ea) {
-  const int w = l + 1;
-  for (int k = 0; k < w * w; ++k) Ea[k] = 0.0;
-  Ea[0] = 1.0;
-  const double o2a = 0.5 / a;
-  for (int n = 1; n <= l; ++n)
-    for (int t = 0; t <= n; ++t) {
-      double v = 0.0;
-      if (t > 0) v += o2a * Ea[(n - 1) * w + t - 1];
-      if (t + 1 <= n - 1) v += (t + 1) * Ea[(n - 1) * w + t + 1];
-      Ea[n * w + t] = v;
+// x^n exp(-a x^2) = sum_t c[n][t] (2a)^(-(n + t) / 2) Lambda_t about its own centre,
+// c[n][t] = n! / (t! m! 2^m) with 2 m = n - t (zero for odd n - t).
+struct AuxTable {
+  double c[kJMaxLAux + 1][kJMaxLAux + 1];
+};
+constexpr AuxTable make_aux_table() {
+  AuxTable a{};
+  a.c[0][0] = 1.0;
+  for (int n = 1; n <= kJMaxLAux; ++n)
+    for (int t = 0; t <= n; ++t)
+      a.c[n][t] = (t > 0 ? a.c[n - 1][t - 1] : 0.0) + (t + 1 <= n - 1 ? (t + 1) * a.c[n - 1][t + 1] : 0.0);
+  return a;
+}
+__device__ constexpr AuxTable kAux = make_aux_table();
+
+// Cartesian functions of a class's shells and Hermite functions of their pairs.  A wavefront's pairs
+// are of one class, so the angular transforms are the same for every lane (scalar loads).
+template <int LA, int LB>
+struct PairDims {
+  static constexpr int NA = (LA + 1) * (LA + 2) / 2, NB = (LB + 1) * (LB + 2) / 2, H = hcount_c(LA + LB);
+  typedef double ETab[LA + 1][LB + 1][LA + LB + 1];
+};
+
+// One Cartesian function I of A at a time (recursion instead of a loop, which for f shells would be
+// too long to unroll): the row's part of the Hermite density, or the row of J from the potential.
+template <int LA, int LB, int I>
+__device__ __forceinline__ void hermite_row_in(const typename PairDims<LA, LB>::ETab& Ex,
+                                               const typename PairDims<LA, LB>::ETab& Ey,
+                                               const typename PairDims<LA, LB>::ETab& Ez,
+                                               const double (&Pc)[PairDims<LA, LB>::NA][PairDims<LA, LB>::NB],
+                                               double (&out)[PairDims<LA, LB>::H]) {
+  using Dim = PairDims<LA, LB>;
+  constexpr int ax = kCart.x[LA][I], ay = kCart.y[LA][I], az = kCart.z[LA][I];
+#pragma unroll
+  for (int j = 0; j < Dim::NB; ++j) {
+    const int bx = kCart.x[LB][j], by = kCart.y[LB][j], bz = kCart.z[LB][j];
+#pragma unroll
+    for (int k = 0; k < Dim::H; ++k) {
+      const int t = kHerm.t[k], u = kHerm.u[k], v = kHerm.v[k];
+      if (t <= ax + bx && u <= ay + by && v <= az + bz)
+        out[k] += Pc[I][j] * (Ex[ax][bx][t] * (Ey[ay][by][u] * Ez[az][bz][v]));
     }
+  }
+  if constexpr (I + 1 < Dim::NA) hermite_row_in<LA, LB, I + 1>(Ex, Ey, Ez, Pc, out);
+}
+template <int LA, int LB, int I>
+__device__ __forceinline__ void hermite_row_out(const typename PairDims<LA, LB>::ETab& Ex,
+                                                const typename PairDims<LA, LB>::ETab& Ey,
+                                                const typename PairDims<LA, LB>::ETab& Ez,
+                                                const double (&in)[PairDims<LA, LB>::H],
+                                                double (&Jc)[PairDims<LA, LB>::NA][PairDims<LA, LB>::NB]) {
+  using Dim = PairDims<LA, LB>;
+  constexpr int ax = kCart.x[LA][I], ay = kCart.y[LA][I], az = kCart.z[LA][I];
+#pragma unroll
+  for (int j = 0; j < Dim::NB; ++j) {
+    const int bx = kCart.x[LB][j], by = kCart.y[LB][j], bz = kCart.z[LB][j];
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < Dim::H; ++k) {
+      const int t = kHerm.t[k], u = kHerm.u[k], v = kHerm.v[k];
+      if (t <= ax + bx && u <= ay + by && v <= az + bz) s += in[k] * (Ex[ax][bx][t] * (Ey[ay][by][u] * Ez[az][bz][v]));
+    }
+    Jc[I][j] = s;
+  }
+  if constexpr (I + 1 < Dim::NA) hermite_row_out<LA, LB, I + 1>(Ex, Ey, Ez, in, Jc);
 }
 
-// 1. Hermite density of each primitive pair
-__global__ __launch_bounds__(128) void jdens_kernel(const JPair* __restrict__ pairs, int npair,
-                                                    const DevShell* __restrict__ shells,
-                                                    const double* __restrict__ ang, const double* __restrict__ P,
-                                                    int n, double* __restrict__ D) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= npair) return;
-  const JPair pr = pairs[q];
-  const DevShell A = shells[pr.A], B = shells[pr.B];
-  const int la = A.l, lb = B.l, L = la + lb;
-  double Pc[kJMaxNcart * kJMaxNcart];
-  for (int i = 0; i < A.ncart; ++i)
-    for (int j = 0; j < B.ncart; ++j) {
+// 1. Hermite density of each primitive pair, over the pair's exponent (step 2 wants D / p)
+template <int LA, int LB>
+__device__ __forceinline__ void jdens_pair(const JPair& pr, const DevShell& A, const DevShell& B,
+                                           const double* __restrict__ angA, const double* __restrict__ angB,
+                                           const double* __restrict__ P, int n, double* __restrict__ D) {
+  using Dim = PairDims<LA, LB>;
+  double Pc[Dim::NA][Dim::NB];
+#pragma unroll
+  for (int i = 0; i < Dim::NA; ++i)
+#pragma unroll
+    for (int j = 0; j < Dim::NB; ++j) Pc[i][j] = 0.0;
+  const gmem<const double>* Pg = to_global(P) + A.ao_off + (int64_t)n * B.ao_off;
+  const int nfa = A.nfunc, nfb = B.nfunc;
+  for (int f = 0; f < nfa; ++f) {
+    double row[Dim::NB];
+#pragma unroll
+    for (int j = 0; j < Dim::NB; ++j) row[j] = 0.0;
+    for (int h = 0; h < nfb; ++h) {
+      const double v = Pg[f + (int64_t)n * h];
+#pragma unroll
+      for (int j = 0; j < Dim::NB; ++j) row[j] += v * angB[h * Dim::NB + j];
+    }
+#pragma unroll
+    for (int i = 0; i < Dim::NA; ++i)
+#pragma unroll
+      for (int j = 0; j < Dim::NB; ++j) Pc[i][j] += angA[f * Dim::NA + i] * row[j];
+  }
+  double Ex[LA + 1][LB + 1][LA + LB + 1], Ey[LA + 1][LB + 1][LA + LB + 1], Ez[LA + 1][LB + 1][LA + LB + 1];
+  hermite_E<LA, LB>(pr.p, pr.PA[0], pr.PB[0], Ex);
+  hermite_E<LA, LB>(pr.p, pr.PA[1], pr.PB[1], Ey);
+  hermite_E<LA, LB>(pr.p, pr.PA[2], pr.PB[2], Ez);
+  double out[Dim::H];
+#pragma unroll
+  for (int k = 0; k < Dim::H; ++k) out[k] = 0.0;
+  hermite_row_in<LA, LB, 0>(Ex, Ey, Ez, Pc, out);
+  const double scale = pr.sym * pr.K / pr.p;
+  gmem<double>* dst = to_global(D) + pr.herm_off;
+#pragma unroll
+  for (int k = 0; k < Dim::H; ++k) dst[k] = scale * out[k];
+}
+
+// 5. J block of each primitive pair from its Hermite potential, added to both triangles of J
+template <int LA, int LB>
+__device__ __forceinline__ void jassemble_pair(const JPair& pr, const DevShell& A, const DevShell& B,
+                                               const double* __restrict__ angA, const double* __restrict__ angB,
+                                               const gmem<const double>* __restrict__ V, int64_t stride, int n,
+                                               double* __restrict__ J) {
+  using Dim = PairDims<LA, LB>;
+  double Ex[LA + 1][LB + 1][LA + LB + 1], Ey[LA + 1][LB + 1][LA + LB + 1], Ez[LA + 1][LB + 1][LA + LB + 1];
+  hermite_E<LA, LB>(pr.p, pr.PA[0], pr.PB[0], Ex);
+  hermite_E<LA, LB>(pr.p, pr.PA[1], pr.PB[1], Ey);
+  hermite_E<LA, LB>(pr.p, pr.PA[2], pr.PB[2], Ez);
+  double in[Dim::H];
+#pragma unroll
+  for (int k = 0; k < Dim::H; ++k) in[k] = pr.K * V[k * stride];
+  double Jc[Dim::NA][Dim::NB];
+  hermite_row_out<LA, LB, 0>(Ex, Ey, Ez, in, Jc);
+  const int nfa = A.nfunc, nfb = B.nfunc;
+  const bool off = pr.A != pr.B;
+  for (int f = 0; f < nfa; ++f) {
+    double row[Dim::NB];
+#pragma unroll
+    for (int j = 0; j < Dim::NB; ++j) {
+      row[j] = 0.0;
+#pragma unroll
+      for (int i = 0; i < Dim::NA; ++i) row[j] += angA[f * Dim::NA + i] * Jc[i][j];
+    }
+    for (int h = 0; h < nfb; ++h) {
       double s = 0.0;
-      for (int f = 0; f < A.nfunc; ++f) {
-        const double ma = ang[A.ang_off + f * A.ncart + i];
-        if (ma == 0.0) continue;
-        for (int h = 0; h < B.nfunc; ++h)
-          s += ma * P[(A.ao_off + f) + (int64_t)n * (B.ao_off + h)] * ang[B.ang_off + h * B.ncart + j];
-      }
-      Pc[i * B.ncart + j] = pr.sym * s;
-    }
-  double Ex[kJMaxE], Ey[kJMaxE], Ez[kJMaxE];
-  hermite_E(la, lb, pr.p, pr.PA[0], pr.PB[0], Ex);
-  hermite_E(la, lb, pr.p, pr.PA[1], pr.PB[1], Ey);
-  hermite_E(la, lb, pr.p, pr.PA[2], pr.PB[2], Ez);
-  const int nt = L + 1;
-  double* out = D + pr.herm_off;
-  for (int k = 0; k < hcount(L); ++k) out[k] = 0.0;
-  for (int i = 0; i < A.ncart; ++i) {
-    int ax, ay, az;
-    cart_of(la, i, ax, ay, az);
-    for (int j = 0; j < B.ncart; ++j) {
-      int bx, by, bz;
-      cart_of(lb, j, bx, by, bz);
-      const double pc = pr.K * Pc[i * B.ncart + j];
-      if (pc == 0.0) continue;
-      const double* ex = Ex + (ax * (lb + 1) + bx) * nt;
-      const double* ey = Ey + (ay * (lb + 1) + by) * nt;
-      const double* ez = Ez + (az * (lb + 1) + bz) * nt;
-      for (int t = 0; t <= ax + bx; ++t)
-        for (int u = 0; u <= ay + by; ++u)
-          for (int v = 0; v <= az + bz; ++v) out[hidx(t, u, v)] += pc * ex[t] * ey[u] * ez[v];
-    }
-  }
-}
-
-// 2. fitting right-hand side: one workgroup per (auxiliary shell, chunk of pairs)
-__global__ __launch_bounds__(256) void jrhs_kernel(const JPair* __restrict__ pairs, int npair, int chunk,
-                                                   const double* __restrict__ D,
-                                                   const DevShell* __restrict__ aux,
-                                                   const double* __restrict__ aux_alpha,
-                                                   const double* __restrict__ aux_coef,
-                                                   const int* __restrict__ aux_cart_off, double* __restrict__ bc) {
-  __shared__ double red[kJMaxNcartAux][256];
-  const int s = blockIdx.x;
-  const DevShell S = aux[s];
-  const int ls = S.l, ncs = S.ncart;
-  double acc[kJMaxNcartAux];
-  for (int k = 0; k < ncs; ++k) acc[k] = 0.0;
-  double R[kJMaxH], buf[2 * kJMaxH], W[kJMaxHs], Ea[(kJMaxLAux + 1) * (kJMaxLAux + 1)];
-  const int q0 = blockIdx.y * chunk, q1 = min(npair, q0 + chunk);
-  for (int q = q0 + threadIdx.x; q < q1; q += 256) {
-    const JPair pr = pairs[q];
-    const int Lab = pr.L, L = Lab + ls;
-    const double* Dq = D + pr.herm_off;
-    for (int k = 0; k < S.nprim; ++k) {
-      const double a = aux_alpha[S.prim_off + k];
-      const double alpha = pr.p * a / (pr.p + a);
-      const double pref = 2.0 * pow(M_PI, 2.5) / (pr.p * a * sqrt(pr.p + a)) * aux_coef[S.prim_off + k];
-      hermite_R(L, alpha, pr.P[0] - S.cx, pr.P[1] - S.cy, pr.P[2] - S.cz, R, buf);
-      // W[tau nu phi] = (-1)^(tau+nu+phi) sum_tuv D_tuv R_(t+tau, u+nu, v+phi)
-      for (int sh = 0; sh <= ls; ++sh)
-        for (int tt = sh; tt >= 0; --tt)
-          for (int uu = sh - tt; uu >= 0; --uu) {
-            const int vv = sh - tt - uu;
-            double w = 0.0;
-            for (int sab = 0; sab <= Lab; ++sab)
-              for (int t = sab; t >= 0; --t)
-                for (int u = sab - t; u >= 0; --u) {
-                  const int v = sab - t - u;
-                  w += Dq[hidx(t, u, v)] * R[hidx(t + tt, u + uu, v + vv)];
-                }
-            W[hidx(tt, uu, vv)] = (sh & 1) ? -w : w;
-          }
-      aux_E(ls, a, Ea);
-      for (int c = 0; c < ncs; ++c) {
-        int ax, ay, az;
-        cart_of(ls, c, ax, ay, az);
-        double val = 0.0;
-        for (int tt = 0; tt <= ax; ++tt)
-          for (int uu = 0; uu <= ay; ++uu)
-            for (int vv = 0; vv <= az; ++vv)
-              val += Ea[ax * (ls + 1) + tt] * Ea[ay * (ls + 1) + uu] * Ea[az * (ls + 1) + vv] * W[hidx(tt, uu, vv)];
-        acc[c] += pref * val;
-      }
-    }
-  }
-  for (int c = 0; c < ncs; ++c) red[c][threadIdx.x] = acc[c];
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w)
-      for (int c = 0; c < ncs; ++c) red[c][threadIdx.x] += red[c][threadIdx.x + w];
-    __syncthreads();
-  }
-  if ((int)threadIdx.x < ncs) atomicAdd(&bc[aux_cart_off[s] + threadIdx.x], red[threadIdx.x][0]);
-}
-
-// 3. Hermite potential of each primitive pair from the Cartesian fitting coefficients
-__global__ __launch_bounds__(128) void jpot_kernel(const JPair* __restrict__ pairs, int npair,
-                                                   const DevShell* __restrict__ aux, int naux_shell,
-                                                   const double* __restrict__ aux_alpha,
-                                                   const double* __restrict__ aux_coef,
-                                                   const int* __restrict__ aux_cart_off,
-                                                   const double* __restrict__ cc, double* __restrict__ V) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= npair) return;
-  const JPair pr = pairs[q];
-  const int Lab = pr.L;
-  double acc[kJMaxHab];
-  for (int i = 0; i < hcount(Lab); ++i) acc[i] = 0.0;
-  double R[kJMaxH], buf[2 * kJMaxH], U[kJMaxHs], Ea[(kJMaxLAux + 1) * (kJMaxLAux + 1)];
-  for (int s = 0; s < naux_shell; ++s) {
-    const DevShell S = aux[s];
-    const int ls = S.l;
-    const double* c = cc + aux_cart_off[s];
-    for (int k = 0; k < S.nprim; ++k) {
-      const double a = aux_alpha[S.prim_off + k];
-      aux_E(ls, a, Ea);
-      // U[tau nu phi] = (-1)^(tau+nu+phi) sum_c cc_c Ea Ea Ea
-      for (int i = 0; i < hcount(ls); ++i) U[i] = 0.0;
-      for (int ci = 0; ci < S.ncart; ++ci) {
-        int ax, ay, az;
-        cart_of(ls, ci, ax, ay, az);
-        const double cv = c[ci];
-        if (cv == 0.0) continue;
-        for (int tt = 0; tt <= ax; ++tt)
-          for (int uu = 0; uu <= ay; ++uu)
-            for (int vv = 0; vv <= az; ++vv)
-              U[hidx(tt, uu, vv)] +=
-                  cv * Ea[ax * (ls + 1) + tt] * Ea[ay * (ls + 1) + uu] * Ea[az * (ls + 1) + vv];
-      }
-      const double alpha = pr.p * a / (pr.p + a);
-      const double pref = 2.0 * pow(M_PI, 2.5) / (pr.p * a * sqrt(pr.p + a)) * aux_coef[S.prim_off + k];
-      hermite_R(Lab + ls, alpha, pr.P[0] - S.cx, pr.P[1] - S.cy, pr.P[2] - S.cz, R, buf);
-      for (int sab = 0; sab <= Lab; ++sab)
-        for (int t = sab; t >= 0; --t)
-          for (int u = sab - t; u >= 0; --u) {
-            const int v = sab - t - u;
-            double w = 0.0;
-            for (int sh = 0; sh <= ls; ++sh)
-              for (int tt = sh; tt >= 0; --tt)
-                for (int uu = sh - tt; uu >= 0; --uu) {
-                  const int vv = sh - tt - uu;
-                  const double r = R[hidx(t + tt, u + uu, v + vv)];
-                  w += (sh & 1) ? -U[hidx(tt, uu, vv)] * r : U[hidx(tt, uu, vv)] * r;
-                }
-            acc[hidx(t, u, v)] += pref * w;
-          }
-    }
-  }
-  double* out = V + pr.herm_off;
-  for (int i = 0; i < hcount(Lab); ++i) out[i] = acc[i];
-}
-
-// 5. J blocks of each primitive pair, angular transforms, symmetric scatter into J
-__global__ __launch_bounds__(128) void jassemble_kernel(const JPair* __restrict__ pairs, int npair,
-                                                        const DevShell* __restrict__ shells,
-                                                        const double* __restrict__ ang,
-                                                        const double* __restrict__ V, int n,
-                                                        double* __restrict__ J) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= npair) return;
-  const JPair pr = pairs[q];
-  const DevShell A = shells[pr.A], B = shells[pr.B];
-  const int la = A.l, lb = B.l, nt = la + lb + 1;
-  double Ex[kJMaxE], Ey[kJMaxE], Ez[kJMaxE];
-  hermite_E(la, lb, pr.p, pr.PA[0], pr.PB[0], Ex);
-  hermite_E(la, lb, pr.p, pr.PA[1], pr.PB[1], Ey);
-  hermite_E(la, lb, pr.p, pr.PA[2], pr.PB[2], Ez);
-  const double* Vq = V + pr.herm_off;
-  double Jc[kJMaxNcart * kJMaxNcart];
-  for (int i = 0; i < A.ncart; ++i) {
-    int ax, ay, az;
-    cart_of(la, i, ax, ay, az);
-    for (int j = 0; j < B.ncart; ++j) {
-      int bx, by, bz;
-      cart_of(lb, j, bx, by, bz);
-      const double* ex = Ex + (ax * (lb + 1) + bx) * nt;
-      const double* ey = Ey + (ay * (lb + 1) + by) * nt;
-      const double* ez = Ez + (az * (lb + 1) + bz) * nt;
-      double s = 0.0;
-      for (int t = 0; t <= ax + bx; ++t)
-        for (int u = 0; u <= ay + by; ++u)
-          for (int v = 0; v <= az + bz; ++v) s += ex[t] * ey[u] * ez[v] * Vq[hidx(t, u, v)];
-      Jc[i * B.ncart + j] = pr.K * s;
-    }
-  }
-  for (int f = 0; f < A.nfunc; ++f)
-    for (int h = 0; h < B.nfunc; ++h) {
-      double s = 0.0;
-      for (int i = 0; i < A.ncart; ++i) {
-        const double ma = ang[A.ang_off + f * A.ncart + i];
-        if (ma == 0.0) continue;
-        for (int j = 0; j < B.ncart; ++j) s += ma * Jc[i * B.ncart + j] * ang[B.ang_off + h * B.ncart + j];
-      }
+#pragma unroll
+      for (int j = 0; j < Dim::NB; ++j) s += row[j] * angB[h * Dim::NB + j];
       const int mu = A.ao_off + f, nu = B.ao_off + h;
       atomicAdd(&J[mu + (int64_t)n * nu], s);
-      if (pr.A != pr.B) atomicAdd(&J[nu + (int64_t)n * mu], s);
+      if (off) atomicAdd(&J[nu + (int64_t)n * mu], s);
     }
+  }
+}
+
+// One wavefront per item: up to 64 primitive pairs of one (l_A, l_B), shells of one kind each.
+// Straight-line code per class keeps the expansions in registers (with run-time angular momenta
+// they were 3.5 KB of private memory per lane: 1.04 and 0.86 ms at (H2O)32/def2-TZVP).
+template <bool Dens, int Lo, int Hi>
+__global__ __launch_bounds__(64) void jpair_kernel(const JPairItem* __restrict__ items, const JPair* __restrict__ pairs,
+                                                   const DevShell* __restrict__ shells,
+                                                   const double* __restrict__ ang, JView Jv,
+                                                   const double* __restrict__ in, int n, double* __restrict__ out) {
+  const JPairItem it = items[blockIdx.x];
+  const double* angA = ang + it.angA;
+  const double* angB = ang + it.angB;
+  const int q = it.q0 + threadIdx.x;
+  if ((int)threadIdx.x >= it.nq) return;
+  const JPair pr = pairs[q];
+  DevShell A = shells[pr.A], B = shells[pr.B];
+  A.nfunc = it.nfa;  // the class's own, the same for every lane
+  B.nfunc = it.nfb;
+#define SXC_P(LA_, LB_)                                                                                       \
+  if constexpr (LA_ + LB_ >= Lo && LA_ + LB_ <= Hi)                                                           \
+    if (it.la == LA_ && it.lb == LB_) {                                                                       \
+      if constexpr (Dens) {                                                                                   \
+        jdens_pair<LA_, LB_>(pr, A, B, angA, angB, in, n, out);                                               \
+      } else {                                                                                                \
+        constexpr int L_ = LA_ + LB_;                                                                         \
+        jassemble_pair<LA_, LB_>(pr, A, B, angA, angB, to_global(in) + Jv.herm0[L_] + (q - Jv.pair0[L_]),     \
+                                 Jv.pair0[L_ + 1] - Jv.pair0[L_], n, out);                                    \
+      }                                                                                                       \
+      return;                                                                                                 \
+    }
+#define SXC_PL(LA_) SXC_P(LA_, 0) SXC_P(LA_, 1) SXC_P(LA_, 2) SXC_P(LA_, 3)
+  static_assert(kJMaxLPrim == 3, "one case per (l_A, l_B)");
+  SXC_PL(0) SXC_PL(1) SXC_PL(2) SXC_PL(3)
+#undef SXC_PL
+#undef SXC_P
+}
+
+// Steps 2 and 4 meet every primitive pair with every auxiliary primitive.  Work items are one
+// wavefront each, of one (L, l) class (pair and auxiliary angular momentum), so that the recursion
+// and the contraction are straight-line code on registers: per meeting a Boys evaluation, about
+// 3 sum_(n <= L + l) hcount(n) operations of the recursion and 2 hcount(L) hcount(l) of the
+// contraction, all FP64 vector work.  What does not change in a lane's loop is read once, what is the
+// same for all lanes (the pair's density, the auxiliary's coefficients) comes through scalar loads,
+// and no lane meets another before an item's end.  The classes are bundled in three kernels by L + l
+// (<= 3, <= 6, above), because a kernel holds the registers of its widest class (128, 256, 512 and
+// spills: the last hold 0.4 % of the meetings).  At (H2O)32/def2-TZVP (160 297 pairs x 1280
+// auxiliary primitives) step 2 takes 1.5 ms and step 4 1.2 ms, about 20 TFLOP/s (FP64 vector peak
+// 78); with run-time angular momenta, whose arrays live in private memory, and one thread per pair
+// they took 50 and 263 ms.
+
+// acc[j] += sum over i >= I of c[i] R(index i + index j), i < NI, j < NJ (recursion over i: one loop
+// over both would be too long to unroll for the widest classes).
+template <int NI, int NJ, int I, typename Ptr, int NR>
+__device__ __forceinline__ void meet_contract(Ptr c, const double (&R)[NR], double (&acc)[NJ]) {
+  const double d = c[I];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+    acc[j] += d * R[hidx_c(kHerm.t[I] + kHerm.t[j], kHerm.u[I] + kHerm.u[j], kHerm.v[I] + kHerm.v[j])];
+  if constexpr (I + 1 < NI) meet_contract<NI, NJ, I + 1>(c, R, acc);
+}
+
+// 2. W_tau of the auxiliary primitives: lanes are auxiliary primitives (where a class has fewer than
+// 64, groups of lanes take different pairs), the loop runs over the item's pairs.
+template <int L, int l>
+__device__ __forceinline__ void jrhs_item(const JItem& it, const JView& J, const double* __restrict__ D,
+                                          double* __restrict__ W) {
+  constexpr int M = L + l, HL = hcount_c(L), Hl = hcount_c(l);
+  const int lane = threadIdx.x;
+  const int width = it.na;  // lanes per pair: a power of two for the grouped classes
+  const int g = l >= kJGroupL ? lane / width : 0;
+  const int step = l >= kJGroupL ? 64 / width : 1;
+  const int aw = l >= kJGroupL ? lane - g * width : lane;
+  const int a = min(it.a0 + aw, J.aux0[l + 1] - 1);
+  const bool live = it.a0 + aw < J.aux0[l + 1] && aw < width;
+  const gmem<const double>* A = to_global(J.aux) + 4 * (int64_t)a;
+  const double cx = A[0], cy = A[1], cz = A[2], ea = A[3];
+  double acc[Hl];
+#pragma unroll
+  for (int j = 0; j < Hl; ++j) acc[j] = 0.0;
+  const double* D0 = D + J.herm0[L];
+  const int q1 = it.q0 + it.nq;
+  for (int q = it.q0 + g; q < q1; q += step) {
+    const double* Q = J.pair + 4 * (int64_t)q;
+    const double p = Q[3];
+    const double* Dq = D0 + (int64_t)(q - J.pair0[L]) * HL;
+    const double r = rsqrt(p + ea);
+    const double x[3] = {Q[0] - cx, Q[1] - cy, Q[2] - cz};
+    double R[hcount_c(M)];
+    r_tensor<M>(p * ea * r * r, r, x, J.boys, R);
+    meet_contract<HL, Hl, 0>(Dq, R, acc);
+  }
+  if (!live) return;
+  const int nal = J.aux0[l + 1] - J.aux0[l];
+  double* out = W + J.aherm0[l] + (a - J.aux0[l]);
+#pragma unroll
+  for (int j = 0; j < Hl; ++j) atomicAdd(out + (int64_t)j * nal, acc[j]);
+}
+
+// 4. Hermite potential of the pairs: lanes are pairs, the loop runs over the item's auxiliary
+// primitives, whose Hermite coefficients U are the same for every lane.
+template <int L, int l>
+__device__ __forceinline__ void jpot_item(const JItem& it, const JView& J, const double* __restrict__ U,
+                                          double* __restrict__ V) {
+  constexpr int M = L + l, HL = hcount_c(L), Hl = hcount_c(l);
+  const int lane = threadIdx.x;
+  const int q = it.q0 + min(lane, it.nq - 1);
+  const gmem<const double>* Q = to_global(J.pair) + 4 * (int64_t)q;
+  const double px = Q[0], py = Q[1], pz = Q[2], p = Q[3];
+  double acc[HL];
+#pragma unroll
+  for (int i = 0; i < HL; ++i) acc[i] = 0.0;
+  for (int k = 0; k < it.na; ++k) {
+    const int a = it.a0 + k;
+    const double* A = J.aux + 4 * (int64_t)a;
+    const double* Ua = U + J.aherm0[l] + (int64_t)(a - J.aux0[l]) * Hl;
+    const double ea = A[3], r = rsqrt(p + ea);
+    const double x[3] = {px - A[0], py - A[1], pz - A[2]};
+    double R[hcount_c(M)];
+    r_tensor<M>(p * ea * r * r, r, x, J.boys, R);
+    meet_contract<Hl, HL, 0>(Ua, R, acc);
+  }
+  if (lane >= it.nq) return;
+  const double ip = 1.0 / p;
+  const int nql = J.pair0[L + 1] - J.pair0[L];
+  double* out = V + J.herm0[L] + (q - J.pair0[L]);
+#pragma unroll
+  for (int i = 0; i < HL; ++i) atomicAdd(out + (int64_t)i * nql, acc[i] * ip);
+}
+
+template <bool Rhs, int Lo, int Hi>
+__device__ __forceinline__ void jmeet(const JItem& it, const JView& J, const double* __restrict__ in,
+                                      double* __restrict__ out) {
+#define SXC_J(L_, l_)                                                              \
+  if constexpr (L_ + l_ >= Lo && L_ + l_ <= Hi)                                    \
+    if (it.L == L_ && it.l == l_) {                                                \
+      if constexpr (Rhs)                                                           \
+        jrhs_item<L_, l_>(it, J, in, out);                                         \
+      else                                                                         \
+        jpot_item<L_, l_>(it, J, in, out);                                         \
+      return;                                                                      \
+    }
+#define SXC_JL(L_) SXC_J(L_, 0) SXC_J(L_, 1) SXC_J(L_, 2) SXC_J(L_, 3) SXC_J(L_, 4)
+  static_assert(kJMaxLAux == 4 && kJMaxLPrim == 3, "one case per (L, l)");
+  SXC_JL(0) SXC_JL(1) SXC_JL(2) SXC_JL(3) SXC_JL(4) SXC_JL(5) SXC_JL(6)
+#undef SXC_JL
+#undef SXC_J
+}
+
+template <bool Rhs, int Lo, int Hi>
+__global__ __launch_bounds__(64) void jmeet_kernel(const JItem* __restrict__ items, JView J,
+                                                   const double* __restrict__ in, double* __restrict__ out) {
+  const JItem it = items[blockIdx.x];
+  jmeet<Rhs, Lo, Hi>(it, J, in, out);
+}
+
+// 2 pi^(5/2) / a coef (2a)^(-(l + s) / 2): what the Hermite coefficients of order s of an auxiliary
+// primitive share.
+__device__ inline double aux_scale(double a, double coef, int l, int s) {
+  double f = 34.986836655249725693 / a * coef;  // 2 pi^(5/2)
+  for (int k = 0; k < (l + s) / 2; ++k) f *= 0.5 / a;
+  return s & 1 ? -f : f;
+}
+
+// Auxiliary functions between their Cartesian coefficients and the primitives' Hermite ones, one
+// thread per primitive and Hermite index.
+// U[a][tau nu phi] = (-1)^(tau + nu + phi) 2 pi^(5/2) / a coef sum_c cc_c E E E (input of step 4)
+__global__ __launch_bounds__(256) void jaux_in_kernel(JView J, int naux, const int* __restrict__ prim_shell,
+                                                      const DevShell* __restrict__ aux,
+                                                      const double* __restrict__ prim_coef,
+                                                      const int* __restrict__ cart_off, const double* __restrict__ cc,
+                                                      double* __restrict__ U) {
+  const int id = blockIdx.x * 256 + threadIdx.x, a = id / kJMaxHs, i = id - a * kJMaxHs;
+  if (a >= naux) return;
+  const int sh = prim_shell[a], l = aux[sh].l, nc = aux[sh].ncart;
+  if (i >= hcount_c(l)) return;
+  const int t = kHerm.t[i], u = kHerm.u[i], v = kHerm.v[i], s = t + u + v;
+  double sum = 0.0;
+  if (((l - s) & 1) == 0)
+    for (int c = 0; c < nc; ++c) {
+      const int ax = kCart.x[l][c], ay = kCart.y[l][c], az = kCart.z[l][c];
+      if (t <= ax && u <= ay && v <= az)
+        sum += cc[cart_off[sh] + c] * (kAux.c[ax][t] * kAux.c[ay][u] * kAux.c[az][v]);
+    }
+  U[J.aherm0[l] + (int64_t)(a - J.aux0[l]) * hcount_c(l) + i] =
+      aux_scale(J.aux[4 * (int64_t)a + 3], prim_coef[a], l, s) * sum;
+}
+
+// bc[shell][c] = sum over the shell's primitives of the same coefficients times W (output of step 2),
+// one thread per Cartesian function
+__global__ __launch_bounds__(64) void jaux_out_kernel(JView J, const DevShell* __restrict__ aux, int nshell,
+                                                      const int* __restrict__ shell_prim,
+                                                      const double* __restrict__ prim_coef,
+                                                      const int* __restrict__ cart_off, const double* __restrict__ W,
+                                                      double* __restrict__ bc) {
+  const int sh = blockIdx.x * 4 + (threadIdx.x >> 4), c = threadIdx.x & 15;
+  if (sh >= nshell || c >= aux[sh].ncart) return;
+  const int l = aux[sh].l, nal = J.aux0[l + 1] - J.aux0[l];
+  const int ax = kCart.x[l][c], ay = kCart.y[l][c], az = kCart.z[l][c];
+  double sum = 0.0;
+  for (int k = 0; k < aux[sh].nprim; ++k) {
+    const int a = shell_prim[sh] + k;
+    const double ea = J.aux[4 * (int64_t)a + 3];
+    const double* Wa = W + J.aherm0[l] + (a - J.aux0[l]);
+    for (int i = 0; i < hcount_c(l); ++i) {
+      const int t = kHerm.t[i], u = kHerm.u[i], v = kHerm.v[i], s = t + u + v;
+      if (((l - s) & 1) == 0 && t <= ax && u <= ay && v <= az)
+        sum += aux_scale(ea, prim_coef[a], l, s) * (kAux.c[ax][t] * kAux.c[ay][u] * kAux.c[az][v]) *
+               Wa[(int64_t)i * nal];
+    }
+  }
+  bc[cart_off[sh] + c] = sum;
 }
 
 }  // namespace
 
-void launch_jdens(hipStream_t s, const JPair* pairs, int npair, const DevShell* shells, const double* ang,
-                  const double* P, int n, double* D) {
-  if (npair <= 0) return;
-  hipLaunchKernelGGL(jdens_kernel, dim3((npair + 127) / 128), dim3(128), 0, s, pairs, npair, shells, ang, P, n, D);
+template <bool Dens>
+static void launch_jpair(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs,
+                         const DevShell* shells, const double* ang, const JView& Jv, const double* in, int n,
+                         double* out) {
+  if (nitem <= 0) return;
+  if (cls == 0)
+    hipLaunchKernelGGL((jpair_kernel<Dens, 0, kJPairTop>), dim3(nitem), dim3(64), 0, s, items, pairs, shells, ang, Jv,
+                       in, n, out);
+  else
+    hipLaunchKernelGGL((jpair_kernel<Dens, kJPairTop + 1, 2 * kJMaxLPrim>), dim3(nitem), dim3(64), 0, s, items, pairs,
+                       shells, ang, Jv, in, n, out);
 }
 
-void launch_jrhs(hipStream_t s, const JPair* pairs, int npair, const double* D, const DevShell* aux, int naux_shell,
-                 const double* aux_alpha, const double* aux_coef, const int* aux_cart_off, double* bc) {
-  if (npair <= 0 || naux_shell <= 0) return;
-  const int chunk = 2048;
-  const int nchunk = (npair + chunk - 1) / chunk;
-  hipLaunchKernelGGL(jrhs_kernel, dim3(naux_shell, nchunk), dim3(256), 0, s, pairs, npair, chunk, D, aux, aux_alpha,
-                     aux_coef, aux_cart_off, bc);
+void launch_jdens(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs, const DevShell* shells,
+                  const double* ang, const JView& Jv, const double* P, int n, double* D) {
+  launch_jpair<true>(s, cls, items, nitem, pairs, shells, ang, Jv, P, n, D);
 }
 
-void launch_jpot(hipStream_t s, const JPair* pairs, int npair, const DevShell* aux, int naux_shell,
-                 const double* aux_alpha, const double* aux_coef, const int* aux_cart_off, const double* cc,
-                 double* V) {
-  if (npair <= 0) return;
-  hipLaunchKernelGGL(jpot_kernel, dim3((npair + 127) / 128), dim3(128), 0, s, pairs, npair, aux, naux_shell,
-                     aux_alpha, aux_coef, aux_cart_off, cc, V);
+void launch_jassemble(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs,
+                      const DevShell* shells, const double* ang, const JView& Jv, const double* V, int n, double* J) {
+  launch_jpair<false>(s, cls, items, nitem, pairs, shells, ang, Jv, V, n, J);
 }
 
-void launch_jassemble(hipStream_t s, const JPair* pairs, int npair, const DevShell* shells, const double* ang,
-                      const double* V, int n, double* J) {
-  if (npair <= 0) return;
-  hipLaunchKernelGGL(jassemble_kernel, dim3((npair + 127) / 128), dim3(128), 0, s, pairs, npair, shells, ang, V, n,
-                     J);
+template <bool Rhs>
+static void launch_jmeet(hipStream_t s, int cls, const JItem* items, int nitem, const JView& J, const double* in,
+                         double* out) {
+  if (nitem <= 0) return;
+  if (cls == 0)
+    hipLaunchKernelGGL((jmeet_kernel<Rhs, 0, kJClassTop[0]>), dim3(nitem), dim3(64), 0, s, items, J, in, out);
+  else if (cls == 1)
+    hipLaunchKernelGGL((jmeet_kernel<Rhs, kJClassTop[0] + 1, kJClassTop[1]>), dim3(nitem), dim3(64), 0, s, items, J,
+                       in, out);
+  else
+    hipLaunchKernelGGL((jmeet_kernel<Rhs, kJClassTop[1] + 1, kJMaxL>), dim3(nitem), dim3(64), 0, s, items, J, in, out);
+}
+
+void launch_jrhs(hipStream_t s, int cls, const JItem* items, int nitem, const JView& J, const double* D, double* W) {
+  launch_jmeet<true>(s, cls, items, nitem, J, D, W);
+}
+
+void launch_jpot(hipStream_t s, int cls, const JItem* items, int nitem, const JView& J, const double* U, double* V) {
+  launch_jmeet<false>(s, cls, items, nitem, J, U, V);
+}
+
+void launch_jaux_in(hipStream_t s, const JView& J, int naux, const int* prim_shell, const DevShell* aux,
+                    const double* prim_coef, const int* cart_off, const double* cc, double* U) {
+  if (naux <= 0) return;
+  hipLaunchKernelGGL(jaux_in_kernel, dim3((naux * kJMaxHs + 255) / 256), dim3(256), 0, s, J, naux, prim_shell, aux, prim_coef,
+                     cart_off, cc, U);
+}
+
+void launch_jaux_out(hipStream_t s, const JView& J, const DevShell* aux, int nshell, const int* shell_prim,
+                     const double* prim_coef, const int* cart_off, const double* W, double* bc) {
+  if (nshell <= 0) return;
+  hipLaunchKernelGGL(jaux_out_kernel, dim3((nshell + 3) / 4), dim3(64), 0, s, J, aux, nshell, shell_prim, prim_coef,
+                     cart_off, W, bc);
 }
 
 }  // namespace sxc

@@ -283,20 +283,49 @@ constexpr int kJMaxLPrim = 3;                      // orbital shells up to f
 constexpr int kJMaxLAux = 4;                       // auxiliary shells up to g
 constexpr int kJMaxL = 2 * kJMaxLPrim + kJMaxLAux;
 constexpr int kJMaxH = (kJMaxL + 1) * (kJMaxL + 2) * (kJMaxL + 3) / 6;
-constexpr int kJMaxHab = (2 * kJMaxLPrim + 1) * (2 * kJMaxLPrim + 2) * (2 * kJMaxLPrim + 3) / 6;
 constexpr int kJMaxHs = (kJMaxLAux + 1) * (kJMaxLAux + 2) * (kJMaxLAux + 3) / 6;
-constexpr int kJMaxNcart = (kJMaxLPrim + 1) * (kJMaxLPrim + 2) / 2;
 constexpr int kJMaxNcartAux = (kJMaxLAux + 1) * (kJMaxLAux + 2) / 2;
-constexpr int kJMaxE = (kJMaxLPrim + 1) * (kJMaxLPrim + 1) * (2 * kJMaxLPrim + 1);
-void launch_jdens(hipStream_t s, const JPair* pairs, int npair, const DevShell* shells, const double* ang,
-                  const double* P, int n, double* D);
-void launch_jrhs(hipStream_t s, const JPair* pairs, int npair, const double* D, const DevShell* aux, int naux_shell,
-                 const double* aux_alpha, const double* aux_coef, const int* aux_cart_off, double* bc);
-void launch_jpot(hipStream_t s, const JPair* pairs, int npair, const DevShell* aux, int naux_shell,
-                 const double* aux_alpha, const double* aux_coef, const int* aux_cart_off, const double* cc,
-                 double* V);
-void launch_jassemble(hipStream_t s, const JPair* pairs, int npair, const DevShell* shells, const double* ang,
-                      const double* V, int n, double* J);
+// Boys table: rows at T = 0, 0.1, .. kBoysEnd, each e^-T and F_0 .. F_(kJMaxL + 8).
+constexpr double kBoysEnd = 35.0;
+constexpr int kBoysPerUnit = 10;
+constexpr int kBoysRows = 351;
+constexpr int kBoysCols = 1 + kJMaxL + 9;
+// Kernels of the pair x auxiliary meetings: L + l up to kJClassTop[0], up to kJClassTop[1], above.
+constexpr int kJClasses = 3;
+constexpr int kJClassTop[2] = {3, 6};
+constexpr int kJGroupL = 3;  // auxiliary classes from this l on share a wavefront's lanes between pairs
+// One wavefront's meetings: pairs [q0, q0 + nq) of class L with auxiliary primitives of class l,
+// [a0, a0 + na) (step 4) or the na lanes from a0 (step 2).
+struct JItem {
+  int L, l, q0, nq, a0, na;
+};
+// Pairs are sorted by L (class L at [pair0[L], pair0[L + 1])), auxiliary primitives by l; herm0 and
+// aherm0 are the classes' offsets in the Hermite arrays (D and U: by pair or primitive, then Hermite
+// index; V and W: by Hermite index, then pair or primitive).
+struct JView {
+  const double* pair;  // x, y, z, exponent of every pair
+  const double* aux;   // x, y, z, exponent of every auxiliary primitive
+  const double* boys;
+  int pair0[2 * kJMaxLPrim + 2], aux0[kJMaxLAux + 2];
+  int herm0[2 * kJMaxLPrim + 1], aherm0[kJMaxLAux + 1];
+};
+// Steps 1 and 5: one wavefront's pairs [q0, q0 + nq), of one (l_A, l_B) and of shells with nfa and nfb
+// functions, whose angular transforms start at angA and angB; kernels of l_A + l_B <= kJPairTop and above.
+struct JPairItem {
+  int la, lb, q0, nq, nfa, nfb, angA, angB;
+};
+constexpr int kJPairClasses = 2;
+constexpr int kJPairTop = 3;
+void launch_jdens(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs, const DevShell* shells,
+                  const double* ang, const JView& Jv, const double* P, int n, double* D);
+void launch_jrhs(hipStream_t s, int cls, const JItem* items, int nitem, const JView& J, const double* D, double* W);
+void launch_jpot(hipStream_t s, int cls, const JItem* items, int nitem, const JView& J, const double* U, double* V);
+void launch_jaux_in(hipStream_t s, const JView& J, int naux, const int* prim_shell, const DevShell* aux,
+                    const double* prim_coef, const int* cart_off, const double* cc, double* U);
+void launch_jaux_out(hipStream_t s, const JView& J, const DevShell* aux, int nshell, const int* shell_prim,
+                     const double* prim_coef, const int* cart_off, const double* W, double* bc);
+void launch_jassemble(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs,
+                      const DevShell* shells, const double* ang, const JView& Jv, const double* V, int n, double* J);
 
 // Molecular-grid partition weights of ncand candidate points (kernels/grid_kernels.hip).
 void launch_partition(hipStream_t s, int type, unsigned smoothing, int natoms, const double* xyz, const double* dist,

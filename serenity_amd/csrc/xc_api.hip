@@ -347,10 +347,106 @@ struct xc_coulomb {
   int64_t herm_total = 0;
   int ncart_aux = 0;
   std::vector<int> cart_off;  // first Cartesian function of every auxiliary shell
+  int naux = 0;               // auxiliary primitives
+  int64_t aherm_total = 0;
+  JView view{};               // class offsets; its arrays are d_pair, d_aux and d_boys
   DBuf<JPair> d_pairs;
-  DBuf<int> d_cart_off;
-  DBuf<double> d_D, d_V, d_bc, d_cc, d_P, d_J;
+  DBuf<int> d_cart_off, d_prim_shell, d_shell_prim;
+  DBuf<double> d_pair, d_aux, d_prim_coef, d_boys;
+  // work items of [0: the right-hand side, 1: the potential]
+  std::vector<JItem> items[2][kJClasses];
+  DBuf<JItem> d_items[2][kJClasses];
+  std::vector<JPairItem> pair_items[kJPairClasses];
+  DBuf<JPairItem> d_pair_items[kJPairClasses];
+  DBuf<double> d_D, d_V, d_U, d_bc, d_cc, d_P, d_J;
+  void plan_items();
 };
+
+namespace {
+
+// Boys functions at the table's nodes: the confluent series in extended precision.
+std::vector<double> boys_table() {
+  std::vector<double> tab((size_t)kBoysRows * kBoysCols);
+  for (int i = 0; i < kBoysRows; ++i) {
+    const long double T = (long double)i / kBoysPerUnit, e = expl(-T);
+    tab[(size_t)i * kBoysCols] = (double)e;
+    for (int m = 0; m + 1 < kBoysCols; ++m) {
+      long double term = 1.0L / (2 * m + 1), sum = term;
+      for (int k = 1; term > 1e-22L * sum; ++k) {
+        term *= 2.0L * T / (2 * m + 2 * k + 1);
+        sum += term;
+      }
+      tab[(size_t)i * kBoysCols + 1 + m] = (double)(e * sum);
+    }
+  }
+  return tab;
+}
+
+}  // namespace
+
+// Items of the meetings, the largest L + l first.  An item is one wavefront.  Its length is set by
+// the operations of a meeting, so that the items take about the same time and there are about
+// kTarget of them (the chip holds 1024 to 4096 of these wavefronts at once), but at most 64
+// (potential) or 512 (right-hand side) meetings per lane, where the atomic additions at an item's
+// end no longer show, and at least 2.  With one length for all classes the few pairs of f and d
+// shells made a few long items: 32.6 of 51 ms of (H2O)32/def2-TZVP went to 0.4 % of the meetings.
+void xc_coulomb::plan_items() {
+  // steps 1 and 5: runs of at most 64 pairs of one kind of shells
+  const auto& sh = basis->shells;
+  const auto kind = [&](const JPair& q) {
+    return ((sh[q.A].l * 2 + sh[q.A].pure) * (kJMaxLPrim + 1) + sh[q.B].l) * 2 + sh[q.B].pure;
+  };
+  for (size_t q = 0; q < pairs.size();) {
+    size_t e = q + 1;
+    while (e < pairs.size() && e < q + 64 && kind(pairs[e]) == kind(pairs[q])) ++e;
+    const DevShell &A = sh[pairs[q].A], &B = sh[pairs[q].B];
+    pair_items[A.l + B.l > kJPairTop].push_back(
+        JPairItem{A.l, B.l, (int)q, (int)(e - q), A.nfunc, B.nfunc, A.ang_off, B.ang_off});
+    q = e;
+  }
+  constexpr int kTarget = 16384, kMaxLab = 2 * kJMaxLPrim;
+  const auto hcount = [](int L) { return (L + 1) * (L + 2) * (L + 3) / 6; };
+  const auto cost = [&](int L, int l) {
+    double c = 60.0 + 2.0 * hcount(L) * hcount(l);
+    for (int i = 0; i <= L + l; ++i) c += 3.0 * hcount(i);
+    return L + l > kJClassTop[1] ? 4.0 * c : c;  // these spill registers
+  };
+  const auto width_of = [&](int l, int na) {  // lanes per pair in the right-hand side
+    if (l < kJGroupL) return 64;
+    int w = 1;
+    while (w < na && w < 64) w *= 2;
+    return w;
+  };
+  double pot = 0.0, rhs = 0.0;
+  for (int L = 0; L <= kMaxLab; ++L) {
+    const int64_t nq = view.pair0[L + 1] - view.pair0[L];
+    for (int l = 0; l <= kJMaxLAux; ++l) {
+      const int64_t na = view.aux0[l + 1] - view.aux0[l];
+      if (!na || !nq) continue;
+      const int w = width_of(l, (int)na);
+      pot += cost(L, l) * (double)((nq + 63) / 64 * na);
+      rhs += cost(L, l) * (double)((na + w - 1) / w * ((nq * w + 63) / 64));
+    }
+  }
+  const auto length = [&](double total, int L, int l, double hi) {
+    return (int)std::min(std::max(std::round(total / kTarget / cost(L, l)), 2.0), hi);
+  };
+  for (int M = kMaxLab + kJMaxLAux; M >= 0; --M) {
+    const int cls = M <= kJClassTop[0] ? 0 : M <= kJClassTop[1] ? 1 : 2;
+    for (int L = std::max(0, M - kJMaxLAux); L <= std::min(M, kMaxLab); ++L) {
+      const int l = M - L;
+      const int q0 = view.pair0[L], q1 = view.pair0[L + 1], a0 = view.aux0[l], a1 = view.aux0[l + 1];
+      if (q0 == q1 || a0 == a1) continue;
+      const int pot_len = length(pot, L, l, 64.0);
+      for (int q = q0; q < q1; q += 64)
+        for (int a = a0; a < a1; a += pot_len)
+          items[1][cls].push_back(JItem{L, l, q, std::min(64, q1 - q), a, std::min(pot_len, a1 - a)});
+      const int w = width_of(l, a1 - a0), nq = length(rhs, L, l, 512.0) * (64 / w);
+      for (int a = a0; a < a1; a += w)
+        for (int q = q0; q < q1; q += nq) items[0][cls].push_back(JItem{L, l, q, std::min(nq, q1 - q), a, w});
+    }
+  }
+}
 
 struct xc_grid {
   xc_ctx* ctx = nullptr;
@@ -2318,23 +2414,88 @@ int xc_coulomb_create(xc_basis* basis, xc_basis* aux, double threshold, xc_coulo
               jc->pairs.push_back(q);
             }
         }
-      std::stable_sort(jc->pairs.begin(), jc->pairs.end(), [&](const JPair& x, const JPair& y) {
-        return x.L != y.L ? x.L < y.L : sh[x.A].l < sh[y.A].l;
-      });
+      // by L, then l_A and the kinds of the shells, otherwise in order (a counting sort)
+      const auto key = [&](const JPair& q) {
+        return ((q.L * (kJMaxLPrim + 1) + sh[q.A].l) * 2 + sh[q.A].pure) * 2 + sh[q.B].pure;
+      };
+      {
+        std::vector<size_t> at((2 * kJMaxLPrim + 1) * (kJMaxLPrim + 1) * 4 + 1, 0);
+        for (const auto& q : jc->pairs) ++at[key(q) + 1];
+        for (size_t k = 1; k < at.size(); ++k) at[k] += at[k - 1];
+        std::vector<JPair> sorted(jc->pairs.size());
+        for (const auto& q : jc->pairs) sorted[at[key(q)]++] = q;
+        jc->pairs.swap(sorted);
+      }
+      const auto hcount = [](int L) { return (L + 1) * (L + 2) * (L + 3) / 6; };
+      constexpr int kMaxLab = 2 * kJMaxLPrim;
+      JView& view = jc->view;
       int64_t off = 0;
+      int count[kMaxLab + 1] = {};
       for (auto& q : jc->pairs) {
         q.herm_off = (int)off;
-        off += (q.L + 1) * (q.L + 2) * (q.L + 3) / 6;
+        off += hcount(q.L);
+        ++count[q.L];
       }
       require(off < (1LL << 31), XC_ERR_INPUT, "xc_coulomb_create: too many primitive pairs");
       jc->herm_total = off;
+      int64_t h0 = 0;
+      for (int L = 0; L <= kMaxLab; ++L) {
+        view.pair0[L + 1] = view.pair0[L] + count[L];
+        view.herm0[L] = (int)h0;
+        h0 += (int64_t)count[L] * hcount(L);
+      }
       for (const auto& s : aux->shells) {
         jc->cart_off.push_back(jc->ncart_aux);
         jc->ncart_aux += s.ncart;
       }
+      // auxiliary primitives by angular momentum
+      std::vector<double> apos, acoef;
+      std::vector<int> prim_shell, shell_prim(aux->shells.size(), 0);
+      int64_t ah = 0;
+      for (int l = 0; l <= kJMaxLAux; ++l) {
+        view.aux0[l] = (int)prim_shell.size();
+        view.aherm0[l] = (int)ah;
+        for (size_t k = 0; k < aux->shells.size(); ++k) {
+          const DevShell& s = aux->shells[k];
+          if (s.l != l) continue;
+          shell_prim[k] = (int)prim_shell.size();
+          for (int i = 0; i < s.nprim; ++i) {
+            apos.insert(apos.end(), {s.cx, s.cy, s.cz, aux->alpha[s.prim_off + i]});
+            acoef.push_back(aux->coef[s.prim_off + i]);
+            prim_shell.push_back((int)k);
+          }
+        }
+        ah += (int64_t)(prim_shell.size() - view.aux0[l]) * hcount(l);
+      }
+      view.aux0[kJMaxLAux + 1] = jc->naux = (int)prim_shell.size();
+      require(ah < (1LL << 31), XC_ERR_INPUT, "xc_coulomb_create: too many auxiliary primitives");
+      jc->aherm_total = ah;
+      jc->plan_items();
       const int n = basis->nao;
       jc->d_pairs.upload(ctx, jc->pairs.data(), jc->pairs.size());
       jc->d_cart_off.upload(ctx, jc->cart_off.data(), jc->cart_off.size());
+      std::vector<double> ppos(4 * jc->pairs.size());
+      for (size_t q = 0; q < jc->pairs.size(); ++q) {
+        const JPair& pr = jc->pairs[q];
+        const double x[4] = {pr.P[0], pr.P[1], pr.P[2], pr.p};
+        std::copy(x, x + 4, ppos.begin() + 4 * q);
+      }
+      static const std::vector<double> boys = boys_table();
+      jc->d_pair.upload(ctx, ppos.data(), ppos.size());
+      jc->d_aux.upload(ctx, apos.data(), apos.size());
+      jc->d_prim_coef.upload(ctx, acoef.data(), acoef.size());
+      jc->d_prim_shell.upload(ctx, prim_shell.data(), prim_shell.size());
+      jc->d_shell_prim.upload(ctx, shell_prim.data(), shell_prim.size());
+      jc->d_boys.upload(ctx, boys.data(), boys.size());
+      view.pair = jc->d_pair.p;
+      view.aux = jc->d_aux.p;
+      view.boys = jc->d_boys.p;
+      for (int k = 0; k < 2; ++k)
+        for (int c = 0; c < kJClasses; ++c)
+          jc->d_items[k][c].upload(ctx, jc->items[k][c].data(), jc->items[k][c].size());
+      for (int c = 0; c < kJPairClasses; ++c)
+        jc->d_pair_items[c].upload(ctx, jc->pair_items[c].data(), jc->pair_items[c].size());
+      jc->d_U.alloc(ctx, std::max<int64_t>(jc->aherm_total, 1));  // U of step 4, W of step 2
       jc->d_D.alloc(ctx, std::max<int64_t>(off, 1));
       jc->d_V.alloc(ctx, std::max<int64_t>(off, 1));
       jc->d_bc.alloc(ctx, std::max(jc->ncart_aux, 1));
@@ -2375,12 +2536,19 @@ int xc_coulomb_rhs(xc_coulomb* jc, const double* P, double* b) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     hipStream_t s = ctx->stream;
     const int n = jc->basis->nao;
-    const int npair = (int)jc->pairs.size();
     HIPX(hipMemcpyAsync(jc->d_P.p, P, sizeof(double) * n * n, hipMemcpyHostToDevice, s));
-    launch_jdens(s, jc->d_pairs.p, npair, jc->basis->d_shells.p, jc->basis->d_ang.p, jc->d_P.p, n, jc->d_D.p);
-    launch_fill(s, jc->d_bc.p, jc->ncart_aux, 0.0);
-    launch_jrhs(s, jc->d_pairs.p, npair, jc->d_D.p, jc->aux->d_shells.p, jc->aux->nshell, jc->aux->d_alpha.p,
-                jc->aux->d_coef.p, jc->d_cart_off.p, jc->d_bc.p);
+    over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
+               [&](int c, hipStream_t st) {
+      launch_jdens(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p, jc->basis->d_shells.p,
+                   jc->basis->d_ang.p, jc->view, jc->d_P.p, n, jc->d_D.p);
+    });
+    launch_fill(s, jc->d_U.p, jc->aherm_total, 0.0);
+    // the widest classes (the longest items, few of them) beside the others
+    over_lanes(ctx->lanes, kJClasses, [&](int c) { return (int)jc->items[0][c].size(); }, [&](int c, hipStream_t st) {
+      launch_jrhs(st, c, jc->d_items[0][c].p, (int)jc->items[0][c].size(), jc->view, jc->d_D.p, jc->d_U.p);
+    });
+    launch_jaux_out(s, jc->view, jc->aux->d_shells.p, jc->aux->nshell, jc->d_shell_prim.p, jc->d_prim_coef.p,
+                    jc->d_cart_off.p, jc->d_U.p, jc->d_bc.p);
     HIPX(hipGetLastError());
     std::vector<double> bc(jc->ncart_aux);
     HIPX(hipMemcpyAsync(bc.data(), jc->d_bc.p, sizeof(double) * bc.size(), hipMemcpyDeviceToHost, s));
@@ -2404,7 +2572,6 @@ int xc_coulomb_matrix(xc_coulomb* jc, const double* c, double* J) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     hipStream_t s = ctx->stream;
     const int n = jc->basis->nao;
-    const int npair = (int)jc->pairs.size();
     // auxiliary AO -> Cartesian: cc_c = sum_f c_f M[f][c]
     std::vector<double> cc(std::max(jc->ncart_aux, 1), 0.0);
     for (int k = 0; k < jc->aux->nshell; ++k) {
@@ -2414,10 +2581,18 @@ int xc_coulomb_matrix(xc_coulomb* jc, const double* c, double* J) {
           cc[jc->cart_off[k] + q] += c[S.ao_off + f] * jc->aux->ang[S.ang_off + f * S.ncart + q];
     }
     HIPX(hipMemcpyAsync(jc->d_cc.p, cc.data(), sizeof(double) * jc->ncart_aux, hipMemcpyHostToDevice, s));
-    launch_jpot(s, jc->d_pairs.p, npair, jc->aux->d_shells.p, jc->aux->nshell, jc->aux->d_alpha.p, jc->aux->d_coef.p,
-                jc->d_cart_off.p, jc->d_cc.p, jc->d_V.p);
+    launch_jaux_in(s, jc->view, jc->naux, jc->d_prim_shell.p, jc->aux->d_shells.p, jc->d_prim_coef.p,
+                   jc->d_cart_off.p, jc->d_cc.p, jc->d_U.p);
+    launch_fill(s, jc->d_V.p, jc->herm_total, 0.0);
+    over_lanes(ctx->lanes, kJClasses, [&](int c) { return (int)jc->items[1][c].size(); }, [&](int c, hipStream_t st) {
+      launch_jpot(st, c, jc->d_items[1][c].p, (int)jc->items[1][c].size(), jc->view, jc->d_U.p, jc->d_V.p);
+    });
     launch_fill(s, jc->d_J.p, (int64_t)n * n, 0.0);
-    launch_jassemble(s, jc->d_pairs.p, npair, jc->basis->d_shells.p, jc->basis->d_ang.p, jc->d_V.p, n, jc->d_J.p);
+    over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
+               [&](int c, hipStream_t st) {
+      launch_jassemble(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p,
+                       jc->basis->d_shells.p, jc->basis->d_ang.p, jc->view, jc->d_V.p, n, jc->d_J.p);
+    });
     HIPX(hipGetLastError());
     HIPX(hipMemcpyAsync(J, jc->d_J.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, s));
     HIPX(hipStreamSynchronize(s));
