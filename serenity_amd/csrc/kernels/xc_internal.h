@@ -241,14 +241,17 @@ void launch_fock_sub(hipStream_t s, int sc, const FockItem* work, int nwork, con
 // U[j + n i] = sum over the row entries of AO i (block order) of the stored sub-tile values at
 // columns j >= i, for every i of [0, n): the lower triangle of the Fock accumulator, each element
 // written once (its terms meet in LDS in an order that varies from run to run).  Packed:
-// blockIdx.y = system, n = the largest n.  16 wavefronts per row: at (H2O)64/def2-TZVP the reduce
-// takes 0.68 ms against 0.86 ms with 8 and 1.40 ms with 4 (each wavefront's entries form a chain
-// of dependent load-add steps; more wavefronts, shorter chains).
+// blockIdx.y = system, n = the largest n.  16 wavefronts per row: each group's entries form a chain
+// of dependent load-add steps, and more wavefronts make shorter chains (with whole wavefronts per
+// entry 0.68 ms at (H2O)64/def2-TZVP against 0.86 ms with 8 and 1.40 ms with 4).  wide: blocks hold
+// more than 256 AOs on average, so that a row segment (half of them on average) fills the 128
+// columns that 32 lanes take at once; else 16 lanes take an entry.
 constexpr int kReduceWaves = 16;
 constexpr int kReduceWindow = 8192;  // row columns accumulated in LDS per pass
 template <typename T>
 void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
-                        double* U, int n, const PackSys* pack = nullptr, int nsys = 1, bool fixed = false);
+                        double* U, int n, const PackSys* pack = nullptr, int nsys = 1, bool fixed = false,
+                        bool wide = false);
 // Packed elementwise stages over nsys systems (maxnn = largest n^2): P -> FP32,
 // F = mirror of U (+ FP32 rounding partials), E = sum of block energies (+ rounding term).
 constexpr int kPackRoundBlocks = 512;  // finalize workgroups per system of a packed build

@@ -928,15 +928,21 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
 }
 
 // One AO row i of the Fock accumulator per workgroup: its entries (the blocks holding AO i, in
-// block order) are dealt to the kReduceWaves wavefronts round-robin; a wavefront adds each entry's
+// block order) are dealt to groups of Group lanes round-robin; a group adds each entry's
 // stored row segment into the workgroup's LDS copy of the row, and the row is written once to
-// U[j + n i], j >= i.  Each lane takes an aligned group of four columns (256 per pass of the
-// wavefront): one 16-byte load of their AO indices and one of their stored values, the lanes of a
-// wavefront reading one contiguous run of the block's stored row (a block's AO list is padded to
+// U[j + n i], j >= i.  Each lane takes an aligned group of four columns (4 Group per step):
+// one 16-byte load of their AO indices and one of their stored values, the lanes of a group
+// reading one contiguous run of the block's stored row (a block's AO list is padded to
 // a multiple of 32 with -1 and its stored row a runs from column 16 (a / 16) to the padded end,
 // so an aligned group never leaves either; the columns of the group before the segment start are
-// masked).  The loads of a wavefront's next entry are issued before the current entry's LDS
-// additions.  Rows longer than the LDS window are done in several passes over the entries.
+// masked).  A group walks its entries' steps as one sequence: while a step's values are added, the
+// next step's loads and the entry after it are in flight.  What bounds the kernel is the latency of
+// that chain, so short chains (many groups) count: segments hold n_b / 2 columns on average (12 to
+// 170), which left most of a wavefront's 64 lanes idle when a whole wavefront took an entry.  Groups
+// of 16 against whole wavefronts: (H2O)8/def2-SVP 40 -> 21 us, C20H42/def2-SVP 90 -> 76 us (FP64);
+// groups of 32 for blocks of more than 256 AOs: (H2O)64/def2-TZVP 683 -> 599 us in FP32 (631 with
+// 16), where the 2.8 GB of values and AO lists now come at 4.7 TB/s (a device copy: 5.0).
+// Rows longer than the LDS window are done in several passes over the entries.
 // Fixed = false: FP64 additions in LDS, which the wavefronts make in an order that varies from run
 // to run, so F varies at the rounding level.  Fixed = true: each term x is split into integers,
 // x = h 2^-32 + l 2^-72 + e with h = x 2^32 and l = (x - h 2^-32) 2^72 rounded to the nearest
@@ -946,7 +952,7 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
 // in the last place is then 2^-32 (1), and reads the integer from the bit pattern.  Valid for
 // terms of |x| < 2^19 in columns of fewer than 2^23 terms whose absolute values sum to less than
 // 2^30.
-template <typename T, bool Fixed>
+template <typename T, bool Fixed, int Group>
 __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const RowEnt* __restrict__ ent,
                                                                         const int* __restrict__ row_ptr,
                                                                         const T* __restrict__ Tscr,
@@ -966,8 +972,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
   }
   const int i = blockIdx.x;
   if (i >= n) return;  // uniform over the workgroup
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x;
   const gmem<const RowEnt>* entg = to_global(ent);
   const gmem<const T>* Tg = to_global(Tscr);
   const gmem<const int>* idxg = to_global(ao_idx);
@@ -983,86 +988,61 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
       }
     }
     __syncthreads();
-    auto fetch = [&](const RowEnt& E, int c, i32x4& gi, double (&v)[4]) {
-      gi = *reinterpret_cast<const gmem<const i32x4>*>(idxg + E.idx_off + c);
-      const gmem<const T>* src = Tg + E.rowbase + c;
-      if constexpr (sizeof(T) == 4) {
-        const f32x4 f = *reinterpret_cast<const gmem<const f32x4>*>(src);
-        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
-      } else {
-        const f64x2 f0 = *reinterpret_cast<const gmem<const f64x2>*>(src);
-        const f64x2 f1 = *reinterpret_cast<const gmem<const f64x2>*>(src + 2);
-        v[0] = f0.x; v[1] = f0.y; v[2] = f1.x; v[3] = f1.y;
+    // the group's entries e0 + grp + kGroups k; E: the entry of the step in flight, N: the one after it
+    constexpr int kGroups = 64 * kReduceWaves / Group;
+    const int gl = tid & (Group - 1);
+    int k = e0 + tid / Group;
+    RowEnt E = {0, 0, 0, 0, 0}, N = {0, 0, 0, 0, 0};
+    if (k < e1) E = load_global(entg + k);
+    if (k + kGroups < e1) N = load_global(entg + k + kGroups);
+    int c = (E.c0 & ~3) + 4 * gl, base = E.c0 & ~3;
+    i32x4 gi = {-1, -1, -1, -1};
+    T v[4] = {T(0), T(0), T(0), T(0)};
+    auto fetch = [&]() {  // the four columns of this lane in the current step, columns outside [c0, c1) masked
+      gi = i32x4{-1, -1, -1, -1};
+      if (k < e1 && c < E.c1) {
+        gi = *reinterpret_cast<const gmem<const i32x4>*>(idxg + E.idx_off + c);
+        const gmem<const T>* src = Tg + E.rowbase + c;
+        if constexpr (sizeof(T) == 4) {
+          const f32x4 f = *reinterpret_cast<const gmem<const f32x4>*>(src);
+          v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+        } else {
+          const f64x2 f0 = *reinterpret_cast<const gmem<const f64x2>*>(src);
+          const f64x2 f1 = *reinterpret_cast<const gmem<const f64x2>*>(src + 2);
+          v[0] = f0.x; v[1] = f0.y; v[2] = f1.x; v[3] = f1.y;
+        }
       }
     };
-    auto add = [&](const RowEnt& E, int c, const i32x4& gi, const double (&v)[4]) {
-      const int gg[4] = {gi.x, gi.y, gi.z, gi.w};
+    fetch();
+    while (__any(k < e1)) {
+      // this step's values, then the next step's loads, then the additions
+      const i32x4 ga = gi;
+      const double x[4] = {(double)v[0], (double)v[1], (double)v[2], (double)v[3]};
+      const int lo = E.c0 - c, hi = E.c1 - c;
+      base += 4 * Group;
+      if (base >= E.c1) {  // the same for the lanes of a group
+        k += kGroups;
+        E = N;
+        if (k + kGroups < e1) N = load_global(entg + k + kGroups);
+        base = E.c0 & ~3;
+      }
+      c = base + 4 * gl;
+      fetch();
+      const int gg[4] = {ga.x, ga.y, ga.z, ga.w};
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int g = gg[u] - i - w0;
-        if (c + u >= E.c0 && c + u < E.c1 && g >= 0 && g < wl) {
+        if (u >= lo && u < hi && g >= 0 && g < wl) {
           if constexpr (Fixed) {
-            const double t = v[u] + 0x1.8p20;
+            const double t = x[u] + 0x1.8p20;
             const long long h = __double_as_longlong(t) - __double_as_longlong(0x1.8p20);
-            const double rem = v[u] - (t - 0x1.8p20);  // exact, |rem| <= 2^-33
+            const double rem = x[u] - (t - 0x1.8p20);  // exact, |rem| <= 2^-33
             const long long l = __double_as_longlong(rem * 0x1p72 + 0x1.8p52) - __double_as_longlong(0x1.8p52);
             atomicAdd(racc_u + g, (unsigned long long)h);
             atomicAdd(racc_u + window + g, (unsigned long long)l);
           } else {
-            atomicAdd(racc + g, v[u]);
+            atomicAdd(racc + g, x[u]);
           }
-        }
-      }
-    };
-    // this wavefront's entries e0 + w + kReduceWaves k, k < nk: their RowEnts are read 64 at a time,
-    // one per lane, and broadcast from the lanes (scalar registers), so that an entry's loads
-    // depend on no load of its own; the loads of the next kAhead entries are in flight during an
-    // entry's LDS additions
-    constexpr int kAhead = 1;
-    const int nk = e1 - e0 > w ? (e1 - e0 - w + kReduceWaves - 1) / kReduceWaves : 0;
-    for (int kb = 0; kb < nk; kb += 64) {
-      const int cnt = min(64, nk - kb);
-      RowEnt L = {0, 0, 0, 0, 0};
-      if (lane < cnt) L = load_global(entg + e0 + w + kReduceWaves * (kb + lane));
-      RowEnt Eq[kAhead + 1];
-      int cq[kAhead + 1];
-      i32x4 gq[kAhead + 1];
-      double vq[kAhead + 1][4];
-      auto issue = [&](int k, int d) {  // entry k into slot d
-        RowEnt& E = Eq[d];
-        const int lo = __builtin_amdgcn_readlane((int)(L.rowbase & 0xffffffff), k);
-        const int hi = __builtin_amdgcn_readlane((int)(L.rowbase >> 32), k);
-        E.rowbase = (int64_t)(((uint64_t)(unsigned)hi << 32) | (unsigned)lo);
-        E.c0 = __builtin_amdgcn_readlane(L.c0, k);
-        E.c1 = __builtin_amdgcn_readlane(L.c1, k);
-        E.idx_off = __builtin_amdgcn_readlane(L.idx_off, k);
-        E.block = 0;
-        cq[d] = (E.c0 & ~3) + 4 * lane;
-        gq[d] = i32x4{-1, -1, -1, -1};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) vq[d][u] = 0.0;
-        if (cq[d] < E.c1) fetch(E, cq[d], gq[d], vq[d]);
-      };
-#pragma unroll
-      for (int d = 0; d < kAhead; ++d)
-        if (d < cnt) issue(d, d);
-      for (int k = 0; k < cnt; ++k) {
-        if (k + kAhead < cnt) issue(k + kAhead, kAhead);  // wavefront-uniform
-        const RowEnt& E = Eq[0];
-        if (cq[0] < E.c1) add(E, cq[0], gq[0], vq[0]);
-        for (int c2 = cq[0] + 256; c2 < E.c1; c2 += 256) {
-          i32x4 g2;
-          double v2[4];
-          fetch(E, c2, g2, v2);
-          add(E, c2, g2, v2);
-        }
-#pragma unroll
-        for (int d = 0; d < kAhead; ++d) {
-          Eq[d] = Eq[d + 1];
-          cq[d] = cq[d + 1];
-          gq[d] = gq[d + 1];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) vq[d][u] = vq[d + 1][u];
         }
       }
     }
@@ -1487,24 +1467,33 @@ static int reduce_window_limit(bool fixed) {
   return cached[fixed][dev];
 }
 
-template <typename T>
-void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
-                        double* U, int n, const PackSys* pack, int nsys, bool fixed) {
-  if (n <= 0 || nsys <= 0) return;
-  const int lim = reduce_window_limit(fixed);
+template <typename T, bool Fixed>
+static void launch_fock_reduce_f(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr,
+                                 const int* ao_idx, double* U, int n, const PackSys* pack, int nsys, bool wide) {
+  const int lim = reduce_window_limit(Fixed);
   const int window = n < lim ? n : lim;
-  const size_t lds = (fixed ? 16 : 8) * (size_t)window;
-  if (fixed)
-    hipLaunchKernelGGL((fock_reduce_kernel<T, true>), dim3(n, nsys), dim3(64 * kReduceWaves), lds, s, ent, row_ptr,
+  const size_t lds = (Fixed ? 16 : 8) * (size_t)window;
+  if (wide)
+    hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 32>), dim3(n, nsys), dim3(64 * kReduceWaves), lds, s, ent, row_ptr,
                        Tscr, ao_idx, U, n, window, pack);
   else
-    hipLaunchKernelGGL((fock_reduce_kernel<T, false>), dim3(n, nsys), dim3(64 * kReduceWaves), lds, s, ent, row_ptr,
+    hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 16>), dim3(n, nsys), dim3(64 * kReduceWaves), lds, s, ent, row_ptr,
                        Tscr, ao_idx, U, n, window, pack);
 }
+
+template <typename T>
+void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
+                        double* U, int n, const PackSys* pack, int nsys, bool fixed, bool wide) {
+  if (n <= 0 || nsys <= 0) return;
+  if (fixed)
+    launch_fock_reduce_f<T, true>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide);
+  else
+    launch_fock_reduce_f<T, false>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide);
+}
 template void launch_fock_reduce<double>(hipStream_t, const RowEnt*, const int*, const double*, const int*, double*,
-                                         int, const PackSys*, int, bool);
+                                         int, const PackSys*, int, bool, bool);
 template void launch_fock_reduce<float>(hipStream_t, const RowEnt*, const int*, const float*, const int*, double*,
-                                        int, const PackSys*, int, bool);
+                                        int, const PackSys*, int, bool, bool);
 
 void launch_weight_potential(hipStream_t s, int64_t npts, const double* w, const double* v, const double* g,
                              double* vs, double* gw) {

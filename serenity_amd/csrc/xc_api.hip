@@ -620,7 +620,8 @@ void run_fock_tiles(xc_bfogc* bf, const T* tiles, int gga, double thr, const Lan
 template <typename T>
 void run_fock_reduce(xc_bfogc* bf, const Lanes& L) {
   launch_fock_reduce<T>(L.main, bf->d_rowent.p, bf->d_rowptr.p, reinterpret_cast<const T*>(bf->d_T.p),
-                        bf->d_ao_idx.p, bf->d_U.p, bf->basis->nao, nullptr, 1, bf->ctx->deterministic);
+                        bf->d_ao_idx.p, bf->d_U.p, bf->basis->nao, nullptr, 1, bf->ctx->deterministic,
+                        bf->sum_nb > 256 * (int64_t)bf->nblocks);
 }
 
 template <typename T>
