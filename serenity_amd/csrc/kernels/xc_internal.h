@@ -140,21 +140,33 @@ struct FockItem {
   int b0, nb;
   int nsub;
 };
-constexpr int kFockRows = 256;        // rows a sub-tile item may stage
 constexpr int kFockPanel = 128;       // panel height of blocks split into panel pairs
-#ifndef SXC_FOCK_WAVES
-#define SXC_FOCK_WAVES 16
-#endif
-constexpr int kFockWaves = SXC_FOCK_WAVES;  // wavefronts per workgroup of the sub-tile kernel
-#if SXC_FOCK_WAVES == 16
-constexpr int kFockNumS = 5;          // slot-count classes of the sub-tile kernel
-constexpr int kFockS[kFockNumS] = {1, 2, 3, 4, 5};
-inline int fock_smax(int) { return 5; }  // accumulator budget: kFockWaves * 5 sub-tiles per item
-#else
-constexpr int kFockNumS = 9;
-constexpr int kFockS[kFockNumS] = {1, 2, 3, 4, 5, 6, 7, 8, 10};
-inline int fock_smax(int) { return 10; }
-#endif
+// Workgroup shapes of the sub-tile kernel: wavefronts, rows an item may stage (576 bytes of LDS each),
+// 16 x 16 sub-tiles per wavefront, and the widest block (padded AOs) whose triangle is one item of
+// the shape; wider blocks are split into pairs of panels, items of kFockPanelShape.  A compute unit
+// holds three workgroups of the first shape and one of the others: an item of few rows waits for its
+// loads and barriers most of its time, so several run beside each other (26 potentials of the
+// embedding sweep over blocks of up to 64 AOs: 67 -> 34 us each in FP64 with 4 wavefronts instead of
+// 16 and a compute unit's whole LDS).  Blocks of 96 to 128 AOs in 8 wavefronts, two per compute unit,
+// measured no faster (C20H42/def2-SVP 470 against 431 us): there the matrix cores are the bound.
+// The others differ in the slots of a wavefront alone, whose registers every item of a kernel holds.
+struct FockShape {
+  int waves, rows, slots, npad;
+};
+constexpr int kFockShapes = 4;
+constexpr FockShape kFockShape[kFockShapes] = {{4, 64, 3, 64}, {16, 256, 3, 128}, {16, 256, 4, 160}, {16, 256, 5, 192}};
+constexpr int kFockPanelShape = 2;
+constexpr bool fock_shapes_fit() {
+  for (int k = 0; k < kFockShapes; ++k) {
+    const int nt = kFockShape[k].npad / 16;
+    if (nt * (nt + 1) / 2 > kFockShape[k].waves * kFockShape[k].slots || kFockShape[k].npad > kFockShape[k].rows)
+      return false;
+  }
+  const int np = kFockPanel / 16;
+  const FockShape p = kFockShape[kFockPanelShape];
+  return 2 * kFockPanel <= p.rows && np * np <= p.waves * p.slots;
+}
+static_assert(fock_shapes_fit(), "every item's sub-tiles and rows fit its shape");
 
 // Work item of the density kernel: block, a = first column of the pass,
 // b = columns of the pass (multiple of 16), pass = partial-density slot.
@@ -170,7 +182,7 @@ void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, const in
                     const DevShell* shells, const double* alpha, const double* coef, const double* ang,
                     const double* pts, double radial_thr, double exp_thr, int ncomp, double* tiles64, float* tiles32);
 
-// Sub-tile density kernel: 8 wavefronts, S = pass columns / 16 (1..kDensMaxS).
+// Sub-tile density kernel: 8 wavefronts per pass of at most 16 kDensMaxS columns.
 // Partial densities: part[(pass * 4 + c) * npts + q], c = rho, d/dx, d/dy, d/dz
 // (gradient slots hold sum T grad phi without the factor 2).
 constexpr int kDensMaxS = 6;
@@ -182,30 +194,30 @@ constexpr int kDensIdxLds = 2048;  // AO index lists up to this length are stage
 // With nwork_dev, the launch covers a list filled on the device: only its first *nwork_dev
 // items run (nwork is the list's capacity).
 template <typename T>
-void launch_density_sub(hipStream_t s, int S, const WorkItem* work, int nwork, const DevBlock* blocks,
-                        const int* ao_idx, const T* tiles, const T* P, int n, int want_grad, double* part,
-                        int64_t npts, const PackSys* pack = nullptr, const int* nwork_dev = nullptr,
+void launch_density_sub(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
+                        const T* tiles, const T* P, int n, int want_grad, double* part, int64_t npts,
+                        const PackSys* pack = nullptr, const int* nwork_dev = nullptr,
                         const unsigned char* skip = nullptr);
 
-// Dense-block refinement of the mixed-precision density: the work lists (one per column-tile
-// class) and their device-side counts, filled by launch_mark_dense.
-struct DenseLists {
-  WorkItem* item[kDensMaxS + 1];
-  int* count;  // kDensMaxS + 1 counters
+// Dense-block refinement of the mixed-precision density: a work list and its device-side count, filled
+// by launch_mark_dense.
+struct DenseList {
+  WorkItem* item;
+  int* count;
 };
-// Clears the counts, then appends the density items of every block whose largest density in the
+// Clears the count, then appends the density items of every block whose largest density in the
 // partials part (one pass per item, 128-point blocks) exceeds rho_thr; by_block holds every block's
-// items contiguously from item0[b] (blocks[b].npass of them), cls[b] is their class.
+// items contiguously from item0[b] (blocks[b].npass of them).
 // With a mask (one byte per block: the blocks the first pass skipped because the previous build
 // found them dense), only the blocks outside it are tested and the listed ones join it;
 // launch_list_masked lists the mask's own blocks (before the first pass, so that their second pass
 // can run beside it), and launch_refresh_dense, after the second passes, keeps in the mask only the
 // blocks whose density from them still exceeds rho_thr.
 void launch_mark_dense(hipStream_t s, const DevBlock* blocks, int nblocks, int64_t npts, const double* part,
-                       double rho_thr, const WorkItem* by_block, const int* item0, const int* cls,
-                       const DenseLists& lists, unsigned char* mask = nullptr);
+                       double rho_thr, const WorkItem* by_block, const int* item0, const DenseList& list,
+                       unsigned char* mask = nullptr);
 void launch_list_masked(hipStream_t s, const DevBlock* blocks, int nblocks, const WorkItem* by_block,
-                        const int* item0, const int* cls, const DenseLists& lists, const unsigned char* mask);
+                        const int* item0, const DenseList& list, const unsigned char* mask);
 void launch_refresh_dense(hipStream_t s, const DevBlock* blocks, int nblocks, int64_t npts, const double* part,
                           double rho_thr, unsigned char* mask);
 void launch_to_double(hipStream_t s, const float* src, double* dst, int64_t n);
@@ -231,13 +243,13 @@ void launch_functional_pol(hipStream_t s, int func, const XcParams& prm, int64_t
                            const double* ra2 = nullptr, const double* ga2 = nullptr, const double* rb2 = nullptr,
                            const double* gb2 = nullptr);
 
-// Sub-tile Fock kernel: kFockWaves wavefronts, slot class sc (kFockS[sc] sub-tiles per wavefront).
+// Sub-tile Fock kernel over items of one workgroup shape.
 // Each item stores its sub-tiles of phi^T G + G^T phi into the block's scratch slice Tscr + toff
 // (zeros when the block-average test skips the block).
 template <typename T>
-void launch_fock_sub(hipStream_t s, int sc, const FockItem* work, int nwork, const DevBlock* blocks,
-                     const int* ao_idx, const T* tiles, const double* vs, const double* gw, int gga,
-                     double block_ave_thr, T* Tscr, int64_t npts, const PackSys* pack = nullptr);
+void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, const DevBlock* blocks, const T* tiles,
+                     const double* vs, const double* gw, int gga, double block_ave_thr, T* Tscr, int64_t npts,
+                     const PackSys* pack = nullptr);
 // U[j + n i] = sum over the row entries of AO i (block order) of the stored sub-tile values at
 // columns j >= i, for every i of [0, n): the lower triangle of the Fock accumulator, each element
 // written once (its terms meet in LDS in an order that varies from run to run).  Packed:

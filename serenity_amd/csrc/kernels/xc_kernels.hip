@@ -202,17 +202,20 @@ __device__ inline void quad_rows(const gmem<const float>* seg, int lane, double 
 // lane dotting its T entries with the phi / grad phi values of the same
 // (point, column), and summed over the columns by lane shuffles.  (FP64
 // accumulates T transposed, so that its lanes read whole 128-byte point runs.)
+// What the density items of one launch share.
+template <typename T>
+struct DensityArgs {
+  const int* ao_idx;
+  const T* tiles;
+  const T* P;
+  int n, want_grad;
+  double* part;
+  int64_t npts;
+};
+
 template <typename T, int S>
-__global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __restrict__ work,
-                                                          const DevBlock* __restrict__ blocks,
-                                                          const int* __restrict__ ao_idx,
-                                                          const T* __restrict__ tiles, const T* __restrict__ P,
-                                                          int n, int want_grad, double* __restrict__ part,
-                                                          int64_t npts, const PackSys* __restrict__ pack,
-                                                          const int* __restrict__ nwork_dev,
-                                                          const unsigned char* __restrict__ skip) {
-  // a launch over a list filled on the device runs only its first *nwork_dev items
-  if (nwork_dev && (int)blockIdx.x >= *nwork_dev) return;
+__device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock& bk, const DensityArgs<T>& arg,
+                                             unsigned char* smem, int* sIdx) {
   using M = Mfma<T>;
   constexpr int KC = 128 / (int)sizeof(T);      // AOs per chunk (128 bytes of each LDS row)
   constexpr int KV = KC / 4;
@@ -220,25 +223,15 @@ __global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __rest
   constexpr int NC = 16 * S;
   constexpr int NB = (4 * NC + 511) / 512;      // P staging tasks per thread
   constexpr int GS = 2;
-  constexpr int STAGE_BYTES = (kTile + NC) * RS * (int)sizeof(T);
   typedef T vec_t __attribute__((ext_vector_type(KV)));
-  __shared__ __attribute__((aligned(16))) unsigned char smem[STAGE_BYTES];
-  __shared__ int sIdx[kDensIdxLds];
   T(*sA)[RS] = reinterpret_cast<T(*)[RS]>(smem);
   T(*sB)[RS] = reinterpret_cast<T(*)[RS]>(smem + kTile * RS * sizeof(T));
-
-  const WorkItem wk = work[blockIdx.x];
-  if (skip && skip[wk.block]) return;  // a block the caller contracts in another pass
-  const DevBlock bk = blocks[wk.block];
-  if (pack) {
-    const PackSys& ps = pack[bk.sys];
-    tiles = static_cast<const T*>(ps.tiles);
-    P = static_cast<const T*>(ps.P);
-    ao_idx = ps.ao_idx;
-    part = ps.part;
-    npts = ps.npts;
-    n = ps.n;
-  }
+  const int* ao_idx = arg.ao_idx;
+  const T* tiles = arg.tiles;
+  const T* P = arg.P;
+  double* part = arg.part;
+  const int n = arg.n, want_grad = arg.want_grad;
+  const int64_t npts = arg.npts;
   const int col0 = wk.a, ncols = wk.b;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -305,8 +298,9 @@ __global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __rest
   // dependent global load) in windows of kDensIdxLds entries: one window unless the block is
   // wider.  One LDS buffer; the global loads of chunk k + 1 of a window are in flight during the
   // MFMAs of chunk k.
-  for (int wb = 0; wb < npad; wb += kDensIdxLds) {
-    const int wl = min(kDensIdxLds, npad - wb);
+  const int kend = (bk.nb + KC - 1) / KC * KC;  // whole chunks: at most npad, whose last AOs are zero
+  for (int wb = 0; wb < kend; wb += kDensIdxLds) {
+    const int wl = min(kDensIdxLds, kend - wb);
     for (int i = tid; i < wl; i += 512) sIdx[i] = idx[wb + i];
     __syncthreads();
     const int nch = wl / KC;
@@ -438,6 +432,42 @@ __global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __rest
         dst[3 * npts] = zv;
       }
     }
+  }
+}
+
+// Every pass width in one kernel: a launch per width left each of them a tail of its own, and small
+// systems paid the launches and the stream forks more than the work ((H2O)8/def2-SVP: 108 us of
+// which the kernels ran 49).
+template <typename T>
+__global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __restrict__ work,
+                                                          const DevBlock* __restrict__ blocks, DensityArgs<T> arg,
+                                                          const PackSys* __restrict__ pack,
+                                                          const int* __restrict__ nwork_dev,
+                                                          const unsigned char* __restrict__ skip) {
+  // a launch over a list filled on the device runs only its first *nwork_dev items
+  if (nwork_dev && (int)blockIdx.x >= *nwork_dev) return;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[(kTile + 16 * kDensMaxS) * 144];
+  __shared__ int sIdx[kDensIdxLds];
+  const WorkItem wk = work[blockIdx.x];
+  if (skip && skip[wk.block]) return;  // a block the caller contracts in another pass
+  const DevBlock bk = blocks[wk.block];
+  if (pack) {
+    const PackSys& ps = pack[bk.sys];
+    arg.tiles = static_cast<const T*>(ps.tiles);
+    arg.P = static_cast<const T*>(ps.P);
+    arg.ao_idx = ps.ao_idx;
+    arg.part = ps.part;
+    arg.npts = ps.npts;
+    arg.n = ps.n;
+  }
+  static_assert(kDensMaxS == 6, "one case per pass width");
+  switch ((wk.b + 15) / 16) {
+    case 1: return density_item<T, 1>(wk, bk, arg, smem, sIdx);
+    case 2: return density_item<T, 2>(wk, bk, arg, smem, sIdx);
+    case 3: return density_item<T, 3>(wk, bk, arg, smem, sIdx);
+    case 4: return density_item<T, 4>(wk, bk, arg, smem, sIdx);
+    case 5: return density_item<T, 5>(wk, bk, arg, smem, sIdx);
+    default: return density_item<T, 6>(wk, bk, arg, smem, sIdx);
   }
 }
 
@@ -653,7 +683,7 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, XcParams 
   if (t == 0) e_blk[b] = eb;
 }
 
-// Sub-tile Fock contraction.  One workgroup of kFockWaves wavefronts per work item; the
+// Sub-tile Fock contraction.  One workgroup of W wavefronts per work item; the
 // item's 16 x 16 AO sub-tiles (i, j) are dealt to the wavefronts round-robin,
 // S per wavefront, each accumulating S_ij = phi_i^T G_j + G_i^T phi_j over the
 // block's 128 points in registers (dummy slots of a short item compute on row
@@ -664,10 +694,13 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, XcParams 
 // rows of LDS on its way in.  Inside a chunk, k-step t of lane group g takes
 // point KV g + t (KV = KC / 4), so each MFMA operand of a chunk is one 32-byte
 // LDS read of KV consecutive points of one AO row.
-template <typename T, int S>
-__global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockItem* __restrict__ work,
+// One kernel per workgroup shape, with one slot count each: an item's wavefronts stop at the slots
+// they hold, so a shape's smaller items lose nothing but the registers of the widest (FP64 at 5
+// slots spills 4; one kernel of 5 slots for every wide item was 2 to 3 % slower at (H2O)64 and 32).
+template <typename T, int W, int Rows, int S>
+__global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __restrict__ work,
                                                        const DevBlock* __restrict__ blocks,
-                                                       const int* __restrict__ ao_idx, const T* __restrict__ tiles,
+                                                       const T* __restrict__ tiles,
                                                        const double* __restrict__ vs, const double* __restrict__ gw,
                                                        int gga, double thr, T* __restrict__ Tscr, int64_t npts,
                                                        const PackSys* __restrict__ pack) {
@@ -676,16 +709,16 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
   constexpr int KV = KC / 4;
   constexpr int RS = KC + 16 / (int)sizeof(T);  // 144-byte LDS rows: the 16 rows of an operand read hit distinct banks
   constexpr int NCH = kTile / KC;
-  constexpr int NT = 64 * kFockWaves;            // threads
-  constexpr int NTASK = kFockRows * 4 / NT;
+  constexpr int NT = 64 * W;                     // threads
+  constexpr int NTASK = Rows * 4 / NT;
+  static_assert(NTASK * NT == Rows * 4, "whole staging tasks");
   typedef T vec_t __attribute__((ext_vector_type(KV)));
   // Two LDS buffers, one barrier per chunk.  FP32 stages chunk c + 1 after the MFMAs of chunk c
   // (4.25 -> 4.09 ms at (H2O)64/def2-TZVP against one buffer); FP64 stages it in the instruction
   // stream of the MFMAs of slot 0 of chunk c, from registers loaded one chunk earlier (6.22 -> 5.88
   // ms; the same order measured no faster in FP32).
-  constexpr int NBUF = 2;
-  __shared__ __attribute__((aligned(16))) T sPhi2[NBUF][kFockRows][RS];
-  __shared__ __attribute__((aligned(16))) T sG2[NBUF][kFockRows][RS];
+  __shared__ __attribute__((aligned(16))) T sPhi2[2][Rows][RS];
+  __shared__ __attribute__((aligned(16))) T sG2[2][Rows][RS];
   // w v / 2, w g_x, w g_y, w g_z of each point in the contraction type, one plane per quantity:
   // the four point runs a wavefront reads at once then start on distinct banks
   __shared__ __attribute__((aligned(16))) T spot[4][kTile];
@@ -726,12 +759,18 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
     for (int m = 0; m < NTASK; ++m) {
       const int task = tid + NT * m;
       if (task < 4 * R) {
-        const gmem<const T>* src = tb + (int64_t)grow_of(row_of(task)) * kTile + p0 + KV * q;
-        raw[m][0] = *reinterpret_cast<const gmem<const vec_t>*>(src);
+        // one 32-bit byte offset per lane from the planes' wavefront-uniform bases (a 64-bit address
+        // per plane and task took the registers that made the widest FP64 items spill)
+        const unsigned off = (unsigned)((grow_of(row_of(task)) * kTile + p0 + KV * q) * (int)sizeof(T));
+        auto plane = [&](int k) {
+          return *reinterpret_cast<const gmem<const vec_t>*>(reinterpret_cast<const gmem<const char>*>(tb + k * cstride) +
+                                                             off);
+        };
+        raw[m][0] = plane(0);
         if (gga) {
-          raw[m][1] = *reinterpret_cast<const gmem<const vec_t>*>(src + cstride);
-          raw[m][2] = *reinterpret_cast<const gmem<const vec_t>*>(src + 2 * cstride);
-          raw[m][3] = *reinterpret_cast<const gmem<const vec_t>*>(src + 3 * cstride);
+          raw[m][1] = plane(1);
+          raw[m][2] = plane(2);
+          raw[m][3] = plane(3);
         }
       }
     }
@@ -779,7 +818,7 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
   // in its sub-tiles, so the reduce needs no per-block test
   if ((red[0] + red[1]) / bk.npts < thr) {
     gmem<T>* out0 = to_global(Tscr + bk.toff);
-    for (int t = w; t < it.nsub; t += kFockWaves) {
+    for (int t = w; t < it.nsub; t += W) {
       int i, j;
       decode(t, i, j);
       const int I = it.a0 / 16 + i, J = (diag ? it.a0 : it.b0) / 16 + j;
@@ -792,7 +831,7 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
   int li[S], lj[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int t = w + kFockWaves * s;
+    const int t = w + W * s;
     int i = 0, j = 0;
     if (t < it.nsub) decode(t, i, j);
     li[s] = __builtin_amdgcn_readfirstlane(t < it.nsub ? 16 * i : 0);
@@ -800,8 +839,8 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
   }
 
   auto store = [&](int c) {
-    T(*sPhi)[RS] = sPhi2[NBUF == 2 ? (c & 1) : 0];
-    T(*sG)[RS] = sG2[NBUF == 2 ? (c & 1) : 0];
+    T(*sPhi)[RS] = sPhi2[c & 1];
+    T(*sG)[RS] = sG2[c & 1];
     // the KV points of this thread's tasks are the same for every task; their potentials are
     // read as whole vectors, the GGA test taken once (a test per value branches around each
     // LDS read and waits for it)
@@ -838,7 +877,7 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
   for (int s = 0; s < S; ++s) acc[s] = M::zero();
   const int r = lane & 15, g = lane >> 4;
   // slots of this wavefront that hold a sub-tile (an item smaller than its class leaves the rest idle)
-  const int slive = it.nsub > w ? (it.nsub - w + kFockWaves - 1) / kFockWaves : 0;
+  const int slive = it.nsub > w ? (it.nsub - w + W - 1) / W : 0;
   auto slot = [&](int s, T(*sPhi)[RS], T(*sG)[RS]) {
     const vec_t aP = *reinterpret_cast<const vec_t*>(&sPhi[li[s] + r][KV * g]);
     const vec_t aG = *reinterpret_cast<const vec_t*>(&sG[li[s] + r][KV * g]);
@@ -915,7 +954,7 @@ __global__ __launch_bounds__(64 * kFockWaves) void fock_sub_kernel(const FockIte
   gmem<T>* tb_out = to_global(Tscr + bk.toff);
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int t = w + kFockWaves * s;
+    const int t = w + W * s;
     if (t >= it.nsub) continue;
     int i, j;
     decode(t, i, j);
@@ -1228,33 +1267,19 @@ void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, const in
 }
 
 template <typename T>
-void launch_density_sub(hipStream_t s, int S, const WorkItem* work, int nwork, const DevBlock* blocks,
-                        const int* ao_idx, const T* tiles, const T* P, int n, int want_grad, double* part,
-                        int64_t npts, const PackSys* pack, const int* nwork_dev, const unsigned char* skip) {
+void launch_density_sub(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
+                        const T* tiles, const T* P, int n, int want_grad, double* part, int64_t npts,
+                        const PackSys* pack, const int* nwork_dev, const unsigned char* skip) {
   if (nwork <= 0) return;
-  switch (S) {
-#define SXC_DENS_S(SV)                                                                                        \
-  case SV:                                                                                                    \
-    hipLaunchKernelGGL((density_sub_kernel<T, SV>), dim3(nwork), dim3(512), 0, s, work, blocks, ao_idx, tiles, \
-                       P, n, want_grad, part, npts, pack, nwork_dev, skip);                                   \
-    return;
-    static_assert(kDensMaxS == 6, "one case per column-tile class");
-    SXC_DENS_S(1)
-    SXC_DENS_S(2)
-    SXC_DENS_S(3)
-    SXC_DENS_S(4)
-    SXC_DENS_S(5)
-    SXC_DENS_S(6)
-#undef SXC_DENS_S
-  }
-  throw std::runtime_error("launch_density_sub: column-tile count out of range");
+  const DensityArgs<T> arg = {ao_idx, tiles, P, n, want_grad, part, npts};
+  hipLaunchKernelGGL((density_sub_kernel<T>), dim3(nwork), dim3(512), 0, s, work, blocks, arg, pack, nwork_dev, skip);
 }
-template void launch_density_sub<double>(hipStream_t, int, const WorkItem*, int, const DevBlock*, const int*,
-                                         const double*, const double*, int, int, double*, int64_t,
-                                         const PackSys*, const int*, const unsigned char*);
-template void launch_density_sub<float>(hipStream_t, int, const WorkItem*, int, const DevBlock*, const int*,
-                                        const float*, const float*, int, int, double*, int64_t, const PackSys*,
-                                        const int*, const unsigned char*);
+template void launch_density_sub<double>(hipStream_t, const WorkItem*, int, const DevBlock*, const int*, const double*,
+                                         const double*, int, int, double*, int64_t, const PackSys*, const int*,
+                                         const unsigned char*);
+template void launch_density_sub<float>(hipStream_t, const WorkItem*, int, const DevBlock*, const int*, const float*,
+                                        const float*, int, int, double*, int64_t, const PackSys*, const int*,
+                                        const unsigned char*);
 
 // Largest density of block b (128 threads), from the partials of its passes.
 __device__ double block_max_density(const DevBlock& bk, int64_t npts, const double* __restrict__ part, double* red) {
@@ -1272,39 +1297,37 @@ __device__ double block_max_density(const DevBlock& bk, int64_t npts, const doub
 }
 
 // Blocks whose largest density (from the partials of a first pass) exceeds rho_thr have their
-// density work items appended to the list of their column-tile class, for a second pass.  With a
+// density work items appended to the list, for a second pass.  With a
 // mask, only the blocks outside it are tested (the first pass skipped the others) and the listed
 // ones join it.
 __global__ __launch_bounds__(128) void mark_dense_kernel(const DevBlock* __restrict__ blocks, int64_t npts,
                                                          const double* __restrict__ part, double rho_thr,
                                                          const WorkItem* __restrict__ by_block,
-                                                         const int* __restrict__ item0, const int* __restrict__ cls,
-                                                         DenseLists lists, unsigned char* __restrict__ mask) {
+                                                         const int* __restrict__ item0, DenseList list,
+                                                         unsigned char* __restrict__ mask) {
   __shared__ double red[128];
   const int b = blockIdx.x, t = threadIdx.x;
   if (mask && mask[b]) return;  // uniform over the workgroup
   const DevBlock bk = blocks[b];
   const bool dense = bk.npass > 0 && block_max_density(bk, npts, part, red) > rho_thr;
   if (t == 0 && dense) {
-    const int c = cls[b];
-    const int pos = atomicAdd(lists.count + c, bk.npass);
-    for (int k = 0; k < bk.npass; ++k) lists.item[c][pos + k] = by_block[item0[b] + k];
+    const int pos = atomicAdd(list.count, bk.npass);
+    for (int k = 0; k < bk.npass; ++k) list.item[pos + k] = by_block[item0[b] + k];
     if (mask) mask[b] = 1;
   }
 }
 
-// The density work items of the blocks in the mask, appended to the list of their class.
+// The density work items of the blocks in the mask, appended to the list.
 __global__ __launch_bounds__(64) void list_masked_kernel(const DevBlock* __restrict__ blocks, int nblocks,
                                                          const WorkItem* __restrict__ by_block,
-                                                         const int* __restrict__ item0, const int* __restrict__ cls,
-                                                         DenseLists lists, const unsigned char* __restrict__ mask) {
+                                                         const int* __restrict__ item0, DenseList list,
+                                                         const unsigned char* __restrict__ mask) {
   const int b = blockIdx.x * 64 + threadIdx.x;
   if (b >= nblocks || !mask[b]) return;
   const int np = blocks[b].npass;
   if (np <= 0) return;
-  const int c = cls[b];
-  const int pos = atomicAdd(lists.count + c, np);
-  for (int k = 0; k < np; ++k) lists.item[c][pos + k] = by_block[item0[b] + k];
+  const int pos = atomicAdd(list.count, np);
+  for (int k = 0; k < np; ++k) list.item[pos + k] = by_block[item0[b] + k];
 }
 
 // After the second pass: a listed block stays in the mask while its density exceeds rho_thr.
@@ -1329,20 +1352,20 @@ __global__ void to_double_kernel(const float* __restrict__ s, double* __restrict
 }
 
 void launch_mark_dense(hipStream_t s, const DevBlock* blocks, int nblocks, int64_t npts, const double* part,
-                       double rho_thr, const WorkItem* by_block, const int* item0, const int* cls,
-                       const DenseLists& lists, unsigned char* mask) {
+                       double rho_thr, const WorkItem* by_block, const int* item0, const DenseList& list,
+                       unsigned char* mask) {
   if (nblocks <= 0) return;
-  hipLaunchKernelGGL(clear_counts_kernel, dim3(1), dim3(64), 0, s, lists.count, kDensMaxS + 1);
+  hipLaunchKernelGGL(clear_counts_kernel, dim3(1), dim3(64), 0, s, list.count, 1);
   hipLaunchKernelGGL(mark_dense_kernel, dim3(nblocks), dim3(128), 0, s, blocks, npts, part, rho_thr, by_block, item0,
-                     cls, lists, mask);
+                     list, mask);
 }
 
 void launch_list_masked(hipStream_t s, const DevBlock* blocks, int nblocks, const WorkItem* by_block,
-                        const int* item0, const int* cls, const DenseLists& lists, const unsigned char* mask) {
-  hipLaunchKernelGGL(clear_counts_kernel, dim3(1), dim3(64), 0, s, lists.count, kDensMaxS + 1);
+                        const int* item0, const DenseList& list, const unsigned char* mask) {
+  hipLaunchKernelGGL(clear_counts_kernel, dim3(1), dim3(64), 0, s, list.count, 1);
   if (nblocks <= 0) return;
   hipLaunchKernelGGL(list_masked_kernel, dim3((nblocks + 63) / 64), dim3(64), 0, s, blocks, nblocks, by_block, item0,
-                     cls, lists, mask);
+                     list, mask);
 }
 
 void launch_refresh_dense(hipStream_t s, const DevBlock* blocks, int nblocks, int64_t npts, const double* part,
@@ -1412,44 +1435,30 @@ void launch_functional_pol(hipStream_t s, int func, const XcParams& prm, int64_t
                      gwa, vsb, gwb, e_blk, ra2, ga2, rb2, gb2);
 }
 
-template <typename T, int S>
-static void launch_fock_sub_s(hipStream_t s, const FockItem* work, int nwork, const DevBlock* blocks,
-                              const int* ao_idx, const T* tiles, const double* vs, const double* gw, int gga,
-                              double thr, T* Tscr, int64_t npts, const PackSys* pack) {
-  hipLaunchKernelGGL((fock_sub_kernel<T, S>), dim3(nwork), dim3(64 * kFockWaves), 0, s, work, blocks, ao_idx, tiles,
-                     vs, gw, gga, thr, Tscr, npts, pack);
-}
-
 template <typename T>
-void launch_fock_sub(hipStream_t s, int sc, const FockItem* work, int nwork, const DevBlock* blocks,
-                     const int* ao_idx, const T* tiles, const double* vs, const double* gw, int gga, double thr,
-                     T* Tscr, int64_t npts, const PackSys* pack) {
+void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, const DevBlock* blocks, const T* tiles,
+                     const double* vs, const double* gw, int gga, double thr, T* Tscr, int64_t npts,
+                     const PackSys* pack) {
   if (nwork <= 0) return;
-  switch (kFockS[sc]) {
-#define SXC_FOCK_S(SV) \
-  case SV:             \
-    return launch_fock_sub_s<T, SV>(s, work, nwork, blocks, ao_idx, tiles, vs, gw, gga, thr, Tscr, npts, pack);
-    SXC_FOCK_S(1)
-    SXC_FOCK_S(2)
-    SXC_FOCK_S(3)
-    SXC_FOCK_S(4)
-    SXC_FOCK_S(5)
-#if SXC_FOCK_WAVES != 16
-    SXC_FOCK_S(6)
-    SXC_FOCK_S(7)
-    SXC_FOCK_S(8)
-    SXC_FOCK_S(10)
-#endif
-#undef SXC_FOCK_S
+#define SXC_FOCK_SHAPE(k)                                                                                          \
+  if (shape == k) {                                                                                                \
+    hipLaunchKernelGGL((fock_sub_kernel<T, kFockShape[k].waves, kFockShape[k].rows, kFockShape[k].slots>),         \
+                       dim3(nwork), dim3(64 * kFockShape[k].waves), 0, s, work, blocks, tiles, vs, gw, gga, thr,   \
+                       Tscr, npts, pack);                                                                          \
+    return;                                                                                                        \
   }
-  throw std::runtime_error("launch_fock_sub: slot class beyond the accumulator budget of this precision");
+  static_assert(kFockShapes == 4, "one case per shape");
+  SXC_FOCK_SHAPE(0)
+  SXC_FOCK_SHAPE(1)
+  SXC_FOCK_SHAPE(2)
+  SXC_FOCK_SHAPE(3)
+#undef SXC_FOCK_SHAPE
+  throw std::runtime_error("launch_fock_sub: unknown workgroup shape");
 }
-template void launch_fock_sub<double>(hipStream_t, int, const FockItem*, int, const DevBlock*, const int*,
-                                      const double*, const double*, const double*, int, double, double*, int64_t,
-                                      const PackSys*);
-template void launch_fock_sub<float>(hipStream_t, int, const FockItem*, int, const DevBlock*, const int*,
-                                     const float*, const double*, const double*, int, double, float*, int64_t,
-                                     const PackSys*);
+template void launch_fock_sub<double>(hipStream_t, int, const FockItem*, int, const DevBlock*, const double*,
+                                      const double*, const double*, int, double, double*, int64_t, const PackSys*);
+template void launch_fock_sub<float>(hipStream_t, int, const FockItem*, int, const DevBlock*, const float*,
+                                     const double*, const double*, int, double, float*, int64_t, const PackSys*);
 
 // Row columns per LDS pass of the reduce: kReduceWindow, or less where the device's LDS per
 // workgroup cannot hold that many columns of 8 bytes (fixed = false) or 16 bytes (fixed = true).

@@ -26,31 +26,37 @@ namespace {
 /* Work items of one block are consecutive in a list.  Workgroups of a launch are
  * dealt to the 8 XCDs round-robin (workgroup w runs on XCD w mod 8, from some
  * starting XCD), each with its own L2.  Cut the list into 8 contiguous ranges of
- * whole blocks (about a fair share of items each; the blocks are in grid order,
+ * whole blocks (about a fair share of the items' cost each; the blocks are in grid order,
  * so a range is a region of the molecule) and interleave them: one XCD runs a
  * block's items one after another, its re-reads of the block's tiles hit its L2,
  * and the density-matrix rows its region reads stay in that L2 too (density stage
  * at (H2O)64/def2-TZVP: 4.46 -> 4.36 ms FP32 against dealing blocks to the
  * shortest queue). */
-template <typename Item>
-void xcd_order(std::vector<Item>& v) {
+template <typename Item, typename Cost>
+void xcd_order(std::vector<Item>& v, Cost&& cost) {
   constexpr int kXcd = 8;
-  std::vector<std::vector<Item>> q(kXcd);
-  const size_t target = (v.size() + kXcd - 1) / kXcd;
-  size_t x = 0;
-  for (size_t i = 0; i < v.size();) {
-    size_t j = i;
-    while (j < v.size() && v[j].block == v[i].block) ++j;
-    if (q[x].size() >= target && x + 1 < q.size()) ++x;
-    q[x].insert(q[x].end(), v.begin() + i, v.begin() + j);
-    i = j;
+  double total = 0.0;
+  for (const Item& x : v) total += cost(x);
+  size_t begin[kXcd + 1] = {};
+  size_t i = 0;
+  double sum = 0.0;
+  for (int x = 0; x < kXcd; ++x) {
+    begin[x] = i;
+    const double end = total * (x + 1) / kXcd;
+    while (i < v.size() && (x + 1 == kXcd || sum < end)) {  // whole blocks
+      const int block = v[i].block;
+      for (; i < v.size() && v[i].block == block; ++i) sum += cost(v[i]);
+    }
   }
+  begin[kXcd] = v.size();
   size_t len = 0;
-  for (const auto& u : q) len = std::max(len, u.size());
-  v.clear();
+  for (int x = 0; x < kXcd; ++x) len = std::max(len, begin[x + 1] - begin[x]);
+  std::vector<Item> out;
+  out.reserve(v.size());
   for (size_t k = 0; k < len; ++k)
-    for (const auto& u : q)
-      if (k < u.size()) v.push_back(u[k]);
+    for (int x = 0; x < kXcd; ++x)
+      if (begin[x] + k < begin[x + 1]) out.push_back(v[begin[x] + k]);
+  v.swap(out);
 }
 
 thread_local std::string g_last_error;
@@ -298,8 +304,8 @@ struct DBuf {
 struct PackWork {
   DBuf<DevBlock> blocks;
   DBuf<PackSys> sys;
-  DBuf<WorkItem> dens[kDensMaxS + 1];
-  DBuf<FockItem> fock[kFockNumS];
+  DBuf<WorkItem> dens;
+  DBuf<FockItem> fock[kFockShapes];
   DBuf<double> round, E;
   hipGraphExec_t exec = nullptr;  // captured build of a repeated composition
   uint64_t last_use = 0;          // packed-build counter at its last use (least recently used is evicted)
@@ -470,23 +476,22 @@ struct xc_bfogc {
   DBuf<int> d_ao_idx, d_sig_shell, d_sig_pos;
   DBuf<double> d_t64;
   DBuf<float> d_t32;
-  // contraction work lists per size class
+  // contraction work lists
   int npass_max = 0;
-  std::vector<WorkItem> dens_work[kDensMaxS + 1];        // by column tiles per pass
-  std::vector<FockItem> fock_items[2][kFockNumS];       // sub-tile Fock kernel, [fp64][slot class]
-  DBuf<WorkItem> d_dens_work[kDensMaxS + 1];
-  // mixed precision: every block's density items contiguously (from dens_item0[b], class
-  // dens_cls[b]); the device lists of the dense blocks refined in FP64 and their counts; the
-  // FP32-rounded density matrix in FP64
+  std::vector<WorkItem> dens_work;
+  std::vector<FockItem> fock_items[kFockShapes];  // by workgroup shape
+  DBuf<WorkItem> d_dens_work;
+  // mixed precision: every block's density items contiguously (from dens_item0[b]); the device lists
+  // of the dense blocks refined in FP64 and their counts; the FP32-rounded density matrix in FP64
   std::vector<WorkItem> dens_by_block;
-  std::vector<int> dens_item0, dens_cls;
-  DBuf<WorkItem> d_dens_by_block, d_dense_list[kDensMaxS + 1], d_carry_list[kDensMaxS + 1];
-  DBuf<int> d_dens_item0, d_dens_cls, d_dense_cnt, d_carry_cnt;
+  std::vector<int> dens_item0;
+  DBuf<WorkItem> d_dens_by_block, d_dense_list, d_carry_list;
+  DBuf<int> d_dens_item0, d_dense_cnt, d_carry_cnt;
   // mixed precision: the blocks contracted in FP64 by the last mixed build that were still dense
   // (one byte per block); the next mixed build's FP32 pass skips them
   DBuf<unsigned char> d_dense_mask;
   DBuf<double> d_P32d;
-  DBuf<FockItem> d_fock_items[2][kFockNumS];
+  DBuf<FockItem> d_fock_items[kFockShapes];
   // per-build work buffers
   DBuf<double> d_part, d_rho, d_grad, d_vs, d_gw, d_eblk, d_U, d_P, d_F, d_v, d_g, d_E;
   // Fock sub-tile scratch (FP64 size when FP64 tiles are kept, else FP32) and the row entries of
@@ -538,53 +543,37 @@ void over_lanes(const Lanes& L, int nclass, const std::function<int(int)>& count
 
 template <typename T>
 void run_density(xc_bfogc* bf, const T* tiles, const T* P, int want_grad, const Lanes& L) {
-  over_lanes(L, kDensMaxS + 1, [&](int c) { return c >= 1 ? (int)bf->dens_work[c].size() : 0; },
-             [&](int c, hipStream_t s) {
-    launch_density_sub<T>(s, c, bf->d_dens_work[c].p, (int)bf->dens_work[c].size(), bf->d_blocks.p,
-                      bf->d_ao_idx.p, tiles, P, bf->basis->nao, want_grad, bf->d_part.p, bf->grid->npts);
-  });
+  launch_density_sub<T>(L.main, bf->d_dens_work.p, (int)bf->dens_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, tiles,
+                        P, bf->basis->nao, want_grad, bf->d_part.p, bf->grid->npts);
 }
 
 // Mixed precision: the FP32 density pass, and FP64 density items (FP64 tiles, the FP32-rounded P
 // in FP64) for the blocks whose largest density exceeds kMixedRhoThreshold.  The controller's mask
 // holds the blocks the last mixed build found dense: their FP64 items run beside the FP32 pass over
-// the other blocks (on the helper lanes its smaller classes leave free), then the blocks outside
+// the other blocks (on a helper lane), then the blocks outside
 // the mask that the FP32 pass finds dense get theirs, and the mask keeps the blocks whose FP64
 // density exceeds the threshold.  The lists are filled on the device, so those launches cover the
 // lists' capacity and run only the filled part.
 void run_density_mixed(xc_bfogc* bf, int want_grad, const Lanes& L) {
-  DenseLists carry{}, late{};
-  for (int c = 0; c <= kDensMaxS; ++c) {
-    carry.item[c] = bf->d_carry_list[c].p;
-    late.item[c] = bf->d_dense_list[c].p;
-  }
-  carry.count = bf->d_carry_cnt.p;
-  late.count = bf->d_dense_cnt.p;
-  const int n = bf->basis->nao;
+  const DenseList carry = {bf->d_carry_list.p, bf->d_carry_cnt.p}, late = {bf->d_dense_list.p, bf->d_dense_cnt.p};
+  const int n = bf->basis->nao, nwork = (int)bf->dens_work.size();
   const int64_t N = bf->grid->npts;
-  auto fp64_pass = [&](int c, hipStream_t s, const DenseLists& lists) {
-    launch_density_sub<double>(s, c, lists.item[c], (int)bf->dens_work[c].size(), bf->d_blocks.p, bf->d_ao_idx.p,
-                               bf->d_t64.p, bf->d_P32d.p, n, want_grad, bf->d_part.p, N, nullptr, lists.count + c);
+  auto fp64_pass = [&](hipStream_t s, const DenseList& list) {
+    launch_density_sub<double>(s, list.item, nwork, bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t64.p, bf->d_P32d.p, n,
+                               want_grad, bf->d_part.p, N, nullptr, list.count);
   };
-  launch_list_masked(L.main, bf->d_blocks.p, bf->nblocks, bf->d_dens_by_block.p, bf->d_dens_item0.p,
-                     bf->d_dens_cls.p, carry, bf->d_dense_mask.p);
-  const bool par = L.n > 1;
-  if (par) L.fork_all();
-  // FP32 classes from the widest on lanes 0, 1, ...; FP64 classes from the widest on the last
-  // lane backwards, behind the FP32 pass's smallest classes
-  int k = 0, kb = 0;
-  for (int c = kDensMaxS; c >= 1; --c)
-    if (!bf->dens_work[c].empty())
-      launch_density_sub<float>(par ? L.lane(k++) : L.main, c, bf->d_dens_work[c].p, (int)bf->dens_work[c].size(),
-                                bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t32.p, bf->d_P32.p, n, want_grad,
-                                bf->d_part.p, N, nullptr, nullptr, bf->d_dense_mask.p);
-  for (int c = kDensMaxS; c >= 1; --c)
-    if (!bf->dens_work[c].empty()) fp64_pass(c, par ? L.lane(L.n - 1 - kb++ % L.n) : L.main, carry);
-  if (par) L.join_all();
+  launch_list_masked(L.main, bf->d_blocks.p, bf->nblocks, bf->d_dens_by_block.p, bf->d_dens_item0.p, carry,
+                     bf->d_dense_mask.p);
+  over_lanes(L, 2, [&](int) { return nwork; }, [&](int c, hipStream_t s) {
+    if (c == 1)
+      launch_density_sub<float>(s, bf->d_dens_work.p, nwork, bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t32.p, bf->d_P32.p,
+                                n, want_grad, bf->d_part.p, N, nullptr, nullptr, bf->d_dense_mask.p);
+    else
+      fp64_pass(s, carry);
+  });
   launch_mark_dense(L.main, bf->d_blocks.p, bf->nblocks, N, bf->d_part.p, kMixedRhoThreshold, bf->d_dens_by_block.p,
-                    bf->d_dens_item0.p, bf->d_dens_cls.p, late, bf->d_dense_mask.p);
-  over_lanes(L, kDensMaxS + 1, [&](int c) { return c >= 1 ? (int)bf->dens_work[c].size() : 0; },
-             [&](int c, hipStream_t s) { fp64_pass(c, s, late); });
+                    bf->d_dens_item0.p, late, bf->d_dense_mask.p);
+  fp64_pass(L.main, late);
   launch_refresh_dense(L.main, bf->d_blocks.p, bf->nblocks, N, bf->d_part.p, kMixedRhoThreshold,
                        bf->d_dense_mask.p);
 }
@@ -607,13 +596,12 @@ void require_idle(const xc_bfogc* act, int nenv, xc_bfogc* const* env, const cha
 template <typename T>
 void run_fock_tiles(xc_bfogc* bf, const T* tiles, int gga, double thr, const Lanes& L, const double* vs = nullptr,
                     const double* gw = nullptr) {
-  const int f = sizeof(T) == 8 ? 1 : 0;
   if (!vs) vs = bf->d_vs.p;
   if (!gw) gw = bf->d_gw.p;
   T* Tscr = reinterpret_cast<T*>(bf->d_T.p);
-  over_lanes(L, kFockNumS, [&](int c) { return (int)bf->fock_items[f][c].size(); }, [&](int c, hipStream_t s) {
-    launch_fock_sub<T>(s, c, bf->d_fock_items[f][c].p, (int)bf->fock_items[f][c].size(),
-                       bf->d_blocks.p, bf->d_ao_idx.p, tiles, vs, gw, gga, thr, Tscr, bf->grid->npts);
+  over_lanes(L, kFockShapes, [&](int c) { return (int)bf->fock_items[c].size(); }, [&](int c, hipStream_t s) {
+    launch_fock_sub<T>(s, c, bf->d_fock_items[c].p, (int)bf->fock_items[c].size(), bf->d_blocks.p, tiles, vs, gw, gga,
+                       thr, Tscr, bf->grid->npts);
   });
 }
 
@@ -1113,7 +1101,6 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       std::vector<int> sig_shell, sig_pos;
       bf->blocks.resize(nb);
       bf->dens_item0.assign(nb, 0);
-      bf->dens_cls.assign(nb, 1);
       int64_t tile_off = 0;
       for (int b = 0; b < nb; ++b) {
         DevBlock& bk = bf->blocks[b];
@@ -1143,56 +1130,43 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
         bf->sum_B_nb2 += (double)bk.npts * cnt * cnt;
         bk.npass = 0;
         if (cnt > 0) {
+          // what is computed ends with the 16 columns of the last AO (the padding goes to 32)
+          const int nc = (cnt + 15) / 16 * 16;
           // density: balanced passes of at most 16 kDensMaxS columns, 16-column granularity
-          const int npass = (bk.npad + 16 * kDensMaxS - 1) / (16 * kDensMaxS);
-          const int width = ((bk.npad + npass - 1) / npass + 15) / 16 * 16;
+          const int npass = (nc + 16 * kDensMaxS - 1) / (16 * kDensMaxS);
+          const int width = ((nc + npass - 1) / npass + 15) / 16 * 16;
           int s = 0;
-          // every pass of a block in the class of the widest, so that they share a launch
           bf->dens_item0[b] = (int)bf->dens_by_block.size();
-          bf->dens_cls[b] = width / 16;
-          for (int c0 = 0; c0 < bk.npad; c0 += width, ++s) {
-            const int ncols = std::min(width, bk.npad - c0);
-            bf->dens_work[width / 16].push_back(WorkItem{b, c0, ncols, s});
-            bf->dens_by_block.push_back(WorkItem{b, c0, ncols, s});
-          }
+          for (int c0 = 0; c0 < nc; c0 += width, ++s)
+            bf->dens_by_block.push_back(WorkItem{b, c0, std::min(width, nc - c0), s});
           bk.npass = s;
           bf->npass_max = std::max(bf->npass_max, s);
-          // Fock: the whole upper triangle of 16 x 16 sub-tiles as one item where
-          // its accumulators fit, else pairs of 128-row panels
-          // (all items of a block in one slot class, the largest they need, so that they
-          // share a launch and can be ordered for L2 reuse)
-          for (int fp64 = 0; fp64 < 2; ++fp64) {
-            std::vector<FockItem> mine;
-            auto add = [&](int a0, int na, int b0, int nbr) {
-              const int ta = na / 16, tb = nbr / 16;
-              const int nsub = nbr == 0 ? ta * (ta + 1) / 2 : ta * tb;
-              mine.push_back(FockItem{b, a0, na, b0, nbr, nsub});
-            };
-            const int nt16 = bk.npad / 16;
-            if (bk.npad <= kFockRows && nt16 * (nt16 + 1) / 2 <= kFockWaves * fock_smax(fp64)) {
-              add(0, bk.npad, 0, 0);
-            } else {
-              const int np = (bk.npad + kFockPanel - 1) / kFockPanel;
-              for (int P = 0; P < np; ++P) {
-                const int a0 = P * kFockPanel, na = std::min(kFockPanel, bk.npad - a0);
-                add(a0, na, 0, 0);
-                for (int Q = P + 1; Q < np; ++Q) {
-                  const int b0 = Q * kFockPanel;
-                  add(a0, na, b0, std::min(kFockPanel, bk.npad - b0));
-                }
+          // Fock: the whole upper triangle of 16 x 16 sub-tiles as one item of the smallest workgroup
+          // shape that holds it, else pairs of 128-row panels
+          int shape = 0;
+          while (shape < kFockShapes && nc > kFockShape[shape].npad) ++shape;
+          auto add = [&](int k, int a0, int na, int b0, int nbr) {
+            const int ta = na / 16, tb = nbr / 16;
+            bf->fock_items[k].push_back(FockItem{b, a0, na, b0, nbr, nbr == 0 ? ta * (ta + 1) / 2 : ta * tb});
+          };
+          if (shape < kFockShapes) {
+            add(shape, 0, nc, 0, 0);
+          } else {
+            const int np = (nc + kFockPanel - 1) / kFockPanel;
+            for (int P = 0; P < np; ++P) {
+              const int a0 = P * kFockPanel, na = std::min(kFockPanel, nc - a0);
+              add(kFockPanelShape, a0, na, 0, 0);
+              for (int Q = P + 1; Q < np; ++Q) {
+                const int b0 = Q * kFockPanel;
+                add(kFockPanelShape, a0, na, b0, std::min(kFockPanel, nc - b0));
               }
             }
-            int nsub_max = 0;
-            for (const FockItem& it : mine) nsub_max = std::max(nsub_max, it.nsub);
-            int sc = 0;
-            while (kFockWaves * kFockS[sc] < nsub_max) ++sc;
-            for (const FockItem& it : mine) bf->fock_items[fp64][sc].push_back(it);
           }
         }
       }
-      for (int c = 0; c <= kDensMaxS; ++c) xcd_order(bf->dens_work[c]);
-      for (int f = 0; f < 2; ++f)
-        for (int c = 0; c < kFockNumS; ++c) xcd_order(bf->fock_items[f][c]);
+      bf->dens_work = bf->dens_by_block;
+      xcd_order(bf->dens_work, [&](const WorkItem& w) { return (double)w.b * bf->blocks[w.block].npad; });
+      for (auto& items : bf->fock_items) xcd_order(items, [](const FockItem& f) { return (double)f.nsub; });
       bf->tile_elems = tile_off;
       // row entries of the Fock reduce: for every AO, the blocks holding it (in block order) with
       // the position of its row in the scratch
@@ -1234,24 +1208,19 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       bf->d_ao_idx.upload(ctx, bf->ao_idx.data(), bf->ao_idx.size());
       bf->d_sig_shell.upload(ctx, sig_shell.data(), sig_shell.size());
       bf->d_sig_pos.upload(ctx, sig_pos.data(), sig_pos.size());
-      for (int c = 0; c <= kDensMaxS; ++c)
-        bf->d_dens_work[c].upload(ctx, bf->dens_work[c].data(), bf->dens_work[c].size());
+      bf->d_dens_work.upload(ctx, bf->dens_work.data(), bf->dens_work.size());
       if (keep_fp32 == 1) {  // both tile sets: the mixed-precision build is available
         bf->d_dens_by_block.upload(ctx, bf->dens_by_block.data(), bf->dens_by_block.size());
         bf->d_dens_item0.upload(ctx, bf->dens_item0.data(), bf->dens_item0.size());
-        bf->d_dens_cls.upload(ctx, bf->dens_cls.data(), bf->dens_cls.size());
-        for (int c = 1; c <= kDensMaxS; ++c) {
-          bf->d_dense_list[c].alloc(ctx, std::max<size_t>(bf->dens_work[c].size(), 1));
-          bf->d_carry_list[c].alloc(ctx, std::max<size_t>(bf->dens_work[c].size(), 1));
-        }
-        bf->d_dense_cnt.alloc(ctx, kDensMaxS + 1);
-        bf->d_carry_cnt.alloc(ctx, kDensMaxS + 1);
+        bf->d_dense_list.alloc(ctx, std::max<size_t>(bf->dens_work.size(), 1));
+        bf->d_carry_list.alloc(ctx, std::max<size_t>(bf->dens_work.size(), 1));
+        bf->d_dense_cnt.alloc(ctx, 1);
+        bf->d_carry_cnt.alloc(ctx, 1);
         bf->d_dense_mask.alloc(ctx, std::max(bf->nblocks, 1));
         HIPX(hipMemsetAsync(bf->d_dense_mask.p, 0, std::max(bf->nblocks, 1), ctx->stream));
       }
-      for (int f = 0; f < 2; ++f)
-        for (int c = 0; c < kFockNumS; ++c)
-          bf->d_fock_items[f][c].upload(ctx, bf->fock_items[f][c].data(), bf->fock_items[f][c].size());
+      for (int c = 0; c < kFockShapes; ++c)
+        bf->d_fock_items[c].upload(ctx, bf->fock_items[c].data(), bf->fock_items[c].size());
       const size_t nt_el = (size_t)std::max<int64_t>(tile_off, 1);
       if (keep_fp32 != 2) {
         bf->d_t64.alloc(ctx, nt_el);
@@ -2071,8 +2040,8 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
     const bool fp32 = precision == XC_PREC_FP32;
     std::vector<DevBlock> blocks;
     std::vector<PackSys> sys(nsys);
-    std::vector<WorkItem> dens[kDensMaxS + 1];
-    std::vector<FockItem> fock[kFockNumS];
+    std::vector<WorkItem> dens;
+    std::vector<FockItem> fock[kFockShapes];
     int64_t maxnn = 0;
     int maxn = 0;
     for (int i = 0; i < nsys; ++i) {
@@ -2092,13 +2061,12 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
         b.sys = i;
         blocks.push_back(b);
       }
-      for (int c = 1; c <= kDensMaxS; ++c)
-        for (WorkItem w : bf->dens_work[c]) {
-          w.block += blk0;
-          dens[c].push_back(w);
-        }
-      for (int c = 0; c < kFockNumS; ++c)
-        for (FockItem f : bf->fock_items[fp32 ? 0 : 1][c]) {
+      for (WorkItem w : bf->dens_work) {
+        w.block += blk0;
+        dens.push_back(w);
+      }
+      for (int c = 0; c < kFockShapes; ++c)
+        for (FockItem f : bf->fock_items[c]) {
           f.block += blk0;
           fock[c].push_back(f);
         }
@@ -2176,29 +2144,26 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       HIPX(hipGraphLaunch(pw.exec, s));
     } else {
       upload_grow(ctx, pw.blocks, blocks);
-      for (int c = 1; c <= kDensMaxS; ++c) upload_grow(ctx, pw.dens[c], dens[c]);
-      for (int c = 0; c < kFockNumS; ++c) upload_grow(ctx, pw.fock[c], fock[c]);
+      upload_grow(ctx, pw.dens, dens);
+      for (int c = 0; c < kFockShapes; ++c) upload_grow(ctx, pw.fock[c], fock[c]);
       const PackSys* dsys = pw.sys.p;
       // one launch per stage and work class for every system of the pack
       auto enqueue = [&]() {
         if (fp32) launch_pack_to_float(s, dsys, nsys, maxnn);
-        over_lanes(L, kDensMaxS + 1, [&](int c) { return c >= 1 ? (int)dens[c].size() : 0; },
-                   [&](int c, hipStream_t st) {
-          if (fp32)
-            launch_density_sub<float>(st, c, pw.dens[c].p, (int)dens[c].size(), pw.blocks.p, nullptr, nullptr,
-                                      nullptr, 0, g, nullptr, 0, dsys);
-          else
-            launch_density_sub<double>(st, c, pw.dens[c].p, (int)dens[c].size(), pw.blocks.p, nullptr, nullptr,
-                                       nullptr, 0, g, nullptr, 0, dsys);
-        });
+        if (fp32)
+          launch_density_sub<float>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
+                                    nullptr, 0, dsys);
+        else
+          launch_density_sub<double>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
+                                     nullptr, 0, dsys);
         launch_functional_packed(s, functional, ctx->prm, (int)blocks.size(), pw.blocks.p, dsys);
-        over_lanes(L, kFockNumS, [&](int c) { return (int)fock[c].size(); }, [&](int c, hipStream_t st) {
+        over_lanes(L, kFockShapes, [&](int c) { return (int)fock[c].size(); }, [&](int c, hipStream_t st) {
           if (fp32)
-            launch_fock_sub<float>(st, c, pw.fock[c].p, (int)fock[c].size(), pw.blocks.p, nullptr, nullptr,
-                                   nullptr, nullptr, g, thr, nullptr, 0, dsys);
+            launch_fock_sub<float>(st, c, pw.fock[c].p, (int)fock[c].size(), pw.blocks.p, nullptr, nullptr, nullptr, g,
+                                   thr, nullptr, 0, dsys);
           else
-            launch_fock_sub<double>(st, c, pw.fock[c].p, (int)fock[c].size(), pw.blocks.p, nullptr, nullptr,
-                                    nullptr, nullptr, g, thr, nullptr, 0, dsys);
+            launch_fock_sub<double>(st, c, pw.fock[c].p, (int)fock[c].size(), pw.blocks.p, nullptr, nullptr, nullptr, g,
+                                    thr, nullptr, 0, dsys);
         });
         if (fp32)
           launch_fock_reduce<float>(s, nullptr, nullptr, nullptr, nullptr, nullptr, maxn, dsys, nsys,
