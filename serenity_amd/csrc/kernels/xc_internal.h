@@ -192,12 +192,13 @@ constexpr int kDensMaxS = 6;
 constexpr double kMixedRhoThreshold = 2.0;
 constexpr int kDensIdxLds = 2048;  // AO index lists up to this length are staged in LDS
 // With nwork_dev, the launch covers a list filled on the device: only its first *nwork_dev
-// items run (nwork is the list's capacity).
+// items run (nwork is the list's capacity).  form (FP64, no gradient): P is the folded matrix of
+// launch_fold, and the density is its quadratic form.
 template <typename T>
 void launch_density_sub(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
                         const T* tiles, const T* P, int n, int want_grad, double* part, int64_t npts,
                         const PackSys* pack = nullptr, const int* nwork_dev = nullptr,
-                        const unsigned char* skip = nullptr);
+                        const unsigned char* skip = nullptr, bool form = false);
 
 // Dense-block refinement of the mixed-precision density: a work list and its device-side count, filled
 // by launch_mark_dense.
@@ -382,6 +383,8 @@ void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, 
                           double* rho, double* grad);
 // out[0] -= list.rho[i][0] for i in order.
 void launch_subtract_scalars(hipStream_t s, const DensityList& list, double* out);
+// Q[i, j] = P[i, j] + P[j, i], Q[i, i] = P[i, i] (packed: every system's P64 into its U, n the largest)
+void launch_fold(hipStream_t s, const double* P, double* Q, int n, const PackSys* pack = nullptr, int nsys = 1);
 void launch_to_float(hipStream_t s, const double* src, float* dst, int64_t n);
 // F[i + n j] (+)= U[max(i,j) + n min(i,j)] (U holds the lower triangle)
 // F = mirror of U (accumulate: F += it); with P32, part[b] = block b's sum of F (P - P32)

@@ -213,7 +213,7 @@ struct DensityArgs {
   int64_t npts;
 };
 
-template <typename T, int S>
+template <typename T, int S, bool Tri>
 __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock& bk, const DensityArgs<T>& arg,
                                              unsigned char* smem, int* sIdx) {
   using M = Mfma<T>;
@@ -281,7 +281,7 @@ __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock&
       }
     }
   };
-  auto store = [&]() {
+  auto store = [&]([[maybe_unused]] int k0) {
     *reinterpret_cast<vec_t*>(&sA[pa][KV * qa]) = rA;
 #pragma unroll
     for (int m = 0; m < NB; ++m) {
@@ -289,7 +289,10 @@ __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock&
       if (task < 4 * NC) {
         vec_t v = rB[m];
 #pragma unroll
-        for (int e = 0; e < KV; ++e) v[e] *= T(((mu_ok >> e) & 1u) && nu[m] >= 0);
+        for (int e = 0; e < KV; ++e) {
+          const bool ok = ((mu_ok >> e) & 1u) && nu[m] >= 0;
+          v[e] *= T(ok && (!Tri || k0 + KV * qb + e <= col0 + col_of(task)));
+        }
         *reinterpret_cast<vec_t*>(&sB[col_of(task)][KV * qb]) = v;
       }
     }
@@ -298,7 +301,8 @@ __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock&
   // dependent global load) in windows of kDensIdxLds entries: one window unless the block is
   // wider.  One LDS buffer; the global loads of chunk k + 1 of a window are in flight during the
   // MFMAs of chunk k.
-  const int kend = (bk.nb + KC - 1) / KC * KC;  // whole chunks: at most npad, whose last AOs are zero
+  // whole chunks: at most npad, whose last AOs are zero (Tri: up to the pass's last column)
+  const int kend = ((Tri ? min(bk.nb, col0 + ncols) : bk.nb) + KC - 1) / KC * KC;
   for (int wb = 0; wb < kend; wb += kDensIdxLds) {
     const int wl = min(kDensIdxLds, kend - wb);
     for (int i = tid; i < wl; i += 512) sIdx[i] = idx[wb + i];
@@ -306,7 +310,7 @@ __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock&
     const int nch = wl / KC;
     load(wb, 0);
     for (int ch = 0; ch < nch; ++ch) {
-      store();
+      store(wb + ch * KC);
       __syncthreads();
       if (ch + 1 < nch) load(wb + (ch + 1) * KC, (ch + 1) * KC);
       const vec_t av = *reinterpret_cast<const vec_t*>(&sA[16 * w + r][KV * g]);
@@ -438,7 +442,12 @@ __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock&
 // Every pass width in one kernel: a launch per width left each of them a tail of its own, and small
 // systems paid the launches and the stream forks more than the work ((H2O)8/def2-SVP: 108 us of
 // which the kernels ran 49).
-template <typename T>
+// Tri: the density alone (no gradient) is a quadratic form, rho = sum_nu phi_nu sum_(mu <= nu) phi_mu Q_mu,nu
+// with Q = P + P^T above the diagonal and P on it, so a pass contracts only the AOs up to its last
+// column: half the MFMAs and elements of P on average.  The caller passes Q (fold_kernel).  FP64
+// only (the other order of the sum moves FP32 densities by FP32 rounding), and for the builds: the
+// densities handed out or cached are the same bits with and without their gradient.
+template <typename T, bool Tri>
 __global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __restrict__ work,
                                                           const DevBlock* __restrict__ blocks, DensityArgs<T> arg,
                                                           const PackSys* __restrict__ pack,
@@ -462,12 +471,12 @@ __global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __rest
   }
   static_assert(kDensMaxS == 6, "one case per pass width");
   switch ((wk.b + 15) / 16) {
-    case 1: return density_item<T, 1>(wk, bk, arg, smem, sIdx);
-    case 2: return density_item<T, 2>(wk, bk, arg, smem, sIdx);
-    case 3: return density_item<T, 3>(wk, bk, arg, smem, sIdx);
-    case 4: return density_item<T, 4>(wk, bk, arg, smem, sIdx);
-    case 5: return density_item<T, 5>(wk, bk, arg, smem, sIdx);
-    default: return density_item<T, 6>(wk, bk, arg, smem, sIdx);
+    case 1: return density_item<T, 1, Tri>(wk, bk, arg, smem, sIdx);
+    case 2: return density_item<T, 2, Tri>(wk, bk, arg, smem, sIdx);
+    case 3: return density_item<T, 3, Tri>(wk, bk, arg, smem, sIdx);
+    case 4: return density_item<T, 4, Tri>(wk, bk, arg, smem, sIdx);
+    case 5: return density_item<T, 5, Tri>(wk, bk, arg, smem, sIdx);
+    default: return density_item<T, 6, Tri>(wk, bk, arg, smem, sIdx);
   }
 }
 
@@ -697,7 +706,9 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, XcParams 
 // One kernel per workgroup shape, with one slot count each: an item's wavefronts stop at the slots
 // they hold, so a shape's smaller items lose nothing but the registers of the widest (FP64 at 5
 // slots spills 4; one kernel of 5 slots for every wide item was 2 to 3 % slower at (H2O)64 and 32).
-template <typename T, int W, int Rows, int S>
+// One: without gradient terms both products of an element are the same sum phi_i (w v / 2) phi_j, so
+// FP64 takes one of them with w v (FP32 keeps both: its rounding would differ).
+template <typename T, int W, int Rows, int S, bool One>
 __global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __restrict__ work,
                                                        const DevBlock* __restrict__ blocks,
                                                        const T* __restrict__ tiles,
@@ -785,7 +796,7 @@ __global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __rest
     const double v1 = (in && gga) ? gwg[q] : 0.0;
     const double v2 = (in && gga) ? gwg[npts + q] : 0.0;
     const double v3 = (in && gga) ? gwg[2 * npts + q] : 0.0;
-    spot[0][tid] = (T)(0.5 * v0);
+    spot[0][tid] = (T)(One ? v0 : 0.5 * v0);
     spot[1][tid] = (T)v1;
     spot[2][tid] = (T)v2;
     spot[3][tid] = (T)v3;
@@ -880,13 +891,18 @@ __global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __rest
   const int slive = it.nsub > w ? (it.nsub - w + W - 1) / W : 0;
   auto slot = [&](int s, T(*sPhi)[RS], T(*sG)[RS]) {
     const vec_t aP = *reinterpret_cast<const vec_t*>(&sPhi[li[s] + r][KV * g]);
-    const vec_t aG = *reinterpret_cast<const vec_t*>(&sG[li[s] + r][KV * g]);
-    const vec_t bP = *reinterpret_cast<const vec_t*>(&sPhi[lj[s] + r][KV * g]);
     const vec_t bG = *reinterpret_cast<const vec_t*>(&sG[lj[s] + r][KV * g]);
+    if constexpr (One) {
 #pragma unroll
-    for (int t = 0; t < KV; ++t) acc[s] = M::step(aP[t], bG[t], acc[s]);
+      for (int t = 0; t < KV; ++t) acc[s] = M::step(aP[t], bG[t], acc[s]);
+    } else {
+      const vec_t aG = *reinterpret_cast<const vec_t*>(&sG[li[s] + r][KV * g]);
+      const vec_t bP = *reinterpret_cast<const vec_t*>(&sPhi[lj[s] + r][KV * g]);
 #pragma unroll
-    for (int t = 0; t < KV; ++t) acc[s] = M::step(aG[t], bP[t], acc[s]);
+      for (int t = 0; t < KV; ++t) acc[s] = M::step(aP[t], bG[t], acc[s]);
+#pragma unroll
+      for (int t = 0; t < KV; ++t) acc[s] = M::step(aG[t], bP[t], acc[s]);
+    }
   };
   if constexpr (sizeof(T) == 8) {
     static_assert((NCH & (NCH - 1)) == 0, "chunks per item: a power of two");
@@ -1146,6 +1162,31 @@ __global__ void fill_kernel(double* __restrict__ p, int64_t n, double value) {
   if (i < n) p[i] = value;
 }
 
+// Q = P + P^T, on the diagonal P, of one matrix or of every system of a pack (P64 into U).
+constexpr int kFoldTile = 32;
+__global__ __launch_bounds__(256) void fold_kernel(const double* __restrict__ P, double* __restrict__ Q, int n,
+                                                   const PackSys* __restrict__ pack) {
+  __shared__ double t[kFoldTile][kFoldTile + 1];
+  if (pack) {
+    const PackSys& ps = pack[blockIdx.z];
+    P = ps.P64;
+    Q = ps.U;
+    n = ps.n;
+  }
+  const int i0 = blockIdx.x * kFoldTile, j0 = blockIdx.y * kFoldTile, x = threadIdx.x & 31, y0 = threadIdx.x >> 5;
+  if (i0 >= n || j0 >= n) return;  // uniform over the workgroup
+  for (int y = y0; y < kFoldTile; y += 8)
+    t[y][x] = j0 + x < n && i0 + y < n ? P[(j0 + x) + (int64_t)n * (i0 + y)] : 0.0;
+  __syncthreads();
+  for (int y = y0; y < kFoldTile; y += 8) {
+    const int i = i0 + x, j = j0 + y;
+    if (i < n && j < n) {
+      const double p = P[i + (int64_t)n * j];
+      Q[i + (int64_t)n * j] = i == j ? p : p + t[x][y];
+    }
+  }
+}
+
 __global__ void to_float_kernel(const double* __restrict__ s, float* __restrict__ d, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) d[i] = (float)s[i];
@@ -1269,17 +1310,22 @@ void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, const in
 template <typename T>
 void launch_density_sub(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
                         const T* tiles, const T* P, int n, int want_grad, double* part, int64_t npts,
-                        const PackSys* pack, const int* nwork_dev, const unsigned char* skip) {
+                        const PackSys* pack, const int* nwork_dev, const unsigned char* skip, bool form) {
   if (nwork <= 0) return;
   const DensityArgs<T> arg = {ao_idx, tiles, P, n, want_grad, part, npts};
-  hipLaunchKernelGGL((density_sub_kernel<T>), dim3(nwork), dim3(512), 0, s, work, blocks, arg, pack, nwork_dev, skip);
+  if (sizeof(T) == 8 && form)
+    hipLaunchKernelGGL((density_sub_kernel<T, sizeof(T) == 8>), dim3(nwork), dim3(512), 0, s, work, blocks, arg, pack,
+                       nwork_dev, skip);
+  else
+    hipLaunchKernelGGL((density_sub_kernel<T, false>), dim3(nwork), dim3(512), 0, s, work, blocks, arg, pack, nwork_dev,
+                       skip);
 }
 template void launch_density_sub<double>(hipStream_t, const WorkItem*, int, const DevBlock*, const int*, const double*,
                                          const double*, int, int, double*, int64_t, const PackSys*, const int*,
-                                         const unsigned char*);
+                                         const unsigned char*, bool);
 template void launch_density_sub<float>(hipStream_t, const WorkItem*, int, const DevBlock*, const int*, const float*,
                                         const float*, int, int, double*, int64_t, const PackSys*, const int*,
-                                        const unsigned char*);
+                                        const unsigned char*, bool);
 
 // Largest density of block b (128 threads), from the partials of its passes.
 __device__ double block_max_density(const DevBlock& bk, int64_t npts, const double* __restrict__ part, double* red) {
@@ -1440,12 +1486,17 @@ void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, 
                      const double* vs, const double* gw, int gga, double thr, T* Tscr, int64_t npts,
                      const PackSys* pack) {
   if (nwork <= 0) return;
-#define SXC_FOCK_SHAPE(k)                                                                                          \
-  if (shape == k) {                                                                                                \
-    hipLaunchKernelGGL((fock_sub_kernel<T, kFockShape[k].waves, kFockShape[k].rows, kFockShape[k].slots>),         \
-                       dim3(nwork), dim3(64 * kFockShape[k].waves), 0, s, work, blocks, tiles, vs, gw, gga, thr,   \
-                       Tscr, npts, pack);                                                                          \
-    return;                                                                                                        \
+  constexpr bool f64 = sizeof(T) == 8;
+#define SXC_FOCK_SHAPE(k)                                                                                           \
+  if (shape == k) {                                                                                                 \
+    constexpr FockShape sh = kFockShape[k];                                                                         \
+    if (f64 && !gga)                                                                                                \
+      hipLaunchKernelGGL((fock_sub_kernel<T, sh.waves, sh.rows, sh.slots, f64>), dim3(nwork), dim3(64 * sh.waves), 0, \
+                         s, work, blocks, tiles, vs, gw, gga, thr, Tscr, npts, pack);                               \
+    else                                                                                                            \
+      hipLaunchKernelGGL((fock_sub_kernel<T, sh.waves, sh.rows, sh.slots, false>), dim3(nwork), dim3(64 * sh.waves), \
+                         0, s, work, blocks, tiles, vs, gw, gga, thr, Tscr, npts, pack);                            \
+    return;                                                                                                         \
   }
   static_assert(kFockShapes == 4, "one case per shape");
   SXC_FOCK_SHAPE(0)
@@ -1529,6 +1580,12 @@ void launch_copy(hipStream_t s, const void* src, void* dst, int64_t n32) {
 void launch_fill(hipStream_t s, double* p, int64_t n, double value) {
   if (n <= 0) return;
   hipLaunchKernelGGL(fill_kernel, dim3(grid1d(n, 256)), dim3(256), 0, s, p, n, value);
+}
+
+void launch_fold(hipStream_t s, const double* P, double* Q, int n, const PackSys* pack, int nsys) {
+  if (n <= 0 || nsys <= 0) return;
+  const unsigned g = grid1d(n, kFoldTile);
+  hipLaunchKernelGGL(fold_kernel, dim3(g, g, nsys), dim3(256), 0, s, P, Q, n, pack);
 }
 
 void launch_to_float(hipStream_t s, const double* src, float* dst, int64_t n) {

@@ -541,10 +541,15 @@ void over_lanes(const Lanes& L, int nclass, const std::function<int(int)>& count
   if (par) L.join_all();
 }
 
+// A density without its gradient as the quadratic form over half of the folded matrix: where a
+// block can have more than one column pass (a pass contracts everything up to its last column, so one
+// pass saves nothing and the fold's launch costs 4 us).
+bool use_form(bool gga, int n) { return !gga && n > 16 * kDensMaxS; }
+
 template <typename T>
-void run_density(xc_bfogc* bf, const T* tiles, const T* P, int want_grad, const Lanes& L) {
+void run_density(xc_bfogc* bf, const T* tiles, const T* P, int want_grad, const Lanes& L, bool form = false) {
   launch_density_sub<T>(L.main, bf->d_dens_work.p, (int)bf->dens_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, tiles,
-                        P, bf->basis->nao, want_grad, bf->d_part.p, bf->grid->npts);
+                        P, bf->basis->nao, want_grad, bf->d_part.p, bf->grid->npts, nullptr, nullptr, nullptr, form);
 }
 
 // Mixed precision: the FP32 density pass, and FP64 density items (FP64 tiles, the FP32-rounded P
@@ -1504,7 +1509,9 @@ static void enqueue_build(xc_bfogc* bf, int functional, int precision, double th
   if (mixed) launch_to_double(s, bf->d_P32.p, bf->d_P32d.p, (int64_t)n * n);
   if (s == ctx->stream) ctx->mark();
   if (!lowp) {
-    run_density<double>(bf, bf->d_t64.p, dP, gga ? 1 : 0, L);
+    const bool form = use_form(gga, n);  // U is free until the reduce
+    if (form) launch_fold(s, dP, bf->d_U.p, n);
+    run_density<double>(bf, bf->d_t64.p, form ? bf->d_U.p : dP, gga ? 1 : 0, L, form);
   } else {
     if (mixed)
       run_density_mixed(bf, gga ? 1 : 0, L);
@@ -1583,7 +1590,9 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
   float* P32[2] = {bf->d_P32.p, bf->d_P32b.p};
   for (int sp = 0; sp < 2; ++sp) {
     if (precision == XC_PREC_FP64) {
-      run_density<double>(bf, bf->d_t64.p, Ps[sp], gga ? 1 : 0, L);
+      const bool form = use_form(gga, n);
+      if (form) launch_fold(s, Ps[sp], bf->d_U.p, n);
+      run_density<double>(bf, bf->d_t64.p, form ? bf->d_U.p : Ps[sp], gga ? 1 : 0, L, form);
     } else {
       launch_to_float(s, Ps[sp], P32[sp], (int64_t)n * n);
       run_density<float>(bf, bf->d_t32.p, P32[sp], gga ? 1 : 0, L);
@@ -2072,7 +2081,6 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
         }
       PackSys& ps = sys[i];
       ps.tiles = fp32 ? (const void*)bf->d_t32.p : (const void*)bf->d_t64.p;
-      ps.P = fp32 ? (const void*)bf->d_P32.p : (const void*)dP[i];
       ps.P64 = dP[i];
       ps.P32 = fp32 ? bf->d_P32.p : nullptr;
       ps.ao_idx = bf->d_ao_idx.p;
@@ -2093,6 +2101,9 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       maxnn = std::max(maxnn, (int64_t)n * n);
       maxn = std::max(maxn, n);
     }
+    const bool form = !fp32 && use_form(gga, maxn);
+    for (int i = 0; i < nsys; ++i)
+      sys[i].P = fp32 ? (const void*)bfs[i]->d_P32.p : form ? (const void*)bfs[i]->d_U.p : (const void*)dP[i];
     // a composition seen once before runs as a captured graph; the first build is eager
     std::vector<uint64_t> key;
     for (int i = 0; i < nsys; ++i) key.push_back((uint64_t)(uintptr_t)bfs[i]);
@@ -2150,12 +2161,13 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       // one launch per stage and work class for every system of the pack
       auto enqueue = [&]() {
         if (fp32) launch_pack_to_float(s, dsys, nsys, maxnn);
+        if (form) launch_fold(s, nullptr, nullptr, maxn, dsys, nsys);
         if (fp32)
           launch_density_sub<float>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
                                     nullptr, 0, dsys);
         else
           launch_density_sub<double>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
-                                     nullptr, 0, dsys);
+                                     nullptr, 0, dsys, nullptr, nullptr, form);
         launch_functional_packed(s, functional, ctx->prm, (int)blocks.size(), pw.blocks.p, dsys);
         over_lanes(L, kFockShapes, [&](int c) { return (int)fock[c].size(); }, [&](int c, hipStream_t st) {
           if (fp32)

@@ -42,3 +42,33 @@ def test_every_block_width(ctx, atoms, functional):
             assert np.abs(G - F).max() < tol * scale, precision
             assert abs(pot.getEnergy() - E) < tol * max(1.0, abs(E)), precision
     bf._release()
+
+
+@pytest.mark.parametrize("atoms", [4, 20, 39])  # one, two and three column passes
+def test_density_form_of_any_matrix(ctx, atoms):
+    """Without gradient terms only the symmetric part of the matrix counts, alone and packed; the
+    antisymmetric part adds rounding of its size to rho (1e-12 of the oracle's scale is left to it)."""
+    Z, X = hydrogens(atoms)
+    b = xc.BasisController.from_file("DEF2-SVP", Z, X)
+    rng = np.random.default_rng(atoms)
+    grid = xc.GridController(rng.normal(0.0, 1.5, (700, 3)), rng.uniform(0.0, 0.05, 700))
+    C = rng.standard_normal((b.nao, 4)) / np.sqrt(b.nao)
+    P = C @ C.T
+    A = rng.standard_normal(P.shape) / b.nao
+    bf = xc.BasisFunctionOnGridController(ctx, b, grid, 128, 1e-9, 1)
+    pot = xc.FuncPotential(bf, "LDA", "FP64")
+    F, E, _, _ = O.fock_build(b, grid.points, grid.weights, P, "LDA")
+    G = pot.getMatrix(P + A - A.T)
+    scale = max(1.0, np.abs(F).max())
+    assert np.abs(G - F).max() < 1e-9 * scale and abs(pot.getEnergy() - E) < 1e-9 * max(1.0, abs(E))
+    n = b.nao
+    dP, dF = ctx.alloc(8 * n * n), ctx.alloc(8 * n * n)
+    ctx.upload(dP, np.asfortranarray(P + A - A.T).ravel(order="F"))
+    for _ in range(3):  # eager, captured, replayed
+        e = xc.fock_build_packed([pot], [dP], [dF])
+        H = np.zeros(n * n)
+        ctx.download(H, dF)
+        assert np.abs(H.reshape(n, n) - F).max() < 1e-9 * scale and abs(e[0] - E) < 1e-9 * max(1.0, abs(E))
+    ctx.free(dP)
+    ctx.free(dF)
+    bf._release()
