@@ -20,172 +20,240 @@ namespace sxc {
 
 namespace {
 
-// One workgroup of 4 wavefronts per (block, 64-column pass).  Wavefront w owns
-// points 32 w .. 32 w + 31 (two 16-row tiles) and all four 16-column tiles of
-// the pass: 2 x 4 accumulators of phi P and of G P.  The AO (K) dimension
-// streams through LDS in chunks of 16: phi and G point-major (G formed from the
-// value and gradient tiles on the way in), and the pass's 16 x 64 slice of P.
-__global__ __launch_bounds__(256) void gradient_kernel(const GradItem* __restrict__ work,
+// Sum over the 16 lanes of a lane group (rotations within the group).
+template <int Ctrl>
+__device__ __forceinline__ double row_rotate_add(double x) {
+  int2 w = __builtin_bit_cast(int2, x), o;
+  o.x = __builtin_amdgcn_update_dpp(0, w.x, Ctrl, 0xf, 0xf, false);
+  o.y = __builtin_amdgcn_update_dpp(0, w.y, Ctrl, 0xf, 0xf, false);
+  return x + __builtin_bit_cast(double, o);
+}
+__device__ __forceinline__ double row16_sum(double x) {
+  x = row_rotate_add<0x128>(x);  // row_ror:8
+  x = row_rotate_add<0x124>(x);
+  x = row_rotate_add<0x122>(x);
+  return row_rotate_add<0x121>(x);
+}
+
+constexpr int kGradKC = 16;                // AOs per chunk
+constexpr int kGradRS = kGradKC + 2;       // 144-byte LDS rows: the 16 rows of an operand read hit distinct banks
+constexpr int kGradRows = 2 * kTile + 16 * kDensMaxS;  // phi, G and P columns
+
+// One workgroup of 8 wavefronts per (block, pass of 16 S columns): wavefront w owns points 16 w ..
+// 16 w + 15 and the S column tiles of both phi P and G P.  What bounds it is the FP64 matrix
+// cores, 2 x 2 B n_b ncols operations per pass; one workgroup per compute unit (both products'
+// accumulators take 16 S registers a lane), so the AOs stream in chunks of 16 through two LDS
+// buffers with one barrier a chunk: the next chunk is loaded before the chunk's MFMAs and stored
+// after them, G formed from the value and gradient tiles on its way.  The accumulators are transposed
+// (rows: AO columns, columns: points), so that the column dots read 16 consecutive points of a
+// tile row.  At C8H18/def2-TZVP/PBE the kernel takes 1.00 ms (2.57 with 4 wavefronts per 64 columns,
+// one buffer and one element per LDS read); without its tile loads it would take 0.5 (timing only):
+// the ten planes of a block and the four staged again per pass come at about 4 TB/s.
+template <int S>
+__device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock& bk, const int* __restrict__ ao_idx,
+                                              const double* __restrict__ tiles, const double* __restrict__ P, int n,
+                                              const double* __restrict__ vs, const double* __restrict__ gw, int gga,
+                                              int64_t npts, double* __restrict__ acc,
+                                              double (*buf)[kGradRows][kGradRS], double (*spot)[kTile],
+                                              double (*red)[16 * kDensMaxS][3]) {
+  using M = Mfma<double>;
+  constexpr int KC = kGradKC, KV = KC / 4, NP = (16 * S + 31) / 32;
+  typedef double vec_t __attribute__((ext_vector_type(KV)));
+  const int col0 = wk.a, ncols = wk.b;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const gmem<const double>* tb = to_global(tiles + bk.tile_off);
+  const int64_t cs = (int64_t)bk.npad * kTile;
+  const gmem<const int>* idx = to_global(ao_idx + bk.idx_off);
+  const gmem<const double>* Pg = to_global(P);
+  // staging: point pa, AO quad qa of phi and G; P elements (AO tid % 16, columns tid / 16 + 32 m)
+  const int pa = tid & (kTile - 1), qa = tid >> 7, ka = tid & 15;
+  double vp = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
+  if (pa < bk.npts) {
+    const int64_t q = bk.first + pa;
+    vp = to_global(vs)[q];
+    if (gga) {
+      gx = to_global(gw)[q];
+      gy = to_global(gw)[npts + q];
+      gz = to_global(gw)[2 * npts + q];
+    }
+  }
+  if (tid < kTile) {
+    spot[0][tid] = gx;
+    spot[1][tid] = gy;
+    spot[2][tid] = gz;
+  }
+  int nu[NP];
+#pragma unroll
+  for (int m = 0; m < NP; ++m) {
+    const int c = (tid >> 4) + 32 * m;
+    nu[m] = c < ncols ? idx[col0 + c] : -1;
+  }
+  const int kend = (bk.nb + KC - 1) / KC * KC;  // whole chunks: at most npad, whose last AOs are zero
+  double ph[KV], dx[KV], dy[KV], dz[KV], rp[NP];
+#pragma unroll
+  for (int e = 0; e < KV; ++e) dx[e] = dy[e] = dz[e] = 0.0;
+  int mu = idx[ka], mu_now = mu;
+  auto load = [&](int k0) {
+    mu_now = mu;
+#pragma unroll
+    for (int m = 0; m < NP; ++m) rp[m] = Pg[max(mu, 0) + (int64_t)n * max(nu[m], 0)];
+    if (k0 + KC < kend) mu = idx[k0 + KC + ka];  // the next chunk's P addresses depend on no load of it
+#pragma unroll
+    for (int e = 0; e < KV; ++e) {
+      const int64_t o = (int64_t)(k0 + KV * qa + e) * kTile + pa;
+      ph[e] = tb[o];
+      if (gga) {
+        dx[e] = tb[cs + o];
+        dy[e] = tb[2 * cs + o];
+        dz[e] = tb[3 * cs + o];
+      }
+    }
+  };
+  auto store = [&](int b) {
+    vec_t f, h;
+#pragma unroll
+    for (int e = 0; e < KV; ++e) {
+      f[e] = ph[e];
+      h[e] = vp * ph[e] + gx * dx[e] + gy * dy[e] + gz * dz[e];
+    }
+    *reinterpret_cast<vec_t*>(&buf[b][pa][KV * qa]) = f;
+    *reinterpret_cast<vec_t*>(&buf[b][kTile + pa][KV * qa]) = h;
+#pragma unroll
+    for (int m = 0; m < NP; ++m) {
+      const int c = (tid >> 4) + 32 * m;
+      // padding read P[0][0]; a zero for it (a select at the load would wait for it there)
+      if (c < 16 * S) buf[b][2 * kTile + c][ka] = mu_now >= 0 && nu[m] >= 0 ? rp[m] : 0.0;
+    }
+  };
+  M::acc_t T[S], TG[S];
+#pragma unroll
+  for (int c = 0; c < S; ++c) {
+    T[c] = M::zero();
+    TG[c] = M::zero();
+  }
+  load(0);
+  store(0);
+  __syncthreads();
+  int b = 0;
+  for (int k0 = 0; k0 < kend; k0 += KC, b ^= 1) {
+    const bool more = k0 + KC < kend;
+    if (more) load(k0 + KC);
+    const vec_t af = *reinterpret_cast<const vec_t*>(&buf[b][16 * w + r][KV * g]);
+    const vec_t ag = *reinterpret_cast<const vec_t*>(&buf[b][kTile + 16 * w + r][KV * g]);
+#pragma unroll
+    for (int c = 0; c < S; ++c) {
+      const vec_t bv = *reinterpret_cast<const vec_t*>(&buf[b][2 * kTile + 16 * c + r][KV * g]);
+#pragma unroll
+      for (int t = 0; t < KV; ++t) {
+        T[c] = M::step(bv[t], af[t], T[c]);
+        TG[c] = M::step(bv[t], ag[t], TG[c]);
+      }
+    }
+    if (more) store(b ^ 1);
+    __syncthreads();
+  }
+
+  // column dots: lane (r, g) holds point 16 w + r of columns 16 c + g + 4 e
+  const int p = 16 * w + r;  // rows of points beyond the block are zero in the tiles
+  const double wx = spot[0][p], wy = spot[1][p], wz = spot[2][p];
+#pragma unroll
+  for (int c = 0; c < S; ++c) {
+    if (16 * c >= ncols) break;  // uniform
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int cl = 16 * c + g + 4 * e;
+      const gmem<const double>* row = tb + (int64_t)(col0 + cl) * kTile + p;
+      const double tg = TG[c][e];
+      double ax = tg * row[cs], ay = tg * row[2 * cs], az = tg * row[3 * cs];
+      if (gga) {
+        const double tv = T[c][e];
+        const double hxx = row[4 * cs], hxy = row[5 * cs], hxz = row[6 * cs];
+        const double hyy = row[7 * cs], hyz = row[8 * cs], hzz = row[9 * cs];
+        ax += tv * (wx * hxx + wy * hxy + wz * hxz);
+        ay += tv * (wx * hxy + wy * hyy + wz * hyz);
+        az += tv * (wx * hxz + wy * hyz + wz * hzz);
+      }
+      ax = row16_sum(ax);
+      ay = row16_sum(ay);
+      az = row16_sum(az);
+      if (r == 0) {
+        red[w][cl][0] = ax;
+        red[w][cl][1] = ay;
+        red[w][cl][2] = az;
+      }
+    }
+  }
+  __syncthreads();
+  if (tid < 3 * ncols) {
+    const int cl = tid / 3, c = tid - 3 * cl;
+    const int nucol = idx[col0 + cl];
+    if (nucol >= 0) {
+      double s = 0.0;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) s += red[v][cl][c];
+      atomicAdd(&acc[3 * (int64_t)nucol + c], s);
+    }
+  }
+}
+
+__global__ __launch_bounds__(512) void gradient_kernel(const WorkItem* __restrict__ work,
                                                        const DevBlock* __restrict__ blocks,
                                                        const int* __restrict__ ao_idx,
                                                        const double* __restrict__ tiles,
                                                        const double* __restrict__ P, int n,
                                                        const double* __restrict__ vs, const double* __restrict__ gw,
                                                        int gga, int64_t npts, double* __restrict__ acc) {
-  using M = Mfma<double>;
-  constexpr int KC = 16, RS = KC + 1, NC = 64, PR = NC + 1;
-  __shared__ double sPhi[kTile][RS];
-  __shared__ double sG[kTile][RS];
-  __shared__ double sP[KC][PR];
-  __shared__ double sRed[4][NC][3];
-  const GradItem it = work[blockIdx.x];
-  const DevBlock bk = blocks[it.block];
-  const int npad = bk.npad, col0 = it.col0;
-  const int ncols = min(NC, npad - col0);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r16 = lane & 15, g4 = lane >> 4;
-  const double* tb = tiles + bk.tile_off;
-  const int64_t cs = (int64_t)npad * kTile;
-  const int* idx = ao_idx + bk.idx_off;
-  // staging role: point sp, AO half sh (8 AOs of the chunk)
-  const int sp = tid & (kTile - 1), shf = tid >> 7;
-  const bool pin = sp < bk.npts;
-  const int64_t q = bk.first + sp;
-  const double vsp = pin ? vs[q] : 0.0;
-  const double gxp = (pin && gga) ? gw[q] : 0.0;
-  const double gyp = (pin && gga) ? gw[npts + q] : 0.0;
-  const double gzp = (pin && gga) ? gw[2 * npts + q] : 0.0;
-
-  M::acc_t T[2][4], TG[2][4];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      T[a][b] = M::zero();
-      TG[a][b] = M::zero();
-    }
-
-  for (int k0 = 0; k0 < npad; k0 += KC) {
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int kk = shf * 8 + j;
-      const int64_t o = (int64_t)(k0 + kk) * kTile + sp;
-      const double phi = tb[o];
-      double g = vsp * phi;
-      if (gga) g += gxp * tb[cs + o] + gyp * tb[2 * cs + o] + gzp * tb[3 * cs + o];
-      sPhi[sp][kk] = phi;
-      sG[sp][kk] = g;
-    }
-    for (int e = tid; e < KC * NC; e += 256) {
-      const int kk = e & (KC - 1), c = e >> 4;
-      const int mu = idx[k0 + kk];
-      const int nu = c < ncols ? idx[col0 + c] : -1;
-      sP[kk][c] = (mu >= 0 && nu >= 0) ? P[mu + (int64_t)n * nu] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < KC / 4; ++t) {
-      const int k = 4 * t + g4;
-      double ap[2], ag[2], bp[4];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        ap[a] = sPhi[32 * wv + 16 * a + r16][k];
-        ag[a] = sG[32 * wv + 16 * a + r16][k];
-      }
-#pragma unroll
-      for (int b = 0; b < 4; ++b) bp[b] = sP[k][16 * b + r16];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          T[a][b] = M::step(ap[a], bp[b], T[a][b]);
-          TG[a][b] = M::step(ag[a], bp[b], TG[a][b]);
-        }
-    }
+  __shared__ __attribute__((aligned(16))) double buf[2][kGradRows][kGradRS];
+  __shared__ double spot[3][kTile];
+  __shared__ double red[8][16 * kDensMaxS][3];
+  const WorkItem wk = work[blockIdx.x];
+  const DevBlock bk = blocks[wk.block];
+  static_assert(kDensMaxS == 6 && 3 * 16 * kDensMaxS <= 512, "one case per pass width");
+#define SXC_GRAD(S_) \
+  case S_:           \
+    return gradient_item<S_>(wk, bk, ao_idx, tiles, P, n, vs, gw, gga, npts, acc, buf, spot, red);
+  switch ((wk.b + 15) / 16) {
+    SXC_GRAD(1)
+    SXC_GRAD(2)
+    SXC_GRAD(3)
+    SXC_GRAD(4)
+    SXC_GRAD(5)
+    SXC_GRAD(6)
   }
-
-  // column dots: lane (r16, g4) holds column 16 b + r16, rows 16 a + g4 + 4 r of the wavefront
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int cl = 16 * b + r16;  // column within the pass
-    const int i = col0 + cl;      // compact AO index
-    double ax = 0.0, ay = 0.0, az = 0.0;
-    if (cl < ncols) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int p = 32 * wv + 16 * a + g4 + 4 * r;
-          if (p >= bk.npts) continue;
-          const int64_t o = (int64_t)i * kTile + p;
-          const double tg = TG[a][b][r], tv = T[a][b][r];
-          const double dx = tb[cs + o], dy = tb[2 * cs + o], dz = tb[3 * cs + o];
-          ax += tg * dx;
-          ay += tg * dy;
-          az += tg * dz;
-          if (gga) {
-            const int64_t qp = bk.first + p;
-            const double wx = gw[qp], wy = gw[npts + qp], wz = gw[2 * npts + qp];
-            const double hxx = tb[4 * cs + o], hxy = tb[5 * cs + o], hxz = tb[6 * cs + o];
-            const double hyy = tb[7 * cs + o], hyz = tb[8 * cs + o], hzz = tb[9 * cs + o];
-            ax += tv * (wx * hxx + wy * hxy + wz * hxz);
-            ay += tv * (wx * hxy + wy * hyy + wz * hyz);
-            az += tv * (wx * hxz + wy * hyz + wz * hzz);
-          }
-        }
-    }
-    // the four lane groups hold the same column
-    ax += __shfl_xor(ax, 16);
-    ay += __shfl_xor(ay, 16);
-    az += __shfl_xor(az, 16);
-    ax += __shfl_xor(ax, 32);
-    ay += __shfl_xor(ay, 32);
-    az += __shfl_xor(az, 32);
-    if (g4 == 0) {
-      sRed[wv][cl][0] = ax;
-      sRed[wv][cl][1] = ay;
-      sRed[wv][cl][2] = az;
-    }
-  }
-  __syncthreads();
-  if (tid < 3 * ncols) {
-    const int cl = tid / 3, c = tid - 3 * cl;
-    const int mu = idx[col0 + cl];
-    if (mu >= 0) {
-      const double s = sRed[0][cl][c] + sRed[1][cl][c] + sRed[2][cl][c] + sRed[3][cl][c];
-      atomicAdd(&acc[3 * (int64_t)mu + c], s);
-    }
-  }
+#undef SXC_GRAD
 }
 
-// grad[A + natoms c] = -2 sum_{nu : atom(nu) = A} acc[nu][c], AOs in order.
-__global__ void gradient_atoms_kernel(const double* __restrict__ acc, const int* __restrict__ ao_atom, int n,
-                                      int natoms, double* __restrict__ grad) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 3 * natoms) return;
-  const int A = t % natoms, c = t / natoms;
-  double s = 0.0;
-  for (int nu = 0; nu < n; ++nu)
-    if (ao_atom[nu] == A) s += acc[3 * (int64_t)nu + c];
-  grad[t] = -2.0 * s;
+// grad[A + natoms c] = -2 sum_{nu : atom(nu) = A} acc[nu][c]: one wavefront per atom, each lane its
+// AOs in order, the lanes in a fixed tree.
+__global__ __launch_bounds__(64) void gradient_atoms_kernel(const double* __restrict__ acc,
+                                                            const int* __restrict__ ao_atom, int n, int natoms,
+                                                            double* __restrict__ grad) {
+  const int A = blockIdx.x;
+  double s[3] = {0.0, 0.0, 0.0};
+  for (int nu = threadIdx.x; nu < n; nu += 64)
+    if (ao_atom[nu] == A)
+      for (int c = 0; c < 3; ++c) s[c] += acc[3 * (int64_t)nu + c];
+  for (int c = 0; c < 3; ++c) {
+    for (int m = 1; m < 64; m <<= 1) s[c] += __shfl_xor(s[c], m);
+    if (threadIdx.x == 0) grad[A + natoms * c] = -2.0 * s[c];
+  }
 }
 
 }  // namespace
 
-void launch_gradient(hipStream_t s, const GradItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
+void launch_gradient(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
                      const double* tiles, const double* P, int n, const double* vs, const double* gw, int gga,
                      int64_t npts, double* acc) {
   if (nwork <= 0) return;
-  hipLaunchKernelGGL(gradient_kernel, dim3(nwork), dim3(256), 0, s, work, blocks, ao_idx, tiles, P, n, vs, gw, gga,
+  hipLaunchKernelGGL(gradient_kernel, dim3(nwork), dim3(512), 0, s, work, blocks, ao_idx, tiles, P, n, vs, gw, gga,
                      npts, acc);
 }
 
 void launch_gradient_atoms(hipStream_t s, const double* acc, const int* ao_atom, int n, int natoms, double* grad) {
-  const int nt = 3 * natoms;
-  if (nt <= 0) return;
-  hipLaunchKernelGGL(gradient_atoms_kernel, dim3((nt + 127) / 128), dim3(128), 0, s, acc, ao_atom, n, natoms, grad);
+  if (natoms <= 0) return;
+  hipLaunchKernelGGL(gradient_atoms_kernel, dim3(natoms), dim3(64), 0, s, acc, ao_atom, n, natoms, grad);
 }
 
 }  // namespace sxc

@@ -272,14 +272,10 @@ void launch_pack_to_float(hipStream_t s, const PackSys* pack, int nsys, int64_t 
 void launch_pack_finalize(hipStream_t s, const PackSys* pack, int nsys, int fp32);
 void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int fp32);
 
-// Work item of the gradient kernel: the block's AO columns [col0, col0 + 64).
-struct GradItem {
-  int block, col0;
-};
-constexpr int kGradCols = 64;
-// a[nu][c] += sum over the item's points of (G P)_p,nu d_c phi_nu + (phi P)_p,nu H^c_nu
-// (kernels/gradient_kernels.hip); tiles need 4 planes (LDA) or 10 (GGA).
-void launch_gradient(hipStream_t s, const GradItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
+// a[nu][c] += sum over the points of a density work item's block of (G P)_p,nu d_c phi_nu +
+// (phi P)_p,nu H^c_nu for the item's columns nu (kernels/gradient_kernels.hip); tiles need 4 planes
+// (LDA) or 10 (GGA).
+void launch_gradient(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
                      const double* tiles, const double* P, int n, const double* vs, const double* gw, int gga,
                      int64_t npts, double* acc);
 // grad[A + natoms c] = -2 sum_{nu on A} acc[nu][c].

@@ -507,9 +507,7 @@ struct xc_bfogc {
   // cached grid density (xc_bfogc_update_density) and the energies of it per functional
   DBuf<double> d_rho_c, d_grad_c, d_ecache;
   bool rho_c_valid = false, rho_c_grad = false;
-  // nuclear gradient (allocated on first use): work items, per-AO partials, atom map, result
-  std::vector<GradItem> grad_work;
-  DBuf<GradItem> d_grad_work;
+  // nuclear gradient (allocated on first use): per-AO partials, atom map, result
   DBuf<double> d_gacc, d_gout;
   DBuf<int> d_ao_atom;
   // unrestricted builds (allocated on first use): beta density, potential, P and F
@@ -2235,10 +2233,7 @@ void geom_gradient(xc_bfogc* bf, int functional, const double* Pa, const double*
   const int nxc = (int)((N + kTile - 1) / kTile);
   for (int i = 0; i < n; ++i)
     require(ao_atom[i] >= 0 && ao_atom[i] < natoms, XC_ERR_INPUT, "xc_geom_gradient: AO atom index out of range");
-  if (bf->grad_work.empty()) {
-    for (int b = 0; b < bf->nblocks; ++b)
-      for (int c0 = 0; c0 < bf->blocks[b].npad; c0 += kGradCols) bf->grad_work.push_back(GradItem{b, c0});
-    if (!bf->grad_work.empty()) bf->d_grad_work.upload(ctx, bf->grad_work.data(), bf->grad_work.size());
+  if (!bf->d_gacc.p) {
     bf->d_gacc.alloc(ctx, (size_t)3 * std::max(n, 1));
     bf->d_ao_atom.alloc(ctx, (size_t)std::max(n, 1));
   }
@@ -2272,10 +2267,10 @@ void geom_gradient(xc_bfogc* bf, int functional, const double* Pa, const double*
   }
   launch_fill(s, bf->d_gacc.p, (int64_t)3 * n, 0.0);
   // restricted: -2 P_mu,nu with the total-density potential; unrestricted: the same per spin
-  launch_gradient(s, bf->d_grad_work.p, (int)bf->grad_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t64.p,
+  launch_gradient(s, bf->d_dens_work.p, (int)bf->dens_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t64.p,
                   bf->d_P.p, n, bf->d_vs.p, bf->d_gw.p, gga ? 1 : 0, N, bf->d_gacc.p);
   if (Pb)
-    launch_gradient(s, bf->d_grad_work.p, (int)bf->grad_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t64.p,
+    launch_gradient(s, bf->d_dens_work.p, (int)bf->dens_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t64.p,
                     bf->d_Pb.p, n, bf->d_vs_b.p, bf->d_gw_b.p, gga ? 1 : 0, N, bf->d_gacc.p);
   launch_gradient_atoms(s, bf->d_gacc.p, bf->d_ao_atom.p, n, natoms, bf->d_gout.p);
   launch_sum(s, bf->d_eblk.p, nxc, ctx->d_energy);

@@ -72,3 +72,22 @@ def test_density_form_of_any_matrix(ctx, atoms):
     ctx.free(dP)
     ctx.free(dF)
     bf._release()
+
+
+@pytest.mark.parametrize("functional", ["LDA", "PBE"])
+@pytest.mark.parametrize("atoms", [3, 4, 13, 19, 20, 39])
+def test_gradient_at_every_pass_width(ctx, atoms, functional):
+    """15 to 195 AOs a block: one to three column passes, even and odd sub-tile counts."""
+    Z, X = hydrogens(atoms)
+    b = xc.BasisController.from_file("DEF2-SVP", Z, X)
+    rng = np.random.default_rng(atoms)
+    grid = xc.GridController(rng.normal(0.0, 1.5, (700, 3)), rng.uniform(0.0, 0.05, 700))
+    C = rng.standard_normal((b.nao, 4)) / np.sqrt(b.nao)
+    P = C @ C.T
+    G, E = O.xc_gradient(b, grid.points, grid.weights, P, functional, b.getAtomIndicesOfBasis(), atoms)
+    bf = xc.BasisFunctionOnGridController(ctx, b, grid, 128, 1e-9, 2)
+    pot = xc.FuncPotential(bf, functional, "FP64")
+    for _ in range(2):
+        assert np.abs(pot.getGeomGradients(P) - G).max() < 1e-9 * max(1.0, np.abs(G).max())
+        assert abs(pot.getEnergy() - E) < 1e-9 * max(1.0, abs(E))
+    bf._release()
