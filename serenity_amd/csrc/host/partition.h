@@ -24,6 +24,23 @@ SXC_PART_HD inline double part_dist(const double* a, const double* b) {
   return sqrt(dx * dx + dy * dy + dz * dz);
 }
 
+SXC_PART_HD inline double part_dist2(const double* a, const double* b) {
+#pragma clang fp contract(off)
+  const double dx = a[0] - b[0], dy = a[1] - b[1], dz = a[2] - b[2];
+  return dx * dx + dy * dy + dz * dz;
+}
+
+// (ra - rj) / d certainly below 0.64, or certainly above it, from rj^2
+constexpr double kPartOver = 0.64 + 1e-9, kPartUnder = 0.64 - 1e-9;
+SXC_PART_HD inline bool part_below(double ra, double d, double rj2) {
+  const double t = ra - kPartUnder * d;
+  return t < 0.0 || rj2 > t * t * (1.0 + 1e-9);
+}
+SXC_PART_HD inline bool part_above(double ra, double d, double rj2) {
+  const double t = ra - kPartOver * d;
+  return t > 0.0 && rj2 < t * t * (1.0 - 1e-9);
+}
+
 // Becke's cell function s(nu) = (1 - p_k(nu)) / 2, p_k = p applied k times,
 // p(nu) = (3 - nu^2) nu / 2 (applied once for k <= 1).
 SXC_PART_HD inline double becke_cell(double nu, unsigned k) {
@@ -70,18 +87,28 @@ SXC_PART_HD inline double partition_weight(int type, unsigned smoothing, int n, 
       }
     }
   } else {
+    // Most of the n^2 quotients nu = (ra - rj) / dist only need their side of +-0.64.  That is decided
+    // without the root of rj and the division where rj^2 is clearly on one side (margins of 1e-9, far
+    // above the rounding of nu); the others take the quotient itself, so the result is the same bit
+    // for bit.  A cell that the point's own atom k makes zero is skipped before its loop.
     const double rk = part_dist(xyz + 3 * k, gp);
     if (rk >= 0.5 * (1.0 - 0.64) * min_dist_k) {
       for (int j = 0; j < n; ++j) {
-        const double nu = (rk - part_dist(xyz + 3 * j, gp)) / dist[k + (size_t)n * j];
+        const double d = dist[k + (size_t)n * j], r2 = part_dist2(xyz + 3 * j, gp);
+        if (part_below(rk, d, r2)) continue;
+        const double nu = (rk - sqrt(r2)) / d;
         if (nu >= 0.64) return -1.0;
       }
       for (int a = 0; a < n; ++a) {
         const double ra = part_dist(xyz + 3 * a, gp);
+        if (a != k && part_above(ra, dist[a + (size_t)n * k], part_dist2(xyz + 3 * k, gp))) continue;  // cell = 0
         double cell = 1.0;
         for (int j = 0; j < n; ++j) {
           if (a == j) continue;
-          double nu = (ra - part_dist(xyz + 3 * j, gp)) / dist[a + (size_t)n * j];
+          const double d = dist[a + (size_t)n * j], r2 = part_dist2(xyz + 3 * j, gp);
+          const double far = ra + kPartOver * d;
+          if (r2 > far * far * (1.0 + 1e-9)) continue;  // nu < -0.64
+          double nu = (ra - sqrt(r2)) / d;
           if (nu <= -0.64) continue;
           if (nu >= 0.64) {
             cell = 0.0;

@@ -127,16 +127,20 @@ __global__ __launch_bounds__(256) void bbox_partial_kernel(const double* __restr
   if (t < 6) part[6 * blockIdx.x + t] = red[t][0];
 }
 
-// one thread: the box from the partials, then mn and spread = length / (hi - lo) as the host sort
-__global__ void bbox_final_kernel(const double* __restrict__ part, int nparts, int64_t length,
-                                  double* __restrict__ box) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// one wavefront: the box from the partials, then mn and spread = length / (hi - lo) as the host sort
+__global__ __launch_bounds__(64) void bbox_final_kernel(const double* __restrict__ part, int nparts, int64_t length,
+                                                        double* __restrict__ box) {
   for (int d = 0; d < 3; ++d) {
     double lo = HUGE_VAL, hi = -HUGE_VAL;
-    for (int b = 0; b < nparts; ++b) {
+    for (int b = threadIdx.x; b < nparts; b += 64) {
       lo = fmin(lo, part[6 * b + d]);
       hi = fmax(hi, part[6 * b + 3 + d]);
     }
+    for (int m = 1; m < 64; m <<= 1) {
+      lo = fmin(lo, __shfl_xor(lo, m));
+      hi = fmax(hi, __shfl_xor(hi, m));
+    }
+    if (threadIdx.x != 0) continue;
     box[d] = lo;
     box[3 + d] = double(length) / (hi - lo);
   }

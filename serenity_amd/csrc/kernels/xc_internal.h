@@ -175,10 +175,20 @@ struct WorkItem {
 };
 
 // ---- launchers (xc_kernels.hip) -------------------------------------------
+// pos[b nshell + s]: compact position of shell s in block b, -1 where it is negligible; count[2 b],
+// count[2 b + 1]: the block's AOs and significant shells.
 void launch_screen(hipStream_t s, const double* pts, int64_t npts, int bs, int nblocks, const DevShell* shells,
-                   int nshell, const double* alpha, const double* coef, double radial_thr, unsigned char* flags);
+                   int nshell, const double* alpha, const double* coef, double radial_thr, int* pos, int* count);
+// The blocks' lists (from DevBlock's offsets) and the row entries of the reduce; cnt: scratch of
+// row_chunks(nblocks) x nshell.
+int row_chunks(int nblocks);
+void launch_block_lists(hipStream_t s, const DevBlock* blocks, int nblocks, const DevShell* shells, int nshell, int nao,
+                        const int* pos, int* sig_shell, int* sig_pos, int* ao_idx, int* cnt, int* row_ptr,
+                        RowEnt* ent);
 
-void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, const int* sig_shell, const int* sig_pos,
+// max_nshell: the most significant shells of any block
+void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, int max_nshell, const int* sig_shell,
+                    const int* sig_pos,
                     const DevShell* shells, const double* alpha, const double* coef, const double* ang,
                     const double* pts, double radial_thr, double exp_thr, int ncomp, double* tiles64, float* tiles32);
 

@@ -28,50 +28,162 @@ __global__ __launch_bounds__(64) void screen_kernel(const double* __restrict__ p
                                                     const DevShell* __restrict__ shells, int nshell,
                                                     const double* __restrict__ alpha,
                                                     const double* __restrict__ coef, double thr,
-                                                    unsigned char* __restrict__ flags) {
-  __shared__ double c[4];
-  const int b = blockIdx.x;
+                                                    int* __restrict__ pos, int* __restrict__ count) {
+  __shared__ double c[4], xyz[3 * kTile];
+  const int b = blockIdx.x, t = threadIdx.x;
   const int64_t first = (int64_t)b * bs;
   const int B = (int)min((int64_t)bs, npts - first);
-  if (threadIdx.x == 0) {
-    // block centre (mean) and spread (largest distance to the centre),
-    // accumulated point by point in order
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    for (int p = 0; p < B; ++p) {
-      sx += pts[3 * (first + p) + 0];
-      sy += pts[3 * (first + p) + 1];
-      sz += pts[3 * (first + p) + 2];
-    }
-    const double cx = sx / B, cy = sy / B, cz = sz / B;
-    double sp = 0.0;
-    for (int p = 0; p < B; ++p) {
-      const double dx = pts[3 * (first + p) + 0] - cx;
-      const double dy = pts[3 * (first + p) + 1] - cy;
-      const double dz = pts[3 * (first + p) + 2] - cz;
-      sp = fmax(sp, sqrt(dx * dx + dy * dy + dz * dz));
-    }
-    c[0] = cx;
-    c[1] = cy;
-    c[2] = cz;
-    c[3] = sp;
+  for (int i = t; i < 3 * B; i += 64) xyz[i] = pts[3 * first + i];
+  __syncthreads();
+  // block centre (mean), accumulated point by point in order, one lane per coordinate; spread
+  // (largest distance to the centre)
+  if (t < 3) {
+    double s = 0.0;
+    for (int p = 0; p < B; ++p) s += xyz[3 * p + t];
+    c[t] = s / B;
   }
   __syncthreads();
-  for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
-    const DevShell sh = shells[s];
-    const double dx = c[0] - sh.cx, dy = c[1] - sh.cy, dz = c[2] - sh.cz;
-    double d = sqrt(dx * dx + dy * dy + dz * dz) - c[3];
-    unsigned char significant = 1;
-    if (!(d < 1.0)) {
-      // radial part at the closest possible distance of any block point
-      d = d * d;
-      double radial = 0.0;
-      for (int q = 0; q < sh.nprim; ++q) radial += coef[sh.prim_off + q] * exp(-alpha[sh.prim_off + q] * d);
-      if (fabs(radial) < thr) significant = 0;
+  double sp = 0.0;
+  for (int p = t; p < B; p += 64) {
+    const double dx = xyz[3 * p] - c[0], dy = xyz[3 * p + 1] - c[1], dz = xyz[3 * p + 2] - c[2];
+    sp = fmax(sp, sqrt(dx * dx + dy * dy + dz * dz));
+  }
+  for (int m = 1; m < 64; m <<= 1) sp = fmax(sp, __shfl_xor(sp, m));
+  if (t == 0) c[3] = sp;
+  __syncthreads();
+  // 64 shells at a time; a significant shell's compact position is the functions of those before it
+  int nao = 0, nsig = 0;
+  for (int s0 = 0; s0 < nshell; s0 += 64) {
+    const int s = s0 + t;
+    int nf = 0;
+    if (s < nshell) {
+      const DevShell sh = shells[s];
+      const double dx = c[0] - sh.cx, dy = c[1] - sh.cy, dz = c[2] - sh.cz;
+      double d = sqrt(dx * dx + dy * dy + dz * dz) - c[3];
+      nf = sh.nfunc;
+      if (!(d < 1.0)) {
+        // radial part at the closest possible distance of any block point
+        d = d * d;
+        double radial = 0.0;
+        for (int q = 0; q < sh.nprim; ++q) radial += coef[sh.prim_off + q] * exp(-alpha[sh.prim_off + q] * d);
+        if (fabs(radial) < thr) nf = 0;
+      }
     }
-    flags[(int64_t)b * nshell + s] = significant;
+    int sum = nf;  // inclusive prefix over the lanes
+    for (int m = 1; m < 64; m <<= 1) {
+      const int v = __shfl_up(sum, m);
+      if (t >= m) sum += v;
+    }
+    if (s < nshell) pos[(int64_t)b * nshell + s] = nf > 0 ? nao + sum - nf : -1;
+    nao += __shfl(sum, 63);
+    nsig += __popcll(__ballot(nf > 0));
+  }
+  if (t == 0) {
+    count[2 * b] = nao;
+    count[2 * b + 1] = nsig;
   }
 }
 
+// The lists of the blocks from their shells' compact positions: significant shells with their
+// positions, and the AO index list padded with -1.
+__global__ __launch_bounds__(64) void block_lists_kernel(const DevBlock* __restrict__ blocks,
+                                                         const DevShell* __restrict__ shells, int nshell,
+                                                         const int* __restrict__ pos, int* __restrict__ sig_shell,
+                                                         int* __restrict__ sig_pos, int* __restrict__ ao_idx) {
+  const int b = blockIdx.x, t = threadIdx.x;
+  const DevBlock bk = blocks[b];
+  int rank = bk.shell_off;
+  for (int s0 = 0; s0 < nshell; s0 += 64) {
+    const int s = s0 + t, p = s < nshell ? pos[(int64_t)b * nshell + s] : -1;
+    const unsigned long long sig = __ballot(p >= 0);
+    if (p >= 0) {
+      const int at = rank + __popcll(sig & ((1ull << t) - 1));
+      sig_shell[at] = s;
+      sig_pos[at] = p;
+      const int ao = shells[s].ao_off, nf = shells[s].nfunc;
+      for (int f = 0; f < nf; ++f) ao_idx[bk.idx_off + p + f] = ao + f;
+    }
+    rank += __popcll(sig);
+  }
+  for (int i = bk.nb + t; i < bk.npad; i += 64) ao_idx[bk.idx_off + i] = -1;
+}
+
+// Row entries of the Fock reduce, for every AO the blocks holding it in block order, in three steps
+// over chunks of kRowChunk blocks: the blocks of each chunk that hold a shell are counted, the counts
+// become offsets (per shell over the chunks, then over the AOs), and the entries are written.
+constexpr int kRowChunk = 64;
+__global__ __launch_bounds__(256) void row_count_kernel(const int* __restrict__ pos, int nblocks, int nshell,
+                                                        int* __restrict__ cnt) {
+  const int s = blockIdx.y * 256 + threadIdx.x, b0 = blockIdx.x * kRowChunk;
+  if (s >= nshell) return;
+  int n = 0;
+  for (int b = b0; b < min(b0 + kRowChunk, nblocks); ++b) n += pos[(int64_t)b * nshell + s] >= 0;
+  cnt[(int64_t)blockIdx.x * nshell + s] = n;
+}
+
+__global__ __launch_bounds__(1024) void row_offsets_kernel(const DevShell* __restrict__ shells, int nshell, int nchunk,
+                                                           int nao, int* __restrict__ cnt, int* __restrict__ row_ptr) {
+  __shared__ int part[1024];
+  const int t = threadIdx.x;
+  int base = 0;
+  for (int s0 = 0; s0 < nshell; s0 += 1024) {
+    const int s = s0 + t;
+    int total = 0, nf = 0, ao = 0;
+    if (s < nshell) {
+      nf = shells[s].nfunc;
+      ao = shells[s].ao_off;
+      for (int k = 0; k < nchunk; ++k) {
+        const int n = cnt[(int64_t)k * nshell + s];
+        cnt[(int64_t)k * nshell + s] = total;
+        total += n;
+      }
+    }
+    part[t] = total * nf;
+    __syncthreads();
+    for (int m = 1; m < 1024; m <<= 1) {
+      const int v = t >= m ? part[t - m] : 0;
+      __syncthreads();
+      part[t] += v;
+      __syncthreads();
+    }
+    for (int f = 0; f < nf; ++f) row_ptr[ao + f] = base + part[t] - total * (nf - f);
+    base += part[1023];
+    __syncthreads();
+  }
+  if (t == 0) row_ptr[nao] = base;
+}
+
+__global__ __launch_bounds__(256) void row_entries_kernel(const DevBlock* __restrict__ blocks, int nblocks,
+                                                          const DevShell* __restrict__ shells, int nshell,
+                                                          const int* __restrict__ pos, const int* __restrict__ cnt,
+                                                          const int* __restrict__ row_ptr, RowEnt* __restrict__ ent) {
+  const int s = blockIdx.y * 256 + threadIdx.x, b0 = blockIdx.x * kRowChunk;
+  if (s >= nshell) return;
+  const int ao = shells[s].ao_off, nf = shells[s].nfunc;
+  int k = cnt[(int64_t)blockIdx.x * nshell + s];
+  for (int b = b0; b < min(b0 + kRowChunk, nblocks); ++b) {
+    const int p = pos[(int64_t)b * nshell + s];
+    if (p < 0) continue;
+    const DevBlock bk = blocks[b];
+    for (int f = 0; f < nf; ++f) {
+      const int l = p + f;
+      RowEnt e;
+      e.rowbase = bk.toff + fock_row_start(l, bk.npad) - 16 * (l / 16);
+      e.c0 = l;
+      e.c1 = bk.nb;
+      e.idx_off = bk.idx_off;
+      e.block = b;
+      ent[row_ptr[ao + f] + k] = e;
+    }
+    ++k;
+  }
+}
+
+// One workgroup per block and kAoShells of its shells, one thread per point: the exponentials of a
+// shell's primitives bound it, so a block's shells are spread over workgroups (one after another
+// they left most of the chip idle: (H2O)12/def2-SVP, 1175 blocks, AO_NOW).  Every element of
+// the block's tiles is written, so they need no clearing.
+constexpr int kAoShells = 8;
 __global__ __launch_bounds__(128) void ao_kernel(const DevBlock* __restrict__ blocks, const int* __restrict__ sig_shell,
                                                  const int* __restrict__ sig_pos, const DevShell* __restrict__ shells,
                                                  const double* __restrict__ alpha, const double* __restrict__ coef,
@@ -80,12 +192,22 @@ __global__ __launch_bounds__(128) void ao_kernel(const DevBlock* __restrict__ bl
                                                  float* __restrict__ t32) {
   const DevBlock bk = blocks[blockIdx.x];
   const int p = threadIdx.x;
-  if (p >= bk.npts) return;
-  const double px = pts[3 * (bk.first + p) + 0];
-  const double py = pts[3 * (bk.first + p) + 1];
-  const double pz = pts[3 * (bk.first + p) + 2];
+  const int k0 = blockIdx.y * kAoShells, k1 = min(k0 + kAoShells, bk.nshell);
+  if (k0 >= max(bk.nshell, 1)) return;  // uniform over the workgroup
   const int64_t cstride = (int64_t)bk.npad * kTile;
-  for (int k = 0; k < bk.nshell; ++k) {
+  // rows that no AO fills (padding) and points beyond the block are zero
+  auto zero = [&](int64_t o) {
+    for (int c = 0; c < ncomp; ++c) {
+      if (t64) t64[o + c * cstride] = 0.0;
+      if (t32) t32[o + c * cstride] = 0.0f;
+    }
+  };
+  if (k0 == 0)
+    for (int i = bk.nb; i < bk.npad; ++i) zero(bk.tile_off + (int64_t)i * kTile + p);
+  const bool in = p < bk.npts;
+  const int64_t q = bk.first + (in ? p : 0);
+  const double px = pts[3 * q + 0], py = pts[3 * q + 1], pz = pts[3 * q + 2];
+  for (int k = k0; k < k1; ++k) {
     const int s = sig_shell[bk.shell_off + k];
     const int pos = sig_pos[bk.shell_off + k];
     const DevShell sh = shells[s];
@@ -104,12 +226,8 @@ __global__ __launch_bounds__(128) void ao_kernel(const DevBlock* __restrict__ bl
       }
     }
     const int64_t base = bk.tile_off + (int64_t)pos * kTile + p;
-    if (fabs(R) < thr) {
-      for (int f = 0; f < sh.nfunc; ++f)
-        for (int c = 0; c < ncomp; ++c) {
-          if (t64) t64[base + (int64_t)f * kTile + c * cstride] = 0.0;
-          if (t32) t32[base + (int64_t)f * kTile + c * cstride] = 0.0f;
-        }
+    if (!in || fabs(R) < thr) {
+      for (int f = 0; f < sh.nfunc; ++f) zero(base + (int64_t)f * kTile);
       continue;
     }
     double xp[kMaxL + 1], yp[kMaxL + 1], zp[kMaxL + 1];
@@ -1293,18 +1411,33 @@ inline unsigned grid1d(int64_t n, int bsz) { return (unsigned)((n + bsz - 1) / b
 }  // namespace
 
 void launch_screen(hipStream_t s, const double* pts, int64_t npts, int bs, int nblocks, const DevShell* shells,
-                   int nshell, const double* alpha, const double* coef, double radial_thr, unsigned char* flags) {
+                   int nshell, const double* alpha, const double* coef, double radial_thr, int* pos, int* count) {
   if (nblocks <= 0) return;
   hipLaunchKernelGGL(screen_kernel, dim3(nblocks), dim3(64), 0, s, pts, npts, bs, shells, nshell, alpha, coef,
-                     radial_thr, flags);
+                     radial_thr, pos, count);
 }
 
-void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, const int* sig_shell, const int* sig_pos,
-                    const DevShell* shells, const double* alpha, const double* coef, const double* ang,
-                    const double* pts, double radial_thr, double exp_thr, int ncomp, double* t64, float* t32) {
+int row_chunks(int nblocks) { return (nblocks + kRowChunk - 1) / kRowChunk; }
+
+void launch_block_lists(hipStream_t s, const DevBlock* blocks, int nblocks, const DevShell* shells, int nshell, int nao,
+                        const int* pos, int* sig_shell, int* sig_pos, int* ao_idx, int* cnt, int* row_ptr,
+                        RowEnt* ent) {
   if (nblocks <= 0) return;
-  hipLaunchKernelGGL(ao_kernel, dim3(nblocks), dim3(kTile), 0, s, blocks, sig_shell, sig_pos, shells, alpha, coef,
-                     ang, pts, radial_thr, exp_thr, ncomp, t64, t32);
+  const dim3 chunks(row_chunks(nblocks), (nshell + 255) / 256);
+  hipLaunchKernelGGL(block_lists_kernel, dim3(nblocks), dim3(64), 0, s, blocks, shells, nshell, pos, sig_shell, sig_pos,
+                     ao_idx);
+  hipLaunchKernelGGL(row_count_kernel, chunks, dim3(256), 0, s, pos, nblocks, nshell, cnt);
+  hipLaunchKernelGGL(row_offsets_kernel, dim3(1), dim3(1024), 0, s, shells, nshell, (int)chunks.x, nao, cnt, row_ptr);
+  hipLaunchKernelGGL(row_entries_kernel, chunks, dim3(256), 0, s, blocks, nblocks, shells, nshell, pos, cnt, row_ptr,
+                     ent);
+}
+
+void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, int max_nshell, const int* sig_shell,
+                    const int* sig_pos, const DevShell* shells, const double* alpha, const double* coef, const double* ang,
+                    const double* pts, double radial_thr, double exp_thr, int ncomp, double* t64, float* t32) {
+  if (nblocks <= 0 || max_nshell <= 0) return;
+  hipLaunchKernelGGL(ao_kernel, dim3(nblocks, (max_nshell + kAoShells - 1) / kAoShells), dim3(kTile), 0, s, blocks,
+                     sig_shell, sig_pos, shells, alpha, coef, ang, pts, radial_thr, exp_thr, ncomp, t64, t32);
 }
 
 template <typename T>

@@ -468,7 +468,6 @@ struct xc_bfogc {
   double radial_thr = 1e-9;
   int deriv = 1, ncomp = 4, nblocks = 0;
   std::vector<DevBlock> blocks;
-  std::vector<int> ao_idx;
   int64_t tile_elems = 0;
   int64_t sum_nb = 0;
   double sum_B_nb2 = 0.0;
@@ -1092,39 +1091,32 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       bf->nblocks = nb;
       const int ns = basis->nshell;
       // 1. shell screening per block on the device
-      DBuf<unsigned char> d_flags;
-      d_flags.alloc(ctx, (size_t)nb * ns);
+      DBuf<int> d_pos, d_count;
+      d_pos.alloc(ctx, (size_t)nb * ns);
+      d_count.alloc(ctx, 2 * (size_t)nb);
       launch_screen(ctx->stream, grid->d_pts.p, N, max_block_size, nb, basis->d_shells.p, ns, basis->d_alpha.p,
-                    basis->d_coef.p, radial_threshold, d_flags.p);
+                    basis->d_coef.p, radial_threshold, d_pos.p, d_count.p);
       HIPX(hipGetLastError());
-      std::vector<unsigned char> flags((size_t)nb * ns);
-      HIPX(hipMemcpyAsync(flags.data(), d_flags.p, flags.size(), hipMemcpyDeviceToHost, ctx->stream));
+      std::vector<int> count(2 * (size_t)nb);
+      HIPX(hipMemcpyAsync(count.data(), d_count.p, sizeof(int) * count.size(), hipMemcpyDeviceToHost, ctx->stream));
       HIPX(hipStreamSynchronize(ctx->stream));
-      // 2. block lists (compact AO index lists padded to kAoPad) and tile offsets
-      std::vector<int> sig_shell, sig_pos;
+      // 2. the blocks' offsets and work items; their lists (compact AO indices padded to kAoPad,
+      // significant shells, row entries) are filled on the device
       bf->blocks.resize(nb);
       bf->dens_item0.assign(nb, 0);
-      int64_t tile_off = 0;
+      int64_t tile_off = 0, idx_off = 0, shell_off = 0;
       for (int b = 0; b < nb; ++b) {
         DevBlock& bk = bf->blocks[b];
         bk.first = (int64_t)b * max_block_size;
         bk.npts = (int)std::min<int64_t>(max_block_size, N - bk.first);
-        bk.idx_off = (int)bf->ao_idx.size();
-        bk.shell_off = (int)sig_shell.size();
-        int cnt = 0, nsh = 0;
-        for (int s = 0; s < ns; ++s) {
-          if (!flags[(size_t)b * ns + s]) continue;
-          const DevShell& sh = basis->shells[s];
-          sig_shell.push_back(s);
-          sig_pos.push_back(cnt);
-          for (int f = 0; f < sh.nfunc; ++f) bf->ao_idx.push_back(sh.ao_off + f);
-          cnt += sh.nfunc;
-          ++nsh;
-        }
+        const int cnt = count[2 * b], nsh = count[2 * b + 1];
+        bk.idx_off = (int)idx_off;
+        bk.shell_off = (int)shell_off;
         bk.nb = cnt;
         bk.nshell = nsh;
         bk.npad = (cnt + kAoPad - 1) / kAoPad * kAoPad;
-        for (int i = cnt; i < bk.npad; ++i) bf->ao_idx.push_back(-1);
+        idx_off += bk.npad;
+        shell_off += nsh;
         bk.tile_off = tile_off;
         tile_off += (int64_t)bk.npad * kTile * bf->ncomp;
         bk.toff = bf->t_elems;
@@ -1171,29 +1163,8 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       xcd_order(bf->dens_work, [&](const WorkItem& w) { return (double)w.b * bf->blocks[w.block].npad; });
       for (auto& items : bf->fock_items) xcd_order(items, [](const FockItem& f) { return (double)f.nsub; });
       bf->tile_elems = tile_off;
-      // row entries of the Fock reduce: for every AO, the blocks holding it (in block order) with
-      // the position of its row in the scratch
+      require(idx_off < (1LL << 31), XC_ERR_ARG, "xc_bfogc_create: too many AOs over the blocks");
       const int nao = basis->nao;
-      std::vector<int> rowptr(nao + 1, 0);
-      for (int b = 0; b < nb; ++b)
-        for (int l = 0; l < bf->blocks[b].nb; ++l) ++rowptr[bf->ao_idx[bf->blocks[b].idx_off + l] + 1];
-      for (int i = 0; i < nao; ++i) rowptr[i + 1] += rowptr[i];
-      std::vector<RowEnt> rowent(std::max(rowptr[nao], 1));
-      {
-        std::vector<int> fill(rowptr.begin(), rowptr.end() - 1);
-        for (int b = 0; b < nb; ++b) {
-          const DevBlock& bk = bf->blocks[b];
-          for (int l = 0; l < bk.nb; ++l) {
-            RowEnt e;
-            e.rowbase = bk.toff + fock_row_start(l, bk.npad) - 16 * (l / 16);
-            e.c0 = l;
-            e.c1 = bk.nb;
-            e.idx_off = bk.idx_off;
-            e.block = b;
-            rowent[fill[bf->ao_idx[bk.idx_off + l]]++] = e;
-          }
-        }
-      }
       // 3. admission by footprint (the context's cached blocks count as free)
       size_t free_b = 0, total_b = 0;
       HIPX(hipMemGetInfo(&free_b, &total_b));
@@ -1206,11 +1177,15 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
                   std::to_string(free_b / 1e9) + " GB free");
       // 4. upload lists, evaluate AO tiles
       bf->d_blocks.upload(ctx, bf->blocks.data(), bf->blocks.size());
-      bf->d_rowptr.upload(ctx, rowptr.data(), rowptr.size());
-      bf->d_rowent.upload(ctx, rowent.data(), rowent.size());
-      bf->d_ao_idx.upload(ctx, bf->ao_idx.data(), bf->ao_idx.size());
-      bf->d_sig_shell.upload(ctx, sig_shell.data(), sig_shell.size());
-      bf->d_sig_pos.upload(ctx, sig_pos.data(), sig_pos.size());
+      bf->d_rowptr.alloc(ctx, (size_t)nao + 1);
+      bf->d_rowent.alloc(ctx, (size_t)std::max<int64_t>(bf->sum_nb, 1));
+      bf->d_ao_idx.alloc(ctx, (size_t)std::max<int64_t>(idx_off, 1));
+      bf->d_sig_shell.alloc(ctx, (size_t)std::max<int64_t>(shell_off, 1));
+      bf->d_sig_pos.alloc(ctx, (size_t)std::max<int64_t>(shell_off, 1));
+      DBuf<int> d_rowcnt;
+      d_rowcnt.alloc(ctx, (size_t)row_chunks(nb) * ns);
+      launch_block_lists(ctx->stream, bf->d_blocks.p, nb, basis->d_shells.p, ns, nao, d_pos.p, bf->d_sig_shell.p,
+                         bf->d_sig_pos.p, bf->d_ao_idx.p, d_rowcnt.p, bf->d_rowptr.p, bf->d_rowent.p);
       bf->d_dens_work.upload(ctx, bf->dens_work.data(), bf->dens_work.size());
       if (keep_fp32 == 1) {  // both tile sets: the mixed-precision build is available
         bf->d_dens_by_block.upload(ctx, bf->dens_by_block.data(), bf->dens_by_block.size());
@@ -1225,15 +1200,11 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       for (int c = 0; c < kFockShapes; ++c)
         bf->d_fock_items[c].upload(ctx, bf->fock_items[c].data(), bf->fock_items[c].size());
       const size_t nt_el = (size_t)std::max<int64_t>(tile_off, 1);
-      if (keep_fp32 != 2) {
-        bf->d_t64.alloc(ctx, nt_el);
-        HIPX(hipMemsetAsync(bf->d_t64.p, 0, sizeof(double) * nt_el, ctx->stream));
-      }
-      if (keep_fp32) {
-        bf->d_t32.alloc(ctx, nt_el);
-        HIPX(hipMemsetAsync(bf->d_t32.p, 0, sizeof(float) * nt_el, ctx->stream));
-      }
-      launch_ao_eval(ctx->stream, bf->d_blocks.p, nb, bf->d_sig_shell.p, bf->d_sig_pos.p, basis->d_shells.p,
+      if (keep_fp32 != 2) bf->d_t64.alloc(ctx, nt_el);
+      if (keep_fp32) bf->d_t32.alloc(ctx, nt_el);
+      int max_nshell = 0;
+      for (const DevBlock& bk : bf->blocks) max_nshell = std::max(max_nshell, bk.nshell);
+      launch_ao_eval(ctx->stream, bf->d_blocks.p, nb, max_nshell, bf->d_sig_shell.p, bf->d_sig_pos.p, basis->d_shells.p,
                      basis->d_alpha.p, basis->d_coef.p, basis->d_ang.p, grid->d_pts.p, radial_threshold,
                      radial_threshold > 0.0 ? -std::log(radial_threshold) : HUGE_VAL, bf->ncomp, bf->d_t64.p,
                      keep_fp32 ? bf->d_t32.p : nullptr);
@@ -1315,7 +1286,10 @@ int xc_bfogc_block_data(const xc_bfogc* bf, int block, double* values, double* g
     const int n = bf->basis->nao;
     const int64_t cnt = (int64_t)bk.npad * kTile * bf->ncomp;
     std::vector<double> t((size_t)std::max<int64_t>(cnt, 1));
+    std::vector<int> idx((size_t)bk.npad);
     if (cnt) {
+      HIPX(hipMemcpyAsync(idx.data(), bf->d_ao_idx.p + bk.idx_off, sizeof(int) * idx.size(), hipMemcpyDeviceToHost,
+                          bf->ctx->stream));
       HIPX(hipMemcpyAsync(t.data(), bf->d_t64.p + bk.tile_off, sizeof(double) * cnt, hipMemcpyDeviceToHost,
                           bf->ctx->stream));
       HIPX(hipStreamSynchronize(bf->ctx->stream));
@@ -1327,7 +1301,7 @@ int xc_bfogc_block_data(const xc_bfogc* bf, int block, double* values, double* g
       if (outs[c]) std::fill(outs[c], outs[c] + (size_t)B * n, 0.0);
     if (negligible) std::fill(negligible, negligible + n, 1);
     for (int i = 0; i < bk.nb; ++i) {
-      const int mu = bf->ao_idx[bk.idx_off + i];
+      const int mu = idx[i];
       if (negligible) negligible[mu] = 0;
       for (int c = 0; c < std::min(bf->ncomp, 4); ++c) {
         if (!outs[c]) continue;
@@ -1350,14 +1324,17 @@ int xc_bfogc_block_hessian(const xc_bfogc* bf, int block, double* hess) {
     const int B = bk.npts;
     const int64_t cnt = (int64_t)bk.npad * kTile * 6;
     std::vector<double> t((size_t)std::max<int64_t>(cnt, 1));
+    std::vector<int> idx((size_t)bk.npad);
     if (cnt) {
+      HIPX(hipMemcpyAsync(idx.data(), bf->d_ao_idx.p + bk.idx_off, sizeof(int) * idx.size(), hipMemcpyDeviceToHost,
+                          bf->ctx->stream));
       HIPX(hipMemcpyAsync(t.data(), bf->d_t64.p + bk.tile_off + (int64_t)4 * bk.npad * kTile, sizeof(double) * cnt,
                           hipMemcpyDeviceToHost, bf->ctx->stream));
       HIPX(hipStreamSynchronize(bf->ctx->stream));
     }
     std::fill(hess, hess + (size_t)6 * B * n, 0.0);
     for (int i = 0; i < bk.nb; ++i) {
-      const int mu = bf->ao_idx[bk.idx_off + i];
+      const int mu = idx[i];
       for (int c = 0; c < 6; ++c)
         for (int p = 0; p < B; ++p)
           hess[((size_t)c * n + mu) * B + p] = t[((size_t)c * bk.npad + i) * kTile + p];
