@@ -349,11 +349,6 @@ void launch_jaux_out(hipStream_t s, const JView& J, const DevShell* aux, int nsh
 void launch_jassemble(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs,
                       const DevShell* shells, const double* ang, const JView& Jv, const double* V, int n, double* J);
 
-// Molecular-grid partition weights of ncand candidate points (kernels/grid_kernels.hip).
-void launch_partition(hipStream_t s, int type, unsigned smoothing, int natoms, const double* xyz, const double* dist,
-                      const double* apair, const double* min_dist, int64_t ncand, const double* cand_xyz,
-                      const double* cand_w, const int* cand_atom, double* w);
-
 // The device grid build (kernels/grid_kernels.hip): partition weights of every candidate generated
 // from the reference grids (keep[c] = w[c] > thr), the cut (exclusive scan of keep into pos, the
 // kept points in candidate order), the bounding box (mn, spread) and the Hilbert order.
