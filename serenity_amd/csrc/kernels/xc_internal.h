@@ -269,18 +269,35 @@ void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, 
 // entry 0.68 ms at (H2O)64/def2-TZVP against 0.86 ms with 8 and 1.40 ms with 4).  wide: blocks hold
 // more than 256 AOs on average, so that a row segment (half of them on average) fills the 128
 // columns that 32 lanes take at once; else 16 lanes take an entry.
+// With out.direct the rows go to both triangles of F instead (no finalize), each row leaves its part of
+// the FP32 rounding term sum F (P - P32) in round[row] where P32 is given (packed: where round is
+// not null), and one more workgroup sums the block energies into E (a second rounding sum, where
+// there is one, is launch_sum's).  For matrices of up to kDirectRows rows: the upper triangle's writes
+// go one element per line (n^2 / 2 of them), which costs less than the finalize's launch only while
+// they are few ((H2O)8/def2-SVP, 192 rows: reduce, finalize and sum 30 us, together 19 us).
+struct ReduceOut {
+  bool direct;
+  double* F;
+  const double* P;
+  const float* P32;
+  double* round;
+  const double* eblk;
+  int nxc;
+  double* E;
+};
+constexpr int kDirectRows = 512;
 constexpr int kReduceWaves = 16;
 constexpr int kReduceWindow = 8192;  // row columns accumulated in LDS per pass
 template <typename T>
 void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
                         double* U, int n, const PackSys* pack = nullptr, int nsys = 1, bool fixed = false,
-                        bool wide = false);
+                        bool wide = false, const ReduceOut& out = ReduceOut{});
 // Packed elementwise stages over nsys systems (maxnn = largest n^2): P -> FP32,
 // F = mirror of U (+ FP32 rounding partials), E = sum of block energies (+ rounding term).
 constexpr int kPackRoundBlocks = 512;  // finalize workgroups per system of a packed build
 void launch_pack_to_float(hipStream_t s, const PackSys* pack, int nsys, int64_t maxnn);
 void launch_pack_finalize(hipStream_t s, const PackSys* pack, int nsys, int fp32);
-void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int fp32);
+void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int nround);
 
 // a[nu][c] += sum over the points of a density work item's block of (G P)_p,nu d_c phi_nu +
 // (phi P)_p,nu H^c_nu for the item's columns nu (kernels/gradient_kernels.hip); tiles need 4 planes

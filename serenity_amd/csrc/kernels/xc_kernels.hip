@@ -743,6 +743,24 @@ __global__ __launch_bounds__(128) void functional_kernel(int func, XcParams prm,
   if (t == 0) e_blk[b] = eb;
 }
 
+// Sum of x[0..n) and x2[0..n2) by the first 256 threads of a workgroup, in a fixed order (every thread
+// of the workgroup calls it).
+__device__ double sum_256(const double* x, int64_t n, const double* x2, int64_t n2, double* red) {
+  const int t = threadIdx.x;
+  if (t < 256) {
+    double s = 0.0;
+    for (int64_t i = t; i < n; i += 256) s += x[i];
+    for (int64_t i = t; i < n2; i += 256) s += x2[i];
+    red[t] = s;
+  }
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (t < k) red[t] += red[t + k];
+    __syncthreads();
+  }
+  return red[0];
+}
+
 // Unrestricted functional on 128-point blocks: spin densities and gradients in,
 // w v_s and w g_s (the Fock kernel's inputs) per spin and the block energies out.
 // The block is skipped when both spin densities are negligible (sum |rho_s| <
@@ -1132,7 +1150,8 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
                                                                         const T* __restrict__ Tscr,
                                                                         const int* __restrict__ ao_idx,
                                                                         double* __restrict__ U, int n, int window,
-                                                                        const PackSys* __restrict__ pack) {
+                                                                        const PackSys* __restrict__ pack,
+                                                                        ReduceOut out) {
   extern __shared__ unsigned long long racc_u[];  // window (FP64 sums) or 2 window (Fixed: h, then l sums)
   double* racc = reinterpret_cast<double*>(racc_u);
   if (pack) {
@@ -1143,10 +1162,26 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
     ao_idx = ps.ao_idx;
     U = ps.U;
     n = ps.n;
+    if (out.direct) {
+      out.F = ps.F;
+      out.P = ps.P64;
+      out.P32 = out.round ? ps.P32 : nullptr;
+      out.round = ps.round;
+      out.eblk = ps.eblk;
+      out.nxc = ps.nxc;
+      out.E = ps.E;
+    }
   }
   const int i = blockIdx.x;
-  if (i >= n) return;  // uniform over the workgroup
   const int tid = threadIdx.x;
+  if (i >= n) {  // uniform over the workgroup
+    if (i == n && out.direct && out.E) {
+      const double e = sum_256(out.eblk, out.nxc, nullptr, 0, reinterpret_cast<double*>(racc_u));
+      if (tid == 0) out.E[0] = e;
+    }
+    return;
+  }
+  double c_round = 0.0;
   const gmem<const RowEnt>* entg = to_global(ent);
   const gmem<const T>* Tg = to_global(Tscr);
   const gmem<const int>* idxg = to_global(ao_idx);
@@ -1227,9 +1262,34 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
         f = (double)(long long)racc_u[j] * 0x1p-32 + (double)(long long)racc_u[window + j] * 0x1p-72;
       else
         f = racc[j];
-      to_global(U)[(int64_t)(i + w0 + j) + (int64_t)n * i] = f;
+      const int64_t lo = (int64_t)(i + w0 + j) + (int64_t)n * i;
+      if (out.direct) {
+        // both triangles of F, and the row's part of the FP32 rounding term (P is read first: a
+        // caller's F may be its P)
+        const int64_t up = i + (int64_t)n * (i + w0 + j);
+        if (out.P32) {
+          c_round += f * (to_global(out.P)[lo] - (double)to_global(out.P32)[lo]);
+          if (lo != up) c_round += f * (to_global(out.P)[up] - (double)to_global(out.P32)[up]);
+        }
+        to_global(out.F)[lo] = f;
+        if (lo != up) to_global(out.F)[up] = f;
+      } else {
+        to_global(U)[lo] = f;
+      }
     }
     __syncthreads();
+  }
+  if (out.direct && out.P32) {
+    double* red = reinterpret_cast<double*>(racc_u);  // one per wavefront (the host asks for that much LDS)
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) c_round += __shfl_xor(c_round, m);
+    if ((tid & 63) == 0) red[tid >> 6] = c_round;
+    __syncthreads();
+    if (tid == 0) {
+      double s = 0.0;
+      for (int v = 0; v < kReduceWaves; ++v) s += red[v];
+      out.round[i] = s;
+    }
   }
 }
 
@@ -1344,17 +1404,8 @@ __global__ __launch_bounds__(256) void sum_kernel(const double* __restrict__ x, 
                                                   const double* __restrict__ x2, int64_t n2, double* __restrict__ out,
                                                   int mode) {
   __shared__ double red[256];
-  const int t = threadIdx.x;
-  double s = 0.0;
-  for (int64_t i = t; i < n; i += 256) s += x[i];
-  for (int64_t i = t; i < n2; i += 256) s += x2[i];
-  red[t] = s;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if (t < k) red[t] += red[t + k];
-    __syncthreads();
-  }
-  if (t == 0) out[0] = mode == 0 ? red[0] : out[0] - red[0];
+  const double s = sum_256(x, n, x2, n2, red);
+  if (threadIdx.x == 0) out[0] = mode == 0 ? s : out[0] - s;
 }
 
 // ---- packed builds: elementwise stages over the systems of a pack (blockIdx.y = system) ----
@@ -1389,22 +1440,13 @@ __global__ __launch_bounds__(256) void pack_finalize_kernel(const PackSys* __res
   if (t == 0) ps.round[blockIdx.x] = red[0];
 }
 
-// E_xc of each system: its block energies (+ the FP32 rounding term), in a fixed order
-__global__ __launch_bounds__(256) void pack_sum_kernel(const PackSys* __restrict__ pack, int fp32) {
+// E_xc of each system: its block energies and nround partials of the FP32 rounding term (one per
+// AO row for nround < 0), in a fixed order
+__global__ __launch_bounds__(256) void pack_sum_kernel(const PackSys* __restrict__ pack, int nround) {
   const PackSys& ps = pack[blockIdx.x];
   __shared__ double red[256];
-  const int t = threadIdx.x;
-  double s = 0.0;
-  for (int i = t; i < ps.nxc; i += 256) s += ps.eblk[i];
-  if (fp32)
-    for (int i = t; i < kPackRoundBlocks; i += 256) s += ps.round[i];
-  red[t] = s;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if (t < k) red[t] += red[t + k];
-    __syncthreads();
-  }
-  if (t == 0) ps.E[0] = red[0];
+  const double s = sum_256(ps.eblk, ps.nxc, ps.round, nround < 0 ? ps.n : nround, red);
+  if (threadIdx.x == 0) ps.E[0] = s;
 }
 
 inline unsigned grid1d(int64_t n, int bsz) { return (unsigned)((n + bsz - 1) / bsz); }
@@ -1600,9 +1642,9 @@ void launch_pack_finalize(hipStream_t s, const PackSys* pack, int nsys, int fp32
   hipLaunchKernelGGL(pack_finalize_kernel, dim3(kPackRoundBlocks, nsys), dim3(256), 0, s, pack, fp32);
 }
 
-void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int fp32) {
+void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int nround) {
   if (nsys <= 0) return;
-  hipLaunchKernelGGL(pack_sum_kernel, dim3(nsys), dim3(256), 0, s, pack, fp32);
+  hipLaunchKernelGGL(pack_sum_kernel, dim3(nsys), dim3(256), 0, s, pack, nround);
 }
 
 void launch_functional_pol(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* ra,
@@ -1663,31 +1705,36 @@ static int reduce_window_limit(bool fixed) {
 
 template <typename T, bool Fixed>
 static void launch_fock_reduce_f(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr,
-                                 const int* ao_idx, double* U, int n, const PackSys* pack, int nsys, bool wide) {
+                                 const int* ao_idx, double* U, int n, const PackSys* pack, int nsys, bool wide,
+                                 const ReduceOut& out) {
   const int lim = reduce_window_limit(Fixed);
   const int window = n < lim ? n : lim;
-  const size_t lds = (Fixed ? 16 : 8) * (size_t)window;
+  size_t lds = (Fixed ? 16 : 8) * (size_t)window;
+  // one workgroup more for the energy sum, whose 256 terms need LDS (the rounding term's 16 less)
+  const dim3 grid(n + (out.direct && (out.E || pack) ? 1 : 0), nsys);
+  if (out.direct && lds < 256 * sizeof(double)) lds = 256 * sizeof(double);
   if (wide)
-    hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 32>), dim3(n, nsys), dim3(64 * kReduceWaves), lds, s, ent, row_ptr,
-                       Tscr, ao_idx, U, n, window, pack);
+    hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 32>), grid, dim3(64 * kReduceWaves), lds, s, ent, row_ptr, Tscr,
+                       ao_idx, U, n, window, pack, out);
   else
-    hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 16>), dim3(n, nsys), dim3(64 * kReduceWaves), lds, s, ent, row_ptr,
-                       Tscr, ao_idx, U, n, window, pack);
+    hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 16>), grid, dim3(64 * kReduceWaves), lds, s, ent, row_ptr, Tscr,
+                       ao_idx, U, n, window, pack, out);
 }
 
 template <typename T>
 void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
-                        double* U, int n, const PackSys* pack, int nsys, bool fixed, bool wide) {
+                        double* U, int n, const PackSys* pack, int nsys, bool fixed, bool wide,
+                        const ReduceOut& out) {
   if (n <= 0 || nsys <= 0) return;
   if (fixed)
-    launch_fock_reduce_f<T, true>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide);
+    launch_fock_reduce_f<T, true>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide, out);
   else
-    launch_fock_reduce_f<T, false>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide);
+    launch_fock_reduce_f<T, false>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide, out);
 }
 template void launch_fock_reduce<double>(hipStream_t, const RowEnt*, const int*, const double*, const int*, double*,
-                                         int, const PackSys*, int, bool, bool);
+                                         int, const PackSys*, int, bool, bool, const ReduceOut&);
 template void launch_fock_reduce<float>(hipStream_t, const RowEnt*, const int*, const float*, const int*, double*,
-                                        int, const PackSys*, int, bool, bool);
+                                        int, const PackSys*, int, bool, bool, const ReduceOut&);
 
 void launch_weight_potential(hipStream_t s, int64_t npts, const double* w, const double* v, const double* g,
                              double* vs, double* gw) {

@@ -500,7 +500,7 @@ struct xc_bfogc {
   DBuf<RowEnt> d_rowent;
   DBuf<int> d_rowptr;
   DBuf<float> d_P32;
-  DBuf<double> d_round;  // finalize-block partials of the FP32 rounding term, per spin
+  DBuf<double> d_round;  // row or finalize-block partials of the FP32 rounding term, per spin
   // supersystem density of a non-additive build with this controller active (allocated on first use)
   DBuf<double> d_rho_sup, d_grad_sup, d_rho_sup_b, d_grad_sup_b;
   // cached grid density (xc_bfogc_update_density) and the energies of it per functional
@@ -608,10 +608,34 @@ void run_fock_tiles(xc_bfogc* bf, const T* tiles, int gga, double thr, const Lan
 }
 
 template <typename T>
-void run_fock_reduce(xc_bfogc* bf, const Lanes& L) {
+void run_fock_reduce(xc_bfogc* bf, const Lanes& L, const ReduceOut& out = ReduceOut{}) {
   launch_fock_reduce<T>(L.main, bf->d_rowent.p, bf->d_rowptr.p, reinterpret_cast<const T*>(bf->d_T.p),
                         bf->d_ao_idx.p, bf->d_U.p, bf->basis->nao, nullptr, 1, bf->ctx->deterministic,
-                        bf->sum_nb > 256 * (int64_t)bf->nblocks);
+                        bf->sum_nb > 256 * (int64_t)bf->nblocks, out);
+}
+
+// The reduce and what follows it: F (overwritten), the FP32 rounding partials of one spin (P32 given;
+// the spin's slot of d_round), and E = the sum of the block energies (E given) plus the rounding
+// partials of nspin slots.  Small matrices get their rows and the energy from the reduce itself.
+template <typename T>
+void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, const float* P32, int spin, int nspin,
+                     double* E) {
+  hipStream_t s = L.main;
+  const int n = bf->basis->nao;
+  const int nxc = (int)((bf->grid->npts + kTile - 1) / kTile);
+  const bool direct = n <= kDirectRows;
+  const int nround = direct ? n : finalize_blocks(n);
+  double* round = P32 ? bf->d_round.p + (size_t)spin * nround : nullptr;
+  if (direct) {
+    run_fock_reduce<T>(bf, L, ReduceOut{true, dF, P, P32, round, bf->d_eblk.p, nxc, P32 ? nullptr : E});
+  } else {
+    run_fock_reduce<T>(bf, L);
+    if (s == bf->ctx->stream && nspin == 1) bf->ctx->mark();
+    launch_finalize(s, bf->d_U.p, dF, n, 0, P32 ? P : nullptr, P32, round);
+  }
+  if (s == bf->ctx->stream && nspin == 1 && direct) bf->ctx->mark();
+  if (E && (P32 || !direct))
+    launch_sum(s, bf->d_eblk.p, nxc, E, 0, P32 ? bf->d_round.p : nullptr, P32 ? (int64_t)nspin * nround : 0);
 }
 
 template <typename T>
@@ -1229,7 +1253,7 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       bf->d_E.alloc(ctx, 1);
       if (keep_fp32) {
         bf->d_P32.alloc(ctx, (size_t)n * n);
-        bf->d_round.alloc(ctx, 2 * (size_t)finalize_blocks(n));
+        bf->d_round.alloc(ctx, 2 * (size_t)std::max(finalize_blocks(n), n));
       }
       if (keep_fp32 == 1) bf->d_P32d.alloc(ctx, (size_t)n * n);
       HIPX(hipStreamSynchronize(ctx->stream));
@@ -1508,17 +1532,13 @@ static void enqueue_build(xc_bfogc* bf, int functional, int precision, double th
   else
     run_fock_tiles<float>(bf, bf->d_t32.p, gga ? 1 : 0, thr, L);
   if (s == ctx->stream) ctx->mark();
-  if (!lowp)
-    run_fock_reduce<double>(bf, L);
-  else
-    run_fock_reduce<float>(bf, L);
-  if (s == ctx->stream) ctx->mark();
   // FP32 contractions see fl32(P): E_xc[P] = E_xc[fl32(P)] + tr(F (P - fl32(P))) to first order,
-  // the trace formed by the finalize blocks and added with the energy sum (the mixed form's FP64
+  // the trace formed with F and added with the energy sum (the mixed form's FP64
   // refinement also contracts fl32(P), so the same term applies to every block)
-  const bool fp32 = lowp;
-  launch_finalize(s, bf->d_U.p, dF, n, 0, fp32 ? dP : nullptr, fp32 ? bf->d_P32.p : nullptr, bf->d_round.p);
-  launch_sum(s, bf->d_eblk.p, nxc, d_energy, 0, fp32 ? bf->d_round.p : nullptr, fp32 ? finalize_blocks(n) : 0);
+  if (!lowp)
+    run_fock_finish<double>(bf, L, dF, nullptr, nullptr, 0, 1, d_energy);
+  else
+    run_fock_finish<float>(bf, L, dF, dP, bf->d_P32.p, 0, 1, d_energy);
   if (s == ctx->stream) ctx->mark();
   HIPX(hipGetLastError());
 }
@@ -1581,17 +1601,16 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
   const double* gw[2] = {bf->d_gw.p, bf->d_gw_b.p};
   double* Fs[2] = {dFa, dFb};
   for (int sp = 0; sp < 2; ++sp) {
-    if (precision == XC_PREC_FP64)
-      run_fock<double>(bf, bf->d_t64.p, gga ? 1 : 0, thr, L, vs[sp], gw[sp]);
-    else
-      run_fock<float>(bf, bf->d_t32.p, gga ? 1 : 0, thr, L, vs[sp], gw[sp]);
     // with the first-order FP32 rounding term of each spin density matrix (dE_xc/dP_s = F_s)
-    const bool fp32 = precision == XC_PREC_FP32;
-    launch_finalize(s, bf->d_U.p, Fs[sp], n, 0, fp32 ? Ps[sp] : nullptr, fp32 ? P32[sp] : nullptr,
-                    fp32 ? bf->d_round.p + (size_t)sp * finalize_blocks(n) : nullptr);
+    double* E = sp == 1 ? d_energy : nullptr;
+    if (precision == XC_PREC_FP64) {
+      run_fock_tiles<double>(bf, bf->d_t64.p, gga ? 1 : 0, thr, L, vs[sp], gw[sp]);
+      run_fock_finish<double>(bf, L, Fs[sp], nullptr, nullptr, sp, 2, E);
+    } else {
+      run_fock_tiles<float>(bf, bf->d_t32.p, gga ? 1 : 0, thr, L, vs[sp], gw[sp]);
+      run_fock_finish<float>(bf, L, Fs[sp], Ps[sp], P32[sp], sp, 2, E);
+    }
   }
-  launch_sum(s, bf->d_eblk.p, nxc, d_energy, 0, precision == XC_PREC_FP32 ? bf->d_round.p : nullptr,
-             precision == XC_PREC_FP32 ? 2 * finalize_blocks(n) : 0);
   HIPX(hipGetLastError());
 }
 
@@ -1670,11 +1689,9 @@ static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int func
     run_fock_tiles<double>(act, act->d_t64.p, gga ? 1 : 0, thr, ctx->lanes);
   ctx->mark();
   if (fp32)
-    run_fock_reduce<float>(act, ctx->lanes);
+    run_fock_finish<float>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
   else
-    run_fock_reduce<double>(act, ctx->lanes);
-  ctx->mark();
-  launch_finalize(s, act->d_U.p, dF, n, 0);
+    run_fock_finish<double>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
   ctx->mark();
   HIPX(hipGetLastError());
 }
@@ -1766,11 +1783,13 @@ static void enqueue_nadd_pol(xc_bfogc* act, int nenv, xc_bfogc* const* env, int 
   const double* gw[2] = {act->d_gw.p, act->d_gw_b.p};
   double* Fs[2] = {dFa, dFb};
   for (int sp = 0; sp < 2; ++sp) {
-    if (fp32)
-      run_fock<float>(act, act->d_t32.p, g, thr, ctx->lanes, vs[sp], gw[sp]);
-    else
-      run_fock<double>(act, act->d_t64.p, g, thr, ctx->lanes, vs[sp], gw[sp]);
-    launch_finalize(s, act->d_U.p, Fs[sp], n, 0);
+    if (fp32) {
+      run_fock_tiles<float>(act, act->d_t32.p, g, thr, ctx->lanes, vs[sp], gw[sp]);
+      run_fock_finish<float>(act, ctx->lanes, Fs[sp], nullptr, nullptr, sp, 2, nullptr);
+    } else {
+      run_fock_tiles<double>(act, act->d_t64.p, g, thr, ctx->lanes, vs[sp], gw[sp]);
+      run_fock_finish<double>(act, ctx->lanes, Fs[sp], nullptr, nullptr, sp, 2, nullptr);
+    }
   }
   HIPX(hipGetLastError());
 }
@@ -1936,11 +1955,9 @@ int xc_nadd_fock_build_cached(xc_bfogc* act, int nenv, xc_bfogc* const* env, int
       run_fock_tiles<double>(act, act->d_t64.p, gga ? 1 : 0, thr, ctx->lanes);
     ctx->mark();
     if (precision == XC_PREC_FP32)
-      run_fock_reduce<float>(act, ctx->lanes);
+      run_fock_finish<float>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
     else
-      run_fock_reduce<double>(act, ctx->lanes);
-    ctx->mark();
-    launch_finalize(s, act->d_U.p, dF, n, 0);
+      run_fock_finish<double>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
     ctx->mark();
     HIPX(hipGetLastError());
     if (energy) {
@@ -2152,14 +2169,19 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
             launch_fock_sub<double>(st, c, pw.fock[c].p, (int)fock[c].size(), pw.blocks.p, nullptr, nullptr, nullptr, g,
                                     thr, nullptr, 0, dsys);
         });
+        const bool direct = maxn <= kDirectRows;
+        static_assert(kDirectRows <= kPackRoundBlocks, "a system's rounding partials fit its slots");
+        ReduceOut out{};
+        out.direct = direct;
+        out.round = fp32 ? pw.round.p : nullptr;  // (each system's own slots from the table)
         if (fp32)
           launch_fock_reduce<float>(s, nullptr, nullptr, nullptr, nullptr, nullptr, maxn, dsys, nsys,
-                                    ctx->deterministic);
+                                    ctx->deterministic, false, out);
         else
           launch_fock_reduce<double>(s, nullptr, nullptr, nullptr, nullptr, nullptr, maxn, dsys, nsys,
-                                     ctx->deterministic);
-        launch_pack_finalize(s, dsys, nsys, fp32 ? 1 : 0);
-        launch_pack_sum(s, dsys, nsys, fp32 ? 1 : 0);
+                                     ctx->deterministic, false, out);
+        if (!direct) launch_pack_finalize(s, dsys, nsys, fp32 ? 1 : 0);
+        if (fp32 || !direct) launch_pack_sum(s, dsys, nsys, !fp32 ? 0 : direct ? -1 : kPackRoundBlocks);
       };
       if (capture) {
         // second build of this composition: capture it (kernel nodes only, no memsets) into its own lists
