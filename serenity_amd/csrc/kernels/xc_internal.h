@@ -240,8 +240,7 @@ void launch_reduce_partials(hipStream_t s, const DevBlock* blocks, int bs, int64
 // Functional on rho/grad, or (part != nullptr) on the partials of 128-point blocks.
 void launch_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* rho,
                        const double* grad, const DevBlock* blocks, const double* part, const double* w, double* eps,
-                       double* v, double* g, double* vs, double* gw, double* e_blk,
-                       const double* rho_sub = nullptr, const double* grad_sub = nullptr);
+                       double* v, double* g, double* vs, double* gw, double* e_blk);
 // Functional of a packed build: one 128-point block per workgroup over the merged block list.
 void launch_functional_packed(hipStream_t s, int func, const XcParams& prm, int nblocks, const DevBlock* blocks,
                               const PackSys* pack);
@@ -396,11 +395,23 @@ struct DensityList {
   const double* grad[kListMax];
   int n;
 };
-// rho (+)= sum of list.rho[i] in list order; grad likewise (3 x npts each).
-void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, int want_grad, int accumulate,
-                          double* rho, double* grad);
-// out[0] -= list.rho[i][0] for i in order.
-void launch_subtract_scalars(hipStream_t s, const DensityList& list, double* out);
+// rho = sum of list.rho[i] in list order; grad likewise (3 x npts each).
+void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, int want_grad, double* rho,
+                          double* grad);
+// w v and w g of v[sum of sup] - v[rho_act] and the block energies of the difference (where the
+// potential is wanted); beside it the block energies of the pending densities.
+void launch_nadd_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, bool potential,
+                            const DensityList& sup, const double* rho_act, const double* grad_act,
+                            const DensityList& pending, double* const* pending_eblk, const double* w, double* vs,
+                            double* gw, double* e_blk);
+// Energies subtracted from a non-additive energy, with the block energies of those still to be summed.
+struct EnvEnergies {
+  double* e[kListMax];
+  const double* eblk[kListMax];
+  int n;
+};
+// out = sum of e_blk[0..n) (null: out) minus the listed energies in order (summed first where pending)
+void launch_nadd_energy(hipStream_t s, const double* e_blk, int64_t n, const EnvEnergies& env, double* out);
 // Q[i, j] = P[i, j] + P[j, i], Q[i, i] = P[i, i] (packed: every system's P64 into its U, n the largest)
 void launch_fold(hipStream_t s, const double* P, double* Q, int n, const PackSys* pack = nullptr, int nsys = 1);
 void launch_to_float(hipStream_t s, const double* src, float* dst, int64_t n);

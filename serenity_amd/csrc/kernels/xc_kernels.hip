@@ -655,8 +655,6 @@ __global__ __launch_bounds__(128) void functional_kernel(int func, XcParams prm,
                                                          double* __restrict__ v, double* __restrict__ g,
                                                          double* __restrict__ vs, double* __restrict__ gw,
                                                          double* __restrict__ e_blk,
-                                                         const double* __restrict__ rho_sub,
-                                                         const double* __restrict__ grad_sub,
                                                          const PackSys* __restrict__ pack) {
   __shared__ double red[128];
   const int bm = blockIdx.x, t = threadIdx.x;  // bm: block in the (merged) block list
@@ -706,23 +704,6 @@ __global__ __launch_bounds__(128) void functional_kernel(int func, XcParams prm,
   const bool skip = sumabs < B * 1e-12;
   double e = 0.0, vv = 0.0, gg[3] = {0.0, 0.0, 0.0};
   if (in && !skip) e = xc_point(func, r, gx, gy, gz, prm, &vv, gg);
-  if (rho_sub) {
-    // non-additive form: the same functional of a second density is subtracted
-    // (its own block skip applies to it)
-    const double r2 = in ? rho_sub[q] : 0.0;
-    const bool skip2 = block_sum_128(fabs(r2), red) < B * 1e-12;
-    if (in && !skip2) {
-      double v2 = 0.0, g2[3] = {0.0, 0.0, 0.0};
-      const bool has_g = gga && grad_sub;
-      const double e2 = xc_point(func, r2, has_g ? grad_sub[q] : 0.0, has_g ? grad_sub[npts + q] : 0.0,
-                                 has_g ? grad_sub[2 * npts + q] : 0.0, prm, &v2, g2);
-      e -= e2;
-      vv -= v2;
-      gg[0] -= g2[0];
-      gg[1] -= g2[1];
-      gg[2] -= g2[2];
-    }
-  }
   const double wq = in ? w[q] : 0.0;
   if (in) {
     if (eps) eps[q] = e;
@@ -759,6 +740,83 @@ __device__ double sum_256(const double* x, int64_t n, const double* x2, int64_t 
     __syncthreads();
   }
   return red[0];
+}
+
+// Functional of a non-additive build.  Workgroups of y = 0: one block of v[rho_sup] - v[rho_act] (w v,
+// w g) and its energy, rho_sup summed from the listed densities on the way (in list order, the active
+// one first); of y > 0: a block of the energy of pend.dens.rho[y - 1] alone, into pend.eblk[y - 1]
+// (y = blockIdx.y, one more without the first).  What were a pass over all densities, a launch per
+// functional and one per energy sum took 36 us and as much between them ((H2O)12 in def2-SVP, 103 000
+// points); this launch and nadd_energy_kernel 23 us.
+struct PendingEnergies {
+  DensityList dens;
+  double* eblk[kListMax];
+};
+__global__ __launch_bounds__(128) void nadd_functional_kernel(int func, XcParams prm, int64_t npts, int y0,
+                                                              DensityList sup, const double* __restrict__ rho_act,
+                                                              const double* __restrict__ grad_act,
+                                                              PendingEnergies pend, const double* __restrict__ w,
+                                                              double* __restrict__ vs, double* __restrict__ gw,
+                                                              double* __restrict__ e_blk) {
+  __shared__ double red[128];
+  const int b = blockIdx.x, t = threadIdx.x, y = y0 + blockIdx.y;
+  const int64_t q = (int64_t)b * kTile + t;
+  const int B = (int)min((int64_t)kTile, npts - (int64_t)b * kTile);
+  const bool in = t < B, gga = functional_is_gga(func);
+  double r = 0.0, g[3] = {0.0, 0.0, 0.0};
+  if (in) {
+    if (y == 0) {
+      for (int i = 0; i < sup.n; ++i) r += sup.rho[i][q];
+      if (gga)
+        for (int c = 0; c < 3; ++c)
+          for (int i = 0; i < sup.n; ++i) g[c] += sup.grad[i][c * npts + q];
+    } else {
+      r = pend.dens.rho[y - 1][q];
+      if (gga)
+        for (int c = 0; c < 3; ++c) g[c] = pend.dens.grad[y - 1][c * npts + q];
+    }
+  }
+  const bool skip = block_sum_128(fabs(r), red) < B * 1e-12;
+  double e = 0.0, vv = 0.0, gg[3] = {0.0, 0.0, 0.0};
+  if (in && !skip) e = xc_point(func, r, g[0], g[1], g[2], prm, &vv, gg);
+  if (y == 0) {
+    const double r2 = in ? rho_act[q] : 0.0;
+    const bool skip2 = block_sum_128(fabs(r2), red) < B * 1e-12;
+    if (in && !skip2) {
+      double v2 = 0.0, g2[3] = {0.0, 0.0, 0.0};
+      e -= xc_point(func, r2, gga ? grad_act[q] : 0.0, gga ? grad_act[npts + q] : 0.0,
+                    gga ? grad_act[2 * npts + q] : 0.0, prm, &v2, g2);
+      vv -= v2;
+      for (int c = 0; c < 3; ++c) gg[c] -= g2[c];
+    }
+  }
+  const double wq = in ? w[q] : 0.0;
+  if (in && y == 0) {
+    vs[q] = wq * vv;
+    for (int c = 0; c < 3; ++c) gw[c * npts + q] = wq * gg[c];
+  }
+  const double eb = block_sum_128(wq * e, red);
+  if (t == 0) (y == 0 ? e_blk : pend.eblk[y - 1])[b] = eb;
+}
+
+// out = sum of e_blk (null: out itself) - env.e[0] - env.e[1] ..., where an entry with block
+// energies first becomes their sum (kept where e is given).
+__global__ __launch_bounds__(256) void nadd_energy_kernel(const double* __restrict__ e_blk, int64_t n, EnvEnergies env,
+                                                          double* __restrict__ out) {
+  __shared__ double red[256];
+  double e = e_blk ? sum_256(e_blk, n, nullptr, 0, red) : out[0];
+  __syncthreads();
+  for (int i = 0; i < env.n; ++i) {
+    if (env.eblk[i]) {
+      const double s = sum_256(env.eblk[i], n, nullptr, 0, red);
+      if (threadIdx.x == 0 && env.e[i]) env.e[i][0] = s;
+      e -= s;
+      __syncthreads();
+    } else {
+      e -= env.e[i][0];
+    }
+  }
+  if (threadIdx.x == 0) out[0] = e;
 }
 
 // Unrestricted functional on 128-point blocks: spin densities and gradients in,
@@ -1306,29 +1364,20 @@ __global__ void weight_potential_kernel(int64_t npts, const double* __restrict__
   }
 }
 
-// rho[q] (+)= sum_i list.rho[i][q] in list order (likewise the gradient).
-__global__ void sum_densities_kernel(DensityList list, int64_t npts, int want_grad, int accumulate,
-                                     double* __restrict__ rho, double* __restrict__ grad) {
+// rho[q] = sum_i list.rho[i][q] in list order (likewise the gradient); rho itself may be listed.
+__global__ void sum_densities_kernel(DensityList list, int64_t npts, int want_grad, double* rho, double* grad) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= npts) return;
-  double r = accumulate ? rho[q] : 0.0;
+  double r = 0.0;
   for (int i = 0; i < list.n; ++i) r += list.rho[i][q];
   rho[q] = r;
   if (want_grad) {
     for (int c = 0; c < 3; ++c) {
-      double g = accumulate ? grad[c * npts + q] : 0.0;
+      double g = 0.0;
       for (int i = 0; i < list.n; ++i) g += list.grad[i][c * npts + q];
       grad[c * npts + q] = g;
     }
   }
-}
-
-// out[0] -= list.rho[0][0], then list.rho[1][0], ... (one thread, fixed order).
-__global__ void subtract_scalars_kernel(DensityList list, double* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double e = out[0];
-  for (int i = 0; i < list.n; ++i) e -= list.rho[i][0];
-  out[0] = e;
 }
 
 __global__ void copy_kernel(const double4* __restrict__ src, double4* __restrict__ dst, int64_t n) {
@@ -1610,12 +1659,11 @@ void launch_reduce_partials(hipStream_t s, const DevBlock* blocks, int bs, int64
 
 void launch_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* rho,
                        const double* grad, const DevBlock* blocks, const double* part, const double* w, double* eps,
-                       double* v, double* g, double* vs, double* gw, double* e_blk, const double* rho_sub,
-                       const double* grad_sub) {
+                       double* v, double* g, double* vs, double* gw, double* e_blk) {
   const int nb = (int)((npts + bs - 1) / bs);
   if (nb <= 0) return;
   hipLaunchKernelGGL(functional_kernel, dim3(nb), dim3(128), 0, s, func, prm, npts, bs, rho, grad, blocks, part, w,
-                     eps, v, g, vs, gw, e_blk, rho_sub, grad_sub, (const PackSys*)nullptr);
+                     eps, v, g, vs, gw, e_blk, (const PackSys*)nullptr);
 }
 
 void launch_functional_packed(hipStream_t s, int func, const XcParams& prm, int nblocks, const DevBlock* blocks,
@@ -1624,7 +1672,7 @@ void launch_functional_packed(hipStream_t s, int func, const XcParams& prm, int 
   hipLaunchKernelGGL(functional_kernel, dim3(nblocks), dim3(128), 0, s, func, prm, (int64_t)0, kTile,
                      (const double*)nullptr, (const double*)nullptr, blocks, (const double*)nullptr,
                      (const double*)nullptr, (double*)nullptr, (double*)nullptr, (double*)nullptr, (double*)nullptr,
-                     (double*)nullptr, (double*)nullptr, (const double*)nullptr, (const double*)nullptr, pack);
+                     (double*)nullptr, (double*)nullptr, pack);
 }
 
 static unsigned pack_grid(int64_t maxnn) {
@@ -1742,15 +1790,26 @@ void launch_weight_potential(hipStream_t s, int64_t npts, const double* w, const
   hipLaunchKernelGGL(weight_potential_kernel, dim3(grid1d(npts, 256)), dim3(256), 0, s, npts, w, v, g, vs, gw);
 }
 
-void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, int want_grad, int accumulate,
-                          double* rho, double* grad) {
+void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, int want_grad, double* rho,
+                          double* grad) {
   if (npts <= 0) return;
-  hipLaunchKernelGGL(sum_densities_kernel, dim3(grid1d(npts, 256)), dim3(256), 0, s, list, npts, want_grad,
-                     accumulate, rho, grad);
+  hipLaunchKernelGGL(sum_densities_kernel, dim3(grid1d(npts, 256)), dim3(256), 0, s, list, npts, want_grad, rho, grad);
 }
 
-void launch_subtract_scalars(hipStream_t s, const DensityList& list, double* out) {
-  hipLaunchKernelGGL(subtract_scalars_kernel, dim3(1), dim3(64), 0, s, list, out);
+void launch_nadd_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, bool potential,
+                            const DensityList& sup, const double* rho_act, const double* grad_act,
+                            const DensityList& pending, double* const* pending_eblk, const double* w, double* vs,
+                            double* gw, double* e_blk) {
+  if (npts <= 0 || (!potential && pending.n == 0)) return;
+  PendingEnergies pend{};
+  pend.dens = pending;
+  for (int i = 0; i < pending.n; ++i) pend.eblk[i] = pending_eblk[i];
+  hipLaunchKernelGGL(nadd_functional_kernel, dim3(grid1d(npts, kTile), (potential ? 1 : 0) + pending.n), dim3(kTile), 0,
+                     s, func, prm, npts, potential ? 0 : 1, sup, rho_act, grad_act, pend, w, vs, gw, e_blk);
+}
+
+void launch_nadd_energy(hipStream_t s, const double* e_blk, int64_t n, const EnvEnergies& env, double* out) {
+  hipLaunchKernelGGL(nadd_energy_kernel, dim3(1), dim3(256), 0, s, e_blk, n, env, out);
 }
 
 void launch_copy(hipStream_t s, const void* src, void* dst, int64_t n32) {

@@ -1617,6 +1617,66 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
 /* Non-additive build: rho_sup = rho_act + sum_env rho_env on the shared grid,
  * v = v[rho_sup] - v[rho_act] integrated with the active basis,
  * E = E[rho_sup] - E[rho_act] - sum_env E[rho_env] (left in ctx->d_energy). */
+// The functional stage of a non-additive build of sub[0] among sub[1..]: w v and w g of v[rho_sup] -
+// v[rho_act] into sub[0], and E[rho_sup] - E[rho_act] - E[rho_env] ... into the context's energy.
+// cached: on the cached densities, keeping each E[rho_env] until its density changes.
+static void run_nadd_functional(const std::vector<xc_bfogc*>& sub, int functional, bool cached) {
+  xc_bfogc* act = sub[0];
+  xc_ctx* ctx = act->ctx;
+  hipStream_t s = ctx->stream;
+  const bool gga = functional_is_gga(functional);
+  const int64_t N = act->grid->npts;
+  const int nxc = (int)((N + kTile - 1) / kTile);
+  const double* w = act->grid->d_w.p;
+  // rho_sup = rho_act + rho_env[0] + ... in list order, inside the functional's launch (what exceeds
+  // its list is summed before it)
+  DensityList sup{};
+  const auto append = [](DensityList& L, const DBuf<double>& rho, const DBuf<double>& grad) {
+    L.rho[L.n] = rho.p;
+    L.grad[L.n++] = grad.p;
+  };
+  if (sub.size() > (size_t)kListMax && !act->d_rho_sup.p) {
+    act->d_rho_sup.alloc(ctx, N);
+    act->d_grad_sup.alloc(ctx, 3 * N);
+  }
+  for (xc_bfogc* b : sub) {
+    if (sup.n == kListMax) {
+      launch_sum_densities(s, sup, N, gga ? 1 : 0, act->d_rho_sup.p, act->d_grad_sup.p);
+      sup.n = 0;
+      append(sup, act->d_rho_sup, act->d_grad_sup);
+    }
+    append(sup, cached ? b->d_rho_c : b->d_rho, cached ? b->d_grad_c : b->d_grad);
+  }
+  // the environment's energies that are missing, beside the functional (kListMax of them per launch)
+  std::vector<xc_bfogc*> missing;
+  for (size_t i = 1; i < sub.size(); ++i)
+    if (!cached || !sub[i]->ecache_valid[functional]) missing.push_back(sub[i]);
+  for (size_t i0 = 0; i0 == 0 || i0 < missing.size(); i0 += kListMax) {
+    DensityList pending{};
+    double* eblk[kListMax] = {};
+    for (size_t i = i0; i < std::min(missing.size(), i0 + kListMax); ++i) {
+      eblk[pending.n] = missing[i]->d_eblk.p;
+      append(pending, cached ? missing[i]->d_rho_c : missing[i]->d_rho,
+             cached ? missing[i]->d_grad_c : missing[i]->d_grad);
+    }
+    launch_nadd_functional(s, functional, ctx->prm, N, i0 == 0, sup, cached ? act->d_rho_c.p : act->d_rho.p,
+                           cached ? act->d_grad_c.p : act->d_grad.p, pending, eblk, w, act->d_vs.p, act->d_gw.p,
+                           act->d_eblk.p);
+  }
+  for (size_t i0 = 1; i0 == 1 || i0 < sub.size(); i0 += kListMax) {
+    EnvEnergies env_e{};
+    for (size_t i = i0; i < std::min(sub.size(), i0 + kListMax); ++i) {
+      xc_bfogc* b = sub[i];
+      const bool valid = cached && b->ecache_valid[functional];
+      env_e.e[env_e.n] = cached ? b->d_ecache.p + functional : nullptr;
+      env_e.eblk[env_e.n++] = valid ? nullptr : b->d_eblk.p;
+    }
+    launch_nadd_energy(s, i0 == 1 ? act->d_eblk.p : nullptr, nxc, env_e, ctx->d_energy);
+  }
+  if (cached)
+    for (xc_bfogc* b : missing) b->ecache_valid[functional] = true;
+}
+
 static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int functional, int precision, double thr,
                          const double* dP_act, const double* const* dP_env, double* dF) {
   xc_ctx* ctx = act->ctx;
@@ -1647,15 +1707,8 @@ static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int func
     require(!fp32 || b->d_t32.p, XC_ERR_STATE, "FP32 contractions need keep_fp32 tiles");
     require(fp32 || b->d_t64.p, XC_ERR_STATE, "FP64 contractions need FP64 tiles");
   }
-  const int n = act->basis->nao;
   const int64_t N = act->grid->npts;
-  const int nxc = (int)((N + kTile - 1) / kTile);
-  if (!act->d_rho_sup.p) {
-    act->d_rho_sup.alloc(ctx, N);
-    act->d_grad_sup.alloc(ctx, 3 * N);
-  }
   hipStream_t s = ctx->stream;
-  const double* w = act->grid->d_w.p;
   ctx->mark();
   if (fp32)
     for (size_t i = 0; i < sub.size(); ++i)
@@ -1668,20 +1721,9 @@ static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int func
     else
       run_density<double>(b, b->d_t64.p, Ps[i], gga ? 1 : 0, ctx->lanes);
     launch_reduce_partials(s, b->d_blocks.p, b->bs, N, b->d_part.p, gga ? 1 : 0, b->d_rho.p, b->d_grad.p, 0);
-    launch_reduce_partials(s, b->d_blocks.p, b->bs, N, b->d_part.p, gga ? 1 : 0, act->d_rho_sup.p,
-                           act->d_grad_sup.p, i == 0 ? 0 : 1);
   }
   ctx->mark();
-  launch_functional(s, functional, ctx->prm, N, kTile, act->d_rho_sup.p, gga ? act->d_grad_sup.p : nullptr, nullptr,
-                    nullptr, w, nullptr, nullptr, nullptr, act->d_vs.p, act->d_gw.p, act->d_eblk.p, act->d_rho.p,
-                    gga ? act->d_grad.p : nullptr);
-  launch_sum(s, act->d_eblk.p, nxc, ctx->d_energy, 0);
-  for (size_t i = 1; i < sub.size(); ++i) {
-    xc_bfogc* b = sub[i];
-    launch_functional(s, functional, ctx->prm, N, kTile, b->d_rho.p, gga ? b->d_grad.p : nullptr, nullptr, nullptr, w,
-                      nullptr, nullptr, nullptr, nullptr, nullptr, b->d_eblk.p);
-    launch_sum(s, b->d_eblk.p, nxc, ctx->d_energy, 1);
-  }
+  run_nadd_functional(sub, functional, false);
   ctx->mark();
   if (fp32)
     run_fock_tiles<float>(act, act->d_t32.p, gga ? 1 : 0, thr, ctx->lanes);
@@ -1907,47 +1949,11 @@ int xc_nadd_fock_build_cached(xc_bfogc* act, int nenv, xc_bfogc* const* env, int
       require(!gga || b->rho_c_grad, XC_ERR_STATE,
               "xc_nadd_fock_build_cached: GGA functional needs cached density gradients");
     }
-    const int n = act->basis->nao;
-    const int64_t N = act->grid->npts;
-    const int nxc = (int)((N + kTile - 1) / kTile);
-    if (!act->d_rho_sup.p) {
-      act->d_rho_sup.alloc(ctx, N);
-      act->d_grad_sup.alloc(ctx, 3 * N);
-    }
     hipStream_t s = ctx->stream;
-    const double* w = act->grid->d_w.p;
     ctx->mark();
     ctx->mark();
-    // rho_sup = rho_act + rho_env[0] + ... in list order, kListMax arrays per launch
-    for (size_t i0 = 0; i0 < sub.size(); i0 += kListMax) {
-      DensityList L{};
-      L.n = (int)std::min<size_t>(kListMax, sub.size() - i0);
-      for (int k = 0; k < L.n; ++k) {
-        L.rho[k] = sub[i0 + k]->d_rho_c.p;
-        L.grad[k] = sub[i0 + k]->d_grad_c.p;
-      }
-      launch_sum_densities(s, L, N, gga ? 1 : 0, i0 == 0 ? 0 : 1, act->d_rho_sup.p, act->d_grad_sup.p);
-    }
     ctx->mark();
-    launch_functional(s, functional, ctx->prm, N, kTile, act->d_rho_sup.p, gga ? act->d_grad_sup.p : nullptr, nullptr,
-                      nullptr, w, nullptr, nullptr, nullptr, act->d_vs.p, act->d_gw.p, act->d_eblk.p, act->d_rho_c.p,
-                      gga ? act->d_grad_c.p : nullptr);
-    launch_sum(s, act->d_eblk.p, nxc, ctx->d_energy, 0);
-    // E[rho_env] per environment subsystem, kept until its density changes
-    for (size_t i = 1; i < sub.size(); ++i) {
-      xc_bfogc* b = sub[i];
-      if (b->ecache_valid[functional]) continue;
-      launch_functional(s, functional, ctx->prm, N, kTile, b->d_rho_c.p, gga ? b->d_grad_c.p : nullptr, nullptr,
-                        nullptr, w, nullptr, nullptr, nullptr, nullptr, nullptr, b->d_eblk.p);
-      launch_sum(s, b->d_eblk.p, nxc, b->d_ecache.p + functional, 0);
-      b->ecache_valid[functional] = true;
-    }
-    for (size_t i0 = 1; i0 < sub.size(); i0 += kListMax) {
-      DensityList L{};
-      L.n = (int)std::min<size_t>(kListMax, sub.size() - i0);
-      for (int k = 0; k < L.n; ++k) L.rho[k] = sub[i0 + k]->d_ecache.p + functional;
-      launch_subtract_scalars(s, L, ctx->d_energy);
-    }
+    run_nadd_functional(sub, functional, true);
     ctx->mark();
     if (precision == XC_PREC_FP32)
       run_fock_tiles<float>(act, act->d_t32.p, gga ? 1 : 0, thr, ctx->lanes);
