@@ -123,7 +123,7 @@ struct PackSys {
   double* F;            // XC matrix out
   double* eblk;         // per-block energies
   double* round;        // rounding-term partials (FP32)
-  double* E;            // E_xc out (device)
+  double* E;            // E_xc out (device or mapped host memory)
   int64_t npts;
   int n;
   int blk0;             // first merged block of this system

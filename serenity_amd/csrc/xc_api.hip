@@ -8,6 +8,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <deque>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -170,6 +172,92 @@ struct Lanes {
 
 struct PackWork;
 
+// Pinned memory that host matrices and tables pass through on their way to and from the device: a
+// ring of pieces, so that a long copy's pieces are moved on the host and over the link at once.
+// Pageable memory copied directly goes through the runtime's own staging: 4.6 KB, 2.65 MB and 15 MB to
+// the host take 22, 160 and 907 us, to the device 15, 88 and 416; to and from pinned memory they take 12, 55
+// and 273 us, and the host's share (34 and 190 us) overlaps.  A kernel of the build's stream as the mover
+// measured the same.  Used under the context's lock and on its stream only.
+struct HostStage {
+  static constexpr size_t kPiece = size_t(1) << 20;
+  static constexpr int kPieces = 4;
+  char* p = nullptr;
+  hipEvent_t ev[kPieces] = {};
+  bool pending[kPieces] = {};
+  int piece = 0;
+  size_t off = 0;
+  void create() {
+    HIPX(hipHostMalloc((void**)&p, kPiece * kPieces, hipHostMallocMapped | hipHostMallocCoherent));
+    for (auto& e : ev) HIPX(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  void destroy() {
+    for (auto& e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (p) (void)hipHostFree(p);
+  }
+  // Room for len <= kPiece bytes; enter(i) is called with piece i free before it is used again.
+  template <typename Enter>
+  char* take(hipStream_t s, size_t len, Enter&& enter) {
+    if (off + len > kPiece) {
+      HIPX(hipEventRecord(ev[piece], s));
+      pending[piece] = true;
+      piece = (piece + 1) % kPieces;
+      off = 0;
+      if (pending[piece]) HIPX(hipEventSynchronize(ev[piece]));
+      pending[piece] = false;
+      enter(piece);
+    }
+    char* q = p + (size_t)piece * kPiece + off;
+    off += (len + 63) / 64 * 64;
+    return q;
+  }
+  // Host -> device; the host memory is free again on return.
+  void up(hipStream_t s, void* dst, const void* src, size_t bytes) {
+    for (size_t o = 0; o < bytes; o += kPiece) {
+      const size_t len = std::min(kPiece, bytes - o);
+      char* q = take(s, len, [](int) {});
+      std::memcpy(q, (const char*)src + o, len);
+      HIPX(hipMemcpyAsync((char*)dst + o, q, len, hipMemcpyHostToDevice, s));
+    }
+  }
+  struct Out {
+    void* host;
+    const void* dev;
+    size_t bytes;
+  };
+  // Device -> host; what the stream held is done and everything is in place on return.
+  void down(hipStream_t s, std::initializer_list<Out> outs) {
+    struct Part {
+      int piece;
+      char *host, *q;
+      size_t len;
+    };
+    std::deque<Part> parts;
+    const auto deliver = [&](int i) {
+      while (!parts.empty() && parts.front().piece == i) {
+        std::memcpy(parts.front().host, parts.front().q, parts.front().len);
+        parts.pop_front();
+      }
+    };
+    for (const Out& o : outs)
+      for (size_t k = 0; o.host && k < o.bytes; k += kPiece) {
+        const size_t len = std::min(kPiece, o.bytes - k);
+        char* q = take(s, len, deliver);
+        HIPX(hipMemcpyAsync(q, (const char*)o.dev + k, len, hipMemcpyDeviceToHost, s));
+        parts.push_back({piece, (char*)o.host + k, q, len});
+      }
+    while (!parts.empty() && parts.front().piece != piece) {
+      const int i = parts.front().piece;
+      HIPX(hipEventSynchronize(ev[i]));
+      deliver(i);
+    }
+    HIPX(hipStreamSynchronize(s));
+    deliver(piece);
+    std::fill(pending, pending + kPieces, false);
+    off = 0;
+  }
+};
+
 struct xc_ctx {
   int device = 0;
   PackWork* pack = nullptr;  // device lists of packed builds (allocated on first use)
@@ -181,8 +269,12 @@ struct xc_ctx {
   Lanes lanes;  // helper lanes of builds on the context stream
   std::recursive_mutex mu;
   int64_t bytes = 0;
-  double last_energy = 0.0;
-  double* d_energy = nullptr;
+  // E_xc of the last build: pinned host memory that the kernels write (a copy of 8 bytes back to the
+  // host costs 15 us more than the wait for the stream)
+  double* energy = nullptr;
+  double* pack_energy = nullptr;  // likewise of a packed build's systems (grown on demand)
+  size_t pack_energies = 0;
+  HostStage stage;
   XcParams prm;
   std::map<void*, size_t> user_allocs;  // buffers handed out by xc_device_alloc
   int live_handles = 0;                 // bases, grids and controllers not yet destroyed
@@ -286,7 +378,7 @@ struct DBuf {
   }
   void upload(xc_ctx* c, const T* host, size_t count) {
     alloc(c, count);
-    if (count) HIPX(hipMemcpyAsync(p, host, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
+    c->stage.up(c->stream, p, host, count * sizeof(T));
   }
   void free_() {
     if (p && ctx) ctx->release(p, n * sizeof(T));
@@ -306,7 +398,7 @@ struct PackWork {
   DBuf<PackSys> sys;
   DBuf<WorkItem> dens;
   DBuf<FockItem> fock[kFockShapes];
-  DBuf<double> round, E;
+  DBuf<double> round;
   hipGraphExec_t exec = nullptr;  // captured build of a repeated composition
   uint64_t last_use = 0;          // packed-build counter at its last use (least recently used is evicted)
   ~PackWork() {
@@ -332,7 +424,7 @@ template <typename T>
 void upload_grow(xc_ctx* ctx, DBuf<T>& b, const std::vector<T>& v) {
   if (v.empty()) return;
   if (b.n < v.size()) b.alloc(ctx, std::max(v.size(), 2 * b.n));
-  HIPX(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
+  ctx->stage.up(ctx->stream, b.p, v.data(), v.size() * sizeof(T));
 }
 
 struct xc_basis {
@@ -492,7 +584,7 @@ struct xc_bfogc {
   DBuf<double> d_P32d;
   DBuf<FockItem> d_fock_items[kFockShapes];
   // per-build work buffers
-  DBuf<double> d_part, d_rho, d_grad, d_vs, d_gw, d_eblk, d_U, d_P, d_F, d_v, d_g, d_E;
+  DBuf<double> d_part, d_rho, d_grad, d_vs, d_gw, d_eblk, d_U, d_P, d_F, d_v, d_g;
   // Fock sub-tile scratch (FP64 size when FP64 tiles are kept, else FP32) and the row entries of
   // the reduce (sorted by AO row, then block)
   int64_t t_elems = 0;
@@ -695,7 +787,9 @@ int xc_ctx_create(int device, xc_ctx** out) {
     noalloc_setup_current_device(device);
     HIPX(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     c->lanes.create(c->stream, true);
-    c->d_energy = (double*)c->alloc(sizeof(double));
+    HIPX(hipHostMalloc((void**)&c->energy, sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
+    *c->energy = 0.0;
+    c->stage.create();
     *out = c;
   });
 }
@@ -708,7 +802,9 @@ int xc_ctx_destroy(xc_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     for (auto e : ctx->ev_pool) (void)hipEventDestroy(e);
-    ctx->release(ctx->d_energy, sizeof(double));
+    ctx->stage.destroy();
+    (void)hipHostFree(ctx->energy);
+    if (ctx->pack_energy) (void)hipHostFree(ctx->pack_energy);
     delete ctx->pack;
     ctx->pack = nullptr;
     for (auto& kv : ctx->pack_graphs) delete kv.second;
@@ -866,11 +962,8 @@ int xc_molecular_grid_device(xc_ctx* ctx, int natoms, const int* Z, const double
                scan_bytes, d_pts.p, d_pw.p);
     HIPX(hipGetLastError());
     int last[2] = {0, 0};
-    if (nc) {
-      HIPX(hipMemcpyAsync(&last[0], d_pos.p + nc - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-      HIPX(hipMemcpyAsync(&last[1], d_keep.p + nc - 1, sizeof(int), hipMemcpyDeviceToHost, st));
-    }
-    HIPX(hipStreamSynchronize(st));
+    if (nc)
+      ctx->stage.down(st, {{&last[0], d_pos.p + nc - 1, sizeof(int)}, {&last[1], d_keep.p + nc - 1, sizeof(int)}});
     const int64_t n = (int64_t)last[0] + last[1];
     const double* res_pts = d_pts.p;
     const double* res_w = d_pw.p;
@@ -896,11 +989,7 @@ int xc_molecular_grid_device(xc_ctx* ctx, int natoms, const int* Z, const double
     *npoints = n;
     *points = (double*)std::malloc(sizeof(double) * 3 * std::max<int64_t>(n, 1));
     *weights = (double*)std::malloc(sizeof(double) * std::max<int64_t>(n, 1));
-    if (n) {
-      HIPX(hipMemcpyAsync(*points, res_pts, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, st));
-      HIPX(hipMemcpyAsync(*weights, res_w, sizeof(double) * n, hipMemcpyDeviceToHost, st));
-    }
-    HIPX(hipStreamSynchronize(st));
+    ctx->stage.down(st, {{*points, res_pts, sizeof(double) * 3 * n}, {*weights, res_w, sizeof(double) * n}});
     if (npoints_before_cut) *npoints_before_cut = nc;
   });
 }
@@ -1122,8 +1211,7 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
                     basis->d_coef.p, radial_threshold, d_pos.p, d_count.p);
       HIPX(hipGetLastError());
       std::vector<int> count(2 * (size_t)nb);
-      HIPX(hipMemcpyAsync(count.data(), d_count.p, sizeof(int) * count.size(), hipMemcpyDeviceToHost, ctx->stream));
-      HIPX(hipStreamSynchronize(ctx->stream));
+      ctx->stage.down(ctx->stream, {{count.data(), d_count.p, sizeof(int) * count.size()}});
       // 2. the blocks' offsets and work items; their lists (compact AO indices padded to kAoPad,
       // significant shells, row entries) are filled on the device
       bf->blocks.resize(nb);
@@ -1249,8 +1337,7 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       const int64_t t_doubles = keep_fp32 != 2 ? bf->t_elems : (bf->t_elems + 1) / 2;
       bf->d_T.alloc(ctx, (size_t)std::max<int64_t>(t_doubles, 1));
       bf->d_P.alloc(ctx, (size_t)n * n);
-      bf->d_F.alloc(ctx, (size_t)n * n);
-      bf->d_E.alloc(ctx, 1);
+      bf->d_F.alloc(ctx, (size_t)n * n + 1);  // a server build's E_xc behind it
       if (keep_fp32) {
         bf->d_P32.alloc(ctx, (size_t)n * n);
         bf->d_round.alloc(ctx, 2 * (size_t)std::max(finalize_blocks(n), n));
@@ -1376,14 +1463,12 @@ int xc_density(xc_bfogc* bf, const double* P, double* rho, double* grad, int* no
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     const int n = bf->basis->nao;
     const int64_t N = bf->grid->npts;
-    HIPX(hipMemcpyAsync(bf->d_P.p, P, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
+    ctx->stage.up(ctx->stream, bf->d_P.p, P, sizeof(double) * n * n);
     run_density<double>(bf, bf->d_t64.p, bf->d_P.p, grad ? 1 : 0, ctx->lanes);
     launch_reduce_partials(ctx->stream, bf->d_blocks.p, bf->bs, N, bf->d_part.p, grad ? 1 : 0, bf->d_rho.p,
                            bf->d_grad.p);
     HIPX(hipGetLastError());
-    HIPX(hipMemcpyAsync(rho, bf->d_rho.p, sizeof(double) * N, hipMemcpyDeviceToHost, ctx->stream));
-    if (grad) HIPX(hipMemcpyAsync(grad, bf->d_grad.p, sizeof(double) * 3 * N, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
+    ctx->stage.down(ctx->stream, {{rho, bf->d_rho.p, sizeof(double) * N}, {grad, bf->d_grad.p, sizeof(double) * 3 * N}});
     if (nonneg)
       for (int b = 0; b < bf->nblocks; ++b) nonneg[b] = bf->blocks[b].nb > 0 ? 1 : 0;
   });
@@ -1412,17 +1497,12 @@ int xc_functional(xc_ctx* ctx, int functional, int64_t npts, int block_size, con
                       d_eps.p, d_v.p, d_g.p, nullptr, nullptr, d_eblk.p);
     launch_sum(ctx->stream, d_eblk.p, nxc, d_E.p);
     HIPX(hipGetLastError());
-    if (eps) HIPX(hipMemcpyAsync(eps, d_eps.p, sizeof(double) * npts, hipMemcpyDeviceToHost, ctx->stream));
-    if (v) HIPX(hipMemcpyAsync(v, d_v.p, sizeof(double) * npts, hipMemcpyDeviceToHost, ctx->stream));
-    if (g) {
-      if (gga)
-        HIPX(hipMemcpyAsync(g, d_g.p, sizeof(double) * 3 * npts, hipMemcpyDeviceToHost, ctx->stream));
-      else
-        std::fill(g, g + 3 * npts, 0.0);
-    }
+    if (g && !gga) std::fill(g, g + 3 * npts, 0.0);
     double E = 0.0;
-    HIPX(hipMemcpyAsync(&E, d_E.p, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
+    ctx->stage.down(ctx->stream, {{eps, d_eps.p, sizeof(double) * npts},
+                                  {v, d_v.p, sizeof(double) * npts},
+                                  {gga ? g : nullptr, d_g.p, sizeof(double) * 3 * npts},
+                                  {&E, d_E.p, sizeof(double)}});
     if (energy) *energy = E;
   });
 }
@@ -1453,8 +1533,7 @@ int xc_functional_device_noalloc(xc_ctx* ctx, int functional, int64_t npts, int 
     launch_sum(ctx->stream, scr, nxc, scr + kNoallocBlocks);
     HIPX(hipGetLastError());
     if (energy) {
-      HIPX(hipMemcpyAsync(energy, scr + kNoallocBlocks, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-      HIPX(hipStreamSynchronize(ctx->stream));
+      ctx->stage.down(ctx->stream, {{energy, scr + kNoallocBlocks, sizeof(double)}});
     }
   });
 }
@@ -1469,16 +1548,15 @@ int xc_fock_add(xc_bfogc* bf, double thr, const double* v, const double* g, doub
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     const int n = bf->basis->nao;
     const int64_t N = bf->grid->npts;
-    HIPX(hipMemcpyAsync(bf->d_v.p, v, sizeof(double) * N, hipMemcpyHostToDevice, ctx->stream));
-    if (g) HIPX(hipMemcpyAsync(bf->d_g.p, g, sizeof(double) * 3 * N, hipMemcpyHostToDevice, ctx->stream));
+    ctx->stage.up(ctx->stream, bf->d_v.p, v, sizeof(double) * N);
+    if (g) ctx->stage.up(ctx->stream, bf->d_g.p, g, sizeof(double) * 3 * N);
     launch_weight_potential(ctx->stream, N, bf->grid->d_w.p, bf->d_v.p, g ? bf->d_g.p : nullptr, bf->d_vs.p,
                             bf->d_gw.p);
     run_fock<double>(bf, bf->d_t64.p, g ? 1 : 0, thr, ctx->lanes);
-    HIPX(hipMemcpyAsync(bf->d_F.p, F, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
+    ctx->stage.up(ctx->stream, bf->d_F.p, F, sizeof(double) * n * n);
     launch_finalize(ctx->stream, bf->d_U.p, bf->d_F.p, n, 1);
     HIPX(hipGetLastError());
-    HIPX(hipMemcpyAsync(F, bf->d_F.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
+    ctx->stage.down(ctx->stream, {{F, bf->d_F.p, sizeof(double) * n * n}});
   });
 }
 
@@ -1616,7 +1694,7 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
 
 /* Non-additive build: rho_sup = rho_act + sum_env rho_env on the shared grid,
  * v = v[rho_sup] - v[rho_act] integrated with the active basis,
- * E = E[rho_sup] - E[rho_act] - sum_env E[rho_env] (left in ctx->d_energy). */
+ * E = E[rho_sup] - E[rho_act] - sum_env E[rho_env] (left in ctx->energy). */
 // The functional stage of a non-additive build of sub[0] among sub[1..]: w v and w g of v[rho_sup] -
 // v[rho_act] into sub[0], and E[rho_sup] - E[rho_act] - E[rho_env] ... into the context's energy.
 // cached: on the cached densities, keeping each E[rho_env] until its density changes.
@@ -1671,7 +1749,7 @@ static void run_nadd_functional(const std::vector<xc_bfogc*>& sub, int functiona
       env_e.e[env_e.n] = cached ? b->d_ecache.p + functional : nullptr;
       env_e.eblk[env_e.n++] = valid ? nullptr : b->d_eblk.p;
     }
-    launch_nadd_energy(s, i0 == 1 ? act->d_eblk.p : nullptr, nxc, env_e, ctx->d_energy);
+    launch_nadd_energy(s, i0 == 1 ? act->d_eblk.p : nullptr, nxc, env_e, ctx->energy);
   }
   if (cached)
     for (xc_bfogc* b : missing) b->ecache_valid[functional] = true;
@@ -1741,7 +1819,7 @@ static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int func
 /* Unrestricted non-additive build (NAddFuncPotential<UNRESTRICTED>::getMatrix): spin
  * densities of every subsystem on the shared grid, rho_sup^s = sum of them,
  * v^s = v^s[rho_sup] - v^s[rho_act] integrated with the active basis per spin,
- * E = E[sup] - E[act] - sum_env E[env] (left in ctx->d_energy). */
+ * E = E[sup] - E[act] - sum_env E[env] (left in ctx->energy). */
 static void enqueue_nadd_pol(xc_bfogc* act, int nenv, xc_bfogc* const* env, int functional, int precision,
                              double thr, const double* dPa_act, const double* dPb_act, const double* const* dPa_env,
                              const double* const* dPb_env, double* dFa, double* dFb) {
@@ -1814,12 +1892,12 @@ static void enqueue_nadd_pol(xc_bfogc* act, int nenv, xc_bfogc* const* env, int 
   launch_functional_pol(s, functional, ctx->prm, N, kTile, sup_r[0], sup_g[0], sup_r[1], sup_g[1], w, act->d_vs.p,
                         act->d_gw.p, act->d_vs_b.p, act->d_gw_b.p, act->d_eblk.p, act->d_rho.p, act->d_grad.p,
                         act->d_rho_b.p, act->d_grad_b.p);
-  launch_sum(s, act->d_eblk.p, nxc, ctx->d_energy, 0);
+  launch_sum(s, act->d_eblk.p, nxc, ctx->energy, 0);
   for (size_t i = 1; i < sub.size(); ++i) {
     xc_bfogc* b = sub[i];
     launch_functional_pol(s, functional, ctx->prm, N, kTile, b->d_rho.p, b->d_grad.p, b->d_rho_b.p, b->d_grad_b.p, w,
                           nullptr, nullptr, nullptr, nullptr, b->d_eblk.p);
-    launch_sum(s, b->d_eblk.p, nxc, ctx->d_energy, 1);
+    launch_sum(s, b->d_eblk.p, nxc, ctx->energy, 1);
   }
   const double* vs[2] = {act->d_vs.p, act->d_vs_b.p};
   const double* gw[2] = {act->d_gw.p, act->d_gw_b.p};
@@ -1862,8 +1940,8 @@ int xc_nadd_fock_build_unrestricted(xc_bfogc* active, int nenv, xc_bfogc* const*
       const int m = b->basis->nao;
       const double* ha = i == 0 ? Pa_active : Pa_env[i - 1];
       const double* hb = i == 0 ? Pb_active : Pb_env[i - 1];
-      HIPX(hipMemcpyAsync(b->d_P.p, ha, sizeof(double) * m * m, hipMemcpyHostToDevice, ctx->stream));
-      HIPX(hipMemcpyAsync(b->d_Pb.p, hb, sizeof(double) * m * m, hipMemcpyHostToDevice, ctx->stream));
+      ctx->stage.up(ctx->stream, b->d_P.p, ha, sizeof(double) * m * m);
+      ctx->stage.up(ctx->stream, b->d_Pb.p, hb, sizeof(double) * m * m);
       if (i > 0) {
         dPa[i - 1] = b->d_P.p;
         dPb[i - 1] = b->d_Pb.p;
@@ -1872,11 +1950,8 @@ int xc_nadd_fock_build_unrestricted(xc_bfogc* active, int nenv, xc_bfogc* const*
     enqueue_nadd_pol(active, nenv, env, functional, precision, thr, active->d_P.p, active->d_Pb.p, dPa.data(),
                      dPb.data(), active->d_F.p, active->d_Fb.p);
     const int n = active->basis->nao;
-    HIPX(hipMemcpyAsync(Fa, active->d_F.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipMemcpyAsync(Fb, active->d_Fb.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
-    if (energy) *energy = ctx->last_energy;
+    ctx->stage.down(ctx->stream, {{Fa, active->d_F.p, sizeof(double) * n * n}, {Fb, active->d_Fb.p, sizeof(double) * n * n}});
+    if (energy) *energy = *ctx->energy;
   });
 }
 
@@ -1967,9 +2042,8 @@ int xc_nadd_fock_build_cached(xc_bfogc* act, int nenv, xc_bfogc* const* env, int
     ctx->mark();
     HIPX(hipGetLastError());
     if (energy) {
-      HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, s));
       HIPX(hipStreamSynchronize(s));
-      *energy = ctx->last_energy;
+      *energy = *ctx->energy;
     }
   });
 }
@@ -1984,9 +2058,8 @@ int xc_nadd_fock_build_device(xc_bfogc* active, int nenv, xc_bfogc* const* env, 
     require_idle(active, nenv, env, "xc_nadd_fock_build_device");
     enqueue_nadd(active, nenv, env, functional, precision, thr, dP_active, dP_env, dF);
     if (energy) {
-      HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
       HIPX(hipStreamSynchronize(ctx->stream));
-      *energy = ctx->last_energy;
+      *energy = *ctx->energy;
     }
   });
 }
@@ -2000,20 +2073,18 @@ int xc_nadd_fock_build(xc_bfogc* active, int nenv, xc_bfogc* const* env, int fun
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     require_idle(active, nenv, env, "xc_nadd_fock_build");
     const int n = active->basis->nao;
-    HIPX(hipMemcpyAsync(active->d_P.p, P_active, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
+    ctx->stage.up(ctx->stream, active->d_P.p, P_active, sizeof(double) * n * n);
     std::vector<const double*> dP(nenv);
     for (int i = 0; i < nenv; ++i) {
       require(env[i] && P_env[i], XC_ERR_ARG, "xc_nadd_fock_build: null environment controller or density");
       require(env[i]->ctx == ctx, XC_ERR_ARG, "xc_nadd_fock_build: controllers live on different contexts");
       const int m = env[i]->basis->nao;
-      HIPX(hipMemcpyAsync(env[i]->d_P.p, P_env[i], sizeof(double) * m * m, hipMemcpyHostToDevice, ctx->stream));
+      ctx->stage.up(ctx->stream, env[i]->d_P.p, P_env[i], sizeof(double) * m * m);
       dP[i] = env[i]->d_P.p;
     }
     enqueue_nadd(active, nenv, env, functional, precision, thr, active->d_P.p, dP.data(), active->d_F.p);
-    HIPX(hipMemcpyAsync(F, active->d_F.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
-    if (energy) *energy = ctx->last_energy;
+    ctx->stage.down(ctx->stream, {{F, active->d_F.p, sizeof(double) * n * n}});
+    if (energy) *energy = *ctx->energy;
   });
 }
 
@@ -2023,11 +2094,10 @@ int xc_fock_build_device(xc_bfogc* bf, int functional, int precision, double thr
     require(bf && dP && dF, XC_ERR_ARG, "xc_fock_build_device: null argument");
     xc_ctx* ctx = bf->ctx;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-    enqueue_build(bf, functional, precision, thr, dP, dF, ctx->lanes, ctx->d_energy);
+    enqueue_build(bf, functional, precision, thr, dP, dF, ctx->lanes, ctx->energy);
     if (energy) {
-      HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
       HIPX(hipStreamSynchronize(ctx->stream));
-      *energy = ctx->last_energy;
+      *energy = *ctx->energy;
     }
   });
 }
@@ -2139,10 +2209,18 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
     }
     PackWork& pw = *pwp;
     if (pw.round.n < (size_t)nsys * kPackRoundBlocks) pw.round.alloc(ctx, (size_t)2 * nsys * kPackRoundBlocks);
-    if (pw.E.n < (size_t)nsys) pw.E.alloc(ctx, (size_t)2 * nsys);
+    if (ctx->pack_energies < (size_t)nsys) {
+      HIPX(hipStreamSynchronize(ctx->stream));
+      if (ctx->pack_energy) (void)hipHostFree(ctx->pack_energy);
+      ctx->pack_energy = nullptr;
+      ctx->pack_energies = 0;
+      const size_t want = std::max<size_t>(2 * (size_t)nsys, 64);
+      HIPX(hipHostMalloc((void**)&ctx->pack_energy, sizeof(double) * want, hipHostMallocMapped | hipHostMallocCoherent));
+      ctx->pack_energies = want;
+    }
     for (int i = 0; i < nsys; ++i) {
       sys[i].round = pw.round.p + (size_t)i * kPackRoundBlocks;
-      sys[i].E = pw.E.p + i;
+      sys[i].E = ctx->pack_energy + i;
     }
     hipStream_t s = ctx->stream;
     const Lanes& L = ctx->lanes;
@@ -2212,9 +2290,8 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       }
     }
     HIPX(hipGetLastError());
-    HIPX(hipMemcpyAsync(energies, pw.E.p, sizeof(double) * nsys, hipMemcpyDeviceToHost, s));
     HIPX(hipStreamSynchronize(s));
-    ctx->last_energy = energies[nsys - 1];
+    std::copy(ctx->pack_energy, ctx->pack_energy + nsys, energies);
   });
 }
 
@@ -2244,9 +2321,9 @@ void geom_gradient(xc_bfogc* bf, int functional, const double* Pa, const double*
   }
   if ((int64_t)bf->d_gout.n < 3 * (int64_t)natoms) bf->d_gout.alloc(ctx, (size_t)3 * natoms);
   if (Pb) ensure_pol_buffers(bf, false);
-  HIPX(hipMemcpyAsync(bf->d_ao_atom.p, ao_atom, sizeof(int) * n, hipMemcpyHostToDevice, s));
-  HIPX(hipMemcpyAsync(bf->d_P.p, Pa, sizeof(double) * n * n, hipMemcpyHostToDevice, s));
-  if (Pb) HIPX(hipMemcpyAsync(bf->d_Pb.p, Pb, sizeof(double) * n * n, hipMemcpyHostToDevice, s));
+  ctx->stage.up(s, bf->d_ao_atom.p, ao_atom, sizeof(int) * n);
+  ctx->stage.up(s, bf->d_P.p, Pa, sizeof(double) * n * n);
+  if (Pb) ctx->stage.up(s, bf->d_Pb.p, Pb, sizeof(double) * n * n);
   // density and functional as in a Fock build (FP64), then the gradient contractions
   if (!Pb) {
     run_density<double>(bf, bf->d_t64.p, bf->d_P.p, gga ? 1 : 0, ctx->lanes);
@@ -2278,12 +2355,10 @@ void geom_gradient(xc_bfogc* bf, int functional, const double* Pa, const double*
     launch_gradient(s, bf->d_dens_work.p, (int)bf->dens_work.size(), bf->d_blocks.p, bf->d_ao_idx.p, bf->d_t64.p,
                     bf->d_Pb.p, n, bf->d_vs_b.p, bf->d_gw_b.p, gga ? 1 : 0, N, bf->d_gacc.p);
   launch_gradient_atoms(s, bf->d_gacc.p, bf->d_ao_atom.p, n, natoms, bf->d_gout.p);
-  launch_sum(s, bf->d_eblk.p, nxc, ctx->d_energy);
+  launch_sum(s, bf->d_eblk.p, nxc, ctx->energy);
   HIPX(hipGetLastError());
-  HIPX(hipMemcpyAsync(grad, bf->d_gout.p, sizeof(double) * 3 * natoms, hipMemcpyDeviceToHost, s));
-  HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, s));
-  HIPX(hipStreamSynchronize(s));
-  if (energy) *energy = ctx->last_energy;
+  ctx->stage.down(s, {{grad, bf->d_gout.p, sizeof(double) * 3 * natoms}});
+  if (energy) *energy = *ctx->energy;
 }
 }  // namespace
 
@@ -2308,15 +2383,12 @@ int xc_fock_build_unrestricted(xc_bfogc* bf, int functional, int precision, doub
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     const int n = bf->basis->nao;
     ensure_pol_buffers(bf, precision == XC_PREC_FP32);
-    HIPX(hipMemcpyAsync(bf->d_P.p, Pa, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    HIPX(hipMemcpyAsync(bf->d_Pb.p, Pb, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
+    ctx->stage.up(ctx->stream, bf->d_P.p, Pa, sizeof(double) * n * n);
+    ctx->stage.up(ctx->stream, bf->d_Pb.p, Pb, sizeof(double) * n * n);
     enqueue_build_pol(bf, functional, precision, thr, bf->d_P.p, bf->d_Pb.p, bf->d_F.p, bf->d_Fb.p, ctx->lanes,
-                      ctx->d_energy);
-    HIPX(hipMemcpyAsync(Fa, bf->d_F.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipMemcpyAsync(Fb, bf->d_Fb.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
-    if (energy) *energy = ctx->last_energy;
+                      ctx->energy);
+    ctx->stage.down(ctx->stream, {{Fa, bf->d_F.p, sizeof(double) * n * n}, {Fb, bf->d_Fb.p, sizeof(double) * n * n}});
+    if (energy) *energy = *ctx->energy;
   });
 }
 
@@ -2326,11 +2398,10 @@ int xc_fock_build_unrestricted_device(xc_bfogc* bf, int functional, int precisio
     require(bf && dPa && dPb && dFa && dFb, XC_ERR_ARG, "xc_fock_build_unrestricted_device: null argument");
     xc_ctx* ctx = bf->ctx;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-    enqueue_build_pol(bf, functional, precision, thr, dPa, dPb, dFa, dFb, ctx->lanes, ctx->d_energy);
+    enqueue_build_pol(bf, functional, precision, thr, dPa, dPb, dFa, dFb, ctx->lanes, ctx->energy);
     if (energy) {
-      HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
       HIPX(hipStreamSynchronize(ctx->stream));
-      *energy = ctx->last_energy;
+      *energy = *ctx->energy;
     }
   });
 }
@@ -2514,7 +2585,7 @@ int xc_coulomb_rhs(xc_coulomb* jc, const double* P, double* b) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     hipStream_t s = ctx->stream;
     const int n = jc->basis->nao;
-    HIPX(hipMemcpyAsync(jc->d_P.p, P, sizeof(double) * n * n, hipMemcpyHostToDevice, s));
+    ctx->stage.up(s, jc->d_P.p, P, sizeof(double) * n * n);
     over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
                [&](int c, hipStream_t st) {
       launch_jdens(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p, jc->basis->d_shells.p,
@@ -2529,8 +2600,7 @@ int xc_coulomb_rhs(xc_coulomb* jc, const double* P, double* b) {
                     jc->d_cart_off.p, jc->d_U.p, jc->d_bc.p);
     HIPX(hipGetLastError());
     std::vector<double> bc(jc->ncart_aux);
-    HIPX(hipMemcpyAsync(bc.data(), jc->d_bc.p, sizeof(double) * bc.size(), hipMemcpyDeviceToHost, s));
-    HIPX(hipStreamSynchronize(s));
+    ctx->stage.down(s, {{bc.data(), jc->d_bc.p, sizeof(double) * bc.size()}});
     // Cartesian -> auxiliary AO: b_f = sum_c M[f][c] b_c
     for (int k = 0; k < jc->aux->nshell; ++k) {
       const DevShell& S = jc->aux->shells[k];
@@ -2558,7 +2628,7 @@ int xc_coulomb_matrix(xc_coulomb* jc, const double* c, double* J) {
         for (int q = 0; q < S.ncart; ++q)
           cc[jc->cart_off[k] + q] += c[S.ao_off + f] * jc->aux->ang[S.ang_off + f * S.ncart + q];
     }
-    HIPX(hipMemcpyAsync(jc->d_cc.p, cc.data(), sizeof(double) * jc->ncart_aux, hipMemcpyHostToDevice, s));
+    ctx->stage.up(s, jc->d_cc.p, cc.data(), sizeof(double) * jc->ncart_aux);
     launch_jaux_in(s, jc->view, jc->naux, jc->d_prim_shell.p, jc->aux->d_shells.p, jc->d_prim_coef.p,
                    jc->d_cart_off.p, jc->d_cc.p, jc->d_U.p);
     launch_fill(s, jc->d_V.p, jc->herm_total, 0.0);
@@ -2572,8 +2642,7 @@ int xc_coulomb_matrix(xc_coulomb* jc, const double* c, double* J) {
                        jc->basis->d_shells.p, jc->basis->d_ang.p, jc->view, jc->d_V.p, n, jc->d_J.p);
     });
     HIPX(hipGetLastError());
-    HIPX(hipMemcpyAsync(J, jc->d_J.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, s));
-    HIPX(hipStreamSynchronize(s));
+    ctx->stage.down(s, {{J, jc->d_J.p, sizeof(double) * n * n}});
   });
 }
 
@@ -2581,9 +2650,8 @@ int xc_last_energy(xc_ctx* ctx, double* energy) {
   return guarded([&] {
     require(ctx && energy, XC_ERR_ARG, "null argument");
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-    HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPX(hipStreamSynchronize(ctx->stream));
-    *energy = ctx->last_energy;
+    *energy = *ctx->energy;
   });
 }
 
@@ -2594,12 +2662,10 @@ int xc_fock_build(xc_bfogc* bf, int functional, int precision, double thr, const
     xc_ctx* ctx = bf->ctx;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     const int n = bf->basis->nao;
-    HIPX(hipMemcpyAsync(bf->d_P.p, P, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, ctx->lanes, ctx->d_energy);
-    HIPX(hipMemcpyAsync(F, bf->d_F.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipMemcpyAsync(&ctx->last_energy, ctx->d_energy, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPX(hipStreamSynchronize(ctx->stream));
-    if (energy) *energy = ctx->last_energy;
+    ctx->stage.up(ctx->stream, bf->d_P.p, P, sizeof(double) * n * n);
+    enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, ctx->lanes, ctx->energy);
+    ctx->stage.down(ctx->stream, {{F, bf->d_F.p, sizeof(double) * n * n}});
+    if (energy) *energy = *ctx->energy;
   });
 }
 
@@ -2690,9 +2756,8 @@ struct xc_server {
     hipStream_t stream = nullptr;
     Lanes lanes;
     hipEvent_t done = nullptr;
-    double* h_P = nullptr;  // pinned staging of P, F and E
+    double* h_P = nullptr;  // pinned staging of P, and of F with E behind it
     double* h_F = nullptr;
-    double* h_E = nullptr;
     size_t cap = 0;
     bool busy = false;
     int64_t ticket = -1;
@@ -2718,7 +2783,7 @@ void server_slot_release(xc_server::Slot& sl) {
 
 void server_finish(xc_server::Slot& sl, int n) {
   std::memcpy(sl.user_F, sl.h_F, sizeof(double) * (size_t)n * n);
-  if (sl.user_E) *sl.user_E = *sl.h_E;
+  if (sl.user_E) *sl.user_E = sl.h_F[(size_t)n * n];
   sl.bf->in_flight = false;
   sl.busy = false;
   sl.bf = nullptr;
@@ -2749,14 +2814,12 @@ int xc_server_create(xc_ctx* ctx, int nslots, int use_graphs, xc_server** out) {
         // concurrency comes from the slots: a slot's build stays on its own stream
         sl.lanes.create(sl.stream, false);
         HIPX(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
-        HIPX(hipHostMalloc((void**)&sl.h_E, sizeof(double), hipHostMallocDefault));
       }
     } catch (...) {
       for (auto& sl : srv->slots) {
         sl.lanes.destroy();
         if (sl.stream) (void)hipStreamDestroy(sl.stream);
         if (sl.done) (void)hipEventDestroy(sl.done);
-        if (sl.h_E) (void)hipHostFree(sl.h_E);
       }
       delete srv;
       throw;
@@ -2777,7 +2840,6 @@ int xc_server_destroy(xc_server* srv) {
         sl.busy = false;
       }
       server_slot_release(sl);
-      (void)hipHostFree(sl.h_E);
       (void)hipEventDestroy(sl.done);
       sl.lanes.destroy();
       (void)hipStreamDestroy(sl.stream);
@@ -2808,7 +2870,7 @@ int xc_server_submit(xc_server* srv, xc_bfogc* bf, int functional, int precision
     if (sl->cap < nn) {
       server_slot_release(*sl);
       HIPX(hipHostMalloc((void**)&sl->h_P, sizeof(double) * nn, hipHostMallocDefault));
-      HIPX(hipHostMalloc((void**)&sl->h_F, sizeof(double) * nn, hipHostMallocDefault));
+      HIPX(hipHostMalloc((void**)&sl->h_F, sizeof(double) * (nn + 1), hipHostMallocDefault));
       sl->cap = nn;
     }
     std::memcpy(sl->h_P, P, sizeof(double) * nn);
@@ -2823,7 +2885,7 @@ int xc_server_submit(xc_server* srv, xc_bfogc* bf, int functional, int precision
         hipGraph_t graph = nullptr;
         HIPX(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
-          enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, sl->lanes, bf->d_E.p);
+          enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, sl->lanes, bf->d_F.p + nn);
         } catch (...) {
           (void)hipStreamEndCapture(s, &graph);
           if (graph) (void)hipGraphDestroy(graph);
@@ -2839,10 +2901,9 @@ int xc_server_submit(xc_server* srv, xc_bfogc* bf, int functional, int precision
       HIPX(hipGraphLaunch(it->second, s));
       ++srv->graph_launches;
     } else {
-      enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, sl->lanes, bf->d_E.p);
+      enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, sl->lanes, bf->d_F.p + nn);
     }
-    HIPX(hipMemcpyAsync(sl->h_F, bf->d_F.p, sizeof(double) * nn, hipMemcpyDeviceToHost, s));
-    HIPX(hipMemcpyAsync(sl->h_E, bf->d_E.p, sizeof(double), hipMemcpyDeviceToHost, s));
+    HIPX(hipMemcpyAsync(sl->h_F, bf->d_F.p, sizeof(double) * (nn + 1), hipMemcpyDeviceToHost, s));
     HIPX(hipEventRecord(sl->done, s));
     sl->busy = true;
     sl->bf = bf;

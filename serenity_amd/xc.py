@@ -191,6 +191,24 @@ def overlap_matrix(basis):
     return S
 
 
+class _LibraryBuffer:
+    """Host memory that the library allocated, freed with the last array that views it."""
+
+    def __init__(self, pointer, shape):
+        self._pointer = C.cast(pointer, C.c_void_p)
+        self.__array_interface__ = dict(shape=shape, typestr="<f8", data=(self._pointer.value, False), version=3)
+
+    def __del__(self):
+        try:
+            _lib.lib().xc_free_host(self._pointer)
+        except Exception:
+            pass
+
+
+def _library_array(pointer, shape):
+    return np.asarray(_LibraryBuffer(pointer, shape))
+
+
 class GridController:
     """Grid points (N x 3 here; 3 x N column-major in memory) and weights."""
 
@@ -230,13 +248,9 @@ def molecular_grid(Z, coords_bohr, grid_type="SSF", radial_type="AHLRICHS", accu
         check(L.xc_molecular_grid(*args))
     else:
         check(L.xc_molecular_grid_device(ctx.handle, *args))
-    try:
-        N = n.value
-        pts = np.ctypeslib.as_array(pp, shape=(N * 3,)).copy().reshape(N, 3)
-        w = np.ctypeslib.as_array(pw, shape=(N,)).copy()
-    finally:
-        L.xc_free_host(C.cast(pp, C.c_void_p))
-        L.xc_free_host(C.cast(pw, C.c_void_p))
+    N = n.value
+    pts = _library_array(pp, (N, 3))
+    w = _library_array(pw, (N,))
     g = GridController(pts, w)
     if return_before_cut:
         return g, nb.value
@@ -518,7 +532,7 @@ class FuncPotential:
         Pf = np.asfortranarray(P, dtype=np.float64)
         if Pf.shape != (n, n):
             raise XCError(1, "FuncPotential: density matrix is %s, basis has %d functions" % (Pf.shape, n))
-        F = np.zeros((n, n), order="F")
+        F = np.empty((n, n), order="F")
         E = C.c_double()
         check(_lib.lib().xc_fock_build(self.bfogc.handle, FUNCTIONALS[self.functional], PRECISIONS[self.precision],
                                        float(self.blockAveThreshold), Pf.ctypes.data_as(_lib.dp),
@@ -539,8 +553,8 @@ class FuncPotential:
         if Pa.shape != (n, n) or Pb.shape != (n, n):
             raise XCError(1, "FuncPotential: spin density matrices are %s and %s, basis has %d functions"
                           % (Pa.shape, Pb.shape, n))
-        Fa = np.zeros((n, n), order="F")
-        Fb = np.zeros((n, n), order="F")
+        Fa = np.empty((n, n), order="F")
+        Fb = np.empty((n, n), order="F")
         E = C.c_double()
         check(_lib.lib().xc_fock_build_unrestricted(self.bfogc.handle, FUNCTIONALS[self.functional],
                                                     PRECISIONS[self.precision], float(self.blockAveThreshold),
@@ -652,7 +666,7 @@ class NAddFuncPotential:
                               % (Pf.shape, m))
             Pe.append(Pf)
         ptrs = (_lib.dp * max(1, len(Pe)))(*[p.ctypes.data_as(_lib.dp) for p in Pe])
-        F = np.zeros((n, n), order="F")
+        F = np.empty((n, n), order="F")
         E = C.c_double()
         check(_lib.lib().xc_nadd_fock_build(self.active.handle, len(Pe), self._env_handles(),
                                             FUNCTIONALS[self.functional], PRECISIONS[self.precision],
@@ -680,7 +694,7 @@ class NAddFuncPotential:
         Peb = [mat(P, c.getNBasisFunctions(), "environment beta") for c, P in zip(self.environment, Pb_environment)]
         pa = (_lib.dp * max(1, len(Pea)))(*[p.ctypes.data_as(_lib.dp) for p in Pea])
         pb = (_lib.dp * max(1, len(Peb)))(*[p.ctypes.data_as(_lib.dp) for p in Peb])
-        Fa, Fb = np.zeros((n, n), order="F"), np.zeros((n, n), order="F")
+        Fa, Fb = np.empty((n, n), order="F"), np.empty((n, n), order="F")
         E = C.c_double()
         check(_lib.lib().xc_nadd_fock_build_unrestricted(
             self.active.handle, len(Pea), self._env_handles(), FUNCTIONALS[self.functional],
@@ -746,7 +760,7 @@ class Server(_Handle):
         Pf = np.asfortranarray(P, dtype=np.float64)
         if Pf.shape != (n, n):
             raise XCError(1, "Server.submit: density matrix is %s, basis has %d functions" % (Pf.shape, n))
-        F = np.zeros((n, n), order="F")
+        F = np.empty((n, n), order="F")
         E = (C.c_double * 1)()
         t = C.c_int64()
         rc = _lib.lib().xc_server_submit(self.handle, bfogc.handle, FUNCTIONALS[functional], PRECISIONS[precision],
