@@ -766,10 +766,28 @@ __global__ __launch_bounds__(128) void nadd_functional_kernel(int func, XcParams
   double r = 0.0, g[3] = {0.0, 0.0, 0.0};
   if (in) {
     if (y == 0) {
-      for (int i = 0; i < sup.n; ++i) r += sup.rho[i][q];
-      if (gga)
-        for (int c = 0; c < 3; ++c)
-          for (int i = 0; i < sup.n; ++i) g[c] += sup.grad[i][c * npts + q];
+      // four densities' loads at a time (one after another they are a chain of memory latencies:
+      // 44 us for PBE over 13 densities with gradients at 103 000 points, 37 so)
+      constexpr int U = 4;
+      for (int i0 = 0; i0 < sup.n; i0 += U) {
+        double x[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int i = min(i0 + u, sup.n - 1);
+          x[u][0] = to_global(sup.rho[i])[q];
+          if (gga)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) x[u][1 + c] = to_global(sup.grad[i])[c * npts + q];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (i0 + u < sup.n) {
+            r += x[u][0];
+            if (gga)
+#pragma unroll
+              for (int c = 0; c < 3; ++c) g[c] += x[u][1 + c];
+          }
+      }
     } else {
       r = pend.dens.rho[y - 1][q];
       if (gga)
@@ -804,17 +822,18 @@ __global__ __launch_bounds__(128) void nadd_functional_kernel(int func, XcParams
 __global__ __launch_bounds__(256) void nadd_energy_kernel(const double* __restrict__ e_blk, int64_t n, EnvEnergies env,
                                                           double* __restrict__ out) {
   __shared__ double red[256];
+  __shared__ double known[kListMax];
+  if ((int)threadIdx.x < env.n && !env.eblk[threadIdx.x]) known[threadIdx.x] = env.e[threadIdx.x][0];
   double e = e_blk ? sum_256(e_blk, n, nullptr, 0, red) : out[0];
   __syncthreads();
   for (int i = 0; i < env.n; ++i) {
+    double x = known[i];
     if (env.eblk[i]) {
-      const double s = sum_256(env.eblk[i], n, nullptr, 0, red);
-      if (threadIdx.x == 0 && env.e[i]) env.e[i][0] = s;
-      e -= s;
+      x = sum_256(env.eblk[i], n, nullptr, 0, red);
+      if (threadIdx.x == 0 && env.e[i]) env.e[i][0] = x;
       __syncthreads();
-    } else {
-      e -= env.e[i][0];
     }
+    e -= x;
   }
   if (threadIdx.x == 0) out[0] = e;
 }
