@@ -238,16 +238,16 @@ void launch_reduce_partials(hipStream_t s, const DevBlock* blocks, int bs, int64
                             int want_grad, double* rho, double* grad, int accumulate = 0);
 
 // Functional on rho/grad, or (part != nullptr) on the partials of 128-point blocks.
-void launch_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* rho,
+void launch_functional(hipStream_t s, int func, int64_t npts, int bs, const double* rho,
                        const double* grad, const DevBlock* blocks, const double* part, const double* w, double* eps,
                        double* v, double* g, double* vs, double* gw, double* e_blk);
 // Functional of a packed build: one 128-point block per workgroup over the merged block list.
-void launch_functional_packed(hipStream_t s, int func, const XcParams& prm, int nblocks, const DevBlock* blocks,
+void launch_functional_packed(hipStream_t s, int func, int nblocks, const DevBlock* blocks,
                               const PackSys* pack);
 
 // Unrestricted functional: spin densities/gradients (3 x npts each) in; w v_s, w g_s and
 // block energies out.
-void launch_functional_pol(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* ra,
+void launch_functional_pol(hipStream_t s, int func, int64_t npts, int bs, const double* ra,
                            const double* ga, const double* rb, const double* gb, const double* w, double* vsa,
                            double* gwa, double* vsb, double* gwb, double* e_blk,
                            const double* ra2 = nullptr, const double* ga2 = nullptr, const double* rb2 = nullptr,
@@ -400,7 +400,7 @@ void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, 
                           double* grad);
 // w v and w g of v[sum of sup] - v[rho_act] and the block energies of the difference (where the
 // potential is wanted); beside it the block energies of the pending densities.
-void launch_nadd_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, bool potential,
+void launch_nadd_functional(hipStream_t s, int func, int64_t npts, bool potential,
                             const DensityList& sup, const double* rho_act, const double* grad_act,
                             const DensityList& pending, double* const* pending_eblk, const double* w, double* vs,
                             double* gw, double* e_blk);

@@ -646,7 +646,7 @@ __device__ inline double block_sum_128(double x, double* red) {
   return r;
 }
 
-__global__ __launch_bounds__(128) void functional_kernel(int func, XcParams prm, int64_t npts, int bs,
+__global__ __launch_bounds__(128) void functional_kernel(int func, int64_t npts, int bs,
                                                          const double* __restrict__ rho,
                                                          const double* __restrict__ grad,
                                                          const DevBlock* __restrict__ blocks,
@@ -703,7 +703,7 @@ __global__ __launch_bounds__(128) void functional_kernel(int func, XcParams prm,
   const double sumabs = block_sum_128(fabs(r), red);
   const bool skip = sumabs < B * 1e-12;
   double e = 0.0, vv = 0.0, gg[3] = {0.0, 0.0, 0.0};
-  if (in && !skip) e = xc_point(func, r, gx, gy, gz, prm, &vv, gg);
+  if (in && !skip) e = xc_point(func, r, gx, gy, gz, &vv, gg);
   const double wq = in ? w[q] : 0.0;
   if (in) {
     if (eps) eps[q] = e;
@@ -747,12 +747,12 @@ __device__ double sum_256(const double* x, int64_t n, const double* x2, int64_t 
 // one first); of y > 0: a block of the energy of pend.dens.rho[y - 1] alone, into pend.eblk[y - 1]
 // (y = blockIdx.y, one more without the first).  What were a pass over all densities, a launch per
 // functional and one per energy sum took 36 us and as much between them ((H2O)12 in def2-SVP, 103 000
-// points); this launch and nadd_energy_kernel 23 us.
+// points, Thomas-Fermi); this launch and nadd_energy_kernel 19 us.
 struct PendingEnergies {
   DensityList dens;
   double* eblk[kListMax];
 };
-__global__ __launch_bounds__(128) void nadd_functional_kernel(int func, XcParams prm, int64_t npts, int y0,
+__global__ __launch_bounds__(128) void nadd_functional_kernel(int func, int64_t npts, int y0,
                                                               DensityList sup, const double* __restrict__ rho_act,
                                                               const double* __restrict__ grad_act,
                                                               PendingEnergies pend, const double* __restrict__ w,
@@ -767,7 +767,7 @@ __global__ __launch_bounds__(128) void nadd_functional_kernel(int func, XcParams
   if (in) {
     if (y == 0) {
       // four densities' loads at a time (one after another they are a chain of memory latencies:
-      // 44 us for PBE over 13 densities with gradients at 103 000 points, 37 so)
+      // 27 us for PBE over 13 densities with gradients at 103 000 points, 7 more one after another)
       constexpr int U = 4;
       for (int i0 = 0; i0 < sup.n; i0 += U) {
         double x[U][4];
@@ -796,14 +796,14 @@ __global__ __launch_bounds__(128) void nadd_functional_kernel(int func, XcParams
   }
   const bool skip = block_sum_128(fabs(r), red) < B * 1e-12;
   double e = 0.0, vv = 0.0, gg[3] = {0.0, 0.0, 0.0};
-  if (in && !skip) e = xc_point(func, r, g[0], g[1], g[2], prm, &vv, gg);
+  if (in && !skip) e = xc_point(func, r, g[0], g[1], g[2], &vv, gg);
   if (y == 0) {
     const double r2 = in ? rho_act[q] : 0.0;
     const bool skip2 = block_sum_128(fabs(r2), red) < B * 1e-12;
     if (in && !skip2) {
       double v2 = 0.0, g2[3] = {0.0, 0.0, 0.0};
       e -= xc_point(func, r2, gga ? grad_act[q] : 0.0, gga ? grad_act[npts + q] : 0.0,
-                    gga ? grad_act[2 * npts + q] : 0.0, prm, &v2, g2);
+                    gga ? grad_act[2 * npts + q] : 0.0, &v2, g2);
       vv -= v2;
       for (int c = 0; c < 3; ++c) gg[c] -= g2[c];
     }
@@ -842,7 +842,7 @@ __global__ __launch_bounds__(256) void nadd_energy_kernel(const double* __restri
 // w v_s and w g_s (the Fock kernel's inputs) per spin and the block energies out.
 // The block is skipped when both spin densities are negligible (sum |rho_s| <
 // B 1e-12 for each spin), as the reference's for_spin test does.
-__global__ __launch_bounds__(128) void functional_pol_kernel(int func, XcParams prm, int64_t npts, int bs,
+__global__ __launch_bounds__(128) void functional_pol_kernel(int func, int64_t npts, int bs,
                                                              const double* __restrict__ ra,
                                                              const double* __restrict__ ga,
                                                              const double* __restrict__ rb,
@@ -871,7 +871,7 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, XcParams 
   const bool skip_a = block_sum_128(fabs(a), red) < B * 1e-12;
   const bool skip_b = block_sum_128(fabs(bb), red) < B * 1e-12;
   double e = 0.0, v[2] = {0.0, 0.0}, g[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  if (in && !(skip_a && skip_b)) e = xc_point_pol(func, a, bb, xa, xb, prm, v, g);
+  if (in && !(skip_a && skip_b)) e = xc_point_pol(func, a, bb, xa, xb, v, g);
   if (ra2) {
     // non-additive form: the same functional of a second pair of spin densities is subtracted
     // (its own block skip applies to it)
@@ -886,7 +886,7 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, XcParams 
     const bool skip2_b = block_sum_128(fabs(b2), red) < B * 1e-12;
     if (in && !(skip2_a && skip2_b)) {
       double v2[2] = {0.0, 0.0}, g2[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-      e -= xc_point_pol(func, a2, b2, ya, yb, prm, v2, g2);
+      e -= xc_point_pol(func, a2, b2, ya, yb, v2, g2);
       v[0] -= v2[0];
       v[1] -= v2[1];
       for (int c = 0; c < 6; ++c) g[c] -= g2[c];
@@ -1676,19 +1676,19 @@ void launch_reduce_partials(hipStream_t s, const DevBlock* blocks, int bs, int64
                      want_grad, rho, grad, accumulate);
 }
 
-void launch_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* rho,
+void launch_functional(hipStream_t s, int func, int64_t npts, int bs, const double* rho,
                        const double* grad, const DevBlock* blocks, const double* part, const double* w, double* eps,
                        double* v, double* g, double* vs, double* gw, double* e_blk) {
   const int nb = (int)((npts + bs - 1) / bs);
   if (nb <= 0) return;
-  hipLaunchKernelGGL(functional_kernel, dim3(nb), dim3(128), 0, s, func, prm, npts, bs, rho, grad, blocks, part, w,
+  hipLaunchKernelGGL(functional_kernel, dim3(nb), dim3(128), 0, s, func, npts, bs, rho, grad, blocks, part, w,
                      eps, v, g, vs, gw, e_blk, (const PackSys*)nullptr);
 }
 
-void launch_functional_packed(hipStream_t s, int func, const XcParams& prm, int nblocks, const DevBlock* blocks,
+void launch_functional_packed(hipStream_t s, int func, int nblocks, const DevBlock* blocks,
                               const PackSys* pack) {
   if (nblocks <= 0) return;
-  hipLaunchKernelGGL(functional_kernel, dim3(nblocks), dim3(128), 0, s, func, prm, (int64_t)0, kTile,
+  hipLaunchKernelGGL(functional_kernel, dim3(nblocks), dim3(128), 0, s, func, (int64_t)0, kTile,
                      (const double*)nullptr, (const double*)nullptr, blocks, (const double*)nullptr,
                      (const double*)nullptr, (double*)nullptr, (double*)nullptr, (double*)nullptr, (double*)nullptr,
                      (double*)nullptr, (double*)nullptr, pack);
@@ -1714,13 +1714,13 @@ void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int nround) {
   hipLaunchKernelGGL(pack_sum_kernel, dim3(nsys), dim3(256), 0, s, pack, nround);
 }
 
-void launch_functional_pol(hipStream_t s, int func, const XcParams& prm, int64_t npts, int bs, const double* ra,
+void launch_functional_pol(hipStream_t s, int func, int64_t npts, int bs, const double* ra,
                            const double* ga, const double* rb, const double* gb, const double* w, double* vsa,
                            double* gwa, double* vsb, double* gwb, double* e_blk, const double* ra2,
                            const double* ga2, const double* rb2, const double* gb2) {
   const int nb = (int)((npts + bs - 1) / bs);
   if (nb <= 0) return;
-  hipLaunchKernelGGL(functional_pol_kernel, dim3(nb), dim3(128), 0, s, func, prm, npts, bs, ra, ga, rb, gb, w, vsa,
+  hipLaunchKernelGGL(functional_pol_kernel, dim3(nb), dim3(128), 0, s, func, npts, bs, ra, ga, rb, gb, w, vsa,
                      gwa, vsb, gwb, e_blk, ra2, ga2, rb2, gb2);
 }
 
@@ -1815,7 +1815,7 @@ void launch_sum_densities(hipStream_t s, const DensityList& list, int64_t npts, 
   hipLaunchKernelGGL(sum_densities_kernel, dim3(grid1d(npts, 256)), dim3(256), 0, s, list, npts, want_grad, rho, grad);
 }
 
-void launch_nadd_functional(hipStream_t s, int func, const XcParams& prm, int64_t npts, bool potential,
+void launch_nadd_functional(hipStream_t s, int func, int64_t npts, bool potential,
                             const DensityList& sup, const double* rho_act, const double* grad_act,
                             const DensityList& pending, double* const* pending_eblk, const double* w, double* vs,
                             double* gw, double* e_blk) {
@@ -1824,7 +1824,7 @@ void launch_nadd_functional(hipStream_t s, int func, const XcParams& prm, int64_
   pend.dens = pending;
   for (int i = 0; i < pending.n; ++i) pend.eblk[i] = pending_eblk[i];
   hipLaunchKernelGGL(nadd_functional_kernel, dim3(grid1d(npts, kTile), (potential ? 1 : 0) + pending.n), dim3(kTile), 0,
-                     s, func, prm, npts, potential ? 0 : 1, sup, rho_act, grad_act, pend, w, vs, gw, e_blk);
+                     s, func, npts, potential ? 0 : 1, sup, rho_act, grad_act, pend, w, vs, gw, e_blk);
 }
 
 void launch_nadd_energy(hipStream_t s, const double* e_blk, int64_t n, const EnvEnergies& env, double* out) {

@@ -275,7 +275,6 @@ struct xc_ctx {
   double* pack_energy = nullptr;  // likewise of a packed build's systems (grown on demand)
   size_t pack_energies = 0;
   HostStage stage;
-  XcParams prm;
   std::map<void*, size_t> user_allocs;  // buffers handed out by xc_device_alloc
   int live_handles = 0;                 // bases, grids and controllers not yet destroyed
   // stage timing: XC_NSTAGES + 1 events per profiled build
@@ -1493,7 +1492,7 @@ int xc_functional(xc_ctx* ctx, int functional, int64_t npts, int block_size, con
     if (gga) d_g.alloc(ctx, 3 * npts);
     d_eblk.alloc(ctx, nxc);
     d_E.alloc(ctx, 1);
-    launch_functional(ctx->stream, functional, ctx->prm, npts, block_size, d_rho.p, d_grad.p, nullptr, nullptr, d_w.p,
+    launch_functional(ctx->stream, functional, npts, block_size, d_rho.p, d_grad.p, nullptr, nullptr, d_w.p,
                       d_eps.p, d_v.p, d_g.p, nullptr, nullptr, d_eblk.p);
     launch_sum(ctx->stream, d_eblk.p, nxc, d_E.p);
     HIPX(hipGetLastError());
@@ -1527,7 +1526,7 @@ int xc_functional_device_noalloc(xc_ctx* ctx, int functional, int64_t npts, int 
     double* scr = noalloc_scratch(ctx->device);
     // every per-block slot [0, nxc) is written by the functional kernel and the sum slot by the
     // sum kernel, so nothing left from an earlier call is read
-    launch_functional(ctx->stream, functional, ctx->prm, npts, block_size, d_rho, gga ? d_grad : nullptr, nullptr,
+    launch_functional(ctx->stream, functional, npts, block_size, d_rho, gga ? d_grad : nullptr, nullptr,
                       nullptr, d_weights, d_eps, d_v, gga ? d_g : nullptr, nullptr, nullptr, scr);
     if (!gga && d_g) launch_fill(ctx->stream, d_g, 3 * npts, 0.0);
     launch_sum(ctx->stream, scr, nxc, scr + kNoallocBlocks);
@@ -1597,11 +1596,11 @@ static void enqueue_build(xc_bfogc* bf, int functional, int precision, double th
   }
   if (s == ctx->stream) ctx->mark();
   if (bf->bs == kTile) {
-    launch_functional(s, functional, ctx->prm, N, kTile, nullptr, nullptr, bf->d_blocks.p, bf->d_part.p,
+    launch_functional(s, functional, N, kTile, nullptr, nullptr, bf->d_blocks.p, bf->d_part.p,
                       bf->grid->d_w.p, nullptr, nullptr, nullptr, bf->d_vs.p, bf->d_gw.p, bf->d_eblk.p);
   } else {
     launch_reduce_partials(s, bf->d_blocks.p, bf->bs, N, bf->d_part.p, gga ? 1 : 0, bf->d_rho.p, bf->d_grad.p);
-    launch_functional(s, functional, ctx->prm, N, kTile, bf->d_rho.p, gga ? bf->d_grad.p : nullptr, nullptr,
+    launch_functional(s, functional, N, kTile, bf->d_rho.p, gga ? bf->d_grad.p : nullptr, nullptr,
                       nullptr, bf->grid->d_w.p, nullptr, nullptr, nullptr, bf->d_vs.p, bf->d_gw.p, bf->d_eblk.p);
   }
   if (s == ctx->stream) ctx->mark();
@@ -1672,7 +1671,7 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
     }
     launch_reduce_partials(s, bf->d_blocks.p, bf->bs, N, bf->d_part.p, gga ? 1 : 0, rho[sp], grad[sp]);
   }
-  launch_functional_pol(s, functional, ctx->prm, N, kTile, bf->d_rho.p, bf->d_grad.p, bf->d_rho_b.p,
+  launch_functional_pol(s, functional, N, kTile, bf->d_rho.p, bf->d_grad.p, bf->d_rho_b.p,
                         bf->d_grad_b.p, bf->grid->d_w.p, bf->d_vs.p, bf->d_gw.p, bf->d_vs_b.p, bf->d_gw_b.p,
                         bf->d_eblk.p);
   const double* vs[2] = {bf->d_vs.p, bf->d_vs_b.p};
@@ -1737,7 +1736,7 @@ static void run_nadd_functional(const std::vector<xc_bfogc*>& sub, int functiona
       append(pending, cached ? missing[i]->d_rho_c : missing[i]->d_rho,
              cached ? missing[i]->d_grad_c : missing[i]->d_grad);
     }
-    launch_nadd_functional(s, functional, ctx->prm, N, i0 == 0, sup, cached ? act->d_rho_c.p : act->d_rho.p,
+    launch_nadd_functional(s, functional, N, i0 == 0, sup, cached ? act->d_rho_c.p : act->d_rho.p,
                            cached ? act->d_grad_c.p : act->d_grad.p, pending, eblk, w, act->d_vs.p, act->d_gw.p,
                            act->d_eblk.p);
   }
@@ -1889,13 +1888,13 @@ static void enqueue_nadd_pol(xc_bfogc* act, int nenv, xc_bfogc* const* env, int 
     }
   }
   // v^s[sup] - v^s[act] and E[sup] - E[act]
-  launch_functional_pol(s, functional, ctx->prm, N, kTile, sup_r[0], sup_g[0], sup_r[1], sup_g[1], w, act->d_vs.p,
+  launch_functional_pol(s, functional, N, kTile, sup_r[0], sup_g[0], sup_r[1], sup_g[1], w, act->d_vs.p,
                         act->d_gw.p, act->d_vs_b.p, act->d_gw_b.p, act->d_eblk.p, act->d_rho.p, act->d_grad.p,
                         act->d_rho_b.p, act->d_grad_b.p);
   launch_sum(s, act->d_eblk.p, nxc, ctx->energy, 0);
   for (size_t i = 1; i < sub.size(); ++i) {
     xc_bfogc* b = sub[i];
-    launch_functional_pol(s, functional, ctx->prm, N, kTile, b->d_rho.p, b->d_grad.p, b->d_rho_b.p, b->d_grad_b.p, w,
+    launch_functional_pol(s, functional, N, kTile, b->d_rho.p, b->d_grad.p, b->d_rho_b.p, b->d_grad_b.p, w,
                           nullptr, nullptr, nullptr, nullptr, b->d_eblk.p);
     launch_sum(s, b->d_eblk.p, nxc, ctx->energy, 1);
   }
@@ -2244,7 +2243,7 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
         else
           launch_density_sub<double>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
                                      nullptr, 0, dsys, nullptr, nullptr, form);
-        launch_functional_packed(s, functional, ctx->prm, (int)blocks.size(), pw.blocks.p, dsys);
+        launch_functional_packed(s, functional, (int)blocks.size(), pw.blocks.p, dsys);
         over_lanes(L, kFockShapes, [&](int c) { return (int)fock[c].size(); }, [&](int c, hipStream_t st) {
           if (fp32)
             launch_fock_sub<float>(st, c, pw.fock[c].p, (int)fock[c].size(), pw.blocks.p, nullptr, nullptr, nullptr, g,
@@ -2328,11 +2327,11 @@ void geom_gradient(xc_bfogc* bf, int functional, const double* Pa, const double*
   if (!Pb) {
     run_density<double>(bf, bf->d_t64.p, bf->d_P.p, gga ? 1 : 0, ctx->lanes);
     if (bf->bs == kTile) {
-      launch_functional(s, functional, ctx->prm, N, kTile, nullptr, nullptr, bf->d_blocks.p, bf->d_part.p,
+      launch_functional(s, functional, N, kTile, nullptr, nullptr, bf->d_blocks.p, bf->d_part.p,
                         bf->grid->d_w.p, nullptr, nullptr, nullptr, bf->d_vs.p, bf->d_gw.p, bf->d_eblk.p);
     } else {
       launch_reduce_partials(s, bf->d_blocks.p, bf->bs, N, bf->d_part.p, gga ? 1 : 0, bf->d_rho.p, bf->d_grad.p);
-      launch_functional(s, functional, ctx->prm, N, kTile, bf->d_rho.p, gga ? bf->d_grad.p : nullptr, nullptr,
+      launch_functional(s, functional, N, kTile, bf->d_rho.p, gga ? bf->d_grad.p : nullptr, nullptr,
                         nullptr, bf->grid->d_w.p, nullptr, nullptr, nullptr, bf->d_vs.p, bf->d_gw.p, bf->d_eblk.p);
     }
   } else {
@@ -2343,7 +2342,7 @@ void geom_gradient(xc_bfogc* bf, int functional, const double* Pa, const double*
       run_density<double>(bf, bf->d_t64.p, Ps[sp], gga ? 1 : 0, ctx->lanes);
       launch_reduce_partials(s, bf->d_blocks.p, bf->bs, N, bf->d_part.p, gga ? 1 : 0, rho[sp], grd[sp]);
     }
-    launch_functional_pol(s, functional, ctx->prm, N, kTile, bf->d_rho.p, bf->d_grad.p, bf->d_rho_b.p,
+    launch_functional_pol(s, functional, N, kTile, bf->d_rho.p, bf->d_grad.p, bf->d_rho_b.p,
                           bf->d_grad_b.p, bf->grid->d_w.p, bf->d_vs.p, bf->d_gw.p, bf->d_vs_b.p, bf->d_gw_b.p,
                           bf->d_eblk.p);
   }
