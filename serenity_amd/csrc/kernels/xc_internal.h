@@ -260,6 +260,13 @@ template <typename T>
 void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, const DevBlock* blocks, const T* tiles,
                      const double* vs, const double* gw, int gga, double block_ave_thr, T* Tscr, int64_t npts,
                      const PackSys* pack = nullptr);
+constexpr int kListMax = 32;  // entries of the lists passed by value (kernel arguments)
+// Energies subtracted from a non-additive energy, with the block energies of those still to be summed.
+struct EnvEnergies {
+  double* e[kListMax];
+  const double* eblk[kListMax];
+  int n;
+};
 // U[j + n i] = sum over the row entries of AO i (block order) of the stored sub-tile values at
 // columns j >= i, for every i of [0, n): the lower triangle of the Fock accumulator, each element
 // written once (its terms meet in LDS in an order that varies from run to run).  Packed:
@@ -270,10 +277,11 @@ void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, 
 // columns that 32 lanes take at once; else 16 lanes take an entry.
 // With out.direct the rows go to both triangles of F instead (no finalize), each row leaves its part of
 // the FP32 rounding term sum F (P - P32) in round[row] where P32 is given (packed: where round is
-// not null), and one more workgroup sums the block energies into E (a second rounding sum, where
-// there is one, is launch_sum's).  For matrices of up to kDirectRows rows: the upper triangle's writes
-// go one element per line (n^2 / 2 of them), which costs less than the finalize's launch only while
-// they are few ((H2O)8/def2-SVP, 192 rows: reduce, finalize and sum 30 us, together 19 us).
+// not null), and one more workgroup sums the block energies into E, less the energies of env (a
+// rounding sum, where there is one, is launch_sum's).  For matrices of up to kDirectRows rows: the
+// upper triangle's writes go one element per line (n^2 / 2 of them), which costs less than the
+// finalize's launch only while they are few ((H2O)8/def2-SVP, 192 rows: reduce, finalize and sum 30
+// us, together 19 us).
 struct ReduceOut {
   bool direct;
   double* F;
@@ -290,7 +298,7 @@ constexpr int kReduceWindow = 8192;  // row columns accumulated in LDS per pass
 template <typename T>
 void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
                         double* U, int n, const PackSys* pack = nullptr, int nsys = 1, bool fixed = false,
-                        bool wide = false, const ReduceOut& out = ReduceOut{});
+                        bool wide = false, const ReduceOut& out = ReduceOut{}, const EnvEnergies& env = EnvEnergies{});
 // Packed elementwise stages over nsys systems (maxnn = largest n^2): P -> FP32,
 // F = mirror of U (+ FP32 rounding partials), E = sum of block energies (+ rounding term).
 constexpr int kPackRoundBlocks = 512;  // finalize workgroups per system of a packed build
@@ -388,8 +396,7 @@ void launch_weight_potential(hipStream_t s, int64_t npts, const double* w, const
 void launch_fill(hipStream_t s, double* p, int64_t n, double value);
 void launch_copy(hipStream_t s, const void* src, void* dst, int64_t n32);  // n32 units of 32 bytes
 
-// Up to kListMax device arrays passed by value (kernel argument).
-constexpr int kListMax = 32;
+// Up to kListMax densities passed by value (kernel argument).
 struct DensityList {
   const double* rho[kListMax];
   const double* grad[kListMax];
@@ -404,12 +411,6 @@ void launch_nadd_functional(hipStream_t s, int func, int64_t npts, bool potentia
                             const DensityList& sup, const double* rho_act, const double* grad_act,
                             const DensityList& pending, double* const* pending_eblk, const double* w, double* vs,
                             double* gw, double* e_blk);
-// Energies subtracted from a non-additive energy, with the block energies of those still to be summed.
-struct EnvEnergies {
-  double* e[kListMax];
-  const double* eblk[kListMax];
-  int n;
-};
 // out = sum of e_blk[0..n) (null: out) minus the listed energies in order (summed first where pending)
 void launch_nadd_energy(hipStream_t s, const double* e_blk, int64_t n, const EnvEnergies& env, double* out);
 // Q[i, j] = P[i, j] + P[j, i], Q[i, i] = P[i, i] (packed: every system's P64 into its U, n the largest)

@@ -818,24 +818,29 @@ __global__ __launch_bounds__(128) void nadd_functional_kernel(int func, int64_t 
 }
 
 // out = sum of e_blk (null: out itself) - env.e[0] - env.e[1] ..., where an entry with block
-// energies first becomes their sum (kept where e is given).
-__global__ __launch_bounds__(256) void nadd_energy_kernel(const double* __restrict__ e_blk, int64_t n, EnvEnergies env,
-                                                          double* __restrict__ out) {
-  __shared__ double red[256];
-  __shared__ double known[kListMax];
-  if ((int)threadIdx.x < env.n && !env.eblk[threadIdx.x]) known[threadIdx.x] = env.e[threadIdx.x][0];
+// energies first becomes their sum (kept where e is given); every thread of the workgroup calls it.
+// red: 256 + kListMax.
+__device__ void nadd_energy(const double* e_blk, int64_t n, const EnvEnergies& env, double* out, double* red) {
+  double* known = red + 256;
+  const int t = threadIdx.x;
+  if (t < env.n && !env.eblk[t]) known[t] = env.e[t][0];
   double e = e_blk ? sum_256(e_blk, n, nullptr, 0, red) : out[0];
   __syncthreads();
   for (int i = 0; i < env.n; ++i) {
     double x = known[i];
     if (env.eblk[i]) {
       x = sum_256(env.eblk[i], n, nullptr, 0, red);
-      if (threadIdx.x == 0 && env.e[i]) env.e[i][0] = x;
+      if (t == 0 && env.e[i]) env.e[i][0] = x;
       __syncthreads();
     }
     e -= x;
   }
-  if (threadIdx.x == 0) out[0] = e;
+  if (t == 0) out[0] = e;
+}
+__global__ __launch_bounds__(256) void nadd_energy_kernel(const double* __restrict__ e_blk, int64_t n, EnvEnergies env,
+                                                          double* __restrict__ out) {
+  __shared__ double red[256 + kListMax];
+  nadd_energy(e_blk, n, env, out, red);
 }
 
 // Unrestricted functional on 128-point blocks: spin densities and gradients in,
@@ -1228,7 +1233,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
                                                                         const int* __restrict__ ao_idx,
                                                                         double* __restrict__ U, int n, int window,
                                                                         const PackSys* __restrict__ pack,
-                                                                        ReduceOut out) {
+                                                                        ReduceOut out, EnvEnergies env) {
   extern __shared__ unsigned long long racc_u[];  // window (FP64 sums) or 2 window (Fixed: h, then l sums)
   double* racc = reinterpret_cast<double*>(racc_u);
   if (pack) {
@@ -1253,8 +1258,7 @@ __global__ __launch_bounds__(64 * kReduceWaves) void fock_reduce_kernel(const Ro
   const int tid = threadIdx.x;
   if (i >= n) {  // uniform over the workgroup
     if (i == n && out.direct && out.E) {
-      const double e = sum_256(out.eblk, out.nxc, nullptr, 0, reinterpret_cast<double*>(racc_u));
-      if (tid == 0) out.E[0] = e;
+      nadd_energy(out.eblk, out.nxc, env, out.E, reinterpret_cast<double*>(racc_u));
     }
     return;
   }
@@ -1773,35 +1777,37 @@ static int reduce_window_limit(bool fixed) {
 template <typename T, bool Fixed>
 static void launch_fock_reduce_f(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr,
                                  const int* ao_idx, double* U, int n, const PackSys* pack, int nsys, bool wide,
-                                 const ReduceOut& out) {
+                                 const ReduceOut& out, const EnvEnergies& env) {
   const int lim = reduce_window_limit(Fixed);
   const int window = n < lim ? n : lim;
   size_t lds = (Fixed ? 16 : 8) * (size_t)window;
-  // one workgroup more for the energy sum, whose 256 terms need LDS (the rounding term's 16 less)
+  // one workgroup more for the energy sum, whose terms need LDS (the rounding term's 16 less)
   const dim3 grid(n + (out.direct && (out.E || pack) ? 1 : 0), nsys);
-  if (out.direct && lds < 256 * sizeof(double)) lds = 256 * sizeof(double);
+  if (out.direct) lds = std::max(lds, (256 + kListMax) * sizeof(double));
   if (wide)
     hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 32>), grid, dim3(64 * kReduceWaves), lds, s, ent, row_ptr, Tscr,
-                       ao_idx, U, n, window, pack, out);
+                       ao_idx, U, n, window, pack, out, env);
   else
     hipLaunchKernelGGL((fock_reduce_kernel<T, Fixed, 16>), grid, dim3(64 * kReduceWaves), lds, s, ent, row_ptr, Tscr,
-                       ao_idx, U, n, window, pack, out);
+                       ao_idx, U, n, window, pack, out, env);
 }
 
 template <typename T>
 void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
                         double* U, int n, const PackSys* pack, int nsys, bool fixed, bool wide,
-                        const ReduceOut& out) {
+                        const ReduceOut& out, const EnvEnergies& env) {
   if (n <= 0 || nsys <= 0) return;
   if (fixed)
-    launch_fock_reduce_f<T, true>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide, out);
+    launch_fock_reduce_f<T, true>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide, out, env);
   else
-    launch_fock_reduce_f<T, false>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide, out);
+    launch_fock_reduce_f<T, false>(s, ent, row_ptr, Tscr, ao_idx, U, n, pack, nsys, wide, out, env);
 }
 template void launch_fock_reduce<double>(hipStream_t, const RowEnt*, const int*, const double*, const int*, double*,
-                                         int, const PackSys*, int, bool, bool, const ReduceOut&);
+                                         int, const PackSys*, int, bool, bool, const ReduceOut&,
+                                         const EnvEnergies&);
 template void launch_fock_reduce<float>(hipStream_t, const RowEnt*, const int*, const float*, const int*, double*,
-                                        int, const PackSys*, int, bool, bool, const ReduceOut&);
+                                        int, const PackSys*, int, bool, bool, const ReduceOut&,
+                                         const EnvEnergies&);
 
 void launch_weight_potential(hipStream_t s, int64_t npts, const double* w, const double* v, const double* g,
                              double* vs, double* gw) {

@@ -699,18 +699,20 @@ void run_fock_tiles(xc_bfogc* bf, const T* tiles, int gga, double thr, const Lan
 }
 
 template <typename T>
-void run_fock_reduce(xc_bfogc* bf, const Lanes& L, const ReduceOut& out = ReduceOut{}) {
+void run_fock_reduce(xc_bfogc* bf, const Lanes& L, const ReduceOut& out = ReduceOut{},
+                     const EnvEnergies& env = EnvEnergies{}) {
   launch_fock_reduce<T>(L.main, bf->d_rowent.p, bf->d_rowptr.p, reinterpret_cast<const T*>(bf->d_T.p),
                         bf->d_ao_idx.p, bf->d_U.p, bf->basis->nao, nullptr, 1, bf->ctx->deterministic,
-                        bf->sum_nb > 256 * (int64_t)bf->nblocks, out);
+                        bf->sum_nb > 256 * (int64_t)bf->nblocks, out, env);
 }
 
 // The reduce and what follows it: F (overwritten), the FP32 rounding partials of one spin (P32 given;
 // the spin's slot of d_round), and E = the sum of the block energies (E given) plus the rounding
-// partials of nspin slots.  Small matrices get their rows and the energy from the reduce itself.
+// partials of nspin slots (less the environment's energies: small matrices only).  Small matrices get
+// their rows and the energy from the reduce itself.
 template <typename T>
 void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, const float* P32, int spin, int nspin,
-                     double* E) {
+                     double* E, const EnvEnergies& env = EnvEnergies{}) {
   hipStream_t s = L.main;
   const int n = bf->basis->nao;
   const int nxc = (int)((bf->grid->npts + kTile - 1) / kTile);
@@ -718,7 +720,7 @@ void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, 
   const int nround = direct ? n : finalize_blocks(n);
   double* round = P32 ? bf->d_round.p + (size_t)spin * nround : nullptr;
   if (direct) {
-    run_fock_reduce<T>(bf, L, ReduceOut{true, dF, P, P32, round, bf->d_eblk.p, nxc, P32 ? nullptr : E});
+    run_fock_reduce<T>(bf, L, ReduceOut{true, dF, P, P32, round, bf->d_eblk.p, nxc, P32 ? nullptr : E}, env);
   } else {
     run_fock_reduce<T>(bf, L);
     if (s == bf->ctx->stream && nspin == 1) bf->ctx->mark();
@@ -1695,9 +1697,10 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
  * v = v[rho_sup] - v[rho_act] integrated with the active basis,
  * E = E[rho_sup] - E[rho_act] - sum_env E[rho_env] (left in ctx->energy). */
 // The functional stage of a non-additive build of sub[0] among sub[1..]: w v and w g of v[rho_sup] -
-// v[rho_act] into sub[0], and E[rho_sup] - E[rho_act] - E[rho_env] ... into the context's energy.
-// cached: on the cached densities, keeping each E[rho_env] until its density changes.
-static void run_nadd_functional(const std::vector<xc_bfogc*>& sub, int functional, bool cached) {
+// v[rho_act] into sub[0].  E[rho_sup] - E[rho_act] - E[rho_env] ... goes into the context's energy, here or
+// (small matrices) with the returned list in run_nadd_fock.  cached: on the cached densities, keeping
+// each E[rho_env] until its density changes.
+static EnvEnergies run_nadd_functional(const std::vector<xc_bfogc*>& sub, int functional, bool cached) {
   xc_bfogc* act = sub[0];
   xc_ctx* ctx = act->ctx;
   hipStream_t s = ctx->stream;
@@ -1740,18 +1743,41 @@ static void run_nadd_functional(const std::vector<xc_bfogc*>& sub, int functiona
                            cached ? act->d_grad_c.p : act->d_grad.p, pending, eblk, w, act->d_vs.p, act->d_gw.p,
                            act->d_eblk.p);
   }
+  EnvEnergies env_e{};
   for (size_t i0 = 1; i0 == 1 || i0 < sub.size(); i0 += kListMax) {
-    EnvEnergies env_e{};
+    env_e.n = 0;
     for (size_t i = i0; i < std::min(sub.size(), i0 + kListMax); ++i) {
       xc_bfogc* b = sub[i];
       const bool valid = cached && b->ecache_valid[functional];
       env_e.e[env_e.n] = cached ? b->d_ecache.p + functional : nullptr;
       env_e.eblk[env_e.n++] = valid ? nullptr : b->d_eblk.p;
     }
-    launch_nadd_energy(s, i0 == 1 ? act->d_eblk.p : nullptr, nxc, env_e, ctx->energy);
+    // one list of a small matrix goes with its row reduce, in the workgroup that sums the energy
+    if (sub.size() > (size_t)kListMax + 1 || act->basis->nao > kDirectRows)
+      launch_nadd_energy(s, i0 == 1 ? act->d_eblk.p : nullptr, nxc, env_e, ctx->energy);
   }
+  return env_e;
+}
+
+// The Fock stage of a non-additive build, with the energy where the functional stage left its sum.
+static void run_nadd_fock(const std::vector<xc_bfogc*>& sub, int functional, int precision, double thr,
+                          const EnvEnergies& env, bool cached, double* dF) {
+  xc_bfogc* act = sub[0];
+  xc_ctx* ctx = act->ctx;
+  const int g = functional_is_gga(functional) ? 1 : 0;
+  const bool with_energy = act->basis->nao <= kDirectRows && sub.size() <= (size_t)kListMax + 1;
+  double* E = with_energy ? ctx->energy : nullptr;
+  if (precision == XC_PREC_FP32)
+    run_fock_tiles<float>(act, act->d_t32.p, g, thr, ctx->lanes);
+  else
+    run_fock_tiles<double>(act, act->d_t64.p, g, thr, ctx->lanes);
+  ctx->mark();
+  if (precision == XC_PREC_FP32)
+    run_fock_finish<float>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, E, env);
+  else
+    run_fock_finish<double>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, E, env);
   if (cached)
-    for (xc_bfogc* b : missing) b->ecache_valid[functional] = true;
+    for (size_t i = 1; i < sub.size(); ++i) sub[i]->ecache_valid[functional] = true;
 }
 
 static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int functional, int precision, double thr,
@@ -1800,17 +1826,9 @@ static void enqueue_nadd(xc_bfogc* act, int nenv, xc_bfogc* const* env, int func
     launch_reduce_partials(s, b->d_blocks.p, b->bs, N, b->d_part.p, gga ? 1 : 0, b->d_rho.p, b->d_grad.p, 0);
   }
   ctx->mark();
-  run_nadd_functional(sub, functional, false);
+  const EnvEnergies env_e = run_nadd_functional(sub, functional, false);
   ctx->mark();
-  if (fp32)
-    run_fock_tiles<float>(act, act->d_t32.p, gga ? 1 : 0, thr, ctx->lanes);
-  else
-    run_fock_tiles<double>(act, act->d_t64.p, gga ? 1 : 0, thr, ctx->lanes);
-  ctx->mark();
-  if (fp32)
-    run_fock_finish<float>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
-  else
-    run_fock_finish<double>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
+  run_nadd_fock(sub, functional, precision, thr, env_e, false, dF);
   ctx->mark();
   HIPX(hipGetLastError());
 }
@@ -2027,17 +2045,9 @@ int xc_nadd_fock_build_cached(xc_bfogc* act, int nenv, xc_bfogc* const* env, int
     ctx->mark();
     ctx->mark();
     ctx->mark();
-    run_nadd_functional(sub, functional, true);
+    const EnvEnergies env_e = run_nadd_functional(sub, functional, true);
     ctx->mark();
-    if (precision == XC_PREC_FP32)
-      run_fock_tiles<float>(act, act->d_t32.p, gga ? 1 : 0, thr, ctx->lanes);
-    else
-      run_fock_tiles<double>(act, act->d_t64.p, gga ? 1 : 0, thr, ctx->lanes);
-    ctx->mark();
-    if (precision == XC_PREC_FP32)
-      run_fock_finish<float>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
-    else
-      run_fock_finish<double>(act, ctx->lanes, dF, nullptr, nullptr, 0, 1, nullptr);
+    run_nadd_fock(sub, functional, precision, thr, env_e, true, dF);
     ctx->mark();
     HIPX(hipGetLastError());
     if (energy) {
