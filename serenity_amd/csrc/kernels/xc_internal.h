@@ -208,7 +208,7 @@ template <typename T>
 void launch_density_sub(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
                         const T* tiles, const T* P, int n, int want_grad, double* part, int64_t npts,
                         const PackSys* pack = nullptr, const int* nwork_dev = nullptr,
-                        const unsigned char* skip = nullptr, bool form = false);
+                        const unsigned char* skip = nullptr, bool form = false, bool pairs = false);
 
 // Dense-block refinement of the mixed-precision density: a work list and its device-side count, filled
 // by launch_mark_dense.
@@ -251,7 +251,8 @@ void launch_functional_pol(hipStream_t s, int func, int64_t npts, int bs, const 
                            const double* ga, const double* rb, const double* gb, const double* w, double* vsa,
                            double* gwa, double* vsb, double* gwb, double* e_blk,
                            const double* ra2 = nullptr, const double* ga2 = nullptr, const double* rb2 = nullptr,
-                           const double* gb2 = nullptr);
+                           const double* gb2 = nullptr, const DevBlock* blocks = nullptr,
+                           const double* part_a = nullptr, const double* part_b = nullptr);
 
 // Sub-tile Fock kernel over items of one workgroup shape.
 // Each item stores its sub-tiles of phi^T G + G^T phi into the block's scratch slice Tscr + toff
@@ -259,7 +260,7 @@ void launch_functional_pol(hipStream_t s, int func, int64_t npts, int bs, const 
 template <typename T>
 void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, const DevBlock* blocks, const T* tiles,
                      const double* vs, const double* gw, int gga, double block_ave_thr, T* Tscr, int64_t npts,
-                     const PackSys* pack = nullptr);
+                     const PackSys* pack = nullptr, bool pairs = false);
 constexpr int kListMax = 32;  // entries of the lists passed by value (kernel arguments)
 // Energies subtracted from a non-additive energy, with the block energies of those still to be summed.
 struct EnvEnergies {
@@ -299,6 +300,13 @@ template <typename T>
 void launch_fock_reduce(hipStream_t s, const RowEnt* ent, const int* row_ptr, const T* Tscr, const int* ao_idx,
                         double* U, int n, const PackSys* pack = nullptr, int nsys = 1, bool fixed = false,
                         bool wide = false, const ReduceOut& out = ReduceOut{}, const EnvEnergies& env = EnvEnergies{});
+// The two spins of an unrestricted build as a pack of two systems on one controller: launches with pairs
+// run each work item once per spin, with entry block.sys + spin of the table.  The table goes to the
+// device as a kernel argument, so that a caller's captured build keeps its own.
+struct PackPair {
+  PackSys s[2];
+};
+void launch_set_pair(hipStream_t s, const PackPair& pair, PackSys* out);
 // Packed elementwise stages over nsys systems (maxnn = largest n^2): P -> FP32,
 // F = mirror of U (+ FP32 rounding partials), E = sum of block energies (+ rounding term).
 constexpr int kPackRoundBlocks = 512;  // finalize workgroups per system of a packed build

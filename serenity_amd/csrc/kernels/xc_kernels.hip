@@ -321,6 +321,14 @@ __device__ inline void quad_rows(const gmem<const float>* seg, int lane, double 
 // lane dotting its T entries with the phi / grad phi values of the same
 // (point, column), and summed over the columns by lane shuffles.  (FP64
 // accumulates T transposed, so that its lanes read whole 128-byte point runs.)
+// Work item and spin of workgroup x of a launch of pairs items for two spins (0: one pass, item x):
+// eight items of one spin, then the same eight of the other, so that an item's two passes run on one
+// XCD shortly after each other and the second finds the tiles in its L2.
+__device__ __forceinline__ int pair_item(int pairs, int x, int& spin) {
+  spin = pairs ? (x >> 3) & 1 : 0;
+  return pairs ? (x >> 4) * 8 + (x & 7) : x;
+}
+
 // What the density items of one launch share.
 template <typename T>
 struct DensityArgs {
@@ -571,16 +579,19 @@ __global__ __launch_bounds__(512) void density_sub_kernel(const WorkItem* __rest
                                                           const DevBlock* __restrict__ blocks, DensityArgs<T> arg,
                                                           const PackSys* __restrict__ pack,
                                                           const int* __restrict__ nwork_dev,
-                                                          const unsigned char* __restrict__ skip) {
+                                                          const unsigned char* __restrict__ skip, int pairs) {
   // a launch over a list filled on the device runs only its first *nwork_dev items
   if (nwork_dev && (int)blockIdx.x >= *nwork_dev) return;
+  int spin;
+  const int item = pair_item(pairs, blockIdx.x, spin);
+  if (pairs && item >= pairs) return;
   __shared__ __attribute__((aligned(16))) unsigned char smem[(kTile + 16 * kDensMaxS) * 144];
   __shared__ int sIdx[kDensIdxLds];
-  const WorkItem wk = work[blockIdx.x];
+  const WorkItem wk = work[item];
   if (skip && skip[wk.block]) return;  // a block the caller contracts in another pass
   const DevBlock bk = blocks[wk.block];
   if (pack) {
-    const PackSys& ps = pack[bk.sys];
+    const PackSys& ps = pack[bk.sys + spin];
     arg.tiles = static_cast<const T*>(ps.tiles);
     arg.P = static_cast<const T*>(ps.P);
     arg.ao_idx = ps.ao_idx;
@@ -858,7 +869,10 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, int64_t n
                                                              const double* __restrict__ ra2,
                                                              const double* __restrict__ ga2,
                                                              const double* __restrict__ rb2,
-                                                             const double* __restrict__ gb2) {
+                                                             const double* __restrict__ gb2,
+                                                             const DevBlock* __restrict__ blocks,
+                                                             const double* __restrict__ part_a,
+                                                             const double* __restrict__ part_b) {
   __shared__ double red[128];
   const int b = blockIdx.x, t = threadIdx.x;
   const int64_t first = (int64_t)b * bs;
@@ -866,13 +880,34 @@ __global__ __launch_bounds__(128) void functional_pol_kernel(int func, int64_t n
   const int64_t q = first + t;
   const bool in = t < B;
   const bool gga = functional_is_gga(func);
-  const double a = in ? ra[q] : 0.0, bb = in ? rb[q] : 0.0;
+  double a = 0.0, bb = 0.0;
   double xa[3] = {0.0, 0.0, 0.0}, xb[3] = {0.0, 0.0, 0.0};
-  if (in && gga)
-    for (int c = 0; c < 3; ++c) {
-      xa[c] = ga[c * npts + q];
-      xb[c] = gb[c * npts + q];
+  if (in && part_a) {
+    // sum the density passes of this block (blocks of 128 points)
+    const int np = blocks[b].npass;
+    for (int s = 0; s < np; ++s) {
+      const int64_t o = (int64_t)s * 4 * npts + q;
+      a += part_a[o];
+      bb += part_b[o];
+      if (gga)
+        for (int c = 0; c < 3; ++c) {
+          xa[c] += part_a[o + (c + 1) * npts];
+          xb[c] += part_b[o + (c + 1) * npts];
+        }
     }
+    for (int c = 0; c < 3; ++c) {
+      xa[c] *= 2.0;
+      xb[c] *= 2.0;
+    }
+  } else if (in) {
+    a = ra[q];
+    bb = rb[q];
+    if (gga)
+      for (int c = 0; c < 3; ++c) {
+        xa[c] = ga[c * npts + q];
+        xb[c] = gb[c * npts + q];
+      }
+  }
   const bool skip_a = block_sum_128(fabs(a), red) < B * 1e-12;
   const bool skip_b = block_sum_128(fabs(bb), red) < B * 1e-12;
   double e = 0.0, v[2] = {0.0, 0.0}, g[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -933,7 +968,7 @@ __global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __rest
                                                        const T* __restrict__ tiles,
                                                        const double* __restrict__ vs, const double* __restrict__ gw,
                                                        int gga, double thr, T* __restrict__ Tscr, int64_t npts,
-                                                       const PackSys* __restrict__ pack) {
+                                                       const PackSys* __restrict__ pack, int pairs) {
   using M = Mfma<T>;
   constexpr int KC = 128 / (int)sizeof(T);       // points per chunk: one 128-byte line of each AO row
   constexpr int KV = KC / 4;
@@ -954,10 +989,13 @@ __global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __rest
   __shared__ __attribute__((aligned(16))) T spot[4][kTile];
   __shared__ double red[2];
 
-  const FockItem it = work[blockIdx.x];
+  int spin;
+  const int item = pair_item(pairs, blockIdx.x, spin);
+  if (pairs && item >= pairs) return;
+  const FockItem it = work[item];
   const DevBlock bk = blocks[it.block];
   if (pack) {
-    const PackSys& ps = pack[bk.sys];
+    const PackSys& ps = pack[bk.sys + spin];
     tiles = static_cast<const T*>(ps.tiles);
     vs = ps.vs;
     gw = ps.gw;
@@ -1558,22 +1596,25 @@ void launch_ao_eval(hipStream_t s, const DevBlock* blocks, int nblocks, int max_
 template <typename T>
 void launch_density_sub(hipStream_t s, const WorkItem* work, int nwork, const DevBlock* blocks, const int* ao_idx,
                         const T* tiles, const T* P, int n, int want_grad, double* part, int64_t npts,
-                        const PackSys* pack, const int* nwork_dev, const unsigned char* skip, bool form) {
+                        const PackSys* pack, const int* nwork_dev, const unsigned char* skip, bool form,
+                        bool pairs) {
   if (nwork <= 0) return;
   const DensityArgs<T> arg = {ao_idx, tiles, P, n, want_grad, part, npts};
+  const dim3 grid(pairs ? (nwork + 7) / 8 * 16 : nwork);
+  const int np = pairs ? nwork : 0;
   if (sizeof(T) == 8 && form)
-    hipLaunchKernelGGL((density_sub_kernel<T, sizeof(T) == 8>), dim3(nwork), dim3(512), 0, s, work, blocks, arg, pack,
-                       nwork_dev, skip);
+    hipLaunchKernelGGL((density_sub_kernel<T, sizeof(T) == 8>), grid, dim3(512), 0, s, work, blocks, arg, pack,
+                       nwork_dev, skip, np);
   else
-    hipLaunchKernelGGL((density_sub_kernel<T, false>), dim3(nwork), dim3(512), 0, s, work, blocks, arg, pack, nwork_dev,
-                       skip);
+    hipLaunchKernelGGL((density_sub_kernel<T, false>), grid, dim3(512), 0, s, work, blocks, arg, pack, nwork_dev,
+                       skip, np);
 }
 template void launch_density_sub<double>(hipStream_t, const WorkItem*, int, const DevBlock*, const int*, const double*,
                                          const double*, int, int, double*, int64_t, const PackSys*, const int*,
-                                         const unsigned char*, bool);
+                                         const unsigned char*, bool, bool);
 template void launch_density_sub<float>(hipStream_t, const WorkItem*, int, const DevBlock*, const int*, const float*,
                                         const float*, int, int, double*, int64_t, const PackSys*, const int*,
-                                        const unsigned char*, bool);
+                                        const unsigned char*, bool, bool);
 
 // Largest density of block b (128 threads), from the partials of its passes.
 __device__ double block_max_density(const DevBlock& bk, int64_t npts, const double* __restrict__ part, double* red) {
@@ -1703,6 +1744,13 @@ static unsigned pack_grid(int64_t maxnn) {
   return (unsigned)(g < 1 ? 1 : g > 1024 ? 1024 : g);
 }
 
+__global__ void set_pair_kernel(PackPair pair, PackSys* __restrict__ out) {
+  if (threadIdx.x < 2) out[threadIdx.x] = pair.s[threadIdx.x];
+}
+void launch_set_pair(hipStream_t s, const PackPair& pair, PackSys* out) {
+  hipLaunchKernelGGL(set_pair_kernel, dim3(1), dim3(64), 0, s, pair, out);
+}
+
 void launch_pack_to_float(hipStream_t s, const PackSys* pack, int nsys, int64_t maxnn) {
   if (nsys <= 0) return;
   hipLaunchKernelGGL(pack_to_float_kernel, dim3(pack_grid(maxnn), nsys), dim3(256), 0, s, pack);
@@ -1721,29 +1769,32 @@ void launch_pack_sum(hipStream_t s, const PackSys* pack, int nsys, int nround) {
 void launch_functional_pol(hipStream_t s, int func, int64_t npts, int bs, const double* ra,
                            const double* ga, const double* rb, const double* gb, const double* w, double* vsa,
                            double* gwa, double* vsb, double* gwb, double* e_blk, const double* ra2,
-                           const double* ga2, const double* rb2, const double* gb2) {
+                           const double* ga2, const double* rb2, const double* gb2, const DevBlock* blocks,
+                           const double* part_a, const double* part_b) {
   const int nb = (int)((npts + bs - 1) / bs);
   if (nb <= 0) return;
   hipLaunchKernelGGL(functional_pol_kernel, dim3(nb), dim3(128), 0, s, func, npts, bs, ra, ga, rb, gb, w, vsa,
-                     gwa, vsb, gwb, e_blk, ra2, ga2, rb2, gb2);
+                     gwa, vsb, gwb, e_blk, ra2, ga2, rb2, gb2, blocks, part_a, part_b);
 }
 
 template <typename T>
 void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, const DevBlock* blocks, const T* tiles,
                      const double* vs, const double* gw, int gga, double thr, T* Tscr, int64_t npts,
-                     const PackSys* pack) {
+                     const PackSys* pack, bool pairs) {
   if (nwork <= 0) return;
   constexpr bool f64 = sizeof(T) == 8;
-#define SXC_FOCK_SHAPE(k)                                                                                           \
-  if (shape == k) {                                                                                                 \
-    constexpr FockShape sh = kFockShape[k];                                                                         \
-    if (f64 && !gga)                                                                                                \
-      hipLaunchKernelGGL((fock_sub_kernel<T, sh.waves, sh.rows, sh.slots, f64>), dim3(nwork), dim3(64 * sh.waves), 0, \
-                         s, work, blocks, tiles, vs, gw, gga, thr, Tscr, npts, pack);                               \
-    else                                                                                                            \
-      hipLaunchKernelGGL((fock_sub_kernel<T, sh.waves, sh.rows, sh.slots, false>), dim3(nwork), dim3(64 * sh.waves), \
-                         0, s, work, blocks, tiles, vs, gw, gga, thr, Tscr, npts, pack);                            \
-    return;                                                                                                         \
+  const dim3 grid(pairs ? (nwork + 7) / 8 * 16 : nwork);
+  const int np = pairs ? nwork : 0;
+#define SXC_FOCK_SHAPE(k)                                                                                             \
+  if (shape == k) {                                                                                                   \
+    constexpr FockShape sh = kFockShape[k];                                                                           \
+    if (f64 && !gga)                                                                                                  \
+      hipLaunchKernelGGL((fock_sub_kernel<T, sh.waves, sh.rows, sh.slots, f64>), grid, dim3(64 * sh.waves), 0, s,     \
+                         work, blocks, tiles, vs, gw, gga, thr, Tscr, npts, pack, np);                                \
+    else                                                                                                              \
+      hipLaunchKernelGGL((fock_sub_kernel<T, sh.waves, sh.rows, sh.slots, false>), grid, dim3(64 * sh.waves), 0, s,   \
+                         work, blocks, tiles, vs, gw, gga, thr, Tscr, npts, pack, np);                                \
+    return;                                                                                                           \
   }
   static_assert(kFockShapes == 4, "one case per shape");
   SXC_FOCK_SHAPE(0)
@@ -1754,9 +1805,10 @@ void launch_fock_sub(hipStream_t s, int shape, const FockItem* work, int nwork, 
   throw std::runtime_error("launch_fock_sub: unknown workgroup shape");
 }
 template void launch_fock_sub<double>(hipStream_t, int, const FockItem*, int, const DevBlock*, const double*,
-                                      const double*, const double*, int, double, double*, int64_t, const PackSys*);
+                                      const double*, const double*, int, double, double*, int64_t, const PackSys*,
+                                      bool);
 template void launch_fock_sub<float>(hipStream_t, int, const FockItem*, int, const DevBlock*, const float*,
-                                     const double*, const double*, int, double, float*, int64_t, const PackSys*);
+                                     const double*, const double*, int, double, float*, int64_t, const PackSys*, bool);
 
 // Row columns per LDS pass of the reduce: kReduceWindow, or less where the device's LDS per
 // workgroup cannot hold that many columns of 8 bytes (fixed = false) or 16 bytes (fixed = true).

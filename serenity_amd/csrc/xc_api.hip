@@ -602,6 +602,10 @@ struct xc_bfogc {
   DBuf<int> d_ao_atom;
   // unrestricted builds (allocated on first use): beta density, potential, P and F
   DBuf<double> d_rho_b, d_grad_b, d_vs_b, d_gw_b, d_Pb, d_Fb;
+  // the other spin's scratch of a build that runs both spins at once (kPairUnknown until first asked for)
+  DBuf<double> d_part_b, d_T_b, d_U_b;
+  DBuf<PackSys> d_pair;
+  enum { kPairUnknown, kPairYes, kPairNo } pair = kPairUnknown;
   DBuf<float> d_P32b;
   bool ecache_valid[kNumFunctionals] = {};
   // serving: a build of this controller is in flight on a server slot; captured builds
@@ -729,6 +733,90 @@ void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, 
   if (s == bf->ctx->stream && nspin == 1 && direct) bf->ctx->mark();
   if (E && (P32 || !direct))
     launch_sum(s, bf->d_eblk.p, nxc, E, 0, P32 ? bf->d_round.p : nullptr, P32 ? (int64_t)nspin * nround : 0);
+}
+
+// Whether an unrestricted build runs both spins in each launch.  A spin's density and Fock kernels leave a
+// tail of idle compute units and read the same tiles: (H2O)5/def2-TZVP (215 AOs, 31 700
+// points) 600 us one after the other, 482 at once (densities 197 -> 166, Fock stages 200 -> 160).
+// For matrices that take the direct reduce and 128-point blocks; it needs a second scratch of each kind,
+// and a controller that gets none keeps one spin after the other.
+bool pair_buffers(xc_bfogc* bf) {
+  if (bf->pair == xc_bfogc::kPairUnknown) {
+    bf->pair = xc_bfogc::kPairNo;
+    const size_t n = (size_t)bf->basis->nao;
+    if (n <= kDirectRows && bf->bs == kTile) {
+      try {
+        bf->d_part_b.alloc(bf->ctx, bf->d_part.n);
+        bf->d_T_b.alloc(bf->ctx, bf->d_T.n);
+        bf->d_U_b.alloc(bf->ctx, n * n);
+        bf->d_pair.alloc(bf->ctx, 2);
+        bf->pair = xc_bfogc::kPairYes;
+      } catch (const XcError&) {
+        bf->d_part_b.free_();
+        bf->d_T_b.free_();
+        bf->d_U_b.free_();
+      }
+    }
+  }
+  return bf->pair == xc_bfogc::kPairYes;
+}
+
+// Both spins of an unrestricted build in each launch.
+template <typename T>
+void enqueue_build_pair(xc_bfogc* bf, int functional, double thr, const double* const* Ps, double* const* Fs,
+                               const Lanes& L, double* d_energy) {
+  constexpr bool fp32 = sizeof(T) == 4;
+  hipStream_t s = L.main;
+  const int n = bf->basis->nao;
+  const int64_t N = bf->grid->npts;
+  const int nxc = (int)((N + kTile - 1) / kTile);
+  const int g = functional_is_gga(functional) ? 1 : 0;
+  const bool form = !fp32 && use_form(g, n);
+  PackPair pair{};
+  for (int sp = 0; sp < 2; ++sp) {
+    PackSys& ps = pair.s[sp];
+    ps.tiles = fp32 ? (const void*)bf->d_t32.p : (const void*)bf->d_t64.p;
+    ps.P64 = Ps[sp];
+    ps.P32 = fp32 ? (sp ? bf->d_P32b.p : bf->d_P32.p) : nullptr;
+    ps.U = sp ? bf->d_U_b.p : bf->d_U.p;
+    ps.P = fp32 ? (const void*)ps.P32 : form ? (const void*)ps.U : (const void*)Ps[sp];
+    ps.ao_idx = bf->d_ao_idx.p;
+    ps.part = sp ? bf->d_part_b.p : bf->d_part.p;
+    ps.w = bf->grid->d_w.p;
+    ps.vs = sp ? bf->d_vs_b.p : bf->d_vs.p;
+    ps.gw = sp ? bf->d_gw_b.p : bf->d_gw.p;
+    ps.T = sp ? bf->d_T_b.p : bf->d_T.p;
+    ps.ent = bf->d_rowent.p;
+    ps.row_ptr = bf->d_rowptr.p;
+    ps.F = Fs[sp];
+    ps.eblk = bf->d_eblk.p;
+    ps.round = bf->d_round.p + (size_t)sp * (fp32 ? n : 0);
+    ps.E = sp == 1 && !fp32 ? d_energy : nullptr;  // (FP32: with the rounding term below)
+    ps.npts = N;
+    ps.n = n;
+    ps.nxc = nxc;
+  }
+  const PackSys* sys = bf->d_pair.p;
+  launch_set_pair(s, pair, bf->d_pair.p);
+  if (fp32) launch_pack_to_float(s, sys, 2, (int64_t)n * n);
+  if (form) launch_fold(s, nullptr, nullptr, n, sys, 2);
+  launch_density_sub<T>(s, bf->d_dens_work.p, (int)bf->dens_work.size(), bf->d_blocks.p, nullptr, nullptr, nullptr, 0, g,
+                        nullptr, 0, sys, nullptr, nullptr, form, true);
+  launch_functional_pol(s, functional, N, kTile, nullptr, nullptr, nullptr, nullptr, bf->grid->d_w.p, bf->d_vs.p,
+                        bf->d_gw.p, bf->d_vs_b.p, bf->d_gw_b.p, bf->d_eblk.p, nullptr, nullptr, nullptr, nullptr,
+                        bf->d_blocks.p, bf->d_part.p, bf->d_part_b.p);
+  over_lanes(L, kFockShapes, [&](int c) { return (int)bf->fock_items[c].size(); }, [&](int c, hipStream_t st) {
+    launch_fock_sub<T>(st, c, bf->d_fock_items[c].p, (int)bf->fock_items[c].size(), bf->d_blocks.p, nullptr, nullptr,
+                       nullptr, g, thr, nullptr, 0, sys, true);
+  });
+  ReduceOut out{};
+  out.direct = true;
+  out.round = fp32 ? bf->d_round.p : nullptr;
+  launch_fock_reduce<T>(s, nullptr, nullptr, nullptr, nullptr, nullptr, n, sys, 2, bf->ctx->deterministic,
+                        bf->sum_nb > 256 * (int64_t)bf->nblocks, out);
+  // with the first-order FP32 rounding term of each spin density matrix (dE_xc/dP_s = F_s)
+  if (fp32) launch_sum(s, bf->d_eblk.p, nxc, d_energy, 0, bf->d_round.p, 2 * (int64_t)n);
+  HIPX(hipGetLastError());
 }
 
 template <typename T>
@@ -1581,7 +1669,6 @@ static void enqueue_build(xc_bfogc* bf, int functional, int precision, double th
           "mixed precision needs both tile sets (keep_fp32 = 1)");
   const int n = bf->basis->nao;
   const int64_t N = bf->grid->npts;
-  const int nxc = (int)((N + kTile - 1) / kTile);
   if (s == ctx->stream) ctx->mark();
   if (lowp) launch_to_float(s, dP, bf->d_P32.p, (int64_t)n * n);
   if (mixed) launch_to_double(s, bf->d_P32.p, bf->d_P32d.p, (int64_t)n * n);
@@ -1642,7 +1729,6 @@ static void ensure_pol_buffers(xc_bfogc* bf, bool fp32) {
  * spin, each with its own block skip); E_xc left in d_energy. */
 static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, double thr, const double* dPa,
                               const double* dPb, double* dFa, double* dFb, const Lanes& L, double* d_energy) {
-  xc_ctx* ctx = bf->ctx;
   hipStream_t s = L.main;
   require(!bf->in_flight, XC_ERR_STATE, "a server build of this controller is in flight");
   require(functional >= 0 && functional < kNumFunctionals, XC_ERR_ARG, "unknown functional");
@@ -1655,10 +1741,17 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
   require(precision == XC_PREC_FP32 || bf->d_t64.p, XC_ERR_STATE, "FP64 contractions need FP64 tiles");
   const int n = bf->basis->nao;
   const int64_t N = bf->grid->npts;
-  const int nxc = (int)((N + kTile - 1) / kTile);
   ensure_pol_buffers(bf, precision == XC_PREC_FP32);
-  // spin densities: one density pass per spin through the shared partial buffer
   const double* Ps[2] = {dPa, dPb};
+  double* Fs[2] = {dFa, dFb};
+  if (pair_buffers(bf)) {
+    if (precision == XC_PREC_FP64)
+      enqueue_build_pair<double>(bf, functional, thr, Ps, Fs, L, d_energy);
+    else
+      enqueue_build_pair<float>(bf, functional, thr, Ps, Fs, L, d_energy);
+    return;
+  }
+  // spin densities: one density pass per spin through the shared partial buffer
   double* rho[2] = {bf->d_rho.p, bf->d_rho_b.p};
   double* grad[2] = {bf->d_grad.p, bf->d_grad_b.p};
   float* P32[2] = {bf->d_P32.p, bf->d_P32b.p};
@@ -1678,7 +1771,6 @@ static void enqueue_build_pol(xc_bfogc* bf, int functional, int precision, doubl
                         bf->d_eblk.p);
   const double* vs[2] = {bf->d_vs.p, bf->d_vs_b.p};
   const double* gw[2] = {bf->d_gw.p, bf->d_gw_b.p};
-  double* Fs[2] = {dFa, dFb};
   for (int sp = 0; sp < 2; ++sp) {
     // with the first-order FP32 rounding term of each spin density matrix (dE_xc/dP_s = F_s)
     double* E = sp == 1 ? d_energy : nullptr;
@@ -1872,7 +1964,6 @@ static void enqueue_nadd_pol(xc_bfogc* act, int nenv, xc_bfogc* const* env, int 
     require(fp32 || b->d_t64.p, XC_ERR_STATE, "FP64 contractions need FP64 tiles");
     ensure_pol_buffers(b, fp32);
   }
-  const int n = act->basis->nao;
   const int64_t N = act->grid->npts;
   const int nxc = (int)((N + kTile - 1) / kTile);
   if (!act->d_rho_sup.p) {
