@@ -39,16 +39,17 @@ constexpr int kGradKC = 16;                // AOs per chunk
 constexpr int kGradRS = kGradKC + 2;       // 144-byte LDS rows: the 16 rows of an operand read hit distinct banks
 constexpr int kGradRows = 2 * kTile + 16 * kDensMaxS;  // phi, G and P columns
 
-// One workgroup of 8 wavefronts per (block, pass of 16 S columns): wavefront w owns points 16 w ..
-// 16 w + 15 and the S column tiles of both phi P and G P.  What bounds it is the FP64 matrix
-// cores, 2 x 2 B n_b ncols operations per pass; one workgroup per compute unit (both products'
-// accumulators take 16 S registers a lane), so the AOs stream in chunks of 16 through two LDS
+// One workgroup of 16 wavefronts per (block, pass of 16 S columns): wavefront w owns points
+// 16 (w % 8) .. + 15 and half w / 8 of the column tiles of both phi P and G P.  What bounds it is the
+// FP64 matrix cores, 2 x 2 B n_b ncols operations per pass, and the latency of its loads; one workgroup
+// per compute unit (LDS), so the AOs stream in chunks of 16 through two LDS
 // buffers with one barrier a chunk: the next chunk is loaded before the chunk's MFMAs and stored
 // after them, G formed from the value and gradient tiles on its way.  The accumulators are transposed
 // (rows: AO columns, columns: points), so that the column dots read 16 consecutive points of a
-// tile row.  At C8H18/def2-TZVP/PBE the kernel takes 1.00 ms (2.57 with 4 wavefronts per 64 columns,
-// one buffer and one element per LDS read); without its tile loads it would take 0.5 (timing only):
-// the ten planes of a block and the four staged again per pass come at about 4 TB/s.
+// tile row.  At C8H18/def2-TZVP/PBE the kernel takes 0.84 ms (1.00 with 8 wavefronts of all S column
+// tiles: 214 registers, two wavefronts per SIMD; 2.57 with 4 wavefronts per 64 columns, one buffer and
+// one element per LDS read).  The ten planes of a block and the four staged again per pass come at
+// about 3 TB/s, the matrix cores are busy 0.31 ms.
 template <int S>
 __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock& bk, const int* __restrict__ ao_idx,
                                               const double* __restrict__ tiles, const double* __restrict__ P, int n,
@@ -57,17 +58,19 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
                                               double (*buf)[kGradRows][kGradRS], double (*spot)[kTile],
                                               double (*red)[16 * kDensMaxS][3]) {
   using M = Mfma<double>;
-  constexpr int KC = kGradKC, KV = KC / 4, NP = (16 * S + 31) / 32;
+  constexpr int KC = kGradKC, KV = KC / 4, EV = KC / 8, NP = (16 * S + 63) / 64, HS = (S + 1) / 2;
   typedef double vec_t __attribute__((ext_vector_type(KV)));
+  typedef double stage_t __attribute__((ext_vector_type(EV)));
   const int col0 = wk.a, ncols = wk.b;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6) & 7;
+  const int c0 = HS * __builtin_amdgcn_readfirstlane(tid >> 9);  // the wavefront's first column tile
   const int r = lane & 15, g = lane >> 4;
   const gmem<const double>* tb = to_global(tiles + bk.tile_off);
   const int64_t cs = (int64_t)bk.npad * kTile;
   const gmem<const int>* idx = to_global(ao_idx + bk.idx_off);
   const gmem<const double>* Pg = to_global(P);
-  // staging: point pa, AO quad qa of phi and G; P elements (AO tid % 16, columns tid / 16 + 32 m)
+  // staging: point pa, AO pair qa of phi and G; P elements (AO tid % 16, columns tid / 16 + 64 m)
   const int pa = tid & (kTile - 1), qa = tid >> 7, ka = tid & 15;
   double vp = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
   if (pa < bk.npts) {
@@ -87,13 +90,13 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
   int nu[NP];
 #pragma unroll
   for (int m = 0; m < NP; ++m) {
-    const int c = (tid >> 4) + 32 * m;
+    const int c = (tid >> 4) + 64 * m;
     nu[m] = c < ncols ? idx[col0 + c] : -1;
   }
   const int kend = (bk.nb + KC - 1) / KC * KC;  // whole chunks: at most npad, whose last AOs are zero
-  double ph[KV], dx[KV], dy[KV], dz[KV], rp[NP];
+  double ph[EV], dx[EV], dy[EV], dz[EV], rp[NP];
 #pragma unroll
-  for (int e = 0; e < KV; ++e) dx[e] = dy[e] = dz[e] = 0.0;
+  for (int e = 0; e < EV; ++e) dx[e] = dy[e] = dz[e] = 0.0;
   int mu = idx[ka], mu_now = mu;
   auto load = [&](int k0) {
     mu_now = mu;
@@ -101,8 +104,8 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
     for (int m = 0; m < NP; ++m) rp[m] = Pg[max(mu, 0) + (int64_t)n * max(nu[m], 0)];
     if (k0 + KC < kend) mu = idx[k0 + KC + ka];  // the next chunk's P addresses depend on no load of it
 #pragma unroll
-    for (int e = 0; e < KV; ++e) {
-      const int64_t o = (int64_t)(k0 + KV * qa + e) * kTile + pa;
+    for (int e = 0; e < EV; ++e) {
+      const int64_t o = (int64_t)(k0 + EV * qa + e) * kTile + pa;
       ph[e] = tb[o];
       if (gga) {
         dx[e] = tb[cs + o];
@@ -112,24 +115,24 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
     }
   };
   auto store = [&](int b) {
-    vec_t f, h;
+    stage_t f, h;
 #pragma unroll
-    for (int e = 0; e < KV; ++e) {
+    for (int e = 0; e < EV; ++e) {
       f[e] = ph[e];
       h[e] = vp * ph[e] + gx * dx[e] + gy * dy[e] + gz * dz[e];
     }
-    *reinterpret_cast<vec_t*>(&buf[b][pa][KV * qa]) = f;
-    *reinterpret_cast<vec_t*>(&buf[b][kTile + pa][KV * qa]) = h;
+    *reinterpret_cast<stage_t*>(&buf[b][pa][EV * qa]) = f;
+    *reinterpret_cast<stage_t*>(&buf[b][kTile + pa][EV * qa]) = h;
 #pragma unroll
     for (int m = 0; m < NP; ++m) {
-      const int c = (tid >> 4) + 32 * m;
+      const int c = (tid >> 4) + 64 * m;
       // padding read P[0][0]; a zero for it (a select at the load would wait for it there)
       if (c < 16 * S) buf[b][2 * kTile + c][ka] = mu_now >= 0 && nu[m] >= 0 ? rp[m] : 0.0;
     }
   };
-  M::acc_t T[S], TG[S];
+  M::acc_t T[HS], TG[HS];
 #pragma unroll
-  for (int c = 0; c < S; ++c) {
+  for (int c = 0; c < HS; ++c) {
     T[c] = M::zero();
     TG[c] = M::zero();
   }
@@ -143,8 +146,9 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
     const vec_t af = *reinterpret_cast<const vec_t*>(&buf[b][16 * w + r][KV * g]);
     const vec_t ag = *reinterpret_cast<const vec_t*>(&buf[b][kTile + 16 * w + r][KV * g]);
 #pragma unroll
-    for (int c = 0; c < S; ++c) {
-      const vec_t bv = *reinterpret_cast<const vec_t*>(&buf[b][2 * kTile + 16 * c + r][KV * g]);
+    for (int c = 0; c < HS; ++c) {
+      if (c0 + c >= S) break;  // uniform: the last tile of the second half where S is odd
+      const vec_t bv = *reinterpret_cast<const vec_t*>(&buf[b][2 * kTile + 16 * (c0 + c) + r][KV * g]);
 #pragma unroll
       for (int t = 0; t < KV; ++t) {
         T[c] = M::step(bv[t], af[t], T[c]);
@@ -159,11 +163,11 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
   const int p = 16 * w + r;  // rows of points beyond the block are zero in the tiles
   const double wx = spot[0][p], wy = spot[1][p], wz = spot[2][p];
 #pragma unroll
-  for (int c = 0; c < S; ++c) {
-    if (16 * c >= ncols) break;  // uniform
+  for (int c = 0; c < HS; ++c) {
+    if (16 * (c0 + c) >= ncols) break;  // uniform
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int cl = 16 * c + g + 4 * e;
+      const int cl = 16 * (c0 + c) + g + 4 * e;
       const gmem<const double>* row = tb + (int64_t)(col0 + cl) * kTile + p;
       const double tg = TG[c][e];
       double ax = tg * row[cs], ay = tg * row[2 * cs], az = tg * row[3 * cs];
@@ -198,7 +202,7 @@ __device__ __forceinline__ void gradient_item(const WorkItem& wk, const DevBlock
   }
 }
 
-__global__ __launch_bounds__(512) void gradient_kernel(const WorkItem* __restrict__ work,
+__global__ __launch_bounds__(1024) void gradient_kernel(const WorkItem* __restrict__ work,
                                                        const DevBlock* __restrict__ blocks,
                                                        const int* __restrict__ ao_idx,
                                                        const double* __restrict__ tiles,
@@ -247,7 +251,7 @@ void launch_gradient(hipStream_t s, const WorkItem* work, int nwork, const DevBl
                      const double* tiles, const double* P, int n, const double* vs, const double* gw, int gga,
                      int64_t npts, double* acc) {
   if (nwork <= 0) return;
-  hipLaunchKernelGGL(gradient_kernel, dim3(nwork), dim3(512), 0, s, work, blocks, ao_idx, tiles, P, n, vs, gw, gga,
+  hipLaunchKernelGGL(gradient_kernel, dim3(nwork), dim3(1024), 0, s, work, blocks, ao_idx, tiles, P, n, vs, gw, gga,
                      npts, acc);
 }
 
