@@ -173,12 +173,18 @@ int xc_ri_metric(int naux_shell, const int* aux_l, const int* aux_pure, const in
  * integrals.  Orbital shells up to f, auxiliary up to g.
  *   xc_coulomb_rhs:    b_P = sum_mu,nu P_mu,nu (mu nu|P)     (P host n x n, b host naux)
  *   xc_coulomb_matrix: J_mu,nu = sum_P c_P (mu nu|P)         (c host naux, J host n x n)
- * with c = M^-1 b between the two (M from xc_ri_metric). */
+ * with c = M^-1 b between the two (M from xc_ri_metric).
+ *   xc_coulomb_set_metric: keeps M's Cholesky factor on the device (L lower, row-major naux x naux; what
+ *                          is above the diagonal is not read)
+ *   xc_coulomb_build:      J from P in one go, the metric's solves on the device; XC_ERR_INPUT where
+ *                          b is not finite */
 typedef struct xc_coulomb xc_coulomb;
 int xc_coulomb_create(xc_basis* basis, xc_basis* aux, double threshold, xc_coulomb** out);
 int xc_coulomb_info(const xc_coulomb* jc, int64_t* npairs, int64_t* hermite_terms);
 int xc_coulomb_rhs(xc_coulomb* jc, const double* P, double* b);
 int xc_coulomb_matrix(xc_coulomb* jc, const double* c, double* J);
+int xc_coulomb_set_metric(xc_coulomb* jc, const double* L);
+int xc_coulomb_build(xc_coulomb* jc, const double* P, double* J);
 int xc_coulomb_destroy(xc_coulomb* jc);
 
 /* Density-fitted Coulomb integrals over an auxiliary shell list: B3 is

@@ -11,6 +11,7 @@ LIB_PATH = os.path.join(HERE, "libserenity_xc.so")
 
 XC_OK = 0
 XC_BUSY = 6
+XC_ERR_INPUT = 5
 FUNCTIONALS = {"LDA": 0, "PBE": 1, "TF": 2, "SLATER": 3, "VWN5": 4, "PBEX": 5, "PBEC": 6, "PBE_LIBXC": 7, "BP86": 8}
 GGA = {"PBE", "PBEX", "PBEC", "PBE_LIBXC", "BP86"}
 PRECISIONS = {"FP64": 0, "FP32": 1, "MIXED": 2}
@@ -77,6 +78,8 @@ def lib():
     _sig("xc_coulomb_info", C.c_int, vp, C.POINTER(i64), C.POINTER(i64))
     _sig("xc_coulomb_rhs", C.c_int, vp, dp, dp)
     _sig("xc_coulomb_matrix", C.c_int, vp, dp, dp)
+    _sig("xc_coulomb_set_metric", C.c_int, vp, dp)
+    _sig("xc_coulomb_build", C.c_int, vp, dp, dp)
     _sig("xc_coulomb_destroy", C.c_int, vp)
     _sig("xc_basis_create", C.c_int, vp, C.c_int, ip, ip, ip, dp, dp, dp, C.POINTER(vp))
     _sig("xc_basis_destroy", C.c_int, vp)

@@ -378,6 +378,13 @@ void launch_jaux_in(hipStream_t s, const JView& J, int naux, const int* prim_she
                     const double* prim_coef, const int* cart_off, const double* cc, double* U);
 void launch_jaux_out(hipStream_t s, const JView& J, const DevShell* aux, int nshell, const int* shell_prim,
                      const double* prim_coef, const int* cart_off, const double* W, double* bc);
+// cc = the Cartesian form of M^-1 b, b the auxiliary AOs of bc, with M = L L^T (L row-major n x n, dinv the
+// inverses of its diagonal blocks of kSolveBlock, row-major and zero-padded); b, y: n each.  bad is set
+// where b is not finite.
+constexpr int kSolveBlock = 64;
+void launch_metric_solve(hipStream_t s, const double* L, int n, const double* dinv, const DevShell* aux, int nshell,
+                         const double* ang, const int* cart_off, const double* bc, double* b, double* y, double* cc,
+                         int* bad);
 void launch_jassemble(hipStream_t s, int cls, const JPairItem* items, int nitem, const JPair* pairs,
                       const DevShell* shells, const double* ang, const JView& Jv, const double* V, int n, double* J);
 

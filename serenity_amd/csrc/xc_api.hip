@@ -272,6 +272,7 @@ struct xc_ctx {
   // E_xc of the last build: pinned host memory that the kernels write (a copy of 8 bytes back to the
   // host costs 15 us more than the wait for the stream)
   double* energy = nullptr;
+  int* flag = nullptr;  // likewise, for a kernel's report
   double* pack_energy = nullptr;  // likewise of a packed build's systems (grown on demand)
   size_t pack_energies = 0;
   HostStage stage;
@@ -456,6 +457,8 @@ struct xc_coulomb {
   std::vector<JPairItem> pair_items[kJPairClasses];
   DBuf<JPairItem> d_pair_items[kJPairClasses];
   DBuf<double> d_D, d_V, d_U, d_bc, d_cc, d_P, d_J;
+  // the metric's Cholesky factor (lower, row-major), the inverses of its diagonal blocks, and the solves' vectors
+  DBuf<double> d_L, d_dinv, d_b, d_y;
   void plan_items();
 };
 
@@ -876,8 +879,9 @@ int xc_ctx_create(int device, xc_ctx** out) {
     noalloc_setup_current_device(device);
     HIPX(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     c->lanes.create(c->stream, true);
-    HIPX(hipHostMalloc((void**)&c->energy, sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
-    *c->energy = 0.0;
+    HIPX(hipHostMalloc((void**)&c->energy, 2 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
+    c->energy[0] = c->energy[1] = 0.0;
+    c->flag = reinterpret_cast<int*>(c->energy + 1);
     c->stage.create();
     *out = c;
   });
@@ -2678,6 +2682,46 @@ int xc_coulomb_destroy(xc_coulomb* jc) {
   });
 }
 
+// b in Cartesian auxiliary functions (d_bc) from the density in d_P.
+static void enqueue_coulomb_rhs(xc_coulomb* jc) {
+  xc_ctx* ctx = jc->ctx;
+  hipStream_t s = ctx->stream;
+  const int n = jc->basis->nao;
+  over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
+             [&](int c, hipStream_t st) {
+    launch_jdens(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p, jc->basis->d_shells.p,
+                 jc->basis->d_ang.p, jc->view, jc->d_P.p, n, jc->d_D.p);
+  });
+  launch_fill(s, jc->d_U.p, jc->aherm_total, 0.0);
+  // the widest classes (the longest items, few of them) beside the others
+  over_lanes(ctx->lanes, kJClasses, [&](int c) { return (int)jc->items[0][c].size(); }, [&](int c, hipStream_t st) {
+    launch_jrhs(st, c, jc->d_items[0][c].p, (int)jc->items[0][c].size(), jc->view, jc->d_D.p, jc->d_U.p);
+  });
+  launch_jaux_out(s, jc->view, jc->aux->d_shells.p, jc->aux->nshell, jc->d_shell_prim.p, jc->d_prim_coef.p,
+                  jc->d_cart_off.p, jc->d_U.p, jc->d_bc.p);
+  HIPX(hipGetLastError());
+}
+
+// J (d_J) from the Cartesian auxiliary coefficients in d_cc.
+static void enqueue_coulomb_matrix(xc_coulomb* jc) {
+  xc_ctx* ctx = jc->ctx;
+  hipStream_t s = ctx->stream;
+  const int n = jc->basis->nao;
+  launch_jaux_in(s, jc->view, jc->naux, jc->d_prim_shell.p, jc->aux->d_shells.p, jc->d_prim_coef.p, jc->d_cart_off.p,
+                 jc->d_cc.p, jc->d_U.p);
+  launch_fill(s, jc->d_V.p, jc->herm_total, 0.0);
+  over_lanes(ctx->lanes, kJClasses, [&](int c) { return (int)jc->items[1][c].size(); }, [&](int c, hipStream_t st) {
+    launch_jpot(st, c, jc->d_items[1][c].p, (int)jc->items[1][c].size(), jc->view, jc->d_U.p, jc->d_V.p);
+  });
+  launch_fill(s, jc->d_J.p, (int64_t)n * n, 0.0);
+  over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
+             [&](int c, hipStream_t st) {
+    launch_jassemble(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p,
+                     jc->basis->d_shells.p, jc->basis->d_ang.p, jc->view, jc->d_V.p, n, jc->d_J.p);
+  });
+  HIPX(hipGetLastError());
+}
+
 int xc_coulomb_rhs(xc_coulomb* jc, const double* P, double* b) {
   return guarded([&] {
     require(jc && P && b, XC_ERR_ARG, "xc_coulomb_rhs: null argument");
@@ -2686,19 +2730,7 @@ int xc_coulomb_rhs(xc_coulomb* jc, const double* P, double* b) {
     hipStream_t s = ctx->stream;
     const int n = jc->basis->nao;
     ctx->stage.up(s, jc->d_P.p, P, sizeof(double) * n * n);
-    over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
-               [&](int c, hipStream_t st) {
-      launch_jdens(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p, jc->basis->d_shells.p,
-                   jc->basis->d_ang.p, jc->view, jc->d_P.p, n, jc->d_D.p);
-    });
-    launch_fill(s, jc->d_U.p, jc->aherm_total, 0.0);
-    // the widest classes (the longest items, few of them) beside the others
-    over_lanes(ctx->lanes, kJClasses, [&](int c) { return (int)jc->items[0][c].size(); }, [&](int c, hipStream_t st) {
-      launch_jrhs(st, c, jc->d_items[0][c].p, (int)jc->items[0][c].size(), jc->view, jc->d_D.p, jc->d_U.p);
-    });
-    launch_jaux_out(s, jc->view, jc->aux->d_shells.p, jc->aux->nshell, jc->d_shell_prim.p, jc->d_prim_coef.p,
-                    jc->d_cart_off.p, jc->d_U.p, jc->d_bc.p);
-    HIPX(hipGetLastError());
+    enqueue_coulomb_rhs(jc);
     std::vector<double> bc(jc->ncart_aux);
     ctx->stage.down(s, {{bc.data(), jc->d_bc.p, sizeof(double) * bc.size()}});
     // Cartesian -> auxiliary AO: b_f = sum_c M[f][c] b_c
@@ -2729,20 +2761,59 @@ int xc_coulomb_matrix(xc_coulomb* jc, const double* c, double* J) {
           cc[jc->cart_off[k] + q] += c[S.ao_off + f] * jc->aux->ang[S.ang_off + f * S.ncart + q];
     }
     ctx->stage.up(s, jc->d_cc.p, cc.data(), sizeof(double) * jc->ncart_aux);
-    launch_jaux_in(s, jc->view, jc->naux, jc->d_prim_shell.p, jc->aux->d_shells.p, jc->d_prim_coef.p,
-                   jc->d_cart_off.p, jc->d_cc.p, jc->d_U.p);
-    launch_fill(s, jc->d_V.p, jc->herm_total, 0.0);
-    over_lanes(ctx->lanes, kJClasses, [&](int c) { return (int)jc->items[1][c].size(); }, [&](int c, hipStream_t st) {
-      launch_jpot(st, c, jc->d_items[1][c].p, (int)jc->items[1][c].size(), jc->view, jc->d_U.p, jc->d_V.p);
-    });
-    launch_fill(s, jc->d_J.p, (int64_t)n * n, 0.0);
-    over_lanes(ctx->lanes, kJPairClasses, [&](int c) { return (int)jc->pair_items[c].size(); },
-               [&](int c, hipStream_t st) {
-      launch_jassemble(st, c, jc->d_pair_items[c].p, (int)jc->pair_items[c].size(), jc->d_pairs.p,
-                       jc->basis->d_shells.p, jc->basis->d_ang.p, jc->view, jc->d_V.p, n, jc->d_J.p);
-    });
-    HIPX(hipGetLastError());
+    enqueue_coulomb_matrix(jc);
     ctx->stage.down(s, {{J, jc->d_J.p, sizeof(double) * n * n}});
+  });
+}
+
+int xc_coulomb_set_metric(xc_coulomb* jc, const double* L) {
+  return guarded([&] {
+    require(jc && L, XC_ERR_ARG, "xc_coulomb_set_metric: null argument");
+    xc_ctx* ctx = jc->ctx;
+    std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    const int n = jc->aux->nao, B = kSolveBlock, nblk = (n + B - 1) / B;
+    // the diagonal blocks' inverses, column by column (rows and columns beyond n: zero)
+    std::vector<double> inv((size_t)nblk * B * B, 0.0);
+    for (int k = 0; k < nblk; ++k) {
+      const int m = std::min(B, n - k * B);
+      const double* Lk = L + (size_t)k * B * n + (size_t)k * B;
+      double* D = inv.data() + (size_t)k * B * B;
+      for (int j = 0; j < m; ++j)
+        for (int i = j; i < m; ++i) {
+          double v = i == j ? 1.0 : 0.0;
+          for (int q = j; q < i; ++q) v -= Lk[(size_t)i * n + q] * D[q * B + j];
+          D[i * B + j] = v / Lk[(size_t)i * n + i];
+        }
+    }
+    try {
+      jc->d_dinv.upload(ctx, inv.data(), inv.size());
+      jc->d_b.alloc(ctx, (size_t)std::max(n, 1));
+      jc->d_y.alloc(ctx, (size_t)std::max(n, 1));
+      jc->d_L.upload(ctx, L, (size_t)n * n);
+    } catch (...) {
+      jc->d_L.free_();
+      throw;
+    }
+    HIPX(hipStreamSynchronize(ctx->stream));
+  });
+}
+
+int xc_coulomb_build(xc_coulomb* jc, const double* P, double* J) {
+  return guarded([&] {
+    require(jc && P && J, XC_ERR_ARG, "xc_coulomb_build: null argument");
+    require(jc->d_L.p, XC_ERR_STATE, "xc_coulomb_build: no metric (call xc_coulomb_set_metric)");
+    xc_ctx* ctx = jc->ctx;
+    std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    hipStream_t s = ctx->stream;
+    const int n = jc->basis->nao;
+    ctx->stage.up(s, jc->d_P.p, P, sizeof(double) * n * n);
+    enqueue_coulomb_rhs(jc);
+    *ctx->flag = 0;  // (nothing that writes it is in flight: every call that does waits for it)
+    launch_metric_solve(s, jc->d_L.p, jc->aux->nao, jc->d_dinv.p, jc->aux->d_shells.p, jc->aux->nshell,
+                        jc->aux->d_ang.p, jc->d_cart_off.p, jc->d_bc.p, jc->d_b.p, jc->d_y.p, jc->d_cc.p, ctx->flag);
+    enqueue_coulomb_matrix(jc);
+    ctx->stage.down(s, {{J, jc->d_J.p, sizeof(double) * n * n}});
+    require(*ctx->flag == 0, XC_ERR_INPUT, "array must not contain infs or NaNs");
   });
 }
 
