@@ -128,7 +128,7 @@ double* noalloc_scratch(int device) {
 }  // namespace
 
 // Execution lanes of a build: its stream plus kAux helper streams.  The launches
-// of one stage (one per work class) are independent, so they are spread over
+// of one stage (the Fock shapes, the J engine's classes) are independent, so they are spread over
 // the lanes after a fork and joined before the next stage.
 constexpr int kAux = 3;
 struct Lanes {
@@ -2338,7 +2338,7 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       upload_grow(ctx, pw.dens, dens);
       for (int c = 0; c < kFockShapes; ++c) upload_grow(ctx, pw.fock[c], fock[c]);
       const PackSys* dsys = pw.sys.p;
-      // one launch per stage and work class for every system of the pack
+      // one launch per stage (and Fock shape) for every system of the pack
       auto enqueue = [&]() {
         if (fp32) launch_pack_to_float(s, dsys, nsys, maxnn);
         if (form) launch_fold(s, nullptr, nullptr, maxn, dsys, nsys);
