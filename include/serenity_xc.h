@@ -293,7 +293,8 @@ int xc_fock_build_device(xc_bfogc* bfogc, int functional, int precision, double 
  * nsys controllers at once, for callers with many small systems (serving, embedding
  * subsystems).  One functional and precision for all; P_i, F_i device n_i x n_i
  * matrices, energies[i] host.  The work of every system shares one launch per stage
- * and Fock workgroup shape (merged block and work lists with a per-system table); each
+ * and Fock workgroup shape (merged block and work lists with a per-system table; one more
+ * for the density of FP64 LDA or TF packs with systems on both sides of 96 AOs); each
  * F_i and E_xc,i equal those of xc_fock_build_device on the same controller.  The controllers
  * must be distinct, of one context, with 128-point blocks.  Synchronises before
  * returning. */

@@ -428,7 +428,7 @@ void launch_nadd_functional(hipStream_t s, int func, int64_t npts, bool potentia
                             double* gw, double* e_blk);
 // out = sum of e_blk[0..n) (null: out) minus the listed energies in order (summed first where pending)
 void launch_nadd_energy(hipStream_t s, const double* e_blk, int64_t n, const EnvEnergies& env, double* out);
-// Q[i, j] = P[i, j] + P[j, i], Q[i, i] = P[i, i] (packed: every system's P64 into its U, n the largest)
+// Q[i, j] = P[i, j] + P[j, i], Q[i, i] = P[i, i] (packed: P64 into U of the systems whose P is U, n the largest)
 void launch_fold(hipStream_t s, const double* P, double* Q, int n, const PackSys* pack = nullptr, int nsys = 1);
 void launch_to_float(hipStream_t s, const double* src, float* dst, int64_t n);
 // F[i + n j] (+)= U[max(i,j) + n min(i,j)] (U holds the lower triangle)

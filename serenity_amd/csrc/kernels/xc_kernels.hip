@@ -1457,13 +1457,14 @@ __global__ void fill_kernel(double* __restrict__ p, int64_t n, double value) {
   if (i < n) p[i] = value;
 }
 
-// Q = P + P^T, on the diagonal P, of one matrix or of every system of a pack (P64 into U).
+// Q = P + P^T, on the diagonal P, of one matrix or of the systems of a pack whose P is their U (P64 into U).
 constexpr int kFoldTile = 32;
 __global__ __launch_bounds__(256) void fold_kernel(const double* __restrict__ P, double* __restrict__ Q, int n,
                                                    const PackSys* __restrict__ pack) {
   __shared__ double t[kFoldTile][kFoldTile + 1];
   if (pack) {
     const PackSys& ps = pack[blockIdx.z];
+    if (ps.P != ps.U) return;
     P = ps.P64;
     Q = ps.U;
     n = ps.n;

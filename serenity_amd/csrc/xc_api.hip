@@ -396,7 +396,7 @@ struct DBuf {
 struct PackWork {
   DBuf<DevBlock> blocks;
   DBuf<PackSys> sys;
-  DBuf<WorkItem> dens;
+  DBuf<WorkItem> dens[2];  // [1: of the systems whose density is the quadratic form]
   DBuf<FockItem> fock[kFockShapes];
   DBuf<double> round;
   hipGraphExec_t exec = nullptr;  // captured build of a repeated composition
@@ -2221,7 +2221,7 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
     const bool fp32 = precision == XC_PREC_FP32;
     std::vector<DevBlock> blocks;
     std::vector<PackSys> sys(nsys);
-    std::vector<WorkItem> dens;
+    std::vector<WorkItem> dens[2];
     std::vector<FockItem> fock[kFockShapes];
     int64_t maxnn = 0;
     int maxn = 0;
@@ -2242,9 +2242,12 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
         b.sys = i;
         blocks.push_back(b);
       }
+      // each system's density as in its build alone: the form sums in another order, and a
+      // deterministic context's F is the same packed and alone
+      const bool form = !fp32 && use_form(gga, n);
       for (WorkItem w : bf->dens_work) {
         w.block += blk0;
-        dens.push_back(w);
+        dens[form].push_back(w);
       }
       for (int c = 0; c < kFockShapes; ++c)
         for (FockItem f : bf->fock_items[c]) {
@@ -2253,6 +2256,7 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
         }
       PackSys& ps = sys[i];
       ps.tiles = fp32 ? (const void*)bf->d_t32.p : (const void*)bf->d_t64.p;
+      ps.P = fp32 ? (const void*)bf->d_P32.p : form ? (const void*)bf->d_U.p : (const void*)dP[i];
       ps.P64 = dP[i];
       ps.P32 = fp32 ? bf->d_P32.p : nullptr;
       ps.ao_idx = bf->d_ao_idx.p;
@@ -2273,9 +2277,6 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       maxnn = std::max(maxnn, (int64_t)n * n);
       maxn = std::max(maxn, n);
     }
-    const bool form = !fp32 && use_form(gga, maxn);
-    for (int i = 0; i < nsys; ++i)
-      sys[i].P = fp32 ? (const void*)bfs[i]->d_P32.p : form ? (const void*)bfs[i]->d_U.p : (const void*)dP[i];
     // a composition seen once before runs as a captured graph; the first build is eager
     std::vector<uint64_t> key;
     for (int i = 0; i < nsys; ++i) key.push_back((uint64_t)(uintptr_t)bfs[i]);
@@ -2335,19 +2336,21 @@ int xc_fock_build_packed(int nsys, xc_bfogc* const* bfs, int functional, int pre
       HIPX(hipGraphLaunch(pw.exec, s));
     } else {
       upload_grow(ctx, pw.blocks, blocks);
-      upload_grow(ctx, pw.dens, dens);
+      for (int k = 0; k < 2; ++k) upload_grow(ctx, pw.dens[k], dens[k]);
       for (int c = 0; c < kFockShapes; ++c) upload_grow(ctx, pw.fock[c], fock[c]);
       const PackSys* dsys = pw.sys.p;
       // one launch per stage (and Fock shape) for every system of the pack
       auto enqueue = [&]() {
         if (fp32) launch_pack_to_float(s, dsys, nsys, maxnn);
-        if (form) launch_fold(s, nullptr, nullptr, maxn, dsys, nsys);
-        if (fp32)
-          launch_density_sub<float>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
-                                    nullptr, 0, dsys);
-        else
-          launch_density_sub<double>(s, pw.dens.p, (int)dens.size(), pw.blocks.p, nullptr, nullptr, nullptr, 0, g,
-                                     nullptr, 0, dsys, nullptr, nullptr, form);
+        if (!dens[1].empty()) launch_fold(s, nullptr, nullptr, maxn, dsys, nsys);
+        over_lanes(L, 2, [&](int k) { return (int)dens[k].size(); }, [&](int k, hipStream_t st) {
+          if (fp32)
+            launch_density_sub<float>(st, pw.dens[k].p, (int)dens[k].size(), pw.blocks.p, nullptr, nullptr, nullptr, 0,
+                                      g, nullptr, 0, dsys);
+          else
+            launch_density_sub<double>(st, pw.dens[k].p, (int)dens[k].size(), pw.blocks.p, nullptr, nullptr, nullptr, 0,
+                                       g, nullptr, 0, dsys, nullptr, nullptr, k == 1);
+        });
         launch_functional_packed(s, functional, (int)blocks.size(), pw.blocks.p, dsys);
         over_lanes(L, kFockShapes, [&](int c) { return (int)fock[c].size(); }, [&](int c, hipStream_t st) {
           if (fp32)
