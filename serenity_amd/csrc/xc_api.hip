@@ -2488,6 +2488,7 @@ int xc_fock_build_unrestricted(xc_bfogc* bf, int functional, int precision, doub
     require(bf && Pa && Pb && Fa && Fb, XC_ERR_ARG, "xc_fock_build_unrestricted: null argument");
     xc_ctx* ctx = bf->ctx;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    require_idle(bf, "xc_fock_build_unrestricted");
     const int n = bf->basis->nao;
     ensure_pol_buffers(bf, precision == XC_PREC_FP32);
     ctx->stage.up(ctx->stream, bf->d_P.p, Pa, sizeof(double) * n * n);
@@ -2835,6 +2836,7 @@ int xc_fock_build(xc_bfogc* bf, int functional, int precision, double thr, const
     require(bf && P && F, XC_ERR_ARG, "xc_fock_build: null argument");
     xc_ctx* ctx = bf->ctx;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    require_idle(bf, "xc_fock_build");  // a server build reads d_P on its slot's stream to its end
     const int n = bf->basis->nao;
     ctx->stage.up(ctx->stream, bf->d_P.p, P, sizeof(double) * n * n);
     enqueue_build(bf, functional, precision, thr, bf->d_P.p, bf->d_F.p, ctx->lanes, ctx->energy);
