@@ -316,24 +316,33 @@ class DensityFittedCoulomb(_Handle):
         check(_lib.lib().xc_coulomb_info(h, C.byref(np_), C.byref(nh)))
         self.npairs, self.hermite_terms = np_.value, nh.value
 
+    def _density(self, P):
+        Pf = np.asfortranarray(P, dtype=np.float64)
+        if Pf.shape not in ((self.n, self.n), (self.n * self.n,)):
+            raise XCError(1, "DensityFittedCoulomb: density matrix is %s, basis has %d functions" % (Pf.shape, self.n))
+        return Pf
+
     def rhs(self, P):
         """b_Q = sum P_mu,nu (mu nu|Q)."""
         b = np.zeros(self.naux)
-        Pf = np.asfortranarray(P, dtype=np.float64)
+        Pf = self._density(P)
         check(_lib.lib().xc_coulomb_rhs(self.handle, Pf.ctypes.data_as(_lib.dp), _d(b)))
         return b
 
     def matrix(self, c):
         """J_mu,nu = sum_Q c_Q (mu nu|Q)."""
+        c = np.ascontiguousarray(c, dtype=np.float64)
+        if c.size != self.naux:
+            raise XCError(1, "DensityFittedCoulomb: %d fitting coefficients, auxiliary basis has %d functions"
+                          % (c.size, self.naux))
         J = np.zeros((self.n, self.n), order="F")
-        check(_lib.lib().xc_coulomb_matrix(self.handle, _d(np.ascontiguousarray(c, dtype=np.float64)),
-                                           J.ctypes.data_as(_lib.dp)))
+        check(_lib.lib().xc_coulomb_matrix(self.handle, _d(c), J.ctypes.data_as(_lib.dp)))
         return np.array(J)
 
     def coulomb(self, P):
         if self._resident:
             J = np.empty((self.n, self.n), order="F")
-            Pf = np.asfortranarray(P, dtype=np.float64)
+            Pf = self._density(P)
             rc = _lib.lib().xc_coulomb_build(self.handle, Pf.ctypes.data_as(_lib.dp), J.ctypes.data_as(_lib.dp))
             if rc == XC_ERR_INPUT:
                 raise ValueError(_lib.lib().xc_last_error().decode())
