@@ -10,8 +10,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libserenity_xc.so")
 
 XC_OK = 0
+XC_ERR_MEMORY = 3
 XC_BUSY = 6
-XC_ERR_INPUT = 5
 FUNCTIONALS = {"LDA": 0, "PBE": 1, "TF": 2, "SLATER": 3, "VWN5": 4, "PBEX": 5, "PBEC": 6, "PBE_LIBXC": 7, "BP86": 8}
 GGA = {"PBE", "PBEX", "PBEC", "PBE_LIBXC", "BP86"}
 PRECISIONS = {"FP64": 0, "FP32": 1, "MIXED": 2}

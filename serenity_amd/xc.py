@@ -25,7 +25,7 @@ import weakref
 import numpy as np
 
 from . import _lib
-from ._lib import FUNCTIONALS, GGA, PRECISIONS, GRID_TYPES, RADIAL_TYPES, XC_BUSY, XC_ERR_INPUT, XCError, check
+from ._lib import FUNCTIONALS, GGA, PRECISIONS, GRID_TYPES, RADIAL_TYPES, XC_BUSY, XC_ERR_MEMORY, XCError, check
 
 BASIS_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "data", "basis")
 ANGSTROM_TO_BOHR = 1.0 / 0.529177210544
@@ -311,7 +311,10 @@ class DensityFittedCoulomb(_Handle):
         self._cho = scipy.linalg.cho_factor(M)
         # U of M = U^T U in columns is L in rows; a device without room for it leaves the solves here
         U = np.asfortranarray(self._cho[0])
-        self._resident = _lib.lib().xc_coulomb_set_metric(h, U.ctypes.data_as(_lib.dp)) == 0
+        rc = _lib.lib().xc_coulomb_set_metric(h, U.ctypes.data_as(_lib.dp))
+        self._resident = rc != XC_ERR_MEMORY
+        if self._resident:
+            check(rc)
         np_, nh = C.c_int64(), C.c_int64()
         check(_lib.lib().xc_coulomb_info(h, C.byref(np_), C.byref(nh)))
         self.npairs, self.hermite_terms = np_.value, nh.value
@@ -343,10 +346,12 @@ class DensityFittedCoulomb(_Handle):
         if self._resident:
             J = np.empty((self.n, self.n), order="F")
             Pf = self._density(P)
-            rc = _lib.lib().xc_coulomb_build(self.handle, Pf.ctypes.data_as(_lib.dp), J.ctypes.data_as(_lib.dp))
-            if rc == XC_ERR_INPUT:
-                raise ValueError(_lib.lib().xc_last_error().decode())
-            check(rc)
+            try:
+                check(_lib.lib().xc_coulomb_build(self.handle, Pf.ctypes.data_as(_lib.dp), J.ctypes.data_as(_lib.dp)))
+            except XCError as e:
+                if "infs or NaNs" in str(e):  # as the host's solves raise it
+                    raise ValueError(str(e)) from None
+                raise
             return J
         import scipy.linalg
         c = scipy.linalg.cho_solve(self._cho, self.rhs(P))
