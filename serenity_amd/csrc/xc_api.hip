@@ -334,14 +334,15 @@ struct xc_ctx {
     }
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, need);
-    if (e != hipSuccess && cached) {
+    if (e == hipErrorOutOfMemory && cached) {
       (void)hipGetLastError();
       trim();
       e = hipMalloc(&p, need);
     }
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      throw XcError(XC_ERR_MEMORY, "hipMalloc of " + std::to_string(bytes_) + " bytes failed");
+      throw XcError(e == hipErrorOutOfMemory ? XC_ERR_MEMORY : XC_ERR_DEVICE,
+                    "hipMalloc of " + std::to_string(bytes_) + " bytes failed: " + hipGetErrorString(e));
     }
     block_size[p] = need;
     bytes += (int64_t)need;
@@ -742,24 +743,26 @@ void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, 
 // tail of idle compute units and read the same tiles: (H2O)5/def2-TZVP (215 AOs, 31 700
 // points) 600 us one after the other, 482 at once (densities 197 -> 166, Fock stages 200 -> 160).
 // For matrices that take the direct reduce and 128-point blocks; it needs a second scratch of each kind,
-// and a controller that gets none keeps one spin after the other.
+// and a controller that has no room for it keeps one spin after the other.
 bool pair_buffers(xc_bfogc* bf) {
   if (bf->pair == xc_bfogc::kPairUnknown) {
-    bf->pair = xc_bfogc::kPairNo;
     const size_t n = (size_t)bf->basis->nao;
+    auto found = xc_bfogc::kPairNo;
     if (n <= kDirectRows && bf->bs == kTile) {
       try {
         bf->d_part_b.alloc(bf->ctx, bf->d_part.n);
         bf->d_T_b.alloc(bf->ctx, bf->d_T.n);
         bf->d_U_b.alloc(bf->ctx, n * n);
         bf->d_pair.alloc(bf->ctx, 2);
-        bf->pair = xc_bfogc::kPairYes;
-      } catch (const XcError&) {
+        found = xc_bfogc::kPairYes;
+      } catch (const XcError& e) {
         bf->d_part_b.free_();
         bf->d_T_b.free_();
         bf->d_U_b.free_();
+        if (e.code != XC_ERR_MEMORY) throw;
       }
     }
+    bf->pair = found;
   }
   return bf->pair == xc_bfogc::kPairYes;
 }
