@@ -746,6 +746,10 @@ void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, 
 // and a controller that has no room for it keeps one spin after the other.
 bool pair_buffers(xc_bfogc* bf) {
   if (bf->pair == xc_bfogc::kPairUnknown) {
+    // a build that is recorded into a graph allocates nothing: one spin after the other, decided later
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIPX(hipStreamIsCapturing(bf->ctx->stream, &st));
+    if (st != hipStreamCaptureStatusNone) return false;
     const size_t n = (size_t)bf->basis->nao;
     auto found = xc_bfogc::kPairNo;
     if (n <= kDirectRows && bf->bs == kTile) {

@@ -1,4 +1,5 @@
 """What a call does where the device has no room for what makes it faster gives the same results."""
+import ctypes as C
 import subprocess
 import sys
 
@@ -6,7 +7,7 @@ import numpy as np
 import pytest
 
 from common import REPO
-from serenity_amd import xc
+from serenity_amd import _lib, xc
 from serenity_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +58,48 @@ def test_a_device_error_is_not_a_lack_of_memory(ctx):
     with pytest.raises(xc.XCError) as e:
         ctx.alloc(1 << 46)
     assert e.value.code == 3
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FP32"])
+@pytest.mark.parametrize("functional", ["LDA", "PBE"])
+def test_first_unrestricted_device_build_recorded(ctx, functional, precision):
+    """The first unrestricted device build of a controller whose spin buffers exist is recorded into a
+    graph: it allocates nothing, and every replay, with other builds between, gives the eager result
+    (sums of a few thousand terms in another order: 1e-12)."""
+    hip = C.CDLL("libamdhip64.so")
+    Z, X = W.water_chain(2)
+    b = xc.BasisController.from_file("DEF2-SVP", Z, X)
+    g = xc.molecular_grid(Z, X, accuracy=2)
+    n, P = b.nao, W.synthetic_density(b.overlap(), W.n_electrons(Z) // 2)
+    Pa, Pb = np.asfortranarray(0.6 * P), np.asfortranarray(0.4 * P)
+    bf = xc.BasisFunctionOnGridController(ctx, b, g, 128, 1e-9, 1, keep_fp32=True)
+    xc.NAddFuncPotential(bf, [], functional, precision).getMatrixUnrestricted(Pa, Pb, [], [])  # the spin buffers
+    d = [ctx.alloc(8 * n * n) for _ in range(4)]
+    ctx.upload(d[0], Pa)
+    ctx.upload(d[1], Pb)
+    ctx.synchronize()
+    stream, graph, run = C.c_void_p(ctx.stream), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread-local mode
+    rc = _lib.lib().xc_fock_build_unrestricted_device(bf.handle, _lib.FUNCTIONALS[functional],
+                                                      _lib.PRECISIONS[precision], 1e-11, *d, None)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and rc == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    pot = xc.FuncPotential(bf, functional, precision)
+    E = C.c_double()
+    for swap in (False, True, False):
+        ctx.upload(d[0], Pb if swap else Pa)
+        ctx.upload(d[1], Pa if swap else Pb)
+        assert hip.hipGraphLaunch(run, stream) == 0
+        _lib.check(_lib.lib().xc_last_energy(ctx.handle, C.byref(E)))
+        F = [np.zeros((n, n), order="F") for _ in range(2)]
+        for f, p in zip(F, d[2:]):
+            ctx.download(f, p)
+        ref = pot.getMatrixUnrestricted(*((Pb, Pa) if swap else (Pa, Pb)))
+        for f, r in zip(F, ref):
+            assert np.abs(f - r).max() < 1e-12 * max(1.0, np.abs(r).max())
+        assert abs(E.value - pot.getEnergy()) < 1e-12 * abs(E.value)
+    hip.hipGraphExecDestroy(run)
+    hip.hipGraphDestroy(graph)
+    for p in d:
+        ctx.free(p)
+    bf._release()
