@@ -301,7 +301,8 @@ struct xc_ctx {
   // again and again, and hipMalloc / hipFree of their multi-GB buffers cost milliseconds each and
   // now and then stall.  Blocks are sized in 2 MiB steps (256 bytes below 1 MiB); an allocation
   // takes the smallest cached block that fits within 1/8 + 2 MiB of its size, else a new one.
-  // The cache is given back to the device when a hipMalloc fails and when the context ends.
+  // The cache is given back to the device when a hipMalloc fails and when the context ends; where
+  // that is not enough, so are the controllers' spare scratches.
   // `bytes` counts the blocks in use.
   std::multimap<size_t, void*> cache;            // block size -> released block
   std::unordered_map<void*, size_t> block_size;  // every block of this context -> size
@@ -319,7 +320,12 @@ struct xc_ctx {
     cache.clear();
     cached = 0;
   }
-  void* alloc(size_t bytes_) {
+  // Controllers whose second spin scratch no recorded graph holds: reclaim releases it (the controller
+  // then runs one spin after the other), so that it never keeps memory from what has to have it.
+  std::vector<xc_bfogc*> spare;
+  void reclaim();
+  // spare_too: false for what the caller can do without
+  void* alloc(size_t bytes_, bool spare_too = true) {
     if (bytes_ == 0) return nullptr;
     HIPX(hipSetDevice(device));
     const size_t need = block_round(bytes_);
@@ -336,6 +342,12 @@ struct xc_ctx {
     hipError_t e = hipMalloc(&p, need);
     if (e == hipErrorOutOfMemory && cached) {
       (void)hipGetLastError();
+      trim();
+      e = hipMalloc(&p, need);
+    }
+    if (e == hipErrorOutOfMemory && spare_too && !spare.empty()) {
+      (void)hipGetLastError();
+      reclaim();
       trim();
       e = hipMalloc(&p, need);
     }
@@ -371,11 +383,11 @@ struct DBuf {
   T* p = nullptr;
   size_t n = 0;
   xc_ctx* ctx = nullptr;
-  void alloc(xc_ctx* c, size_t count) {
+  void alloc(xc_ctx* c, size_t count, bool spare_too = true) {
     free_();
     ctx = c;
     n = count;
-    p = (T*)c->alloc(count * sizeof(T));
+    p = (T*)c->alloc(count * sizeof(T), spare_too);
   }
   void upload(xc_ctx* c, const T* host, size_t count) {
     alloc(c, count);
@@ -617,8 +629,28 @@ struct xc_bfogc {
   std::map<std::pair<int, double>, hipGraphExec_t> graphs;  // (functional + 16 precision, threshold)
   ~xc_bfogc() {
     for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second);
+    keep_pair();
+  }
+  // no longer among the context's spare scratches
+  void keep_pair() {
+    if (!ctx) return;
+    auto& v = ctx->spare;
+    v.erase(std::remove(v.begin(), v.end(), this), v.end());
+  }
+  void drop_pair() {
+    d_part_b.free_();
+    d_T_b.free_();
+    d_U_b.free_();
   }
 };
+
+void xc_ctx::reclaim() {
+  for (xc_bfogc* bf : spare) {
+    bf->drop_pair();
+    bf->pair = xc_bfogc::kPairNo;
+  }
+  spare.clear();
+}
 
 namespace {
 
@@ -740,35 +772,38 @@ void run_fock_finish(xc_bfogc* bf, const Lanes& L, double* dF, const double* P, 
 }
 
 // Whether an unrestricted build runs both spins in each launch.  A spin's density and Fock kernels leave a
-// tail of idle compute units and read the same tiles: (H2O)5/def2-TZVP (215 AOs, 31 700
+// tail of idle compute units and read the same tiles: (H2O)5/def2-TZVP (215 AOs, 63 392
 // points) 600 us one after the other, 482 at once (densities 197 -> 166, Fock stages 200 -> 160).
 // For matrices that take the direct reduce and 128-point blocks; it needs a second scratch of each kind,
-// and a controller that has no room for it keeps one spin after the other.
+// and a controller that has no room for it, or had to give it back, keeps one spin after the other.
 bool pair_buffers(xc_bfogc* bf) {
-  if (bf->pair == xc_bfogc::kPairUnknown) {
-    // a build that is recorded into a graph allocates nothing: one spin after the other, decided later
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    HIPX(hipStreamIsCapturing(bf->ctx->stream, &st));
-    if (st != hipStreamCaptureStatusNone) return false;
-    const size_t n = (size_t)bf->basis->nao;
-    auto found = xc_bfogc::kPairNo;
-    if (n <= kDirectRows && bf->bs == kTile) {
-      try {
-        bf->d_part_b.alloc(bf->ctx, bf->d_part.n);
-        bf->d_T_b.alloc(bf->ctx, bf->d_T.n);
-        bf->d_U_b.alloc(bf->ctx, n * n);
-        bf->d_pair.alloc(bf->ctx, 2);
-        found = xc_bfogc::kPairYes;
-      } catch (const XcError& e) {
-        bf->d_part_b.free_();
-        bf->d_T_b.free_();
-        bf->d_U_b.free_();
-        if (e.code != XC_ERR_MEMORY) throw;
-      }
-    }
-    bf->pair = found;
+  if (bf->pair == xc_bfogc::kPairNo) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  HIPX(hipStreamIsCapturing(bf->ctx->stream, &st));
+  if (st != hipStreamCaptureStatusNone) {
+    // a build that is recorded into a graph allocates nothing: undecided, it runs one spin after the
+    // other; the scratch that a graph holds stays for the controller's life
+    if (bf->pair == xc_bfogc::kPairYes) bf->keep_pair();
+    return bf->pair == xc_bfogc::kPairYes;
   }
-  return bf->pair == xc_bfogc::kPairYes;
+  if (bf->pair == xc_bfogc::kPairYes) return true;
+  const size_t n = (size_t)bf->basis->nao;
+  auto found = xc_bfogc::kPairNo;
+  if (n <= kDirectRows && bf->bs == kTile) {
+    try {
+      bf->d_part_b.alloc(bf->ctx, bf->d_part.n, false);
+      bf->d_T_b.alloc(bf->ctx, bf->d_T.n, false);
+      bf->d_U_b.alloc(bf->ctx, n * n, false);
+      bf->d_pair.alloc(bf->ctx, 2, false);
+      bf->ctx->spare.push_back(bf);
+      found = xc_bfogc::kPairYes;
+    } catch (const XcError& e) {
+      bf->drop_pair();
+      if (e.code != XC_ERR_MEMORY) throw;
+    }
+  }
+  bf->pair = found;
+  return found == xc_bfogc::kPairYes;
 }
 
 // Both spins of an unrestricted build in each launch.
@@ -1377,13 +1412,20 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       bf->tile_elems = tile_off;
       require(idx_off < (1LL << 31), XC_ERR_ARG, "xc_bfogc_create: too many AOs over the blocks");
       const int nao = basis->nao;
-      // 3. admission by footprint (the context's cached blocks count as free)
+      // 3. admission by footprint (the context's cached blocks count as free; where it does not fit, so
+      // do the spare scratches and the positions, given back before the tiles are allocated)
       size_t free_b = 0, total_b = 0;
       HIPX(hipMemGetInfo(&free_b, &total_b));
       free_b += ctx->cached;
       const double need =
           (double)tile_off * ((keep_fp32 != 2 ? sizeof(double) : 0) + (keep_fp32 ? sizeof(float) : 0)) +
           (double)bf->t_elems * (keep_fp32 != 2 ? sizeof(double) : sizeof(float));
+      const bool tight = !(need < 0.9 * (double)free_b);
+      if (tight) {
+        ctx->reclaim();
+        HIPX(hipMemGetInfo(&free_b, &total_b));
+        free_b += ctx->cached + sizeof(int) * d_pos.n;
+      }
       require(need < 0.9 * (double)free_b, XC_ERR_MEMORY,
               "xc_bfogc_create: AO tiles and Fock scratch need " + std::to_string(need / 1e9) + " GB, " +
                   std::to_string(free_b / 1e9) + " GB free");
@@ -1398,6 +1440,10 @@ int xc_bfogc_create(xc_basis* basis, xc_grid* grid, int max_block_size, double r
       d_rowcnt.alloc(ctx, (size_t)row_chunks(nb) * ns);
       launch_block_lists(ctx->stream, bf->d_blocks.p, nb, basis->d_shells.p, ns, nao, d_pos.p, bf->d_sig_shell.p,
                          bf->d_sig_pos.p, bf->d_ao_idx.p, d_rowcnt.p, bf->d_rowptr.p, bf->d_rowent.p);
+      if (tight) {
+        d_pos.free_();
+        d_rowcnt.free_();
+      }
       bf->d_dens_work.upload(ctx, bf->dens_work.data(), bf->dens_work.size());
       if (keep_fp32 == 1) {  // both tile sets: the mixed-precision build is available
         bf->d_dens_by_block.upload(ctx, bf->dens_by_block.data(), bf->dens_by_block.size());

@@ -103,3 +103,58 @@ def test_first_unrestricted_device_build_recorded(ctx, functional, precision):
     for p in d:
         ctx.free(p)
     bf._release()
+
+
+@pytest.mark.parametrize("recorded", [False, True])
+def test_second_spin_scratch_is_given_back(recorded):
+    """An allocation beyond the device (refused) takes back the scratch with which a controller runs both
+    spins at once; the builds after it run one spin after the other and give the same matrices.  A
+    controller whose build is recorded in a graph keeps its scratch, and the graph its result."""
+    hip = C.CDLL("libamdhip64.so")
+    c = xc.Context(0)
+    Z, X = W.water_chain(3)
+    b = xc.BasisController.from_file("DEF2-SVP", Z, X)
+    g = xc.molecular_grid(Z, X, accuracy=3)
+    n, P = b.nao, W.synthetic_density(b.overlap(), W.n_electrons(Z) // 2)
+    Pa, Pb = np.asfortranarray(0.6 * P), np.asfortranarray(0.4 * P)
+    bf = xc.BasisFunctionOnGridController(c, b, g, 128, 1e-9, 1)
+    pot = xc.FuncPotential(bf, "PBE", "FP64")
+    xc.NAddFuncPotential(bf, [], "PBE", "FP64").getMatrixUnrestricted(Pa, Pb, [], [])  # the spin buffers
+    d = [c.alloc(8 * n * n) for _ in range(4)]
+    c.upload(d[0], Pa)
+    c.upload(d[1], Pb)
+    before = c.memory_in_use()
+    ref = pot.getMatrixUnrestricted(Pa, Pb)
+    E = pot.getEnergy()
+    both = c.memory_in_use()
+    assert both > before
+    stream, graph, run = C.c_void_p(c.stream), C.c_void_p(), C.c_void_p()
+    if recorded:
+        c.synchronize()
+        assert hip.hipStreamBeginCapture(stream, 1) == 0
+        rc = _lib.lib().xc_fock_build_unrestricted_device(bf.handle, 1, 0, 1e-11, *d, None)
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and rc == 0
+        assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    with pytest.raises(xc.XCError):
+        c.alloc(1 << 46)
+    kept = c.memory_in_use()
+    assert kept == both if recorded else before <= kept < both
+    for _ in range(2):
+        F = pot.getMatrixUnrestricted(Pa, Pb)
+        assert c.memory_in_use() == kept
+        for f, r in zip(F, ref):
+            assert np.abs(f - r).max() < 1e-12 * max(1.0, np.abs(r).max())
+        assert abs(pot.getEnergy() - E) < 1e-12 * abs(E)
+        if recorded:
+            assert hip.hipGraphLaunch(run, stream) == 0
+            c.synchronize()
+            for p, r in zip(d[2:], ref):
+                f = np.zeros((n, n), order="F")
+                c.download(f, p)
+                assert np.abs(f - r).max() < 1e-12 * max(1.0, np.abs(r).max())
+    if recorded:
+        hip.hipGraphExecDestroy(run)
+        hip.hipGraphDestroy(graph)
+    for p in d:
+        c.free(p)
+    c.close()
