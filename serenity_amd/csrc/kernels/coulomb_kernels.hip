@@ -11,7 +11,8 @@
 // iteration:
 //   1. D_q = K_q sum_ij Pc_ij E^ij         (Hermite density of each primitive pair)
 //   2. b_k = sum_q (D_q | aux k)           (fitting right-hand side, Cartesian aux)
-//   3. (host) M c = b                      (metric solve)
+//   3. M c = b                             (two triangular solves with M's factor; the host's where it
+//                                           is not resident)
 //   4. V_q = sum_k c_k (Lambda_q | aux k)  (Hermite potential of each pair)
 //   5. J_ab = K_q sum_tuv V_q,tuv E^ab_tuv (then the shells' angular transforms).
 #include <hip/hip_runtime.h>
@@ -347,9 +348,13 @@ __global__ __launch_bounds__(64) void jpair_kernel(const JPairItem* __restrict__
 // and no lane meets another before an item's end.  The classes are bundled in three kernels by L + l
 // (<= 3, <= 6, above), because a kernel holds the registers of its widest class (128, 256, 512 and
 // spills: the last hold 0.4 % of the meetings).  At (H2O)32/def2-TZVP (160 297 pairs x 1280
-// auxiliary primitives) step 2 takes 1.5 ms and step 4 1.2 ms, about 20 TFLOP/s (FP64 vector peak
-// 78); with run-time angular momenta, whose arrays live in private memory, and one thread per pair
-// they took 50 and 263 ms.
+// auxiliary primitives) step 2 takes 1.5 ms and step 4 1.2 ms, the three kernels side by side: 73 GFLOP
+// at 27 TFLOP/s (FP64 vector peak 78).  Alone the kernels run at 22 to 29 TFLOP/s with the vector units
+// busy 40 to 72 % of the time (the widest 11 and 21, 17 and 24 %): a tenth (L + l of 4 to 6) to a
+// fifth (<= 3) of their vector instructions are not FP64, a third to two fifths of the FP64 ones are
+// single multiplies or additions, and a wavefront waits 26 to 47 % of its time, the narrow classes
+// with one vector load in 15 instructions, the rows of the Boys table.  With run-time angular
+// momenta, whose arrays live in private memory, and one thread per pair steps 2 and 4 took 50 and 263 ms.
 
 // acc[j] += sum over i >= I of c[i] R(index i + index j), i < NI, j < NJ (recursion over i: one loop
 // over both would be too long to unroll for the widest classes).

@@ -157,7 +157,7 @@ SXC_HD Dual<N> datan(Dual<N> a) {
 
 // A density (or 1 +- zeta) and the cube root of its value, from which every fractional power of the
 // functionals is a product: FP64 pow takes some 250 instructions, and PBE asked for four of them (the
-// functional stage of PBE at 237 000 points 22 us, of the spin-polarised PBE at 31 700 points 27; 14 and 12 so).
+// functional stage of PBE at 237 000 points 22 us, of the spin-polarised PBE at 63 392 points 27; 14 and 12 so).
 template <class D>
 struct Rooted {
   D n;

@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256) void partition_gen_kernel(int type, unsigned s
 // cells are multiplied and summed in atom order), so the weight is the same bit for bit; dist is
 // symmetric to the bit, and its columns are read along the lanes.  One thread
 // per candidate walked n^2 / 2 dependent steps whose branches the 64 candidates of a wavefront take
-// together (a shell of points around an atom reaches most cells): 725 us for the 174 336 candidates of
-// (H2O)12, 400 us with groups.
+// together (a shell of points around an atom reaches most cells): 696 us for the 174 336 candidates of
+// (H2O)12, 411 us with groups.
 template <int G>
 __global__ __launch_bounds__(256) void ssf_gen_kernel(int n, const double* __restrict__ xyz,
                                                       const double* __restrict__ dist,

@@ -275,14 +275,15 @@ struct EnvEnergies {
 // of dependent load-add steps, and more wavefronts make shorter chains (with whole wavefronts per
 // entry 0.68 ms at (H2O)64/def2-TZVP against 0.86 ms with 8 and 1.40 ms with 4).  wide: blocks hold
 // more than 256 AOs on average, so that a row segment (half of them on average) fills the 128
-// columns that 32 lanes take at once; else 16 lanes take an entry.
+// columns that 32 lanes take at once; else 16 lanes take an entry (both sides: fock_reduce_kernel).
 // With out.direct the rows go to both triangles of F instead (no finalize), each row leaves its part of
 // the FP32 rounding term sum F (P - P32) in round[row] where P32 is given (packed: where round is
 // not null), and one more workgroup sums the block energies into E, less the energies of env (a
 // rounding sum, where there is one, is launch_sum's).  For matrices of up to kDirectRows rows: the
 // upper triangle's writes go one element per line (n^2 / 2 of them), which costs less than the
-// finalize's launch only while they are few ((H2O)8/def2-SVP, 192 rows: reduce, finalize and sum 30
-// us, together 19 us).
+// finalize's launch only while they are few.  Whole builds of def2-SVP waters, PBE, direct / not, in us:
+// FP32 192 rows 210 / 216, 384 rows 465 / 468, 480 rows 606 / 606, 648 rows 963 / 959; FP64, where the
+// energy's launch goes too, 293 / 304, 682 / 692, 894 / 906 and 1452 / 1463.
 struct ReduceOut {
   bool direct;
   double* F;

@@ -10,8 +10,9 @@
 //   fock        S_b = phi_b^T G_b + G_b^T phi_b on matrix cores, the upper-triangle sub-tiles
 //               of every block stored to a scratch (ScalarOperatorToMatrixAdder.cpp:179-303)
 //   fock_reduce F = sum over blocks of S_b scattered by the blocks' AO lists, one AO row per
-//               workgroup summing its blocks in a fixed order (the reference's thread-private
-//               F plus serial sum, ScalarOperatorToMatrixAdder.cpp:101-110)
+//               workgroup adding its blocks' terms in LDS, in an order that varies unless the
+//               context is deterministic (the reference's thread-private F plus serial sum,
+//               ScalarOperatorToMatrixAdder.cpp:101-110)
 #include <hip/hip_runtime.h>
 
 #include <stdexcept>
@@ -308,19 +309,6 @@ __device__ inline void quad_rows(const gmem<const float>* seg, int lane, double 
   f[3] = v.w;
 }
 
-// Density contraction on 16 x 16 sub-tiles.  One workgroup of 8 wavefronts
-// per (block, column pass): T[p][nu] = sum_mu phi[mu][p] P[mu][nu] for the
-// pass's 16 S columns, wavefront w owning points 16 w .. 16 w + 15 and all S
-// column tiles (S independent accumulators).  The AO (K) dimension streams in
-// chunks of KC (32 FP32 / 16 FP64) through an LDS buffer that holds phi
-// point-major and the pass's P columns, both with the AO index fastest: with
-// k-step t of lane group g taking AO KV g + t (KV = KC / 4) every MFMA operand
-// of a chunk is one 32-byte LDS read.  The global loads of chunk k + 1 are
-// issued before the MFMAs of chunk k.  The pass's partial rho and
-// sum_nu T grad phi are then formed from the accumulators in registers, each
-// lane dotting its T entries with the phi / grad phi values of the same
-// (point, column), and summed over the columns by lane shuffles.  (FP64
-// accumulates T transposed, so that its lanes read whole 128-byte point runs.)
 // Work item and spin of workgroup x of a launch of pairs items for two spins (0: one pass, item x):
 // eight items of one spin, then the same eight of the other, so that an item's two passes run on one
 // XCD shortly after each other and the second finds the tiles in its L2.
@@ -340,6 +328,19 @@ struct DensityArgs {
   int64_t npts;
 };
 
+// Density contraction on 16 x 16 sub-tiles.  One workgroup of 8 wavefronts
+// per (block, column pass): T[p][nu] = sum_mu phi[mu][p] P[mu][nu] for the
+// pass's 16 S columns, wavefront w owning points 16 w .. 16 w + 15 and all S
+// column tiles (S independent accumulators).  The AO (K) dimension streams in
+// chunks of KC (32 FP32 / 16 FP64) through an LDS buffer that holds phi
+// point-major and the pass's P columns, both with the AO index fastest: with
+// k-step t of lane group g taking AO KV g + t (KV = KC / 4) every MFMA operand
+// of a chunk is one 32-byte LDS read.  The global loads of chunk k + 1 are
+// issued before the MFMAs of chunk k.  The pass's partial rho and
+// sum_nu T grad phi are then formed from the accumulators in registers, each
+// lane dotting its T entries with the phi / grad phi values of the same
+// (point, column), and summed over the columns by lane shuffles.  (FP64
+// accumulates T transposed, so that its lanes read whole 128-byte point runs.)
 template <typename T, int S, bool Tri>
 __device__ __forceinline__ void density_item(const WorkItem& wk, const DevBlock& bk, const DensityArgs<T>& arg,
                                              unsigned char* smem, int* sIdx) {
@@ -763,8 +764,8 @@ __device__ double sum_256(const double* x, int64_t n, const double* x2, int64_t 
 // w g) and its energy, rho_sup summed from the listed densities on the way (in list order, the active
 // one first); of y > 0: a block of the energy of pend.dens.rho[y - 1] alone, into pend.eblk[y - 1]
 // (y = blockIdx.y, one more without the first).  What were a pass over all densities, a launch per
-// functional and one per energy sum took 36 us and as much between them ((H2O)12 in def2-SVP, 103 000
-// points, Thomas-Fermi); this launch and nadd_energy_kernel 19 us.
+// functional and one per energy sum took 36 us and as much between them (benzene and 12 waters in
+// def2-SVP, 205 486 points, Thomas-Fermi); this launch and nadd_energy_kernel 19 us.
 struct PendingEnergies {
   DensityList dens;
   double* eblk[kListMax];
@@ -784,7 +785,7 @@ __global__ __launch_bounds__(128) void nadd_functional_kernel(int func, int64_t 
   if (in) {
     if (y == 0) {
       // four densities' loads at a time (one after another they are a chain of memory latencies:
-      // 27 us for PBE over 13 densities with gradients at 103 000 points, 7 more one after another)
+      // 27 us for PBE over 13 densities with gradients at 205 486 points, 7 more one after another)
       constexpr int U = 4;
       for (int i0 = 0; i0 < sup.n; i0 += U) {
         double x[U][4];
@@ -1258,8 +1259,12 @@ __global__ __launch_bounds__(64 * W) void fock_sub_kernel(const FockItem* __rest
 // that chain, so short chains (many groups) count: segments hold n_b / 2 columns on average (12 to
 // 170), which left most of a wavefront's 64 lanes idle when a whole wavefront took an entry.  Groups
 // of 16 against whole wavefronts: (H2O)8/def2-SVP 40 -> 21 us, C20H42/def2-SVP 90 -> 76 us (FP64);
-// groups of 32 for blocks of more than 256 AOs: (H2O)64/def2-TZVP 683 -> 599 us in FP32 (631 with
-// 16), where the 2.8 GB of values and AO lists now come at 4.7 TB/s (a device copy: 5.0).
+// groups of 32 for blocks of more than 256 AOs on average.  Wavefronts / 32 / 16 lanes in us, FP64 and
+// FP32: (H2O)64/def2-TZVP (n_b 337) 1007 / 935 / 992 and 792 / 678 / 703, (H2O)32/def2-TZVP (276)
+// 375 / 325 / 337 and 307 / 244 / 241, (H2O)64/def2-SVP (210) 663 / 534 / 529 and 572 / 427 / 392;
+// the best order per precision crosses at an n_b of about 200 in FP64 and 300 in FP32.  (The kernel of
+// whole wavefronts that broadcast their entries from the lanes took 923 and 681 at (H2O)64, 355 and
+// 280 at (H2O)32.)
 // Rows longer than the LDS window are done in several passes over the entries.
 // Fixed = false: FP64 additions in LDS, which the wavefronts make in an order that varies from run
 // to run, so F varies at the rounding level.  Fixed = true: each term x is split into integers,

@@ -3109,8 +3109,7 @@ int xc_server_submit(xc_server* srv, xc_bfogc* bf, int functional, int precision
       const auto key = std::make_pair(functional + 16 * precision, thr);
       auto it = bf->graphs.find(key);
       if (it == bf->graphs.end()) {
-        // capture one build on this controller's resident buffers (no memset nodes: U is
-        // cleared by a fill kernel)
+        // capture one build on this controller's resident buffers (kernel nodes only, no memsets)
         hipGraph_t graph = nullptr;
         HIPX(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
